@@ -131,7 +131,8 @@ extern "C" int fgnn_colsum_plan_create(const int32_t *row_ptr, const int32_t *co
     if (E > 0) {
         char *tmp = nullptr;
         const size_t eb = fgnn_align256((size_t)E * sizeof(int)), rb = fgnn_align256(((size_t)p->n_ranges + 1) * sizeof(int));
-        const size_t sort_b = fgnn_align256(fgnn_rs_sort_workspace(E));
+        const int key_bits = fgnn_rs_key_bits(std::max(p->n_ranges, 2));
+        const size_t sort_b = fgnn_align256(fgnn_rs_sort_workspace(E, key_bits));
         CS_HIP(hipMalloc((void **)&tmp, eb + rb + 256 + sort_b));
         CS_HIP(hipMalloc((void **)&p->tpos_dev, (size_t)E * sizeof(int32_t)));
         CS_HIP(hipMalloc((void **)&p->lcol_dev, (size_t)E * sizeof(uint16_t)));
@@ -146,7 +147,7 @@ extern "C" int fgnn_colsum_plan_create(const int32_t *row_ptr, const int32_t *co
                 rc = fgnn_launch_status("cs_key_kernel");
             }
             const int *skey = nullptr;
-            if (!rc) rc = fgnn_rs_sort_pairs(key, nullptr, E, fgnn_rs_key_bits(std::max(p->n_ranges, 2)), p->tpos_dev, &skey, sort_ws, st);
+            if (!rc) rc = fgnn_rs_sort_pairs(key, nullptr, E, key_bits, p->tpos_dev, &skey, sort_ws, st);
             if (!rc) {
                 hipLaunchKernelGGL(cs_range_ptr_kernel, dim3((unsigned)((E + 256) / 256)), dim3(256), 0, st, E, p->n_ranges, skey, rptr);
                 rc = fgnn_launch_status("cs_range_ptr_kernel");

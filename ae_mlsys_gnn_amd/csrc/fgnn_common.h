@@ -45,7 +45,7 @@ int fgnn_fill_f32(float *p, size_t n, float v, hipStream_t st);
 int fgnn_current_device_has_xcd_mapping();      // 1: workgroup w of a dispatch runs on XCD w % FGNN_NUM_XCD on the current device
 
 // Stable LSD radix sort of (key, payload) pairs and an inclusive int32 scan (fgnn_csr2csc.hip); device pointers.
-size_t fgnn_rs_sort_workspace(int64_t n);
+size_t fgnn_rs_sort_workspace(int64_t n, int key_bits);
 int fgnn_rs_key_bits(int n_keys);
 int fgnn_rs_sort_pairs(const int *keys_in, const int *pay_in, int64_t n, int key_bits, int *pay_out, const int **sorted_keys, void *workspace,
                        hipStream_t st);

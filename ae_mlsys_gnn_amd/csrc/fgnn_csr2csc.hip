@@ -1,210 +1,345 @@
 // GPU CSR -> CSC transpose (stable), replacing the reference's cuSPARSE call
-// (src/csr2csc/csr2csc.cu:10-23).
+// (src/csr2csc/csr2csc.cu:10-23), and the COO -> CSR builder.
 //
-// The transpose is a stable sort of the CSR positions by column: an LSD radix sort with digits of
-// up to 8 bits over key = col_ind[p], payload = p.  Each pass is histogram -> scan -> stable scatter:
-// a workgroup owns a contiguous tile, each of its 4 waves a contiguous quarter of it, and a wave
-// walks its quarter 64 elements at a time, ranking equal digits inside the wave with ballots, so
-// equal keys keep their order (the order of CSR positions).  After the last pass the payload IS
-// `permute`; col_ptr is read off the boundaries of the sorted keys and row_ind by a binary search
-// of each position in row_ptr.  Integer work only, bit-exact and deterministic.
+// Both are stable LSD radix sorts of small records with digits of up to 11 bits (22-bit ids: two passes of
+// 11).  Each pass is histogram -> scan -> stable scatter: a workgroup owns a contiguous tile, each of its 16
+// waves a contiguous sixteenth of it, and a wave walks its part 64 records at a time, ranking equal digits
+// inside the wave with ballots, so equal keys keep their order.  Integer work only, bit-exact and deterministic.
+//
+// What bounds a pass is the scatter: 2048 digits leave about 4 consecutive records of a tile per digit, far
+// less than a 128-byte line.  Two things keep the lines whole: the workgroups of one XCD take a contiguous
+// eighth of the tiles (the next tile of a digit's run is written through the same L2 shortly after, so 2048
+// open lines, 256 KB, complete in it), and a record's words travel together (8-byte stores).  64.3 M records of
+// 8 bytes: the scatter of a pass takes 0.34-0.39 ms (1.03 GB, 2.6-3.0 TB/s) and the pass 0.51; with 8-bit digits,
+// separate 4-byte key and payload streams and the tiles dealt round-robin it was 0.44 and 0.59 ms, and 44 bits took
+// six passes instead of four.  COO -> CSR -> CSC of that graph: 10.3 -> 4.0 ms.
+//
+// A workgroup is 1024 threads with 8 records each: at 512 threads with 16 the records, ranks and counters held 128-168
+// registers, one workgroup lived on a compute unit and the ranking chain had nothing to hide behind (0.67 ms).
 #include "fgnn_common.h"
 
-#define RS_TPB 256
-#define RS_ITEMS 16                    // elements per thread
-#define RS_TILE (RS_TPB * RS_ITEMS)    // 4096 elements per workgroup
-#define RS_SUB (64 * RS_ITEMS)         // 1024 per wave
+#define RS_TPB 1024
+#define RS_WAVES 16
+#define RS_MAX_BITS 11
+#define RS_MAX_DIGITS (1 << RS_MAX_BITS)
+#define RS_DPT (RS_MAX_DIGITS / RS_TPB)      // digits per thread in the per-tile scans
+// Records per thread: tiles of 8192 keep the per-tile digit runs long; small inputs take tiles of 2048 so that they
+// spread over the chip (1 M records: 512 workgroups instead of 128).
+#define RS_SMALL_N (4 << 20)
+static inline int rs_items(int64_t n) { return n < RS_SMALL_N ? 2 : 8; }
+static inline int rs_num_tiles(int64_t n) { const int64_t t = (int64_t)RS_TPB * rs_items(n); return (int)((n + t - 1) / t); }
+static __host__ __device__ inline int rs_hist_ld(int ntiles) { return (ntiles + 7) & ~7; }     // ints per digit of the count array
+static inline unsigned rs_grid(int ntiles) { return (unsigned)(((ntiles + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD) * FGNN_NUM_XCD); }
+// Workgroup b -> tile: the workgroups of an XCD (b % 8) own a contiguous range of tiles.  May be >= ntiles: no work.
+__device__ __forceinline__ int rs_tile_of(int b, int ntiles) { return (b % FGNN_NUM_XCD) * ((ntiles + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD) + b / FGNN_NUM_XCD; }
 
-__global__ __launch_bounds__(RS_TPB) void rs_hist_kernel(const int *__restrict__ keys, int64_t n, int shift, int mask, int nblocks, int *__restrict__ hist)
+// hist[d * rs_hist_ld(ntiles) + t] = records of tile t whose digit is d.  keys: every `stride`-th int.
+template <int ITEMS>
+__global__ __launch_bounds__(RS_TPB) void rs_hist_kernel(const int *__restrict__ keys, int stride, int64_t n, int shift, int mask, int ntiles, int *__restrict__ hist)
 {
-    __shared__ int cnt[4][256];         // one set of counters per wave: a quarter of the collisions
-    for (int i = (int)threadIdx.x; i < 4 * 256; i += RS_TPB) (&cnt[0][0])[i] = 0;
+    __shared__ int cnt[2][RS_MAX_DIGITS];        // two sets of counters: half the collisions
+    const int tile = rs_tile_of((int)blockIdx.x, ntiles);
+    if (tile >= ntiles) return;
+    for (int d = (int)threadIdx.x; d <= mask; d += RS_TPB) { cnt[0][d] = 0; cnt[1][d] = 0; }
     __syncthreads();
-    const int wave = fg_wave(), lane = fg_lane();
-#pragma unroll 4
-    for (int it = 0; it < RS_ITEMS; ++it) {
-        int64_t i = (int64_t)blockIdx.x * RS_TILE + wave * RS_SUB + it * 64 + lane;
-        if (i < n) atomicAdd(&cnt[wave][(keys[i] >> shift) & mask], 1);
+    const int64_t base = (int64_t)tile * (RS_TPB * ITEMS) + threadIdx.x;
+    const int set = (int)threadIdx.x & 1;
+    int key[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const int64_t i = base + it * RS_TPB;
+        key[it] = i < n ? keys[i * stride] : 0;
     }
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+        if (base + it * RS_TPB < n) atomicAdd(&cnt[set][(key[it] >> shift) & mask], 1);
     __syncthreads();
-    if ((int)threadIdx.x <= mask)
-        hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = (cnt[0][threadIdx.x] + cnt[1][threadIdx.x]) + (cnt[2][threadIdx.x] + cnt[3][threadIdx.x]);
+    for (int d = (int)threadIdx.x; d <= mask; d += RS_TPB) hist[(size_t)d * rs_hist_ld(ntiles) + tile] = cnt[0][d] + cnt[1][d];
 }
 
-// One workgroup per digit: exclusive scan of that digit's per-block counts in place.  The row is walked
-// in chunks of RS_TPB * 8 counts: every thread scans 8 consecutive counts serially, the 256 thread totals
+// Inclusive sum over the lanes of a wave.
+__device__ __forceinline__ int rs_wave_incl(int v, int lane)
+{
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        int t = __shfl_up(v, off);
+        if (lane >= off) v += t;
+    }
+    return v;
+}
+
+// One workgroup per digit: exclusive scan of that digit's per-tile counts in place.  The row is walked
+// in chunks of 256 * 8 counts: every thread scans 8 consecutive counts serially, the 256 thread totals
 // are scanned with wave shuffles and one exchange through LDS, and the chunk's total carries over.
-__global__ __launch_bounds__(RS_TPB) void rs_scan_kernel(int *__restrict__ hist, int nblocks, int *__restrict__ digit_total)
+#define RS_SCAN_TPB 256
+__global__ __launch_bounds__(RS_SCAN_TPB) void rs_scan_kernel(int *__restrict__ hist, int ntiles, int *__restrict__ digit_total)
 {
     constexpr int PER = 8;
-    __shared__ int wave_tot[4];
-    int *row = hist + (size_t)blockIdx.x * nblocks;
+    __shared__ int wave_tot[RS_SCAN_TPB / 64];
+    int *row = hist + (size_t)blockIdx.x * rs_hist_ld(ntiles);
     const int lane = fg_lane(), wave = fg_wave();
     int carry = 0;
-    for (int base = 0; base < nblocks; base += RS_TPB * PER) {
-        const int i0 = base + (int)threadIdx.x * PER;
-        int v[PER], tot = 0;
-#pragma unroll
-        for (int j = 0; j < PER; ++j) { v[j] = i0 + j < nblocks ? row[i0 + j] : 0; tot += v[j]; }
-        int incl = tot;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
+    for (int base = 0; base < ntiles; base += RS_SCAN_TPB * PER) {
+        const int i0 = base + (int)threadIdx.x * PER;           // rows are padded to PER counts, whatever the padding holds
+        int v[PER] = {0, 0, 0, 0, 0, 0, 0, 0}, tot = 0;
+        if (i0 < ntiles) {
+            *reinterpret_cast<int4 *>(v) = *reinterpret_cast<const int4 *>(row + i0);
+            *reinterpret_cast<int4 *>(v + 4) = *reinterpret_cast<const int4 *>(row + i0 + 4);
         }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) { if (i0 + j >= ntiles) v[j] = 0; tot += v[j]; }
+        const int incl = rs_wave_incl(tot, lane);
         __syncthreads();                        // the previous chunk's wave totals have been read
         if (lane == 63) wave_tot[wave] = incl;
         __syncthreads();
         int run = carry + incl - tot;
         for (int w = 0; w < wave; ++w) run += wave_tot[w];
 #pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            if (i0 + j < nblocks) row[i0 + j] = run;
-            run += v[j];
+        for (int j = 0; j < PER; ++j) { const int t = v[j]; v[j] = run; run += t; }
+        if (i0 < ntiles) {
+            *reinterpret_cast<int4 *>(row + i0) = *reinterpret_cast<const int4 *>(v);
+            *reinterpret_cast<int4 *>(row + i0 + 4) = *reinterpret_cast<const int4 *>(v + 4);
         }
         carry += wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
     }
     if (threadIdx.x == 0) digit_total[blockIdx.x] = carry;
 }
 
-__global__ __launch_bounds__(256) void rs_digit_base_kernel(const int *__restrict__ digit_total, int n_digits, int *__restrict__ digit_base)
-{
-    __shared__ int sh[256];
-    int v = (int)threadIdx.x < n_digits ? digit_total[threadIdx.x] : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        int t = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
-        sh[threadIdx.x] += t;
-        __syncthreads();
-    }
-    digit_base[threadIdx.x] = sh[threadIdx.x] - v;
-}
+// Where the records of a pass come from.
+//   RS_PAIR:     rec[i] = {x, y}; the key is x, or y with KEY_Y
+//   RS_ARRAYS:   {a[i], b[i]} (b == NULL: {a[i], i}), likewise
+//   RS_TRIPLE:   key[i] and rec[i]
+//   RS_TRIPLE_SWAP: as RS_TRIPLE with key and rec.x exchanged (from here on the other id is sorted)
+//   RS_EDGES:    key b[i], rec {a[i], i} (b: source, a: destination of input edge i)
+//   RS_CSR:      key a[i], rec {i, row of position i}
+enum rs_in { RS_PAIR, RS_ARRAYS, RS_TRIPLE, RS_TRIPLE_SWAP, RS_EDGES, RS_CSR };
+// Where they go: RS_TO_PAIR rec_out[q]; RS_TO_ARRAYS {a_out[q], b_out[q]}; RS_TO_TRIPLE key_out[q], rec_out[q];
+// RS_TO_ARRAYS3 key_out[q], {a_out[q], b_out[q]}.
+enum rs_out { RS_TO_PAIR, RS_TO_ARRAYS, RS_TO_TRIPLE, RS_TO_ARRAYS3 };
+struct rs_args {
+    const int *a, *b;               // separate input arrays
+    const int *key; const int2 *rec;
+    int *a_out, *b_out, *key_out; int2 *rec_out;
+    const int *row_ptr, *hint;      // RS_CSR
+    int n_rows, n_hint;
+};
 
-// Stable scatter of one pass.  pay_in == NULL: the payload is the element's own index (first pass).
-// The tile is first sorted by digit inside LDS (local position = the digit's base inside the tile +
-// rank among the tile's earlier elements of that digit), then written out in local order: all
-// elements of a digit leave as one contiguous run, so neighbouring lanes write neighbouring addresses
-// instead of 4-byte stores scattered over 256 destinations.
-__global__ __launch_bounds__(RS_TPB) void rs_scatter_kernel(const int *__restrict__ keys_in, const int *__restrict__ pay_in, int64_t n, int shift,
-                                                            int bits, int nblocks, const int *__restrict__ hist, const int *__restrict__ digit_base,
-                                                            int *__restrict__ keys_out, int *__restrict__ pay_out)
-{
-    __shared__ int wcnt[4][256];        // per wave and digit: count, then the running local position
-    __shared__ int gofs[256];           // per digit: global position of the tile's run minus its local base
-    __shared__ int wave_tot[4];
-    __shared__ int skey[RS_TILE], spay[RS_TILE];
-    const int wave = fg_wave(), lane = fg_lane();
-    const int mask = (1 << bits) - 1;
-    for (int i = (int)threadIdx.x; i < 4 * 256; i += RS_TPB) (&wcnt[0][0])[i] = 0;
-    __syncthreads();
-    const int64_t tile0 = (int64_t)blockIdx.x * RS_TILE;
-    int key[RS_ITEMS], pay[RS_ITEMS];
-#pragma unroll
-    for (int it = 0; it < RS_ITEMS; ++it) {
-        int64_t i = tile0 + wave * RS_SUB + it * 64 + lane;
-        key[it] = i < n ? keys_in[i] : 0;
-        pay[it] = (pay_in && i < n) ? pay_in[i] : (int)i;      // fetched up front: the ranking loop below is a dependent chain
-        if (i < n) atomicAdd(&wcnt[wave][(key[it] >> shift) & mask], 1);
-    }
-    __syncthreads();
-    {
-        // thread d owns digit d: exclusive scan of the tile's digit counts (inside the wave by shuffles,
-        // across the four waves through LDS), then the per-wave starting positions
-        const int d = (int)threadIdx.x;
-        int c[4], tot = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) { c[w] = wcnt[w][d]; tot += c[w]; }
-        int incl = tot;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-        }
-        if (lane == 63) wave_tot[wave] = incl;
-        __syncthreads();
-        int lbase = incl - tot;
-        for (int w = 0; w < wave; ++w) lbase += wave_tot[w];
-        gofs[d] = d <= mask ? digit_base[d] + hist[(size_t)d * nblocks + blockIdx.x] - lbase : 0;
-        int run = lbase;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) { wcnt[w][d] = run; run += c[w]; }
-    }
-    __syncthreads();
-    const unsigned long long lt = (1ull << lane) - 1ull;
-#pragma unroll
-    for (int it = 0; it < RS_ITEMS; ++it) {
-        int64_t i = tile0 + wave * RS_SUB + it * 64 + lane;
-        bool ok = i < n;
-        int d = (key[it] >> shift) & mask;
-        unsigned long long peers = __builtin_amdgcn_ballot_w64(ok);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            if (bit < bits) {
-                unsigned long long bal = __builtin_amdgcn_ballot_w64(((d >> bit) & 1) != 0);
-                peers &= ((d >> bit) & 1) ? bal : ~bal;
-            }
-        }
-        int rank = __popcll(peers & lt);
-        int base = wcnt[wave][d];
-        if (ok) {
-            skey[base + rank] = key[it];
-            spay[base + rank] = pay[it];
-        }
-        fg_wave_lds_sync();
-        // the highest lane of every peer group advances the wave's counter of that digit
-        if (ok && (peers >> lane) == 1ull) wcnt[wave][d] = base + __popcll(peers);
-        fg_wave_lds_sync();
-    }
-    __syncthreads();
-    const int count = (int)((n - tile0) < (int64_t)RS_TILE ? (n - tile0) : (int64_t)RS_TILE);
-#pragma unroll 4
-    for (int i = (int)threadIdx.x; i < count; i += RS_TPB) {
-        int k = skey[i];
-        int dst = gofs[(k >> shift) & mask] + i;
-        keys_out[dst] = k;
-        pay_out[dst] = spay[i];
-    }
-}
-
-// Row of CSR position p: the last r with row_ptr[r] <= p, searched in [lo, hi) with row_ptr[lo] <= p < row_ptr[hi].
-__device__ __forceinline__ int csc_row_of(const int *__restrict__ row_ptr, int lo, int hi, int p)
-{
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (row_ptr[mid] <= p) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
-// hint[k] = row of position min(k << CSC_HINT_SHIFT, n - 1), k = 0 .. n_hint - 1: a coarse inverse of
-// row_ptr, so that the per-entry search of csc_finalize_kernel covers the few rows of one bucket of
-// positions instead of the whole pointer array.
-#define CSC_HINT_SHIFT 9
+// hint[k] = row of position min(k << CSC_HINT_SHIFT, n - 1): a coarse inverse of row_ptr.  128 = the records a wave of a small
+// tile owns, so that every wave of RS_CSR finds the row of its first record there.
+#define CSC_HINT_SHIFT 7
+static int csc_num_hints(int64_t E) { return E > 0 ? (int)((E - 1) >> CSC_HINT_SHIFT) + 2 : 0; }
 __global__ __launch_bounds__(256) void csc_row_hint_kernel(int64_t n, int n_rows, int n_hint, const int *__restrict__ row_ptr, int *__restrict__ hint)
 {
-    int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (k >= n_hint) return;
     int64_t p = (int64_t)k << CSC_HINT_SHIFT;
     if (p > n - 1) p = n - 1;
-    hint[k] = csc_row_of(row_ptr, 0, n_rows, (int)p);
+    int lo = 0, hi = n_rows;                    // the last r with row_ptr[r] <= p
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (row_ptr[mid] <= (int)p) lo = mid; else hi = mid;
+    }
+    hint[k] = lo;
 }
 
-__global__ __launch_bounds__(256) void csc_finalize_kernel(int64_t n, int n_cols, const int *__restrict__ sorted_keys,
-                                                           const int *__restrict__ permute, const int *__restrict__ row_ptr,
-                                                           const int *__restrict__ hint, int *__restrict__ col_ptr, int *__restrict__ row_ind)
+// Stable scatter of one pass.  The tile is first sorted by digit inside LDS (local position = the digit's base inside
+// the tile + rank among the tile's earlier records of that digit), then written out in local order: the records of a
+// digit leave as one run.  The digit counters and the staged records share the same LDS (72 KB in all: two workgroups
+// of 16 waves per compute unit), and the words of a three-word record are staged one part after the other.
+template <int ITEMS, rs_in IN, rs_out OUT, bool KEY_Y>
+__global__ __launch_bounds__(RS_TPB, 8) void rs_scatter_kernel(rs_args A, int64_t n, int shift, int mask, int ntiles, const int *__restrict__ hist,
+                                                            const int *__restrict__ digit_total)
 {
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    int key = sorted_keys[q];
-    int prev = q > 0 ? sorted_keys[q - 1] : -1;
-    for (int c = prev + 1; c <= key; ++c) col_ptr[c] = (int)q;
-    if (q == n - 1)
-        for (int c = key + 1; c <= n_cols; ++c) col_ptr[c] = (int)n;
-    int p = permute[q];
-    int k = p >> CSC_HINT_SHIFT;
-    row_ind[q] = csc_row_of(row_ptr, hint[k], hint[k + 1] + 1, p);
+    constexpr int TILE = RS_TPB * ITEMS, SUB = 64 * ITEMS;
+    constexpr bool TRIPLE = OUT == RS_TO_TRIPLE || OUT == RS_TO_ARRAYS3;
+    constexpr size_t LDS = TILE * sizeof(int2) > RS_WAVES * RS_MAX_DIGITS * sizeof(uint16_t) ? TILE * sizeof(int2) : RS_WAVES * RS_MAX_DIGITS * sizeof(uint16_t);
+    __shared__ __attribute__((aligned(16))) char buf[LDS];
+    __shared__ int gofs[RS_MAX_DIGITS];          // per digit: global position of the tile's run minus its local base
+    __shared__ int wave_tot[2][RS_WAVES];
+    uint16_t (*wcnt)[RS_MAX_DIGITS] = reinterpret_cast<uint16_t (*)[RS_MAX_DIGITS]>(buf);   // per wave and digit: running count, then the local base
+    const int wave = fg_wave(), lane = fg_lane(), tid = (int)threadIdx.x;
+    const int tile = rs_tile_of((int)blockIdx.x, ntiles);
+    if (tile >= ntiles) return;
+    const int64_t tile0 = (int64_t)tile * TILE;
+    const int64_t first = tile0 + wave * SUB;    // the wave's first record
+    const int count = (int)((n - tile0) < (int64_t)TILE ? (n - tile0) : (int64_t)TILE);
+    const int mine = count - wave * SUB - lane;  // record it * 64 of the lane exists when it lies below this
+    int key[ITEMS];
+    int2 rec[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const int64_t i = tile0 + min(wave * SUB + it * 64 + lane, count - 1);     // past the end: a copy of the last record, never stored
+        int2 r = make_int2(0, 0);
+        int k = 0;
+        if constexpr (IN == RS_PAIR) r = A.rec[i];
+        else if constexpr (IN == RS_ARRAYS) { r.x = A.a[i]; r.y = A.b ? A.b[i] : (int)i; }
+        else if constexpr (IN == RS_EDGES) { k = A.b[i]; r = make_int2(A.a[i], (int)i); }
+        else if constexpr (IN == RS_CSR) { k = A.a[i]; r.x = (int)i; }
+        else { k = A.key[i]; r = A.rec[i]; }
+        if constexpr (IN == RS_TRIPLE_SWAP) { const int t = k; k = r.x; r.x = t; }
+        if constexpr (IN == RS_PAIR || IN == RS_ARRAYS) k = KEY_Y ? r.y : r.x;
+        key[it] = k;
+        rec[it] = r;
+    }
+    if constexpr (IN == RS_CSR) {
+        // row of every position of the tile: the starts of the non-empty rows leave their number in LDS (several rows that
+        // start at one position are empty but for the last, the largest number), then a running maximum over the positions
+        int *mark = reinterpret_cast<int *>(buf);
+        for (int i = tid; i < TILE; i += RS_TPB) mark[i] = 0;
+        __syncthreads();
+        const int64_t last = tile0 + TILE < n ? tile0 + TILE : n - 1;      // rows up to the one that holds the next tile's first position
+        const int r0 = A.hint[tile0 >> CSC_HINT_SHIFT], r1 = A.hint[(last + (1 << CSC_HINT_SHIFT) - 1) >> CSC_HINT_SHIFT];
+        for (int r = r0 + 1 + tid; r <= r1; r += RS_TPB) {
+            const int64_t o = (int64_t)A.row_ptr[r] - tile0;
+            if (o >= 0 && o < TILE) atomicMax(&mark[o], r);
+        }
+        __syncthreads();
+        // a lane takes ITEMS consecutive positions, the lanes of a wave the wave's SUB positions
+        int m[ITEMS];
+        int *own = mark + wave * SUB + lane * ITEMS;
+        int top = 0;
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) { m[it] = own[it]; top = max(top, m[it]); m[it] = top; }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(top, off);
+            if (lane >= off) top = max(top, t);
+        }
+        int run = __shfl_up(top, 1);
+        run = max(lane == 0 ? 0 : run, first < n ? A.hint[first >> CSC_HINT_SHIFT] : 0);
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) own[it] = max(m[it], run);
+        fg_wave_lds_sync();
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) rec[it].y = mark[wave * SUB + it * 64 + lane];
+        __syncthreads();
+    }
+    for (int d = tid; d < RS_WAVES * RS_MAX_DIGITS / 2; d += RS_TPB) reinterpret_cast<int *>(buf)[d] = 0;
+    __syncthreads();
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    int rank[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const bool ok = it * 64 < mine;
+        // opaque here: the ballots of later records stay behind this one (hoisted to the top they cost 60 registers and half the waves)
+        const int d = (int)fg_pin((uint32_t)((key[it] >> shift) & mask));
+        // lanes with the same digit: per bit a sign-extended bit field (0 or -1), its ballot, and peers &= ~(bit ^ ballot) on each half
+        const unsigned long long valid = __builtin_amdgcn_ballot_w64(ok);
+        uint32_t plo = (uint32_t)valid, phi = (uint32_t)(valid >> 32);
+#pragma unroll
+        for (int bit = 0; bit < RS_MAX_BITS; ++bit) {
+            const uint32_t x = (uint32_t)__builtin_amdgcn_sbfe(d, bit, 1);
+            const unsigned long long bal = __builtin_amdgcn_ballot_w64(x != 0);
+            plo &= ~(x ^ (uint32_t)bal);
+            phi &= ~(x ^ (uint32_t)(bal >> 32));
+        }
+        const unsigned long long peers = ((unsigned long long)phi << 32) | plo;
+        const int base = wcnt[wave][d];
+        rank[it] = base + __popcll(peers & lt);
+        fg_wave_lds_sync();
+        // the highest lane of every peer group advances the wave's counter of that digit
+        if (ok && (peers >> lane) == 1ull) wcnt[wave][d] = (uint16_t)(base + __popcll(peers));
+        fg_wave_lds_sync();
+    }
+    __syncthreads();
+    {
+        // thread t owns digits RS_DPT*t ..: exclusive scans of the tile's digit counts and of the digits' totals
+        int c[RS_DPT], g[RS_DPT], ctot = 0, gtot = 0;
+#pragma unroll
+        for (int j = 0; j < RS_DPT; ++j) {
+            const int d = RS_DPT * tid + j;
+            c[j] = 0;
+#pragma unroll 4
+            for (int w = 0; w < RS_WAVES; ++w) c[j] += wcnt[w][d];
+            g[j] = d <= mask ? digit_total[d] : 0;
+            ctot += c[j];
+            gtot += g[j];
+        }
+        const int ci = rs_wave_incl(ctot, lane), gi = rs_wave_incl(gtot, lane);
+        if (lane == 63) { wave_tot[0][wave] = ci; wave_tot[1][wave] = gi; }
+        __syncthreads();
+        int lbase = ci - ctot, gbase = gi - gtot;
+        for (int w = 0; w < wave; ++w) { lbase += wave_tot[0][w]; gbase += wave_tot[1][w]; }
+#pragma unroll
+        for (int j = 0; j < RS_DPT; ++j) {
+            const int d = RS_DPT * tid + j;
+            if (d <= mask) gofs[d] = gbase + hist[(size_t)d * rs_hist_ld(ntiles) + tile] - lbase;
+            int run = lbase;
+#pragma unroll 4
+            for (int w = 0; w < RS_WAVES; ++w) { const int t = wcnt[w][d]; wcnt[w][d] = (uint16_t)run; run += t; }
+            lbase += c[j];
+            gbase += g[j];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) rank[it] += wcnt[wave][(key[it] >> shift) & mask];
+    __syncthreads();                             // the counters have been read: the same LDS now stages the records
+    int2 *stage = reinterpret_cast<int2 *>(buf);
+    if constexpr (!TRIPLE) {
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it)
+            if (it * 64 < mine) stage[rank[it]] = rec[it];
+        __syncthreads();
+#pragma unroll 4
+        for (int i = tid; i < count; i += RS_TPB) {
+            const int2 r = stage[i];
+            const int q = gofs[((KEY_Y ? r.y : r.x) >> shift) & mask] + i;
+            if constexpr (OUT == RS_TO_PAIR) A.rec_out[q] = r;
+            else { A.a_out[q] = r.x; A.b_out[q] = r.y; }
+        }
+    } else {
+        int *kstage = reinterpret_cast<int *>(buf);
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it)
+            if (it * 64 < mine) kstage[rank[it]] = key[it];
+        __syncthreads();
+        int dst[ITEMS];
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) {
+            const int i = it * RS_TPB + tid;
+            dst[it] = 0;
+            if (i < count) {
+                const int k = kstage[i];
+                dst[it] = gofs[(k >> shift) & mask] + i;
+                A.key_out[dst[it]] = k;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it)
+            if (it * 64 < mine) stage[rank[it]] = rec[it];
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) {
+            const int i = it * RS_TPB + tid;
+            if (i < count) {
+                const int2 r = stage[i];
+                if constexpr (OUT == RS_TO_TRIPLE) A.rec_out[dst[it]] = r;
+                else { A.a_out[dst[it]] = r.x; A.b_out[dst[it]] = r.y; }
+            }
+        }
+    }
+}
+
+// col_ptr from the sorted columns.
+__global__ __launch_bounds__(256) void csc_colptr_kernel(int64_t n, int n_cols, const int *__restrict__ sorted_keys, int *__restrict__ col_ptr)
+{
+    const int64_t q0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (q0 >= n) return;
+    int v[4], prev = q0 > 0 ? sorted_keys[q0 - 1] : -1;
+    if (q0 + 4 <= n) *reinterpret_cast<int4 *>(v) = *reinterpret_cast<const int4 *>(sorted_keys + q0);
+    else
+        for (int j = 0; j < 4; ++j) v[j] = q0 + j < n ? sorted_keys[q0 + j] : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int64_t q = q0 + j;
+        if (q >= n) break;
+        for (int c = prev + 1; c <= v[j]; ++c) col_ptr[c] = (int)q;
+        if (q == n - 1)
+            for (int c = v[j] + 1; c <= n_cols; ++c) col_ptr[c] = (int)n;
+        prev = v[j];
+    }
 }
 
 __global__ __launch_bounds__(256) void fill_i32_kernel(int *p, size_t n, int v)
@@ -221,72 +356,92 @@ static int rs_key_bits(int n_cols)
     return bits;
 }
 
-// Scratch of one radix sort of n (key, payload) pairs: two key buffers, one payload buffer,
-// per-block digit counts and two 256-entry tables.
-static size_t rs_sort_workspace(int64_t n)
+// Passes of equal digit width for a key of `key_bits` bits (18 bits: 9 + 9 rather than 11 + 7: fewer digits mean longer runs).
+struct rs_plan { int passes, bits; };
+static rs_plan rs_plan_of(int key_bits)
 {
-    size_t nblocks = (size_t)((n + RS_TILE - 1) / RS_TILE);
-    return 3 * fgnn_align256((size_t)n * sizeof(int)) + fgnn_align256(256 * nblocks * sizeof(int)) + 2 * fgnn_align256(256 * sizeof(int));
+    rs_plan p;
+    p.passes = (key_bits + RS_MAX_BITS - 1) / RS_MAX_BITS;
+    p.bits = (key_bits + p.passes - 1) / p.passes;
+    return p;
+}
+static size_t rs_hist_bytes(int64_t n, int bits)
+{
+    return fgnn_align256(((size_t)rs_hist_ld(rs_num_tiles(n)) << bits) * sizeof(int)) + fgnn_align256(RS_MAX_DIGITS * sizeof(int));
 }
 
-// Stable LSD radix sort of n pairs by the low `key_bits` key bits, in ceil(key_bits / 8) passes of equal
-// digit width (18 bits: 6 + 6 + 6 rather than 8 + 8 + 2 -- fewer digits mean longer contiguous runs per
-// tile in the scatter).  keys_in is not modified; pay_in == NULL sorts the element indices.  The sorted
-// payload lands in pay_out; *sorted_keys points at the sorted keys (inside the workspace).
+// One pass: `keys` / `stride` name the same digits for the histogram that the scatter finds in its records.
+template <rs_in IN, rs_out OUT, bool KEY_Y>
+static int rs_pass(const rs_args &A, const int *keys, int stride, int64_t n, int shift, int bits, int *hist, hipStream_t st)
+{
+    const int ntiles = rs_num_tiles(n), mask = (1 << bits) - 1;
+    int *digit_total = (int *)((char *)hist + fgnn_align256(((size_t)rs_hist_ld(ntiles) << bits) * sizeof(int)));
+    const bool small = rs_items(n) == 2;
+    if (small) hipLaunchKernelGGL(rs_hist_kernel<2>, dim3(rs_grid(ntiles)), dim3(RS_TPB), 0, st, keys, stride, n, shift, mask, ntiles, hist);
+    else hipLaunchKernelGGL(rs_hist_kernel<8>, dim3(rs_grid(ntiles)), dim3(RS_TPB), 0, st, keys, stride, n, shift, mask, ntiles, hist);
+    int rc = fgnn_launch_status("rs_hist_kernel");
+    if (rc) return rc;
+    hipLaunchKernelGGL(rs_scan_kernel, dim3(1 << bits), dim3(RS_SCAN_TPB), 0, st, hist, ntiles, digit_total);
+    rc = fgnn_launch_status("rs_scan_kernel");
+    if (rc) return rc;
+    if (small) hipLaunchKernelGGL((rs_scatter_kernel<2, IN, OUT, KEY_Y>), dim3(rs_grid(ntiles)), dim3(RS_TPB), 0, st, A, n, shift, mask, ntiles, hist, digit_total);
+    else hipLaunchKernelGGL((rs_scatter_kernel<8, IN, OUT, KEY_Y>), dim3(rs_grid(ntiles)), dim3(RS_TPB), 0, st, A, n, shift, mask, ntiles, hist, digit_total);
+    return fgnn_launch_status("rs_scatter_kernel");
+}
+
+// Scratch of rs_sort_pairs: up to two record buffers, the sorted keys, the digit counts.
+static size_t rs_sort_workspace(int64_t n, int key_bits)
+{
+    const rs_plan p = rs_plan_of(key_bits);
+    const size_t nb = fgnn_align256((size_t)n * sizeof(int2));
+    return (size_t)(p.passes > 2 ? 2 : p.passes - 1) * nb + fgnn_align256((size_t)n * sizeof(int)) + rs_hist_bytes(n, p.bits);
+}
+
+// Stable LSD radix sort of n pairs by the low `key_bits` key bits.  keys_in is not modified; pay_in == NULL sorts the element
+// indices.  The sorted payload lands in pay_out; *sorted_keys points at the sorted keys (inside the workspace).
 static int rs_sort_pairs(const int *keys_in, const int *pay_in, int64_t n, int key_bits, int *pay_out, const int **sorted_keys, void *workspace,
                          hipStream_t st)
 {
-    const int passes = (key_bits + 7) / 8;
-    const int bits = (key_bits + passes - 1) / passes;      // digit width of every pass, <= 8
-    const int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
+    const rs_plan p = rs_plan_of(key_bits);
     char *w = (char *)workspace;
-    int *keys[2];
-    keys[0] = (int *)w; w += fgnn_align256((size_t)n * sizeof(int));
-    keys[1] = (int *)w; w += fgnn_align256((size_t)n * sizeof(int));
-    int *pay[2];
-    pay[0] = pay_out;
-    pay[1] = (int *)w; w += fgnn_align256((size_t)n * sizeof(int));
-    int *hist = (int *)w; w += fgnn_align256(256 * (size_t)nblocks * sizeof(int));
-    int *digit_total = (int *)w; w += fgnn_align256(256 * sizeof(int));
-    int *digit_base = (int *)w;
-    const int *kin = keys_in;
-    const int *pin = pay_in;
-    for (int i = 0; i < passes; ++i) {
-        int shift = bits * i;
-        int *kout = keys[i & 1];
-        int *pout = pay[(passes - 1 - i) & 1];      // the last pass lands in pay_out
-        hipLaunchKernelGGL(rs_hist_kernel, dim3(nblocks), dim3(RS_TPB), 0, st, kin, n, shift, (1 << bits) - 1, nblocks, hist);
-        int rc = fgnn_launch_status("rs_hist_kernel");
+    int2 *rec[2] = {nullptr, nullptr};
+    for (int i = 0; i < 2 && i < p.passes - 1; ++i) { rec[i] = (int2 *)w; w += fgnn_align256((size_t)n * sizeof(int2)); }
+    int *keys = (int *)w; w += fgnn_align256((size_t)n * sizeof(int));
+    int *hist = (int *)w;
+    *sorted_keys = keys;
+    for (int i = 0; i < p.passes; ++i) {
+        const bool last = i == p.passes - 1;
+        rs_args A = {};
+        A.a = keys_in; A.b = pay_in; A.a_out = keys; A.b_out = pay_out;
+        if (i > 0) A.rec = rec[(i - 1) & 1];
+        if (!last) A.rec_out = rec[i & 1];
+        int rc;
+        if (i == 0) rc = last ? rs_pass<RS_ARRAYS, RS_TO_ARRAYS, false>(A, keys_in, 1, n, 0, p.bits, hist, st)
+                              : rs_pass<RS_ARRAYS, RS_TO_PAIR, false>(A, keys_in, 1, n, 0, p.bits, hist, st);
+        else rc = last ? rs_pass<RS_PAIR, RS_TO_ARRAYS, false>(A, (const int *)A.rec, 2, n, p.bits * i, p.bits, hist, st)
+                       : rs_pass<RS_PAIR, RS_TO_PAIR, false>(A, (const int *)A.rec, 2, n, p.bits * i, p.bits, hist, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(rs_scan_kernel, dim3(1 << bits), dim3(RS_TPB), 0, st, hist, nblocks, digit_total);
-        rc = fgnn_launch_status("rs_scan_kernel");
-        if (rc) return rc;
-        hipLaunchKernelGGL(rs_digit_base_kernel, dim3(1), dim3(256), 0, st, digit_total, 1 << bits, digit_base);
-        rc = fgnn_launch_status("rs_digit_base_kernel");
-        if (rc) return rc;
-        hipLaunchKernelGGL(rs_scatter_kernel, dim3(nblocks), dim3(RS_TPB), 0, st, kin, pin, n, shift, bits, nblocks, hist, digit_base, kout, pout);
-        rc = fgnn_launch_status("rs_scatter_kernel");
-        if (rc) return rc;
-        kin = kout;
-        pin = pout;
     }
-    *sorted_keys = kin;
     return 0;
 }
 
-static int csc_num_hints(int64_t E) { return E > 0 ? (int)((E - 1) >> CSC_HINT_SHIFT) + 2 : 0; }
-
+// Up to two buffers of (key, two words), the sorted columns, the digit counts, the row hints.
 extern "C" size_t fgnn_csr2csc_workspace_bytes(int n_rows, int n_cols, int64_t E)
 {
-    (void)n_rows; (void)n_cols;
-    return rs_sort_workspace(E) + fgnn_align256((size_t)csc_num_hints(E) * sizeof(int));
+    (void)n_rows;
+    const rs_plan p = rs_plan_of(rs_key_bits(n_cols));
+    const size_t kb = fgnn_align256((size_t)E * sizeof(int)), rb = fgnn_align256((size_t)E * sizeof(int2));
+    return (size_t)(p.passes > 2 ? 2 : p.passes - 1) * (kb + rb) + kb + rs_hist_bytes(E, p.bits) + fgnn_align256((size_t)csc_num_hints(E) * sizeof(int));
 }
 
+// The records are (column, position, row): the row of a position is known where the positions are still in order, in the
+// first pass, and carrying it through the other passes costs 8 bytes per entry and pass; finding it at the end, position by
+// position at random places of row_ptr, took 1.3 ms for 64.3 M entries, as much as two passes.
 extern "C" int fgnn_csr2csc(int n_rows, int n_cols, int64_t E, const int32_t *row_ptr, const int32_t *col_ind, int32_t *col_ptr,
                             int32_t *row_ind, int32_t *permute, void *workspace, size_t workspace_bytes, void *stream)
 {
     FGNN_REQUIRE(n_rows >= 0 && n_cols >= 0 && E >= 0, FGNN_ERR_SHAPE, "fgnn_csr2csc: bad sizes");
-    FGNN_REQUIRE(E <= 2147483647LL - RS_TILE, FGNN_ERR_LIMIT, "fgnn_csr2csc: E=%lld exceeds int32 positions", (long long)E);
+    FGNN_REQUIRE(E <= 2147483647LL - RS_TPB * 8, FGNN_ERR_LIMIT, "fgnn_csr2csc: E=%lld exceeds int32 positions", (long long)E);
     FGNN_REQUIRE(row_ptr && col_ptr && (E == 0 || (col_ind && row_ind && permute)), FGNN_ERR_NULL, "fgnn_csr2csc: NULL argument");
     hipStream_t st = (hipStream_t)stream;
     if (E == 0) {
@@ -296,37 +451,43 @@ extern "C" int fgnn_csr2csc(int n_rows, int n_cols, int64_t E, const int32_t *ro
     FGNN_REQUIRE(n_cols >= 1 && n_rows >= 1, FGNN_ERR_SHAPE, "fgnn_csr2csc: edges without rows or columns");
     size_t need = fgnn_csr2csc_workspace_bytes(n_rows, n_cols, E);
     FGNN_REQUIRE(workspace && workspace_bytes >= need, FGNN_ERR_WORKSPACE, "fgnn_csr2csc: workspace %zu < %zu bytes", workspace_bytes, need);
-    const int *sorted = nullptr;
-    int rc = rs_sort_pairs(col_ind, nullptr, E, rs_key_bits(n_cols), permute, &sorted, workspace, st);
-    if (rc) return rc;
-    int *hint = (int *)((char *)workspace + rs_sort_workspace(E));
+    const rs_plan p = rs_plan_of(rs_key_bits(n_cols));
+    const size_t kb = fgnn_align256((size_t)E * sizeof(int)), rb = fgnn_align256((size_t)E * sizeof(int2));
+    char *w = (char *)workspace;
+    int *key[2] = {nullptr, nullptr};
+    int2 *rec[2] = {nullptr, nullptr};
+    for (int i = 0; i < 2 && i < p.passes - 1; ++i) { key[i] = (int *)w; w += kb; rec[i] = (int2 *)w; w += rb; }
+    int *sorted = (int *)w; w += kb;
+    int *hist = (int *)w; w += rs_hist_bytes(E, p.bits);
+    int *hint = (int *)w;
     const int n_hint = csc_num_hints(E);
     hipLaunchKernelGGL(csc_row_hint_kernel, dim3((unsigned)((n_hint + 255) / 256)), dim3(256), 0, st, E, n_rows, n_hint, row_ptr, hint);
-    rc = fgnn_launch_status("csc_row_hint_kernel");
+    int rc = fgnn_launch_status("csc_row_hint_kernel");
+    for (int i = 0; i < p.passes && !rc; ++i) {
+        const bool last = i == p.passes - 1;
+        rs_args A = {};
+        A.a = col_ind; A.row_ptr = row_ptr; A.hint = hint; A.n_rows = n_rows; A.n_hint = n_hint;
+        if (i > 0) { A.key = key[(i - 1) & 1]; A.rec = rec[(i - 1) & 1]; }
+        A.key_out = last ? sorted : key[i & 1];
+        A.rec_out = last ? nullptr : rec[i & 1];
+        A.a_out = permute; A.b_out = row_ind;
+        if (i == 0) rc = last ? rs_pass<RS_CSR, RS_TO_ARRAYS3, false>(A, col_ind, 1, E, 0, p.bits, hist, st)
+                              : rs_pass<RS_CSR, RS_TO_TRIPLE, false>(A, col_ind, 1, E, 0, p.bits, hist, st);
+        else rc = last ? rs_pass<RS_TRIPLE, RS_TO_ARRAYS3, false>(A, A.key, 1, E, p.bits * i, p.bits, hist, st)
+                       : rs_pass<RS_TRIPLE, RS_TO_TRIPLE, false>(A, A.key, 1, E, p.bits * i, p.bits, hist, st);
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(csc_finalize_kernel, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, st, E, n_cols, sorted, permute, row_ptr, hint, col_ptr, row_ind);
-    return fgnn_launch_status("csc_finalize_kernel");
+    hipLaunchKernelGGL(csc_colptr_kernel, dim3((unsigned)((E + 1023) / 1024)), dim3(256), 0, st, E, n_cols, sorted, col_ptr);
+    return fgnn_launch_status("csc_colptr_kernel");
 }
 
 // ------------------------------------------------------------------------------- COO -> CSR
 // Edge list (dst[e], src[e]) -> CSR by destination with sources ascending inside a row, optionally
 // merging duplicate edges: what the reference does on the host with scipy's csr_matrix
-// (script/train/train_gatconv_our.py:87-91).  Two stable radix sorts (by src, then by dst), a
-// first-of-its-group flag, an inclusive scan of the flags, and a compaction.
-
-__global__ __launch_bounds__(256) void gather_i32_kernel(int64_t n, const int *__restrict__ idx, const int *__restrict__ in, int *__restrict__ out)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = in[idx[i]];
-}
-
-// flag[q] = 1 when sorted entry q starts a new (dst, src) group (always 1 without dedupe)
-__global__ __launch_bounds__(256) void coo_flag_kernel(int64_t n, const int *__restrict__ dsts, const int *__restrict__ srcs, int dedupe, int *__restrict__ flag)
-{
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    flag[q] = (!dedupe || q == 0 || dsts[q] != dsts[q - 1] || srcs[q] != srcs[q - 1]) ? 1 : 0;
-}
+// (script/train/train_gatconv_our.py:87-91).  One LSD sort over the source's digits and then the
+// destination's; both ids travel in the record, so nothing is gathered between the two (through an index
+// payload the two gathers took 2.5 ms for 64.3 M edges).  Where the caller wants the position of every
+// input edge, its index travels too.  The sorted records are then counted (duplicates) and written.
 
 #define SC_ITEMS 16
 #define SC_TILE (256 * SC_ITEMS)
@@ -346,29 +507,34 @@ __global__ __launch_bounds__(256) void scan_tile_sums_kernel(int64_t n, const in
     }
     if (threadIdx.x == 0) sums[blockIdx.x] = sh[0];
 }
-__global__ __launch_bounds__(256) void scan_sums_kernel(int nt, int *__restrict__ sums, int *__restrict__ total)
+// 1024 threads x 8 sums per chunk (64.3 M records: 15.7 k sums in two chunks).
+#define SC_SUMS_TPB 1024
+__global__ __launch_bounds__(SC_SUMS_TPB) void scan_sums_kernel(int nt, int *__restrict__ sums, int *__restrict__ total)
 {
-    __shared__ int sh[256];
-    __shared__ int carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < nt; base += 256) {
-        int i = base + (int)threadIdx.x;
-        int v = i < nt ? sums[i] : 0;
-        sh[threadIdx.x] = v;
+    constexpr int PER = 8;
+    __shared__ int wave_tot[SC_SUMS_TPB / 64];
+    const int lane = fg_lane(), wave = fg_wave();
+    int carry = 0;
+    for (int base = 0; base < nt; base += SC_SUMS_TPB * PER) {
+        const int i0 = base + (int)threadIdx.x * PER;
+        int v[PER], tot = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) { v[j] = i0 + j < nt ? sums[i0 + j] : 0; tot += v[j]; }
+        const int incl = rs_wave_incl(tot, lane);
+        __syncthreads();                        // the previous chunk's wave totals have been read
+        if (lane == 63) wave_tot[wave] = incl;
         __syncthreads();
-        for (int off = 1; off < 256; off <<= 1) {
-            int t = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-            __syncthreads();
-            sh[threadIdx.x] += t;
-            __syncthreads();
+        int run = carry + incl - tot;
+        for (int w = 0; w < SC_SUMS_TPB / 64; ++w) {
+            const int t = wave_tot[w];
+            if (w < wave) run += t;
+            carry += t;
         }
-        int incl = sh[threadIdx.x];
-        int c = carry;
-        if (i < nt) sums[i] = c + incl - v;          // exclusive offset of tile i
-        __syncthreads();
-        if (threadIdx.x == 255) carry = c + incl;
-        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (i0 + j < nt) sums[i0 + j] = run;          // exclusive offset of tile i0 + j
+            run += v[j];
+        }
     }
     if (threadIdx.x == 0) *total = carry;
 }
@@ -397,7 +563,7 @@ __global__ __launch_bounds__(256) void scan_apply_kernel(int64_t n, const int *_
 }
 
 // Library-internal entry points to the sort and the scan (the schedule builder uses them too).
-size_t fgnn_rs_sort_workspace(int64_t n) { return rs_sort_workspace(n); }
+size_t fgnn_rs_sort_workspace(int64_t n, int key_bits) { return rs_sort_workspace(n, key_bits); }
 int fgnn_rs_key_bits(int n_keys) { return rs_key_bits(n_keys); }
 int fgnn_rs_sort_pairs(const int *keys_in, const int *pay_in, int64_t n, int key_bits, int *pay_out, const int **sorted_keys, void *workspace,
                        hipStream_t st)
@@ -412,54 +578,109 @@ int fgnn_inclusive_scan_i32(const int *in, int64_t n, int *out, int *tile_sums, 
     hipLaunchKernelGGL(scan_tile_sums_kernel, dim3(nt), dim3(256), 0, st, n, in, tile_sums);
     int rc = fgnn_launch_status("scan_tile_sums_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(256), 0, st, nt, tile_sums, total_dev);
+    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(SC_SUMS_TPB), 0, st, nt, tile_sums, total_dev);
     rc = fgnn_launch_status("scan_sums_kernel");
     if (rc) return rc;
     hipLaunchKernelGGL(scan_apply_kernel, dim3(nt), dim3(256), 0, st, n, in, tile_sums, out);
     return fgnn_launch_status("scan_apply_kernel");
 }
 
-// Compaction: the first entry of every group writes its source and destination at the group's
-// position; every input edge learns the position of its group.
-__global__ __launch_bounds__(256) void coo_compact_kernel(int64_t n, const int *__restrict__ dsts, const int *__restrict__ srcs,
-                                                          const int *__restrict__ perm, const int *__restrict__ flag, const int *__restrict__ incl,
-                                                          int *__restrict__ col_ind, int *__restrict__ dstc, int *__restrict__ edge_pos)
+// Tile sums of "record q starts a new (dst, src) group" over the sorted records {dst, src} (TRIPLE: key dst, rec {src, edge}).
+template <bool TRIPLE>
+__device__ __forceinline__ int2 coo_at(const int *__restrict__ key, const int2 *__restrict__ rec, int64_t q)
 {
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    int pos = incl[q] - 1;
-    if (flag[q]) { col_ind[pos] = srcs[q]; dstc[pos] = dsts[q]; }
-    if (edge_pos) edge_pos[perm[q]] = pos;
+    if constexpr (TRIPLE) return make_int2(key[q], rec[q].x);
+    else return rec[q];
+}
+template <bool TRIPLE>
+__global__ __launch_bounds__(256) void coo_count_kernel(int64_t n, const int *__restrict__ key, const int2 *__restrict__ rec, int *__restrict__ sums)
+{
+    __shared__ int sh[4];
+    const int64_t base = (int64_t)blockIdx.x * SC_TILE;
+    int acc = 0;
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; ++k) {
+        const int64_t q = base + k * 256 + (int)threadIdx.x;
+        if (q < n) {
+            const int2 r = coo_at<TRIPLE>(key, rec, q);
+            const int2 b = q > 0 ? coo_at<TRIPLE>(key, rec, q - 1) : make_int2(-1, -1);
+            acc += r.x != b.x || r.y != b.y;
+        }
+    }
+    acc = rs_wave_incl(acc, fg_lane());
+    if (fg_lane() == 63) sh[fg_wave()] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// row_ptr from the compacted destinations (ascending); *n_out entries are valid.
-__global__ __launch_bounds__(256) void coo_rowptr_kernel(int n_rows, const int *__restrict__ dstc, const int *__restrict__ n_out_dev,
-                                                         int *__restrict__ row_ptr, int64_t *__restrict__ n_out)
+// The CSR from the sorted records: the first record of every group writes its source at the group's position and, where its
+// destination is a new one, the row pointers up to it; every input edge learns the position of its group.  sums: exclusive
+// tile offsets (NULL: no merging, record q is entry q).
+template <bool TRIPLE>
+__global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, const int *__restrict__ key, const int2 *__restrict__ rec,
+                                                        const int *__restrict__ sums, int *__restrict__ col_ind, int *__restrict__ row_ptr,
+                                                        int64_t *__restrict__ n_out, int *__restrict__ edge_pos)
 {
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = *n_out_dev;
-    if (q == 0 && n_out) *n_out = m;
-    if (q >= m) return;
-    int key = dstc[q];
-    int prev = q > 0 ? dstc[q - 1] : -1;
-    for (int r = prev + 1; r <= key; ++r) row_ptr[r] = (int)q;
-    if (q == m - 1)
-        for (int r = key + 1; r <= n_rows; ++r) row_ptr[r] = m;
+    __shared__ int wave_cnt[SC_ITEMS][4];
+    const int lane = fg_lane(), wave = fg_wave();
+    const int64_t base = (int64_t)blockIdx.x * SC_TILE;
+    const unsigned long long le = lane == 63 ? ~0ull : (1ull << (lane + 1)) - 1ull;
+    int2 r[SC_ITEMS];
+    int before[SC_ITEMS], prev_dst[SC_ITEMS];       // groups started in the wave's 64 records up to and with this one
+    unsigned fl = 0;
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; ++k) {
+        const int64_t q = base + k * 256 + (int)threadIdx.x;
+        r[k] = make_int2(-1, -1);
+        int2 b = make_int2(-1, -1);
+        if (q < n) {
+            r[k] = coo_at<TRIPLE>(key, rec, q);
+            if (q > 0) b = coo_at<TRIPLE>(key, rec, q - 1);
+        }
+        const bool f = q < n && (!sums || r[k].x != b.x || r[k].y != b.y);
+        prev_dst[k] = b.x;
+        fl |= (unsigned)f << k;
+        const unsigned long long m = __ballot(f);
+        before[k] = __popcll(m & le);
+        if (lane == 0) wave_cnt[k][wave] = __popcll(m);
+    }
+    __syncthreads();
+    int run = sums ? sums[blockIdx.x] : (int)base;
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; ++k) {
+        const int64_t q = base + k * 256 + (int)threadIdx.x;
+        int ofs = run;
+        for (int w = 0; w < wave; ++w) ofs += wave_cnt[k][w];
+        const int pos = ofs + before[k] - 1;
+        run += (wave_cnt[k][0] + wave_cnt[k][1]) + (wave_cnt[k][2] + wave_cnt[k][3]);
+        if (q < n) {
+            if ((fl >> k) & 1) {
+                col_ind[pos] = r[k].y;
+                for (int i = prev_dst[k] + 1; i <= r[k].x; ++i) row_ptr[i] = pos;
+            }
+            if (q == n - 1) {
+                for (int i = r[k].x + 1; i <= n_rows; ++i) row_ptr[i] = pos + 1;
+                *n_out = pos + 1;
+            }
+            if constexpr (TRIPLE) edge_pos[rec[q].y] = pos;
+        }
+    }
 }
 
+// With positions: two buffers of (key, two words); without: two of pairs.  The caller's edge_pos is not known here: room for both.
 extern "C" size_t fgnn_coo2csr_workspace_bytes(int n_rows, int n_cols, int64_t E)
 {
-    (void)n_rows; (void)n_cols;
-    size_t nt = (size_t)((E + SC_TILE - 1) / SC_TILE);
-    // sort scratch | perm1 | keys2 / srcs | perm2 | flag | incl | dstc | tile sums | total
-    return rs_sort_workspace(E) + 6 * fgnn_align256((size_t)E * sizeof(int)) + fgnn_align256((nt + 1) * sizeof(int)) + 256;
+    const rs_plan ps = rs_plan_of(rs_key_bits(n_cols)), pd = rs_plan_of(rs_key_bits(n_rows));
+    const size_t nt = (size_t)((E + SC_TILE - 1) / SC_TILE);
+    const size_t kb = fgnn_align256((size_t)E * sizeof(int)), rb = fgnn_align256((size_t)E * sizeof(int2));
+    return 2 * (kb + rb) + rs_hist_bytes(E, ps.bits > pd.bits ? ps.bits : pd.bits) + fgnn_align256((nt + 1) * sizeof(int)) + 256;
 }
 
 extern "C" int fgnn_coo2csr(int n_rows, int n_cols, int64_t E, const int32_t *dst, const int32_t *src, int dedupe, int32_t *row_ptr,
                             int32_t *col_ind, int64_t *n_out, int32_t *edge_pos, void *workspace, size_t workspace_bytes, void *stream)
 {
     FGNN_REQUIRE(n_rows >= 0 && n_cols >= 0 && E >= 0, FGNN_ERR_SHAPE, "fgnn_coo2csr: bad sizes");
-    FGNN_REQUIRE(E <= 2147483647LL - RS_TILE, FGNN_ERR_LIMIT, "fgnn_coo2csr: E=%lld exceeds int32 positions", (long long)E);
+    FGNN_REQUIRE(E <= 2147483647LL - RS_TPB * 8, FGNN_ERR_LIMIT, "fgnn_coo2csr: E=%lld exceeds int32 positions", (long long)E);
     FGNN_REQUIRE(row_ptr && n_out && (E == 0 || (dst && src && col_ind)), FGNN_ERR_NULL, "fgnn_coo2csr: NULL argument");
     hipStream_t st = (hipStream_t)stream;
     if (E == 0) {
@@ -472,47 +693,49 @@ extern "C" int fgnn_coo2csr(int n_rows, int n_cols, int64_t E, const int32_t *ds
     FGNN_REQUIRE(n_cols >= 1 && n_rows >= 1, FGNN_ERR_SHAPE, "fgnn_coo2csr: edges without rows or columns");
     size_t need = fgnn_coo2csr_workspace_bytes(n_rows, n_cols, E);
     FGNN_REQUIRE(workspace && workspace_bytes >= need, FGNN_ERR_WORKSPACE, "fgnn_coo2csr: workspace %zu < %zu bytes", workspace_bytes, need);
+    const rs_plan ps = rs_plan_of(rs_key_bits(n_cols)), pd = rs_plan_of(rs_key_bits(n_rows));
+    const size_t kb = fgnn_align256((size_t)E * sizeof(int)), rb = fgnn_align256((size_t)E * sizeof(int2));
     char *w = (char *)workspace;
-    void *sort_ws = w; w += rs_sort_workspace(E);
-    size_t eb = fgnn_align256((size_t)E * sizeof(int));
-    int *perm1 = (int *)w; w += eb;
-    int *tmp = (int *)w; w += eb;          // dst gathered by perm1, later the sorted sources
-    int *perm2 = (int *)w; w += eb;
-    int *flag = (int *)w; w += eb;
-    int *incl = (int *)w; w += eb;
-    int *dstc = (int *)w; w += eb;
+    int *key[2];
+    int2 *rec[2];
+    for (int i = 0; i < 2; ++i) { key[i] = (int *)w; w += kb; rec[i] = (int2 *)w; w += rb; }
+    int *hist = (int *)w; w += rs_hist_bytes(E, ps.bits > pd.bits ? ps.bits : pd.bits);
     const int nt = (int)((E + SC_TILE - 1) / SC_TILE);
     int *sums = (int *)w; w += fgnn_align256(((size_t)nt + 1) * sizeof(int));
     int *total = (int *)w;
-    const unsigned ge = (unsigned)((E + 255) / 256);
 
-    const int *sorted = nullptr;
-    int rc = rs_sort_pairs(src, nullptr, E, rs_key_bits(n_cols), perm1, &sorted, sort_ws, st);
+    const int passes = ps.passes + pd.passes;
+    int rc = 0;
+    for (int i = 0; i < passes && !rc; ++i) {
+        const bool by_src = i < ps.passes;
+        const int bits = by_src ? ps.bits : pd.bits, shift = bits * (by_src ? i : i - ps.passes);
+        rs_args A = {};
+        A.a = dst; A.b = src;
+        A.key = key[(i - 1) & 1]; A.rec = rec[(i - 1) & 1];
+        A.key_out = key[i & 1]; A.rec_out = rec[i & 1];
+        if (!edge_pos) {                                    // records {dst, src}
+            if (i == 0) rc = rs_pass<RS_ARRAYS, RS_TO_PAIR, true>(A, src, 1, E, shift, bits, hist, st);
+            else if (by_src) rc = rs_pass<RS_PAIR, RS_TO_PAIR, true>(A, (const int *)A.rec + 1, 2, E, shift, bits, hist, st);
+            else rc = rs_pass<RS_PAIR, RS_TO_PAIR, false>(A, (const int *)A.rec, 2, E, shift, bits, hist, st);
+        } else {                                            // src, {dst, edge}; then dst, {src, edge}
+            if (i == 0) rc = rs_pass<RS_EDGES, RS_TO_TRIPLE, false>(A, src, 1, E, shift, bits, hist, st);
+            else if (i == ps.passes) rc = rs_pass<RS_TRIPLE_SWAP, RS_TO_TRIPLE, false>(A, (const int *)A.rec, 2, E, shift, bits, hist, st);
+            else rc = rs_pass<RS_TRIPLE, RS_TO_TRIPLE, false>(A, A.key, 1, E, shift, bits, hist, st);
+        }
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(gather_i32_kernel, dim3(ge), dim3(256), 0, st, E, perm1, dst, tmp);
-    rc = fgnn_launch_status("gather_i32_kernel");
-    if (rc) return rc;
-    const int *dsts = nullptr;
-    rc = rs_sort_pairs(tmp, perm1, E, rs_key_bits(n_rows), perm2, &dsts, sort_ws, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(gather_i32_kernel, dim3(ge), dim3(256), 0, st, E, perm2, src, tmp);       // sources in (dst, src) order
-    rc = fgnn_launch_status("gather_i32_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(coo_flag_kernel, dim3(ge), dim3(256), 0, st, E, dsts, tmp, dedupe, flag);
-    rc = fgnn_launch_status("coo_flag_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(scan_tile_sums_kernel, dim3(nt), dim3(256), 0, st, E, flag, sums);
-    rc = fgnn_launch_status("scan_tile_sums_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(256), 0, st, nt, sums, total);
-    rc = fgnn_launch_status("scan_sums_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(scan_apply_kernel, dim3(nt), dim3(256), 0, st, E, flag, sums, incl);
-    rc = fgnn_launch_status("scan_apply_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(coo_compact_kernel, dim3(ge), dim3(256), 0, st, E, dsts, tmp, perm2, flag, incl, col_ind, dstc, edge_pos);
-    rc = fgnn_launch_status("coo_compact_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(coo_rowptr_kernel, dim3(ge), dim3(256), 0, st, n_rows, dstc, total, row_ptr, n_out);
-    return fgnn_launch_status("coo_rowptr_kernel");
+    const int *skey = key[(passes - 1) & 1];
+    const int2 *srec = rec[(passes - 1) & 1];
+    if (dedupe) {
+        if (edge_pos) hipLaunchKernelGGL(coo_count_kernel<true>, dim3(nt), dim3(256), 0, st, E, skey, srec, sums);
+        else hipLaunchKernelGGL(coo_count_kernel<false>, dim3(nt), dim3(256), 0, st, E, skey, srec, sums);
+        rc = fgnn_launch_status("coo_count_kernel");
+        if (rc) return rc;
+        hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(SC_SUMS_TPB), 0, st, nt, sums, total);
+        rc = fgnn_launch_status("scan_sums_kernel");
+        if (rc) return rc;
+    }
+    if (edge_pos) hipLaunchKernelGGL(coo_write_kernel<true>, dim3(nt), dim3(256), 0, st, E, n_rows, skey, srec, dedupe ? sums : nullptr, col_ind, row_ptr, n_out, edge_pos);
+    else hipLaunchKernelGGL(coo_write_kernel<false>, dim3(nt), dim3(256), 0, st, E, n_rows, skey, srec, dedupe ? sums : nullptr, col_ind, row_ptr, n_out, nullptr);
+    return fgnn_launch_status("coo_write_kernel");
 }

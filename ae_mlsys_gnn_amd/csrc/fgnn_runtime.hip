@@ -473,7 +473,8 @@ static int schedule_build_device(fgnn_schedule *s, const int32_t *ptr_dev, const
     // second stage: sized by the counters
     const size_t pb = fgnn_align256((size_t)std::max(n_part, 1) * sizeof(int)), wb = fgnn_align256((size_t)std::max(n_whole, 1) * sizeof(int));
     const size_t gen_b = fgnn_align256((size_t)std::max(n_part, 1) * sizeof(fgnn_item));
-    const size_t sort_b = fgnn_align256(fgnn_rs_sort_workspace(std::max(std::max(n_part, n_whole), 1)));
+    const int seg_bits = fgnn_rs_key_bits(FGNN_NUM_XCD * (seg_len + 1)), len_bits = fgnn_rs_key_bits(cut + 1);
+    const size_t sort_b = fgnn_align256(std::max(fgnn_rs_sort_workspace(std::max(n_part, 1), seg_bits), fgnn_rs_sort_workspace(std::max(n_whole, 1), len_bits)));
     SCHED_HIP(hipMalloc((void **)&tmp2, gen_b + 2 * pb + 3 * wb + sort_b));
     if (!rc && s->n_items > 0) SCHED_HIP(hipMalloc((void **)&s->items_dev, (size_t)s->n_items * sizeof(fgnn_item)));
     if (!rc && n_split > 0) SCHED_HIP(hipMalloc((void **)&s->split_dev, (size_t)n_split * sizeof(fgnn_split)));
@@ -491,7 +492,7 @@ static int schedule_build_device(fgnn_schedule *s, const int32_t *ptr_dev, const
             rc = fgnn_launch_status("sched_fill_padding_kernel");
             if (!rc && n_part > 0) {
                 const int *sorted_key = nullptr;
-                rc = fgnn_rs_sort_pairs(key, nullptr, n_part, fgnn_rs_key_bits(FGNN_NUM_XCD * (seg_len + 1)), pay, &sorted_key, sort_ws, st);
+                rc = fgnn_rs_sort_pairs(key, nullptr, n_part, seg_bits, pay, &sorted_key, sort_ws, st);
                 if (!rc) {
                     hipLaunchKernelGGL(sched_place_segments_kernel, dim3((unsigned)((n_part + 255) / 256)), dim3(256), 0, st, n_part, pay, sorted_key,
                                        seg_len, bs, gen, s->items_dev);
@@ -501,7 +502,7 @@ static int schedule_build_device(fgnn_schedule *s, const int32_t *ptr_dev, const
         }
         if (!rc && n_whole > 0) {
             const int *sorted_key = nullptr;
-            rc = fgnn_rs_sort_pairs(wkey, wrow, n_whole, fgnn_rs_key_bits(cut + 1), wsorted, &sorted_key, sort_ws, st);
+            rc = fgnn_rs_sort_pairs(wkey, wrow, n_whole, len_bits, wsorted, &sorted_key, sort_ws, st);
             if (!rc) {
                 hipLaunchKernelGGL(sched_place_whole_kernel, dim3((unsigned)((n_whole + 255) / 256)), dim3(256), 0, st, n_whole, wsorted, ptr_dev,
                                    bucketed ? 1 : 0, base2, s->items_dev);

@@ -57,6 +57,33 @@ def test_csr2csc_round_trip_large():
     assert torch.equal(torch.sort(permute).values.long(), torch.arange(g.n_edges, device=DEV))
 
 
+@pytest.mark.parametrize("n,e", [(2048, 2047), (2048, 2048), (2049, 2049), (5, 8192), (4194304, 300001), (4194305, 300000), (700, 4194303),
+                                 (300000, 4194304), (300000, 4202497), (16777217, 4200000)])
+def test_coo2csr_and_csr2csc_at_the_edges_of_the_radix_passes(n, e):
+    # either side of a tile (2048 and 8192 records), of the switch between the two tile sizes (4 Mi) and of one, two and three
+    # passes (11 and 22 bits), against torch's stable sort; one hub row longer than a tile, many empty rows
+    from ae_mlsys_gnn_amd.operators import csr2csc as op
+    gen = torch.Generator(device=DEV).manual_seed(n + e)
+    dst = torch.randint(0, n, (e,), generator=gen, device=DEV, dtype=torch.int32)
+    dst[torch.rand(e, generator=gen, device=DEV) < 0.1] = n // 3
+    src = torch.randint(0, n, (e,), generator=gen, device=DEV, dtype=torch.int32)
+    row_ptr, col_ind, edge_pos = op.coo2csr(dst, src, n, dedupe=False, return_edge_pos=True)
+    keys, order = torch.sort(dst.long() * n + src.long(), stable=True)
+    ref_ptr = torch.zeros(n + 1, dtype=torch.int64, device=DEV)
+    ref_ptr[1:] = torch.cumsum(torch.bincount(dst.long(), minlength=n), 0)
+    assert torch.equal(col_ind.long(), keys % n) and torch.equal(row_ptr.long(), ref_ptr)
+    assert torch.equal(edge_pos.long()[order], torch.arange(e, device=DEV))
+    rp2, ci2 = op.coo2csr(dst, src, n, dedupe=True)
+    uniq = torch.unique(keys)
+    assert torch.equal(ci2.long(), uniq % n) and int(rp2[-1]) == uniq.numel()
+    assert torch.equal((rp2[1:] - rp2[:-1]).long(), torch.bincount(uniq // n, minlength=n))
+    col_ptr, row_ind, permute = op.csr2csc(row_ptr, col_ind)
+    ref = torch.sort(col_ind.long(), stable=True).indices
+    rows = torch.repeat_interleave(torch.arange(n, device=DEV), ref_ptr[1:] - ref_ptr[:-1])
+    assert torch.equal(permute.long(), ref) and torch.equal(row_ind.long(), rows[ref])
+    assert torch.equal((col_ptr[1:] - col_ptr[:-1]).long(), torch.bincount(col_ind.long(), minlength=n)) and int(col_ptr[0]) == 0
+
+
 # ------------------------------------------------------------------ EdgeConv (argmax bit-exact)
 def _edgeconv_case(bsz, npts, k, fin, fout, seed, quantize=False):
     gen = torch.Generator().manual_seed(seed)
