@@ -654,6 +654,24 @@ def test_knn_graph_ties_are_ordered_by_id():
         knn_graph(torch.zeros(1, 200, 3, device=DEV), 129)
 
 
+@pytest.mark.parametrize("p", [33, 64, 129, 256, 500, 1024, 1030])
+@pytest.mark.parametrize("k", [1, 31, 32, 33, 63, 64])
+def test_knn_selection_at_its_limits(p, k):
+    """Neighbour ids fixed by the (distance, id) order, around the group counts of the threshold and with lists that fill, overrun
+    one register or overrun the list: distances that are all different, equal in groups of 3 and of 70, and all equal."""
+    from ae_mlsys_gnn_amd.operators.knn import knn_graph
+    if k > p:
+        pytest.skip("k exceeds the cloud")
+    gen = torch.Generator().manual_seed(p * 100 + k)
+    perm = torch.stack([torch.randperm(p, generator=gen) for _ in range(4)])
+    pts = torch.stack([perm[0], perm[1] // 3, perm[2] // 70, torch.zeros(p, dtype=torch.long)]).float().unsqueeze(2)      # exact in fp32
+    src = knn_graph(pts.to(DEV), k).cpu().long().view(4, p, k)
+    dist = ((pts.double().unsqueeze(2) - pts.double().unsqueeze(1)) ** 2).sum(-1)
+    key = dist * 2048 + torch.arange(p, dtype=torch.float64).view(1, 1, p)
+    want = torch.argsort(key, dim=2)[:, :, :k] + (torch.arange(4) * p).view(4, 1, 1)
+    assert torch.equal(src, want)
+
+
 def test_knn_graph_feeds_edgeconv():
     from ae_mlsys_gnn_amd.layers import EdgeConv
     from ae_mlsys_gnn_amd.operators.knn import knn_graph
