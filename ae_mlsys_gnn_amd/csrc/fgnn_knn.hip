@@ -24,6 +24,7 @@
 // 64 dimensions 1135 -> 436 us.
 #include "fgnn_common.h"
 #include <float.h>
+#include <type_traits>
 
 #define KNN_QW 4         // queries a wave processes together
 #define KNN_WAVES 4      // waves per workgroup
@@ -314,6 +315,250 @@ __global__ __launch_bounds__(KNN_WAVES * 64) void knn_kernel(int P, int D, int k
     }
 }
 
+// Larger clouds of many dimensions: the distances come from the matrix cores as a filter, and only what the filter leaves open
+// is computed exactly.
+//
+// A workgroup of 8 waves takes 32 queries; wave w multiplies its eighth of the tile's candidates (16 x 16 x 4 products, rows =
+// candidates, columns = queries) straight out of global memory: lane (r, q) reads 4 consecutive floats of row r, and the 4
+// products of a chunk take the first, second, third and fourth of them, a permutation of the dimensions that both operands share.
+// The row of the workgroup's first query is taken off all points, so a common offset costs no precision.
+// |c - q|^2 = |c|^2 - 2 c.q + |q|^2 then goes through LDS, 16 queries at a time, to the wave that selects.
+//
+// With u = 2^-24, S = |q|^2 + max |c|^2 (of the shifted points) the product form is within u S (2 D + 11) of the true distance and the
+// exact path's own sum, one subtract and one fma per dimension, within 2 u S (D + 3); E = 2 u S (4 D + 32) covers both twice.  tau, the
+// threshold that at least k approximations pass, thus bounds the k-th smallest exact distance by tau + E, and every candidate
+// that can be among the k best has an approximation of at most tau + 2 E (few more than pass tau).  Sorted by approximation, two
+// neighbours in the list more than 2 E apart are in order; those closer are computed by the exact path's operations in the
+// exact path's order, and the list is sorted once more.  (All 47 candidates of a query at k = 40 cost 24 KB of gathered rows, and
+// the L2 rate was the bound.)  With more candidates than lanes, or more points than a tile, all candidates are computed.  The graph is
+// bit for bit the one of the kernel above.  More than KNN_CAP candidates, or norms that overflow or are no numbers, send the query to
+// the exact path's selection over the exact distances of what passed.
+//
+// Bound by the fp32 matrix rate (1.4 us per dimension of 64 clouds x 1024 points, 95 TFLOP/s) and the selection, 140 us there.
+// Before and after at k = 40: 64 dimensions 634 (379 with the present selection) -> 243 us, 128 dimensions 904 (642) -> 344 us.
+#define KNN_MQ 32        // queries per workgroup
+#define KNN_MW 8         // waves per workgroup
+typedef float knn_f4 __attribute__((ext_vector_type(4)));
+
+// The exact distance of point c from the wave-uniform query q: dimensions in ascending order, NaN last among the real ones.
+__device__ __forceinline__ float knn_exact(const float *cp, int D, int q, int c, int rows_aligned)
+{
+    const float *qr = cp + (size_t)q * D, *cr = cp + (size_t)c * D;
+    float acc = 0.f;
+    int d = 0;
+    if (rows_aligned)
+        for (; d + 32 <= D; d += 32) {              // 8 loads in flight
+            knn_f4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const knn_f4 *>(cr + d + 4 * u);
+#pragma unroll
+            for (int u = 0; u < 32; ++u) { const float df = qr[d + u] - v[u / 4][u % 4]; acc = fmaf(df, df, acc); }
+        }
+#pragma unroll 4
+    for (; d < D; ++d) { const float df = qr[d] - cr[d]; acc = fmaf(df, df, acc); }
+    return fminf(acc, FLT_MAX);
+}
+
+template <int RG, bool WHOLE>
+__global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, int k, int rows_aligned, unsigned per_xcd, unsigned q_blocks, unsigned n_blocks,
+                                                                  const float *__restrict__ pts, int *__restrict__ out)
+{
+    constexpr int NR = 4 * RG, TILE = 256 * RG, NT = 2 * RG, NH = NT < 4 ? NT : 4, ROW = TILE + 4;      // rows 4 banks apart: 16 lanes write 16 rows at once
+    __shared__ __attribute__((aligned(16))) float buf[16 * ROW];
+    __shared__ __attribute__((aligned(16))) float cn[TILE];
+    __shared__ float2 lists[KNN_MW * KNN_CAP];
+    __shared__ float wmax[KNN_MW];
+    const unsigned b = per_xcd ? (blockIdx.x % FGNN_NUM_XCD) * per_xcd + blockIdx.x / FGNN_NUM_XCD : blockIdx.x;
+    if (b >= n_blocks) return;                  // the whole workgroup
+    const int cloud = (int)(b / q_blocks), q0 = (int)(b % q_blocks) * KNN_MQ;
+    const float *cp = pts + (size_t)cloud * P * D;
+    const int lane = fg_lane(), wave = fg_uni(fg_wave()), r16 = lane & 15, kq = lane >> 4;
+    float2 *list = lists + wave * KNN_CAP;
+    float pd[4];                                // the lists of the wave's queries q0 + 16 (a / 2) + 2 wave + a % 2
+    int pi[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) { pd[a] = INFINITY; pi[a] = min(q0 + (a / 2) * 16 + 2 * wave + a % 2, P - 1); }
+
+    // 4 floats of a row from dimension d0 + 4 kq on, zero past the end.  WHOLE: D is a multiple of 16 and rows start on 16 bytes; one
+    // bounds-checked load (rows past the cloud read as zero) then needs no test of its own.
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(cp), 0, WHOLE ? P * D * 4 : 0, 0x00027000);
+    const int lane_off = (r16 * D + 4 * kq) * 4;
+    auto frag = [&](int row0, bool one_row, int d0) {          // row row0 + r16, or row row0 in all lanes
+        if constexpr (WHOLE) {
+            return __builtin_bit_cast(knn_f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (one_row ? 16 * kq : lane_off) + (row0 * D + d0) * 4, 0, 0));
+        } else {
+            const int d = d0 + 4 * kq;
+            const float *src = cp + (size_t)min(row0 + (one_row ? 0 : r16), P - 1) * D + d;
+            knn_f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) if (d + u < D) v[u] = src[u];
+            return v;
+        }
+    };
+    for (int tile0 = 0; tile0 < P; tile0 += TILE) {
+        knn_f4 acc[NT][2];
+        float nrm[NT], qn[2] = {0.f, 0.f};
+        const int crow = tile0 + wave * NT * 16;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            acc[t][0] = acc[t][1] = knn_f4{0.f, 0.f, 0.f, 0.f};
+            nrm[t] = 0.f;
+        }
+        for (int d0 = 0; d0 < D; d0 += 16) {
+            const knn_f4 m = frag(q0, true, d0), b0 = frag(q0, false, d0) - m, b1 = frag(q0 + 16, false, d0) - m;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) { qn[0] = fmaf(b0[u], b0[u], qn[0]); qn[1] = fmaf(b1[u], b1[u], qn[1]); }
+#pragma unroll
+            for (int h = 0; h < NT; h += NH) {          // at most 4 tiles of operands in registers
+                knn_f4 a[NH];
+#pragma unroll
+                for (int t = 0; t < NH; ++t) a[t] = frag(crow + (h + t) * 16, false, d0);
+#pragma unroll
+                for (int t = 0; t < NH; ++t) {
+                    a[t] -= m;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) nrm[h + t] = fmaf(a[t][u], a[t][u], nrm[h + t]);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int t = 0; t < NH; ++t) {
+                        acc[h + t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][u], b0[u], acc[h + t][0], 0, 0, 0);
+                        acc[h + t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][u], b1[u], acc[h + t][1], 0, 0, 0);
+                    }
+            }
+        }
+        // lane (r, q) holds a quarter of the norms of row r: add the quarters up
+        auto quarters = [&](float v) {
+            v += __uint_as_float(knn_xor<16>(__float_as_uint(v), lane));
+            return v + __uint_as_float(knn_xor<32>(__float_as_uint(v), lane));
+        };
+        auto sane = [](float v) { return v < 1e37f ? v : INFINITY; };             // overflow or NaN: the bound becomes infinite
+        qn[0] = quarters(qn[0]);
+        qn[1] = quarters(qn[1]);
+        float mx = 0.f;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const float n = quarters(nrm[t]);
+            if (crow + t * 16 + r16 < P) mx = fmaxf(mx, sane(n));
+            if (kq == 0) cn[(wave * NT + t) * 16 + r16] = n;
+        }
+        mx = fg_wave_max(mx);
+        if (lane == 0) wmax[wave] = mx;
+        fg_wave_lds_sync();                     // a wave reads only the norms that it wrote
+        auto select16 = [&](auto group) {
+            constexpr int gq = decltype(group)::value;
+            const float qg = qn[gq];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int c = (wave * NT + t) * 16 + 4 * kq;                      // the product's rows 4 kq .. 4 kq + 3, column r16
+                const knn_f4 n4 = *reinterpret_cast<const knn_f4 *>(&cn[c]);
+                *reinterpret_cast<knn_f4 *>(&buf[r16 * ROW + c]) = (n4 - 2.f * acc[t][gq]) + qg;
+            }
+            __syncthreads();
+            float cmax = wmax[0];
+#pragma unroll
+            for (int w = 1; w < KNN_MW; ++w) cmax = fmaxf(cmax, wmax[w]);
+#pragma unroll 1
+            for (int j = 0; j < 2; ++j) {
+                const int ql = 2 * wave + j, q = min(q0 + gq * 16 + ql, P - 1);
+                float hd[1] = {j ? pd[2 * gq + 1] : pd[2 * gq]};
+                int hi[1] = {j ? pi[2 * gq + 1] : pi[2 * gq]};
+                float *row = &buf[ql * ROW + lane * 4];
+                float dist[NR];
+                auto fetch = [&]() {
+#pragma unroll
+                    for (int g = 0; g < RG; ++g) {
+                        const knn_f4 v = *reinterpret_cast<const knn_f4 *>(row + g * 256);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) dist[4 * g + u] = tile0 + g * 256 + lane * 4 + u < P ? v[u] : INFINITY;
+                    }
+                };
+                fetch();
+                const float S = sane(fg_readlane(qg, ql)) + cmax;
+                const float E = (float)(4 * D + 32) * 0x1p-23f * S + (float)(D + 1) * 1e-36f;
+                const float tau = knn_threshold<NR>(hd[0], k, lane, [&](int from, int to) {
+                    float m = dist[from];
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) if (r > from && r < to) m = fminf(m, dist[r]);
+                    return m;
+                });
+                const float lim = tau + 2.f * E;
+                int cnt = 0;
+                auto put = [&](bool in, float d, int i) {
+                    const unsigned long long m = __ballot(in);
+                    const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                    if (in && pos < KNN_CAP) list[pos] = make_float2(d, __int_as_float(i));
+                    cnt += __popcll(m);
+                };
+                if (tile0) put(hd[0] <= lim, hd[0], hi[0]);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) put(dist[r] <= lim, dist[r], tile0 + (r / 4) * 256 + lane * 4 + (r % 4));
+                fg_wave_lds_sync();
+                if (lim < INFINITY && cnt <= 64 && P <= TILE) {
+                    const float2 e = lane < cnt ? list[lane] : make_float2(INFINITY, __int_as_float(0x7fffffff));
+                    float cd = e.x;
+                    int ci = __float_as_int(e.y);
+                    KNN_SORT_64(cd, ci, lane);
+                    const float before = fg_bperm(cd, lane ? lane - 1 : 0), after = fg_bperm(cd, lane < 63 ? lane + 1 : 63);
+                    const bool near = lane < cnt && ((lane && cd - before <= 2.f * E) || (lane + 1 < cnt && after - cd <= 2.f * E));
+                    if (__ballot(near)) {
+                        if (near) cd = knn_exact(cp, D, q, ci, rows_aligned);
+                        KNN_SORT_64(cd, ci, lane);
+                    }
+                    hd[0] = lane < k ? cd : INFINITY;
+                    hi[0] = lane < k ? ci : q;
+                } else if (lim < INFINITY && cnt <= KNN_CAP) {
+                    for (int e = lane; e < cnt; e += 64) list[e].x = knn_exact(cp, D, q, __float_as_int(list[e].y), rows_aligned);
+                    fg_wave_lds_sync();
+                    float cd;
+                    int ci;
+                    knn_order(list, cnt, lane, cd, ci);
+                    hd[0] = lane < k ? cd : INFINITY;
+                    hi[0] = lane < k ? ci : q;
+                } else {
+                    _Pragma("unroll 1") for (int r = 0; r < NR; ++r) {
+                        const int c = tile0 + (r / 4) * 256 + lane * 4 + (r % 4);
+                        float &v = row[(r / 4) * 256 + r % 4];
+                        v = c < P && !(v > lim) ? knn_exact(cp, D, q, c, rows_aligned) : INFINITY;
+                    }
+                    fg_wave_lds_sync();
+                    fetch();
+                    knn_select<NR>(dist, tile0, hd, hi, k, lane, q, list);
+                }
+                if (j) { pd[2 * gq + 1] = hd[0]; pi[2 * gq + 1] = hi[0]; }
+                else { pd[2 * gq] = hd[0]; pi[2 * gq] = hi[0]; }
+                fg_wave_lds_sync();
+            }
+            __syncthreads();                    // the rows have been read
+        };
+        select16(std::integral_constant<int, 0>());
+        select16(std::integral_constant<int, 1>());
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const int q = q0 + (a / 2) * 16 + 2 * wave + a % 2;
+        if (q < P && lane < k) out[((size_t)cloud * P + q) * k + lane] = cloud * P + pi[a];
+    }
+}
+
+template <int RG>
+static void knn_mfma_launch(int n_clouds, int P, int D, int k, const float *points, int32_t *src_ind, hipStream_t st)
+{
+    const unsigned q_blocks = (unsigned)((P + KNN_MQ - 1) / KNN_MQ), n_blocks = q_blocks * (unsigned)n_clouds;
+    unsigned grid = n_blocks, per_xcd = 0;
+    if (grid >= 8 * FGNN_NUM_XCD && fgnn_current_device_has_xcd_mapping()) {      // a cloud is read through one XCD's L2
+        per_xcd = (grid + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD;
+        grid = per_xcd * FGNN_NUM_XCD;
+    }
+    const int rows_aligned = D % 4 == 0 && fgnn_aligned16(points) ? 1 : 0;
+    if (rows_aligned && D % 16 == 0 && (int64_t)P * D * 4 <= 0x7fffffff)
+        hipLaunchKernelGGL((knn_mfma_kernel<RG, true>), dim3(grid), dim3(KNN_MW * 64), 0, st, P, D, k, 1, per_xcd, q_blocks, n_blocks, points, src_ind);
+    else
+        hipLaunchKernelGGL((knn_mfma_kernel<RG, false>), dim3(grid), dim3(KNN_MW * 64), 0, st, P, D, k, rows_aligned, per_xcd, q_blocks, n_blocks, points,
+                           src_ind);
+}
+
 template <int RG, int KR>
 static void knn_launch(int n_clouds, int P, int D, int k, const float *points, int32_t *src_ind, hipStream_t st)
 {
@@ -334,7 +579,13 @@ extern "C" int fgnn_knn_graph(int n_clouds, int P, int D, int k, const float *po
     if (n_clouds == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     const int rg = P <= 256 ? 1 : P <= 512 ? 2 : 4;     // tile = 256 * rg candidate points
-    if (k <= 64) {
+    // The matrix form costs less per dimension (64 clouds: 1.4 against 4 us at 1024 points, 0.5 against 0.8 at 512) and more per query
+    // (140 against 115 us, 44 against 30): equal at 10 to 16 and at 45 dimensions.  At 256 points it loses up to 128 dimensions
+    // (46 against 44 us; 34 against 29 at 64).
+    if (k <= 64 && ((rg == 4 && D >= 16) || (rg == 2 && D >= 48))) {
+        if (rg == 2) knn_mfma_launch<2>(n_clouds, P, D, k, points, src_ind, st);
+        else knn_mfma_launch<4>(n_clouds, P, D, k, points, src_ind, st);
+    } else if (k <= 64) {
         if (rg == 1) knn_launch<1, 1>(n_clouds, P, D, k, points, src_ind, st);
         else if (rg == 2) knn_launch<2, 1>(n_clouds, P, D, k, points, src_ind, st);
         else knn_launch<4, 1>(n_clouds, P, D, k, points, src_ind, st);

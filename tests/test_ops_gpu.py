@@ -672,6 +672,32 @@ def test_knn_selection_at_its_limits(p, k):
     assert torch.equal(src, want)
 
 
+@pytest.mark.parametrize("p,d", [(512, 48), (300, 64), (257, 130), (513, 16), (600, 31), (1000, 17), (1024, 64), (1024, 100), (1025, 16), (2100, 36)])
+@pytest.mark.parametrize("k", [1, 20, 40, 64])
+def test_knn_graph_in_many_dimensions(p, d, k):
+    """Integer coordinates make every squared distance exact, so the ids are fixed by the (distance, id) order: many ties, a common
+    offset, an outlier that widens the filter's bound, points that are all the same, and coordinates that are no numbers."""
+    from ae_mlsys_gnn_amd.operators.knn import knn_graph
+    gen = torch.Generator().manual_seed(p * 1000 + d + k)
+    grid = torch.randint(0, 3, (p, d), generator=gen).float()
+    wide = torch.randint(-40, 41, (p, d), generator=gen).float()
+    outlier = grid.clone()
+    outlier[p // 3] = 200.0             # 130 * 200^2 < 2^24: every partial sum is a whole number that fp32 holds
+    broken = wide.clone()
+    broken[p // 2, 0], broken[p // 5, d - 1] = float("nan"), float("inf")
+    pts = torch.stack([grid, wide + 4096.0, outlier, torch.ones(p, d), broken])
+    src = knn_graph(pts.to(DEV), k).cpu().long().view(5, p, k)
+    for c in range(5):
+        x = pts[c].double()
+        clean = torch.nan_to_num(x, nan=0.0, posinf=0.0)
+        dist = torch.cdist(clean, clean, compute_mode="donot_use_mm_for_euclid_dist").square().round()      # whole numbers below 2^53
+        bad = ~torch.isfinite(x).all(1)
+        dist[bad] = 2.0 ** 40           # distances that are infinite or no numbers share the last place
+        dist[:, bad] = 2.0 ** 40
+        want = torch.argsort(dist * 4096 + torch.arange(p, dtype=torch.float64), dim=1)[:, :k] + c * p
+        assert torch.equal(src[c], want), (c, p, d, k)
+
+
 def test_knn_graph_feeds_edgeconv():
     from ae_mlsys_gnn_amd.layers import EdgeConv
     from ae_mlsys_gnn_amd.operators.knn import knn_graph
