@@ -6,8 +6,8 @@ import torch as th
 from torch import nn
 from torch.nn import init
 
-from ..operators.fused_gmmconv import (GmmAggregate, GmmAggregateTwoOrders, GmmConvFuseSum, GmmConvFuseSumTwoOrders, GmmConvStash,
-                                        GmmConvStashSumTwoOrders, gmm_native)
+from ..operators.fused_gmmconv import (GmmAggregate, GmmAggregateLinear, GmmAggregateTwoOrders, GmmConvFuseSum, GmmConvFuseSumTwoOrders, GmmConvStash,
+                                        GmmConvStashSumTwoOrders, gmm_native, project_in_backward)
 from .dense import add_bias, tall_linear
 
 
@@ -105,6 +105,11 @@ class _GMMBase(nn.Module):
         if pseudo_csc is not None or own_order:
             if own_order and pseudo_csc is None and th.is_grad_enabled() and (feat.requires_grad or pseudo.requires_grad):
                 raise ValueError("own_order without pseudo_csc is forward-only")
+        two = pseudo_csc is not None
+        if th.is_grad_enabled() and (two or not own_order) and project_in_backward(k, fin, fout, feat.requires_grad):
+            return GmmAggregateLinear(rowptr, colind, colptr, rowind, None if two else permute, feat, pseudo.detach() if two else pseudo, pseudo_csc,
+                                      self.mu, self.inv_sigma, self.fc.weight, own_order=own_order)
+        if two or own_order:
             agg = GmmAggregateTwoOrders(rowptr, colind, colptr, rowind, feat, pseudo.detach(), pseudo_csc, self.mu, self.inv_sigma,
                                         own_order=own_order)
         else:

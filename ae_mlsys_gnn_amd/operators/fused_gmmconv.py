@@ -333,6 +333,57 @@ class GmmAggregateTwoOrdersFunction(torch.autograd.Function):
         return None, None, None, None, grad_feat, None, grad_pseudo_csc, grad_mu, grad_sigma, None
 
 
+def project_in_backward(k, fin, fout, input_grad):
+    """Which rows the backward of an aggregate-first layer gathers per edge: K x fin floats, the gradient of the aggregate, or the
+    fout floats (rounded up to 4) of the layer's own gradient, for the price of projecting the input again (and of one more
+    product for the input's gradient).  Layer steps, gathering K x fin / fout floats: 169 k nodes, 2.3 M edges, 384 / 64 floats 1.69 ->
+    1.01 ms (1.16 with the input's gradient), 128 / 64 0.76 -> 0.68 (0.74), 96 / 44 0.66 -> 0.66 (0.69), 128 / 84 0.78 -> 0.89 ms (0.99);
+    300 k nodes, 0.9 M edges, 256 / 100 floats 1.53 -> 1.49 (1.70): the lines lie at ratios of 2 and 3."""
+    return k * fin >= (3 if input_grad else 2) * ((fout + 3) // 4 * 4)
+
+
+def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order=False):
+    """sum_k (sum_p w[p,k] * feat[colind[p],:]) @ W_k for feat [N, in] and the fc weight [K*out, in]: [N, out].  The forward aggregates the
+    input (an edge gathers `in` floats); the backward takes the other order of the two linear steps, so an edge gathers the `out`
+    floats of the gradient: T[j,k,:] = sum_p w[p,k] * g[row(p),:] is the gradient of feat @ W_k^T, the derivatives of the Gaussian weights
+    need <g[row(p),:], (feat @ W_k^T)[j,:]>, and the projection is formed again.  Nothing as wide as K x in is kept.
+    pseudo_csc, own_order: as GmmConvFuseSumTwoOrders; pseudo_csc None: one copy, through permute."""
+    return GmmAggregateLinearFunction.apply(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order)
+
+
+class GmmAggregateLinearFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order):
+        k, fin = mu.shape[0], feat.shape[1]
+        fout = weight.shape[0] // k
+        agg = gmm_native.gmmconv_shared(rowptr, colind, feat, pseudo, mu, sigma, own_order=own_order)
+        w = weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)
+        ctx.two_orders, ctx.own_order = pseudo_csc is not None, own_order
+        ctx.save_for_backward(colptr, rowind, None if ctx.two_orders else permute, feat, pseudo_csc if ctx.two_orders else pseudo, mu, sigma, weight)
+        return torch.matmul(agg.view(-1, k * fin), w.t())
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        from ..layers.dense import reduce_over_rows
+        colptr, rowind, permute, feat, pseudo, mu, sigma, weight = ctx.saved_tensors
+        k, fin = mu.shape[0], feat.shape[1]
+        fout = weight.shape[0] // k
+        pad = (-fout) % 4
+        if pad:         # zero columns up to a multiple of 4: the operator then takes its 128-bit row layout
+            weight = torch.nn.functional.pad(weight.view(k, fout, fin), (0, 0, 0, pad)).view(-1, fin)
+            grad_out = torch.nn.functional.pad(grad_out, (0, pad))
+        proj = torch.matmul(feat, weight.t()).view(-1, k, fout + pad)
+        t, grad_pseudo, grad_mu, grad_sigma = gmm_native.gmmconv_backward(colptr, rowind, permute, proj, pseudo, mu, sigma, grad_out.contiguous(),
+                                                                          sum_kernels=True, own_order=ctx.own_order)
+        t = t.view(-1, k * (fout + pad))
+        grad_feat = torch.matmul(t, weight) if ctx.needs_input_grad[5] else None
+        grad_w = reduce_over_rows(t, feat) if ctx.needs_input_grad[10] else None
+        if pad and grad_w is not None:
+            grad_w = grad_w.view(k, fout + pad, fin)[:, :fout].reshape(-1, fin)
+        gp = (None, grad_pseudo) if ctx.two_orders else (grad_pseudo, None)
+        return (None, None, None, None, None, grad_feat) + gp + (grad_mu, grad_sigma, grad_w, None)
+
+
 class GmmFuseSumFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, rowptr, colind, colptr, rowind, permute, node_feat, pseudo, mu, sigma, bias=None, residual=None):

@@ -331,6 +331,48 @@ def test_gmm_layer_matches_dgl_composed(fin, fout, k, dim, variant, agg_first):
         assert_close_sum(got, want, s[key], "GMMConv grad " + name, c=c)
 
 
+@pytest.mark.parametrize("fin,fout,k,dim", [(48, 16, 3, 2), (32, 31, 2, 1), (128, 64, 3, 2), (32, 9, 1, 3), (256, 100, 4, 1)])
+@pytest.mark.parametrize("form", ["permute", "two_orders", "own_order"])
+@pytest.mark.parametrize("input_grad", [False, True])
+def test_gmm_aggregate_linear(fin, fout, k, dim, form, input_grad):
+    """The aggregate-first layer whose backward gathers the layer's own gradient: every output against autograd through the
+    float64 composed layer, on either side of the rule, with one copy of the coordinates and with one per direction."""
+    from ae_mlsys_gnn_amd.operators import fused_gmmconv as fg
+    gen = torch.Generator().manual_seed(fin + fout)
+    g = graphs.add_csc_torch(graphs.rmat_graph(700, 9000, seed=4))
+    gd = g.to(DEV)
+    x, pseudo, go = torch.randn(g.n, fin, generator=gen), torch.rand(g.n_edges, dim, generator=gen), torch.randn(g.n, fout, generator=gen)
+    w, mu, isg = torch.randn(k * fout, fin, generator=gen), torch.rand(k, dim, generator=gen), 0.5 + torch.rand(k, dim, generator=gen)
+    zero = torch.zeros(fout, dtype=torch.float64)
+    leaves = [t.double().requires_grad_(True) for t in (w, mu, isg, x, pseudo)]
+    ref = orc.gmm_layer_dgl(leaves[0], leaves[1], leaves[2], zero, g.row_ptr, g.col_ind, leaves[3], leaves[4], torch.zeros(fout, fin, dtype=torch.float64))
+    ref.backward(go.double())
+    wd, md, sd, xd = (t.to(DEV).requires_grad_(True) for t in (w, mu, isg, x))
+    xd = xd if input_grad else xd.detach()
+    if form == "permute":
+        pd = pseudo.to(DEV).requires_grad_(True)
+        order = torch.arange(g.n_edges, device=DEV)
+        out = fg.GmmAggregateLinear(gd.row_ptr, gd.col_ind, gd.col_ptr, gd.row_ind, gd.permute, xd, pd, None, md, sd, wd)
+    else:
+        own = form == "own_order"
+        pos_r = fg.gmm_edge_positions(gd.row_ptr, gd.col_ind) if own else None
+        pos_c = fg.gmm_edge_positions(gd.col_ptr, gd.row_ind, True) if own else None
+        order = gd.permute.long() if pos_c is None else gd.permute[pos_c.long()].long()
+        fwd = pseudo.to(DEV) if pos_r is None else pseudo.to(DEV)[pos_r.long()].contiguous()
+        pd = pseudo.to(DEV)[order].contiguous().requires_grad_(True)
+        out = fg.GmmAggregateLinear(gd.row_ptr, gd.col_ind, gd.col_ptr, gd.row_ind, None, xd, fwd, pd, md, sd, wd, own_order=own)
+    out.backward(go.to(DEV))
+    d = [t.detach() for t in leaves]
+    s = orc.gmm_layer_abs_sums(d[0], d[1], d[2], zero, g.row_ptr, g.col_ind, d[3], d[4], torch.zeros(fout, fin, dtype=torch.float64), go.double())
+    c = _gmm_c(d[4], d[1], d[2])
+    assert_close_sum(out, ref.detach(), s["out"], "out", c=c)
+    if input_grad:
+        assert_close_sum(xd.grad, leaves[3].grad, s["grad_feat"], "grad feat", c=c)
+    assert_close_sum(pd.grad, leaves[4].grad[order.cpu()], s["grad_pseudo"][order.cpu()], "grad pseudo", c=c)
+    for name, got, want, key in (("fc", wd, leaves[0], "grad_fc"), ("mu", md, leaves[1], "grad_mu"), ("inv_sigma", sd, leaves[2], "grad_sigma")):
+        assert_close_sum(got.grad, want.grad, s[key], "grad " + name, c=c)
+
+
 # ------------------------------------------------------------------ GAT layer vs the DGL-composed layer
 @pytest.mark.parametrize("fin,f,h,variant", [(64, 16, 4, "our"), (30, 47, 1, "our"), (30, 47, 1, "stash"), (20, 6, 3, "fusescatter"),
                                              (12, 128, 1, "our")])
