@@ -56,6 +56,8 @@ _SIGNATURES = {
     "fgnn_edgeconv_forward_lrelu": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 3 + [c_float] + [c_void_p] * 2 + [c_void_p]),
     "fgnn_edgeconv_backward_lrelu": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float] + [c_void_p] * 3
                                      + [c_void_p, c_size_t, c_void_p]),
+    "fgnn_edgeconv_pair_forward": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p]),
+    "fgnn_edgeconv_pair_backward": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "fgnn_edgeconv_backward_blocked_workspace_bytes": (c_size_t, [c_int, c_int]),
     "fgnn_edgeconv_backward_blocked": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 4 + [c_size_t, c_void_p]),
     "fgnn_edgeconv_backward_blocked_static_max_elems": (c_size_t, []),

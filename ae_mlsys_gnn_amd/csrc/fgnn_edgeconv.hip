@@ -15,9 +15,11 @@
 // per_xcd > 0: the workgroups of one XCD (blockIdx.x % FGNN_NUM_XCD) take one contiguous eighth of the nodes.  The neighbours of
 // a node of a batched kNN graph lie in its own cloud; with the workgroups dealt round-robin every XCD gathered from every
 // cloud and the feature matrix crossed the fabric eight times (106 MB fetched for 32 clouds of 1024 points x 64 floats).
+// ld: floats between the rows of h_src and of h_dst.  diff: the destination's term is h_dst[i] - h_src[i] (the layer's phi(x) -
+// theta(x), formed here instead of in a pass of its own).  argmax NULL: nobody will run the backward.
 template <int VEC>
 __global__ __launch_bounds__(256) void edgeconv_fwd_kernel(int N, int F, int k, unsigned per_xcd, const int *__restrict__ src_ind,
-                                                           const float *__restrict__ h_src, const float *__restrict__ h_dst,
+                                                           const float *__restrict__ h_src, const float *__restrict__ h_dst, int ld, int diff,
                                                            float out_slope, float *__restrict__ out, int *__restrict__ argmax)
 {
     const int per = F / VEC;
@@ -27,7 +29,15 @@ __global__ __launch_bounds__(256) void edgeconv_fwd_kernel(int N, int F, int k, 
     const int node = (int)(tid / per);
     const int fo = (int)(tid - (long long)node * per) * VEC;
     fg_vec<VEC> d;
-    d.load(h_dst + (size_t)node * F + fo);
+    d.load(h_dst + (size_t)node * ld + fo);
+    if (diff) {
+        fg_vec<VEC> own;
+        own.load(h_src + (size_t)node * ld + fo);
+        float *dv = reinterpret_cast<float *>(&d);
+        const float *ov = reinterpret_cast<const float *>(&own);
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) dv[c] -= ov[c];
+    }
     const int *nb = src_ind + (size_t)node * k;
     float best[VEC];
     int arg[VEC];
@@ -44,10 +54,10 @@ __global__ __launch_bounds__(256) void edgeconv_fwd_kernel(int N, int F, int k, 
     for (; t + 4 <= k; t += 4) {
         int j0 = nb[t], j1 = nb[t + 1], j2 = nb[t + 2], j3 = nb[t + 3];
         fg_vec<VEC> s0, s1, s2, s3;
-        s0.load(h_src + (size_t)j0 * F + fo);
-        s1.load(h_src + (size_t)j1 * F + fo);
-        s2.load(h_src + (size_t)j2 * F + fo);
-        s3.load(h_src + (size_t)j3 * F + fo);
+        s0.load(h_src + (size_t)j0 * ld + fo);
+        s1.load(h_src + (size_t)j1 * ld + fo);
+        s2.load(h_src + (size_t)j2 * ld + fo);
+        s3.load(h_src + (size_t)j3 * ld + fo);
         consider(j0, s0, t == 0);
         consider(j1, s1, false);
         consider(j2, s2, false);
@@ -56,14 +66,14 @@ __global__ __launch_bounds__(256) void edgeconv_fwd_kernel(int N, int F, int k, 
     for (; t < k; ++t) {
         int j = nb[t];
         fg_vec<VEC> s;
-        s.load(h_src + (size_t)j * F + fo);
+        s.load(h_src + (size_t)j * ld + fo);
         consider(j, s, t == 0);
     }
 #pragma unroll
     for (int c = 0; c < VEC; ++c) {
         // optional LeakyReLU on the way out (out_slope == 1: the identity, bit for bit)
         out[(size_t)node * F + fo + c] = best[c] > 0.f ? best[c] : best[c] * out_slope;
-        argmax[(size_t)node * F + fo + c] = arg[c];
+        if (argmax) argmax[(size_t)node * F + fo + c] = arg[c];
     }
 }
 
@@ -86,14 +96,26 @@ __device__ __forceinline__ float ec_masked(float g, const float *act_out, float 
 }
 __global__ __launch_bounds__(256) void edgeconv_bwd_kernel(long long total, int F, const int *__restrict__ argmax,
                                                            const float *__restrict__ grad_out, const float *__restrict__ act_out, float act_slope,
-                                                           float *__restrict__ grad_src, float *__restrict__ grad_dst)
+                                                           float *__restrict__ grad_src, float *__restrict__ grad_dst, int ld)
 {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
     int f = (int)(i % F);
     const float g = ec_masked(grad_out[i], act_out, act_slope, i);
     if (grad_dst) grad_dst[i] = g;
-    unsafeAtomicAdd(grad_src + (size_t)argmax[i] * F + f, g);     // hardware float add (device memory), no CAS loop
+    unsafeAtomicAdd(grad_src + (size_t)argmax[i] * ld + f, g);    // hardware float add (device memory), no CAS loop
+}
+
+// grad_h [N, 2F] before the scatter of the layer's form: -g in the half of theta, g in that of phi.
+__global__ __launch_bounds__(256) void edgeconv_pair_init_kernel(long long total, int F, const float *__restrict__ grad_out, const float *__restrict__ act_out,
+                                                                 float act_slope, float *__restrict__ grad_h)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= total) return;
+    const long long r = i / F;
+    const float g = ec_masked(grad_out[i], act_out, act_slope, i);
+    grad_h[r * 2 * F + (i - r * F)] = -g;
+    grad_h[r * 2 * F + F + (i - r * F)] = g;
 }
 
 int fgnn_fill_f32(float *p, size_t n, float v, hipStream_t st)
@@ -106,10 +128,10 @@ int fgnn_fill_f32(float *p, size_t n, float v, hipStream_t st)
 }
 
 static int edgeconv_forward_run(const char *fn, int N, int n_src, int F, int k, const int32_t *src_ind, const float *h_src,
-                                const float *h_dst, float out_slope, float *out, int32_t *argmax, void *stream)
+                                const float *h_dst, int ld, int diff, float out_slope, float *out, int32_t *argmax, void *stream)
 {
     FGNN_REQUIRE(N >= 0 && n_src >= 0 && F >= 1 && k >= 1, FGNN_ERR_SHAPE, "%s: bad sizes N=%d n_src=%d F=%d k=%d", fn, N, n_src, F, k);
-    FGNN_REQUIRE(src_ind && h_src && h_dst && out && argmax, FGNN_ERR_NULL, "%s: NULL argument", fn);
+    FGNN_REQUIRE(src_ind && h_src && h_dst && out && (argmax || diff), FGNN_ERR_NULL, "%s: NULL argument", fn);
     FGNN_REQUIRE((int64_t)N * k <= 2147483647LL, FGNN_ERR_LIMIT, "%s: N*k exceeds int32", fn);
     if (N == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
@@ -121,15 +143,15 @@ static int edgeconv_forward_run(const char *fn, int N, int n_src, int F, int k, 
         per_xcd = (grid + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD;
         grid = per_xcd * FGNN_NUM_XCD;
     }
-    if (v4) hipLaunchKernelGGL(edgeconv_fwd_kernel<4>, dim3(grid), dim3(256), 0, st, N, F, k, per_xcd, src_ind, h_src, h_dst, out_slope, out, argmax);
-    else hipLaunchKernelGGL(edgeconv_fwd_kernel<1>, dim3(grid), dim3(256), 0, st, N, F, k, per_xcd, src_ind, h_src, h_dst, out_slope, out, argmax);
+    if (v4) hipLaunchKernelGGL(edgeconv_fwd_kernel<4>, dim3(grid), dim3(256), 0, st, N, F, k, per_xcd, src_ind, h_src, h_dst, ld, diff, out_slope, out, argmax);
+    else hipLaunchKernelGGL(edgeconv_fwd_kernel<1>, dim3(grid), dim3(256), 0, st, N, F, k, per_xcd, src_ind, h_src, h_dst, ld, diff, out_slope, out, argmax);
     return fgnn_launch_status("edgeconv_fwd_kernel");
 }
 
 extern "C" int fgnn_edgeconv_forward(int N, int n_src, int F, int k, const int32_t *src_ind, const float *h_src,
                                      const float *h_dst, float *out, int32_t *argmax, void *stream)
 {
-    return edgeconv_forward_run("fgnn_edgeconv_forward", N, n_src, F, k, src_ind, h_src, h_dst, 1.f, out, argmax, stream);
+    return edgeconv_forward_run("fgnn_edgeconv_forward", N, n_src, F, k, src_ind, h_src, h_dst, F, 0, 1.f, out, argmax, stream);
 }
 
 extern "C" int fgnn_edgeconv_forward_lrelu(int N, int n_src, int F, int k, const int32_t *src_ind, const float *h_src,
@@ -137,7 +159,18 @@ extern "C" int fgnn_edgeconv_forward_lrelu(int N, int n_src, int F, int k, const
 {
     FGNN_REQUIRE(out_slope > 0.f, FGNN_ERR_LIMIT, "fgnn_edgeconv_forward_lrelu: out_slope=%g; the backward reads the sign of the pre-activation "
                  "off the output, which needs a positive slope", (double)out_slope);
-    return edgeconv_forward_run("fgnn_edgeconv_forward_lrelu", N, n_src, F, k, src_ind, h_src, h_dst, out_slope, out, argmax, stream);
+    return edgeconv_forward_run("fgnn_edgeconv_forward_lrelu", N, n_src, F, k, src_ind, h_src, h_dst, F, 0, out_slope, out, argmax, stream);
+}
+
+// The layer's form: h [N, 2F] holds theta(x) and phi(x) of every node side by side, as one product leaves them.  Reading it in place
+// saves the copy of one half and the difference of both (two passes of 4 N F and 6 N F bytes and their launches); without argmax, in
+// inference, a third of what the kernel writes and reads beside the gathered rows.
+extern "C" int fgnn_edgeconv_pair_forward(int N, int F, int k, const int32_t *src_ind, const float *h, float out_slope, float *out, int32_t *argmax,
+                                          void *stream)
+{
+    FGNN_REQUIRE(out_slope > 0.f, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_forward: out_slope=%g must be positive (1: no activation)", (double)out_slope);
+    FGNN_REQUIRE(F >= 1 && F <= (1 << 28), FGNN_ERR_SHAPE, "fgnn_edgeconv_pair_forward: bad sizes F=%d", F);
+    return edgeconv_forward_run("fgnn_edgeconv_pair_forward", N, N, F, k, src_ind, h, h ? h + F : nullptr, 2 * F, 1, out_slope, out, argmax, stream);
 }
 
 // fn: the entry point the caller used, for the error messages
@@ -152,7 +185,7 @@ static int edgeconv_backward_run(const char *fn, int N, int n_src, int F, const 
     long long total = (long long)N * F;
     if (total == 0) return 0;
     unsigned grid = (unsigned)((total + 255) / 256);
-    hipLaunchKernelGGL(edgeconv_bwd_kernel, dim3(grid), dim3(256), 0, st, total, F, argmax, grad_out, act_out, act_slope, grad_src, grad_dst);
+    hipLaunchKernelGGL(edgeconv_bwd_kernel, dim3(grid), dim3(256), 0, st, total, F, argmax, grad_out, act_out, act_slope, grad_src, grad_dst, F);
     return fgnn_launch_status("edgeconv_bwd_kernel");
 }
 
@@ -176,11 +209,13 @@ extern "C" int fgnn_edgeconv_backward(int N, int n_src, int F, const int32_t *ar
 // n_tiles > 0: a one-dimensional grid in which the n_tiles column tiles of a block all run on one XCD (workgroup w runs on XCD
 // w % FGNN_NUM_XCD): a tile row is FS * 4 = 32 bytes of a 128-byte line of grad_out and argmax, and with the tiles of a block
 // spread over the XCDs every line crossed the fabric once per XCD that held one of its four tiles (67 MB fetched for 16.8 MB).
+// ld: floats between the rows of grad_src and of grad_dst.  diff: the forward took h_dst - h_src as the destination's term, so
+// grad_src loses what grad_dst gets.
 template <int FS>
 __global__ __launch_bounds__(EC_BT) void edgeconv_bwd_blocked_kernel(int N, int F, int block, int n_tiles, const int *__restrict__ argmax,
                                                                      const float *__restrict__ grad_out, const float *__restrict__ act_out,
-                                                                     float act_slope, float *__restrict__ grad_src, float *__restrict__ grad_dst,
-                                                                     int *__restrict__ ovf)
+                                                                     float act_slope, float *__restrict__ grad_src, float *grad_dst,
+                                                                     int ld, int diff, int *__restrict__ ovf)
 {
     extern __shared__ float tile[];                 // [rows of the block][FS]
     int b = (int)blockIdx.y, tx = (int)blockIdx.x;
@@ -208,7 +243,7 @@ __global__ __launch_bounds__(EC_BT) void edgeconv_bwd_blocked_kernel(int N, int 
             g[u] = (r0 + r) * F + f0 + ff;           // N*F < 2^31 is checked on the host
             a[u] = ok[u] ? argmax[g[u]] : 0;
             v[u] = ok[u] ? ec_masked(grad_out[g[u]], act_out, act_slope, g[u]) : 0.f;
-            if (ok[u] && grad_dst) grad_dst[g[u]] = v[u];
+            if (ok[u] && grad_dst) grad_dst[(size_t)(r0 + r) * ld + f0 + ff] = v[u];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -227,18 +262,21 @@ __global__ __launch_bounds__(EC_BT) void edgeconv_bwd_blocked_kernel(int N, int 
     __syncthreads();
     for (int i = (int)threadIdx.x; i < total; i += EC_BT) {
         const int r = i / FS, ff = i - r * FS;
-        if (ff < fs) grad_src[(size_t)(r0 + r) * F + f0 + ff] = tile[i];
+        if (ff < fs) {
+            const size_t o = (size_t)(r0 + r) * ld + f0 + ff;
+            grad_src[o] = diff ? tile[i] - grad_dst[o] : tile[i];       // this thread wrote grad_dst[o] above
+        }
     }
 }
 
 __global__ __launch_bounds__(256) void edgeconv_bwd_overflow_kernel(int F, const int *__restrict__ argmax, const float *__restrict__ grad_out,
                                                                     const float *__restrict__ act_out, float act_slope,
-                                                                    float *__restrict__ grad_src, const int *__restrict__ ovf)
+                                                                    float *__restrict__ grad_src, int ld, const int *__restrict__ ovf)
 {
     const int count = ovf[0];
     for (int i = (int)(blockIdx.x * 256 + threadIdx.x); i < count; i += (int)(gridDim.x * 256)) {
         const int g = ovf[EC_OVF_HEADER + i];
-        unsafeAtomicAdd(grad_src + (size_t)argmax[g] * F + (g % F), ec_masked(grad_out[g], act_out, act_slope, g));
+        unsafeAtomicAdd(grad_src + (size_t)argmax[g] * ld + (g % F), ec_masked(grad_out[g], act_out, act_slope, g));
     }
 }
 
@@ -252,8 +290,10 @@ static inline int ec_blocked_fs(int block) { return block <= 2048 ? 8 : block <=
 
 // The two launches of the blocked backward; ovf: (N*F + EC_OVF_HEADER) ints of device scratch.
 static int edgeconv_backward_blocked_run(int N, int F, int block, int fs, const int32_t *argmax, const float *grad_out, float *grad_src,
-                                         int *ovf, hipStream_t st, const float *act_out = nullptr, float act_slope = 1.f, float *grad_dst = nullptr)
+                                         int *ovf, hipStream_t st, const float *act_out = nullptr, float act_slope = 1.f, float *grad_dst = nullptr,
+                                         int ld = 0, int diff = 0)
 {
+    if (ld == 0) ld = F;
     int rc = fgnn_fill_f32((float *)ovf, 1, 0.f, st);        // the counter (bit pattern of 0.0f is integer 0); a kernel, so capturable
     if (rc) return rc;
     const long long n_tiles = (F + fs - 1) / fs, n_blocks = ((long long)N + block - 1) / block;
@@ -265,11 +305,11 @@ static int edgeconv_backward_blocked_run(int N, int F, int block, int fs, const 
         tiles_arg = (int)n_tiles;
     }
     const size_t shm = (size_t)block * fs * sizeof(float);
-    if (fs == 8) hipLaunchKernelGGL(edgeconv_bwd_blocked_kernel<8>, grid, dim3(EC_BT), shm, st, N, F, block, tiles_arg, argmax, grad_out, act_out, act_slope, grad_src, grad_dst, ovf);
-    else hipLaunchKernelGGL(edgeconv_bwd_blocked_kernel<4>, grid, dim3(EC_BT), shm, st, N, F, block, tiles_arg, argmax, grad_out, act_out, act_slope, grad_src, grad_dst, ovf);
+    if (fs == 8) hipLaunchKernelGGL(edgeconv_bwd_blocked_kernel<8>, grid, dim3(EC_BT), shm, st, N, F, block, tiles_arg, argmax, grad_out, act_out, act_slope, grad_src, grad_dst, ld, diff, ovf);
+    else hipLaunchKernelGGL(edgeconv_bwd_blocked_kernel<4>, grid, dim3(EC_BT), shm, st, N, F, block, tiles_arg, argmax, grad_out, act_out, act_slope, grad_src, grad_dst, ld, diff, ovf);
     rc = fgnn_launch_status("edgeconv_bwd_blocked_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(edgeconv_bwd_overflow_kernel, dim3(64), dim3(256), 0, st, F, argmax, grad_out, act_out, act_slope, grad_src, ovf);
+    hipLaunchKernelGGL(edgeconv_bwd_overflow_kernel, dim3(64), dim3(256), 0, st, F, argmax, grad_out, act_out, act_slope, grad_src, ld, ovf);
     return fgnn_launch_status("edgeconv_bwd_overflow_kernel");
 }
 
@@ -361,4 +401,28 @@ extern "C" int fgnn_edgeconv_backward_lrelu(int N, int n_src, int F, int block, 
                  workspace_bytes, need);
     if (N == 0) return 0;
     return edgeconv_backward_blocked_run(N, F, block, fs, argmax, grad_out, grad_src, (int *)workspace, (hipStream_t)stream, out, out_slope, grad_dst);
+}
+
+// Backward of fgnn_edgeconv_pair_forward: grad_h [N, 2F] in one pass over the gradient: phi's half is the (masked) gradient, theta's the
+// scattered gradient less it.  out NULL: the forward had no activation.
+extern "C" int fgnn_edgeconv_pair_backward(int N, int F, int block, const int32_t *argmax, const float *out, float out_slope, const float *grad_out,
+                                           float *grad_h, void *workspace, size_t workspace_bytes, void *stream)
+{
+    FGNN_REQUIRE(N >= 0 && F >= 1 && F <= (1 << 28), FGNN_ERR_SHAPE, "fgnn_edgeconv_pair_backward: bad sizes N=%d F=%d", N, F);
+    FGNN_REQUIRE(argmax && grad_out && grad_h, FGNN_ERR_NULL, "fgnn_edgeconv_pair_backward: NULL argument");
+    FGNN_REQUIRE(out_slope > 0.f, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_backward: out_slope=%g must be positive", (double)out_slope);
+    FGNN_REQUIRE((int64_t)N * F <= 2147483647LL, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_backward: N*F exceeds int32");
+    if (N == 0) return 0;
+    hipStream_t st = (hipStream_t)stream;
+    const int fs = block > 0 ? ec_blocked_fs(block) : 0;
+    if (fs == 0 || (size_t)block * fs * sizeof(float) > 64 * 1024) {
+        const long long total = (long long)N * F;
+        const unsigned grid = (unsigned)((total + 255) / 256);
+        hipLaunchKernelGGL(edgeconv_pair_init_kernel, dim3(grid), dim3(256), 0, st, total, F, grad_out, out, out_slope, grad_h);
+        hipLaunchKernelGGL(edgeconv_bwd_kernel, dim3(grid), dim3(256), 0, st, total, F, argmax, grad_out, out, out_slope, grad_h, nullptr, 2 * F);
+        return fgnn_launch_status("edgeconv_bwd_kernel");
+    }
+    const size_t need = fgnn_edgeconv_backward_blocked_workspace_bytes(N, F);
+    FGNN_REQUIRE(workspace && workspace_bytes >= need, FGNN_ERR_WORKSPACE, "fgnn_edgeconv_pair_backward: workspace %zu < %zu bytes", workspace_bytes, need);
+    return edgeconv_backward_blocked_run(N, F, block, fs, argmax, grad_out, grad_h, (int *)workspace, st, out, out_slope, grad_h + F, 2 * F, 1);
 }

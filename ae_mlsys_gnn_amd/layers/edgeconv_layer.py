@@ -4,7 +4,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from ..operators.fused_edgeconv import fused_edgeconv_op
+from ..operators.fused_edgeconv import fused_edgeconv_pair_op
 from .dense import tall_linear
 
 
@@ -29,10 +29,6 @@ class EdgeConv(nn.Module):
         negative_slope_out: apply LeakyReLU with this slope to the result inside the operator (the activation that
         follows every EdgeConv of the reference's DGCNN, script/train/train_edgeconv_our.py:56)."""
         # theta and phi read the same rows: one product with the stacked weights (its weight gradient
-        # reduced over the points in chunks), split afterwards
-        out_feat = self.theta.out_features
+        # reduced over the points in chunks), which the operator reads as it is
         h = tall_linear(feat, torch.cat([self.theta.weight, self.phi.weight], 0))
-        h_theta, h_phi = h[:, :out_feat], h[:, out_feat:]
-        h_src = h_theta.contiguous()
-        h_dst = h_phi - h_theta
-        return fused_edgeconv_op(k, src_ind, h_src, h_dst, block, negative_slope_out)
+        return fused_edgeconv_pair_op(k, src_ind, h, block, negative_slope_out)

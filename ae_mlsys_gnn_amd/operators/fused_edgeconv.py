@@ -101,3 +101,43 @@ class FusedEdgeConvFunction(torch.autograd.Function):
         max_idx, out_feat = ctx.saved_tensors
         grad_src, grad_dst = edgeconv_native.edgeconv_backward_lrelu(grad_out, max_idx, out_feat, ctx.slope, ctx.n_src, ctx.block)
         return None, None, grad_src, grad_dst, None, None
+
+
+def fused_edgeconv_pair_op(k, src_ind, h, block=None, negative_slope_out=None):
+    """fused_edgeconv_op on theta(x) and phi(x) side by side in h [N, 2F]: h_src = theta, h_dst = phi - theta, formed inside the
+    operator in both passes.  block, negative_slope_out: as fused_edgeconv_op."""
+    return FusedEdgeConvPairFunction.apply(k, src_ind, h, block, negative_slope_out)
+
+
+class FusedEdgeConvPairFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, k, src_ind, h, block=None, negative_slope_out=None):
+        require_cuda(src_ind, h)
+        src_ind, h = as_i32(src_ind), as_f32(h)
+        n, f = h.shape[0], h.shape[1] // 2
+        if h.dim() != 2 or h.shape[1] != 2 * f or src_ind.numel() != n * int(k):
+            raise FgnnError("edgeconv: src_ind has %d entries, expected N*k = %d*%d; h is %s" % (src_ind.numel(), n, int(k), tuple(h.shape)))
+        if negative_slope_out is not None and not negative_slope_out > 0:
+            raise FgnnError("edgeconv: the fused LeakyReLU needs a positive slope, got %s" % (negative_slope_out,))
+        out = torch.empty((n, f), dtype=torch.float32, device=h.device)
+        need = ctx.needs_input_grad[2]
+        max_idx = torch.empty((n, f), dtype=torch.int32, device=h.device) if need else None
+        with torch.cuda.device(h.device):
+            check(lib().fgnn_edgeconv_pair_forward(n, f, int(k), ptr(src_ind), ptr(h), 1.0 if negative_slope_out is None else float(negative_slope_out),
+                                                   ptr(out), ptr(max_idx), stream_ptr()), "fgnn_edgeconv_pair_forward")
+        ctx.block, ctx.slope = block, negative_slope_out
+        if need:
+            ctx.save_for_backward(max_idx, None if negative_slope_out is None else out)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        max_idx, out = ctx.saved_tensors
+        grad_out = as_f32(grad_out)
+        n, f = grad_out.shape
+        grad_h = torch.empty((n, 2 * f), dtype=torch.float32, device=grad_out.device)
+        with torch.cuda.device(grad_out.device):
+            ws, wsb = workspace(lib().fgnn_edgeconv_backward_blocked_workspace_bytes(n, f), grad_out.device) if ctx.block else (None, 0)
+            check(lib().fgnn_edgeconv_pair_backward(n, f, int(ctx.block or 0), ptr(max_idx), ptr(out), 1.0 if ctx.slope is None else float(ctx.slope),
+                                                    ptr(grad_out), ptr(grad_h), ptr(ws), wsb, stream_ptr()), "fgnn_edgeconv_pair_backward")
+        return None, None, grad_h, None, None

@@ -236,6 +236,14 @@ int fgnn_edgeconv_backward_lrelu(int N, int n_src, int F, int block, const int32
                                  float out_slope, const float *grad_out, float *grad_src, float *grad_dst,
                                  void *workspace, size_t workspace_bytes, void *stream);
 
+/* The form in which a layer calls it: h [N, 2F] holds theta(x) and phi(x) of every node side by side, h_src = theta,
+ * h_dst = phi - theta (layers/edgeconv_layer.py:36-43 of the reference).  out_slope = 1: no activation; it must be positive.
+ * argmax may be NULL when no backward follows.  The backward writes grad_h [N, 2F]; out NULL: no activation; block as above. */
+int fgnn_edgeconv_pair_forward(int N, int F, int k, const int32_t *src_ind, const float *h, float out_slope, float *out,
+                               int32_t *argmax, void *stream);
+int fgnn_edgeconv_pair_backward(int N, int F, int block, const int32_t *argmax, const float *out, float out_slope,
+                                const float *grad_out, float *grad_h, void *workspace, size_t workspace_bytes, void *stream);
+
 /* The same backward for batched point clouds.  `block` is a hint that the neighbours of destination
  * rows [b*block, (b+1)*block) lie in source rows of the same range, as in a kNN graph of clouds of
  * `block` points (fgnn_knn_graph): those contributions are accumulated in LDS and written with plain

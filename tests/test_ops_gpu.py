@@ -696,6 +696,32 @@ def test_knn_graph_ties_are_ordered_by_id():
         knn_graph(torch.zeros(1, 200, 3, device=DEV), 129)
 
 
+@pytest.mark.parametrize("b,p,f,k,block", [(3, 100, 8, 5, 100), (3, 100, 8, 5, None), (2, 65, 3, 1, 65), (2, 300, 130, 9, 64), (2, 40, 12, 7, 5000),
+                                           (9, 128, 64, 20, 128), (1, 2049, 5, 3, 2049)])
+@pytest.mark.parametrize("slope", [None, 0.2])
+def test_edgeconv_pair(b, p, f, k, block, slope):
+    """theta and phi side by side against the operator on separate halves: the forward bit for bit, the gradients of both halves
+    against sums in float64 over the forward's own argmax; hints that match the clouds, cut them, or fall back to the scatter."""
+    from ae_mlsys_gnn_amd.operators import fused_edgeconv as fe
+    gen = torch.Generator().manual_seed(b * p + f)
+    n = b * p
+    src = (torch.randint(0, p, (n, k), generator=gen) + (torch.arange(n) // p * p).view(n, 1)).int().view(-1).to(DEV)
+    h = torch.randn(n, 2 * f, generator=gen)
+    go = torch.randn(n, f, generator=gen)
+    hd = h.to(DEV).requires_grad_(True)
+    out = fe.fused_edgeconv_pair_op(k, src, hd, block, slope)
+    theta, phi = h[:, :f].to(DEV).contiguous(), h[:, f:].to(DEV).contiguous()
+    want, arg = fe.edgeconv_native.edgeconv_forward(k, src, theta, phi - theta, out_slope=slope)
+    assert torch.equal(out, want)
+    with torch.no_grad():
+        assert torch.equal(fe.fused_edgeconv_pair_op(k, src, h.to(DEV), block, slope), want)       # no argmax is written
+    out.backward(go.to(DEV))
+    g = go.double() if slope is None else torch.where(want.cpu() > 0, go, go * torch.tensor(slope)).double()
+    scat = lambda t: torch.zeros(n, f, dtype=torch.float64).scatter_add_(0, arg.cpu().long(), t)
+    assert torch.equal(hd.grad[:, f:].cpu().double(), g)
+    assert_close_sum(hd.grad[:, :f], scat(g) - g, scat(g.abs()) + g.abs(), "gradient of theta")
+
+
 @pytest.mark.parametrize("p", [33, 64, 129, 256, 500, 1024, 1030])
 @pytest.mark.parametrize("k", [1, 31, 32, 33, 63, 64])
 def test_knn_selection_at_its_limits(p, k):
