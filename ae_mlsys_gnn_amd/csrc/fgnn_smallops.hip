@@ -441,13 +441,17 @@ extern "C" int fgnn_gather_rows(int64_t E, int W, const int32_t *permute, const 
 // load is a contiguous run of S0 floats.  Rows of up to SO_LONG_ELEMS floats are taken by one wave
 // each, longer ones by a whole workgroup each: a 100 k-entry hub row is then a few hundred trips of a
 // workgroup instead of tens of thousands of trips of one wave.  Both kinds run in ONE launch: its first
-// workgroups each look at SO_CAND candidate rows (the first wave reads their lengths, a ballot names the
+// workgroups each look at 16 or 64 candidate rows (the first wave reads their lengths, a ballot names the
 // long ones, the workgroup takes those one after the other), the workgroups behind them give one short
 // row to each of their waves and fill the machine while the last long rows finish.  (On a 233 k-row
 // power-law graph 31 k rows are long and hold 83 % of the entries; a workgroup per row would start
 // 233 k workgroups of which seven in eight leave at once.)
 #define SO_LONG_ELEMS 8192
-#define SO_CAND 16            // candidate rows per workgroup of a long-row launch
+// Candidate rows per workgroup of a long-row launch: 16 where a good part of the rows is long (the workgroup takes its long rows one
+// after the other), 64 where the mean row is short and most of these workgroups leave at once (169 k rows of 15 entries, 8 heads: row sums 59 -> 43 us, with the loads
+// in flight below).
+#define SO_CAND_DENSE 16
+#define SO_CAND_SPARSE 64
 // Registers a row-reduction kernel spends on a row: CACHE groups of VEC floats per lane kept over both phases by a wave on a short
 // row, CLONG by the workgroup on a long row, STREAM loads in flight per lane in the part of a row that is streamed.  The numbers
 // set the kernel's register count and with it the waves resident per SIMD: rows that mostly fit one trip of a wave want a small
@@ -492,7 +496,8 @@ static inline int so_pick_lanes(int N, int64_t elems, int vec, int W)
 // 3.29 / 2.77 / 2.48, the scatter kernel 3.93 / 3.60 / 4.43, gather-row 4.03 / 4.06 / 4.83, row sums 1.08 / 0.79 / 0.66.
 static inline unsigned so_grid(int N, int64_t elems, int tpb, unsigned *n_long, int lanes_per_row = 64)
 {
-    *n_long = elems > SO_LONG_ELEMS ? (unsigned)((N + SO_CAND - 1) / SO_CAND) : 0u;      // otherwise no row can be long
+    const int cand = so_dense_rows(N, elems) ? SO_CAND_DENSE : SO_CAND_SPARSE;
+    *n_long = elems > SO_LONG_ELEMS ? (unsigned)((N + cand - 1) / cand) : 0u;      // otherwise no row can be long
     const int rows_per_block = (tpb / 64) * (64 / lanes_per_row);
     return *n_long + (unsigned)((N + rows_per_block - 1) / rows_per_block);
 }
@@ -584,14 +589,16 @@ __device__ __forceinline__ bool so_take_short_rows(unsigned u, int N, int W, con
     if (n * VEC > SO_LONG_ELEMS) { n = 0; mine = false; }          // the long launch has it
     return __builtin_amdgcn_ballot_w64(mine) != 0ull;
 }
-// Long launch: bit l of the result is set when candidate blockIdx.x * SO_CAND + l is a long row (uniform over the workgroup).
+// Candidates of a workgroup of the long launch, from the number of those workgroups: they cover all rows, at most 64 each.
+__device__ __forceinline__ unsigned so_candidates(int N, unsigned n_long_blocks) { return ((unsigned)N + n_long_blocks - 1) / n_long_blocks; }
+// Long launch: bit l of the result is set when candidate blockIdx.x * cand + l is a long row (uniform over the workgroup).
 template <int VEC>
-__device__ __forceinline__ unsigned long long so_long_candidates(int N, int W, const int *ptr, unsigned long long *sh_mask)
+__device__ __forceinline__ unsigned long long so_long_candidates(int N, int W, unsigned cand, const int *ptr, unsigned long long *sh_mask)
 {
     if (fg_wave() == 0) {
-        const unsigned u = blockIdx.x * SO_CAND + (unsigned)fg_lane();
+        const unsigned u = blockIdx.x * cand + (unsigned)fg_lane();
         bool lng = false;
-        if (fg_lane() < SO_CAND && u < (unsigned)N) {
+        if ((unsigned)fg_lane() < cand && u < (unsigned)N) {
             const int r = so_scattered_row(u, N);
             lng = (int64_t)(ptr[r + 1] - ptr[r]) * W * VEC > SO_LONG_ELEMS;
         }
@@ -731,7 +738,7 @@ __device__ __forceinline__ void so_softmax_row(int W, int64_t n, const Src &src,
     }
 }
 
-// One launch for both kinds of row: the first n_long_blocks workgroups take the long rows among their SO_CAND candidates
+// One launch for both kinds of row: the first n_long_blocks workgroups take the long rows among their candidates
 // (they start first, so the longest rows are not left for the end), the workgroups after them give one short row to each
 // of their eight waves.
 template <int VEC, int TPB, class CFG>
@@ -741,8 +748,9 @@ __global__ __launch_bounds__(TPB) void edge_softmax_kernel(int N, int W, unsigne
     __shared__ float sh[TPB / 64][64];
     __shared__ unsigned long long sh_mask;
     if (blockIdx.x < n_long_blocks) {
-        for (unsigned long long m = so_long_candidates<VEC>(N, W, ptr, &sh_mask); m; m &= m - 1) {
-            const int row = so_scattered_row(blockIdx.x * SO_CAND + (unsigned)__builtin_ctzll(m), N);
+        const unsigned cand = so_candidates(N, n_long_blocks);
+        for (unsigned long long m = so_long_candidates<VEC>(N, W, cand, ptr, &sh_mask); m; m &= m - 1) {
+            const int row = so_scattered_row(blockIdx.x * cand + (unsigned)__builtin_ctzll(m), N);
             const int pb = fg_uni(ptr[row]);
             so_softmax_row<TPB / 64, VEC, CFG::CLONG, CFG::STREAM>(W, (int64_t)(fg_uni(ptr[row + 1]) - pb) * W, so_from_array<VEC>{in + (size_t)pb * W * VEC},
                                                      out + (size_t)pb * W * VEC, sh);
@@ -782,8 +790,9 @@ __global__ __launch_bounds__(TPB) void gat_scatter_kernel(int N, int W, unsigned
     };
     const int col = fg_lane() % W;
     if (blockIdx.x < n_long_blocks) {
-        for (unsigned long long m = so_long_candidates<VEC>(N, W, ptr, &sh_mask); m; m &= m - 1) {
-            const int row = so_scattered_row(blockIdx.x * SO_CAND + (unsigned)__builtin_ctzll(m), N);
+        const unsigned cand = so_candidates(N, n_long_blocks);
+        for (unsigned long long m = so_long_candidates<VEC>(N, W, cand, ptr, &sh_mask); m; m &= m - 1) {
+            const int row = so_scattered_row(blockIdx.x * cand + (unsigned)__builtin_ctzll(m), N);
             const int pb = fg_uni(ptr[row]);
             so_softmax_row<TPB / 64, VEC, CFG::CLONG, CFG::STREAM>(W, (int64_t)(fg_uni(ptr[row + 1]) - pb) * W, source(row, pb, col), esoft + (size_t)pb * W * VEC, sh);
         }
@@ -933,8 +942,9 @@ __global__ __launch_bounds__(TPB) void edge_softmax_bwd_kernel(int N, int W, uns
     __shared__ float sh[TPB / 64][64];
     __shared__ unsigned long long sh_mask;
     if (blockIdx.x < n_long_blocks) {
-        for (unsigned long long m = so_long_candidates<VEC>(N, W, ptr, &sh_mask); m; m &= m - 1) {
-            const int row = so_scattered_row(blockIdx.x * SO_CAND + (unsigned)__builtin_ctzll(m), N);
+        const unsigned cand = so_candidates(N, n_long_blocks);
+        for (unsigned long long m = so_long_candidates<VEC>(N, W, cand, ptr, &sh_mask); m; m &= m - 1) {
+            const int row = so_scattered_row(blockIdx.x * cand + (unsigned)__builtin_ctzll(m), N);
             const int pb = fg_uni(ptr[row]);
             so_softmax_bwd_row<TPB / 64, VEC, CFG::CACHE, CFG::STREAM>(W, pb, (int64_t)(fg_uni(ptr[row + 1]) - pb) * W, sm, g, gin, so_sign_none<VEC>{}, nullptr, sh);
         }
@@ -978,8 +988,9 @@ __global__ __launch_bounds__(TPB) void gat_gather_row_kernel(int N, int W, unsig
         }
     };
     if (blockIdx.x < n_long_blocks) {
-        for (unsigned long long m = so_long_candidates<VEC>(N, W, ptr, &sh_mask); m; m &= m - 1) {
-            const int row = so_scattered_row(blockIdx.x * SO_CAND + (unsigned)__builtin_ctzll(m), N);
+        const unsigned cand = so_candidates(N, n_long_blocks);
+        for (unsigned long long m = so_long_candidates<VEC>(N, W, cand, ptr, &sh_mask); m; m &= m - 1) {
+            const int row = so_scattered_row(blockIdx.x * cand + (unsigned)__builtin_ctzll(m), N);
             const int pb = fg_uni(ptr[row]);
             run.template operator()<TPB / 64, 64>(row, pb, (int64_t)(fg_uni(ptr[row + 1]) - pb) * W, true, sh);
         }
@@ -1143,49 +1154,78 @@ extern "C" int fgnn_gat_gather_row(int N, int64_t E, int H, const int32_t *row_p
     return fgnn_launch_status("gat_gather_row_kernel");
 }
 
+// so_row_of by a whole wave (every argument uniform): 64 places of ptr are looked at at once, so a search over 169 k rows waits for
+// memory three times instead of eighteen.
+__device__ __forceinline__ int so_wave_row_of(const int *__restrict__ ptr, int lo, int hi, int q, int lane)
+{
+    for (;;) {
+        const int step = (int)(((unsigned)(hi - lo) + 64u) / 64u);
+        const int64_t r = (int64_t)lo + (int64_t)lane * step;
+        const int c = __popcll(__ballot(r <= hi && ptr[r <= hi ? r : hi] <= q));
+        lo += (c > 0 ? c - 1 : 0) * step;
+        if (step == 1) return lo;
+        hi = min(hi, lo + step - 1);
+    }
+}
+
 // out[p,w] = row_val[row(p),w] + col_val[col_ind[p],w]  (src/u_add_v/u_add_v.cu:4-26).  W <= 64: one thread per
-// element of out, a wave takes 2048 consecutive ones; the row of an edge is found by bisection of row_ptr, first
-// for the wave's first and last edge (wave-uniform), then per lane inside that usually one- or two-row window.
-#define UAV_CHUNKS 32           // 64-element chunks per wave
-#define UAV_UJ 8                // chunks in flight; divides UAV_CHUNKS
+// element of out, a wave takes `chunks` x 64 consecutive ones.  The row of the wave's first edge is found by a wave-wide search of
+// row_ptr; from there on the 64 row ends that follow sit in a register, and a lane bisects them by lane exchange.  Only
+// where 512 elements span more than 64 rows is row_ptr itself bisected.  (2.5 M entries in 169 k rows, 8 heads: 85 -> 30 us, 64 M entries 1.09 -> 1.06 ms;
+// before, two searches of 18 dependent loads per wave, 7 more per 512 elements, and 2424 waves.)
+#define UAV_UJ 8                // chunks in flight; divides the chunks of a wave
 // VEC = 4: an element is four consecutive columns (W % 4 == 0, 16-byte aligned arrays), W counts such groups.
 template <int VEC>
-__global__ __launch_bounds__(FGNN_TPB) void u_add_v_kernel(int N, int64_t E, int W, const int *__restrict__ ptr, const int *__restrict__ idx,
+__global__ __launch_bounds__(FGNN_TPB) void u_add_v_kernel(int N, int64_t E, int W, int chunks, const int *__restrict__ ptr, const int *__restrict__ idx,
                                                            const float *__restrict__ rv, const float *__restrict__ cv, float *__restrict__ out)
 {
     const int64_t total = E * W;
-    const int64_t k0 = ((int64_t)blockIdx.x * FGNN_WPB + fg_wave()) * (64 * UAV_CHUNKS);
+    const int64_t k0 = ((int64_t)blockIdx.x * FGNN_WPB + fg_wave()) * (64 * chunks);
     if (k0 >= total) return;
-    const int64_t k1 = min(k0 + 64 * UAV_CHUNKS, total);
+    const int64_t k1 = min(k0 + 64 * chunks, total);
     const int lane = fg_lane();
     const unsigned uw = (unsigned)W;
     const unsigned inv_w = (65536u + uw - 1u) / uw;          // ceil(2^16 / W)
     int qbase = fg_uni((int)(k0 / W));                       // edge of the wave's first element
     unsigned rem = (unsigned)fg_uni((int)(k0 - (int64_t)qbase * W));
     const int qlast = fg_uni((int)((k1 - 1) / W));
-    int rlo = fg_uni(so_row_of(ptr, 0, N - 1, qbase));
-    const int rhi = fg_uni(so_row_of(ptr, rlo, N - 1, qlast));
+    int rlo = fg_uni(so_wave_row_of(ptr, 0, N - 1, qbase, lane));
     constexpr int UJ = UAV_UJ;
     for (int64_t kk = k0; kk < k1; kk += 64 * UJ) {
-        int q[UJ], w[UJ], lo[UJ], hi[UJ];
+        const int ends = ptr[(int)min((int64_t)rlo + 1 + lane, (int64_t)N)];
+        int q[UJ], w[UJ], lo[UJ], src[UJ];
 #pragma unroll
         for (int j = 0; j < UJ; ++j) {
             const unsigned x = rem + (unsigned)(64 * j + lane);           // < W + 64 * UJ <= 320
             const unsigned dq = (x * inv_w) >> 16;                          // = x / W for x < 1024 (W <= 64)
             w[j] = (int)(x - dq * uw);
             q[j] = min(qbase + (int)dq, qlast);
-            lo[j] = rlo; hi[j] = rhi;
+            src[j] = idx[q[j]];
         }
-        for (int span = rhi - rlo; span > 0; span >>= 1) {   // wave-uniform trip count: ceil(log2(window))
+        const int qe = __builtin_amdgcn_readlane(q[UJ - 1], 63);
+        if (__builtin_amdgcn_readlane(ends, 63) > qe) {       // the row of every edge here ends at one of the 64 places
+            int pos[UJ];
 #pragma unroll
-            for (int j = 0; j < UJ; ++j) {
-                const int mid = (lo[j] + hi[j] + 1) >> 1;    // lo == hi: mid == lo, nothing changes
-                if (lo[j] < hi[j]) { if (ptr[mid] <= q[j]) lo[j] = mid; else hi[j] = mid - 1; }
+            for (int j = 0; j < UJ; ++j) pos[j] = 0;
+#pragma unroll
+            for (int s = 32; s > 0; s >>= 1)
+#pragma unroll
+                for (int j = 0; j < UJ; ++j) pos[j] += __builtin_amdgcn_ds_bpermute((pos[j] + s - 1) << 2, ends) <= q[j] ? s : 0;
+#pragma unroll
+            for (int j = 0; j < UJ; ++j) lo[j] = rlo + pos[j];
+        } else {
+            const int rhi = fg_uni(so_wave_row_of(ptr, rlo, N - 1, qe, lane));
+            int hi[UJ];
+#pragma unroll
+            for (int j = 0; j < UJ; ++j) { lo[j] = rlo; hi[j] = rhi; }
+            for (int span = rhi - rlo; span > 0; span >>= 1) {   // wave-uniform trip count: ceil(log2(window))
+#pragma unroll
+                for (int j = 0; j < UJ; ++j) {
+                    const int mid = (lo[j] + hi[j] + 1) >> 1;    // lo == hi: mid == lo, nothing changes
+                    if (lo[j] < hi[j]) { if (ptr[mid] <= q[j]) lo[j] = mid; else hi[j] = mid - 1; }
+                }
             }
         }
-        int src[UJ];
-#pragma unroll
-        for (int j = 0; j < UJ; ++j) src[j] = idx[q[j]];
 #pragma unroll
         for (int j = 0; j < UJ; ++j) {
             const int64_t k = kk + 64 * j + lane;
@@ -1234,17 +1274,26 @@ __device__ __forceinline__ void so_rowsum_row(int W, int row, int pb, int pe, co
     const bool act = sl < S0;
     so_grp<VEC> acc = so_fill<VEC>(0.f);
     if (act) {
-#pragma unroll 8
-        for (int q = pb + (NW > 1 ? fg_wave() * per : 0) + sl / W; q < pe; q += per * nw) {
-            const so_grp<VEC> v = so_load<VEC>(g + ((size_t)q * W + w) * VEC);
+        constexpr int U = 8;
+        const int step = per * nw;
+        int q = pb + (NW > 1 ? fg_wave() * per : 0) + sl / W;
+        auto take = [&](int qq, const so_grp<VEC> &v) {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) acc.c[c] += v.c[c];
             if constexpr (COLS) {
-                float *dst = gcol + ((size_t)idx[q] * W + w) * VEC;
+                float *dst = gcol + ((size_t)idx[qq] * W + w) * VEC;
 #pragma unroll
                 for (int c = 0; c < VEC; ++c) unsafeAtomicAdd(dst + c, v.c[c]);
             }
+        };
+        for (; (int64_t)q + (U - 1) * (int64_t)step < pe; q += U * step) {           // U loads in flight
+            so_grp<VEC> v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = so_load<VEC>(g + ((size_t)(q + u * step) * W + w) * VEC);
+#pragma unroll
+            for (int u = 0; u < U; ++u) take(q + u * step, v[u]);
         }
+        for (; q < pe; q += step) take(q, so_load<VEC>(g + ((size_t)q * W + w) * VEC));
     }
     if constexpr (L < 64) acc = so_group_reduce<VEC, L>(acc, lane, W, S0, so_add());
     else acc = so_column_reduce<NW, VEC>(acc, lane, W, S0, sh, so_add());
@@ -1259,8 +1308,9 @@ __global__ __launch_bounds__(TPB) void edge_rowsum_kernel(int N, int W, unsigned
     __shared__ float sh[TPB / 64][64];
     __shared__ unsigned long long sh_mask;
     if (blockIdx.x < n_long_blocks) {
-        for (unsigned long long m = so_long_candidates<VEC>(N, W, ptr, &sh_mask); m; m &= m - 1) {
-            const int row = so_scattered_row(blockIdx.x * SO_CAND + (unsigned)__builtin_ctzll(m), N);
+        const unsigned cand = so_candidates(N, n_long_blocks);
+        for (unsigned long long m = so_long_candidates<VEC>(N, W, cand, ptr, &sh_mask); m; m &= m - 1) {
+            const int row = so_scattered_row(blockIdx.x * cand + (unsigned)__builtin_ctzll(m), N);
             so_rowsum_row<TPB / 64, VEC, COLS>(W, row, fg_uni(ptr[row]), fg_uni(ptr[row + 1]), idx, g, grow, gcol, sh);
         }
         return;
@@ -1309,14 +1359,14 @@ extern "C" int fgnn_u_add_v(int N, int64_t E, int W, const int32_t *row_ptr, con
         return fgnn_launch_status("u_add_v_wide_kernel");
     }
     FGNN_REQUIRE(E <= 2147483647LL, FGNN_ERR_LIMIT, "fgnn_u_add_v: E=%lld exceeds the 32-bit row_ptr", (long long)E);
-    const int64_t per_block = (int64_t)FGNN_WPB * 64 * UAV_CHUNKS;
-    if (W % 4 == 0 && fgnn_aligned16(row_val) && fgnn_aligned16(col_val) && fgnn_aligned16(out)) {
-        const int64_t blocks = (E * (W / 4) + per_block - 1) / per_block;
-        hipLaunchKernelGGL(u_add_v_kernel<4>, dim3((unsigned)blocks), dim3(FGNN_TPB), 0, st, N, E, W / 4, row_ptr, col_ind, row_val, col_val, out);
-    } else {
-        const int64_t blocks = (E * W + per_block - 1) / per_block;
-        hipLaunchKernelGGL(u_add_v_kernel<1>, dim3((unsigned)blocks), dim3(FGNN_TPB), 0, st, N, E, W, row_ptr, col_ind, row_val, col_val, out);
-    }
+    const bool vec4 = W % 4 == 0 && fgnn_aligned16(row_val) && fgnn_aligned16(col_val) && fgnn_aligned16(out);
+    // 2048 elements per wave where that gives every compute unit 32 waves four times over, else 512
+    const int64_t elems = E * (vec4 ? W / 4 : W);
+    const int chunks = elems >= (int64_t)2048 * 32768 ? 32 : 8;
+    const int64_t per_block = (int64_t)FGNN_WPB * 64 * chunks;
+    const unsigned blocks = (unsigned)((elems + per_block - 1) / per_block);
+    if (vec4) hipLaunchKernelGGL(u_add_v_kernel<4>, dim3(blocks), dim3(FGNN_TPB), 0, st, N, E, W / 4, chunks, row_ptr, col_ind, row_val, col_val, out);
+    else hipLaunchKernelGGL(u_add_v_kernel<1>, dim3(blocks), dim3(FGNN_TPB), 0, st, N, E, W, chunks, row_ptr, col_ind, row_val, col_val, out);
     return fgnn_launch_status("u_add_v_kernel");
 }
 

@@ -1375,3 +1375,27 @@ def test_mhspmm_and_mhsddmm_rows_wider_than_1024_floats(h, f, monkeypatch):
         assert_close_sum(fd.grad, fl.grad, s_feat, "mhspmm grad feat, wide rows, buckets " + buckets)
         assert_close_sum(ad.grad, al.grad, s_att, "mhspmm grad att (mhsddmm), wide rows, buckets " + buckets)
     _lib.clear_schedule_cache()
+
+
+@pytest.mark.parametrize("w", [1, 3, 4, 8, 64])
+@pytest.mark.parametrize("shape", ["short", "empty_runs", "hub", "one_row", "long_rows"])
+def test_u_add_v_row_search_and_row_sums(w, shape):
+    """Rows found by the wave-wide search and inside the window of 64 row ends: runs of empty rows longer than the window, a row that
+    spans many waves, a single row, and enough long rows that a workgroup finds several among its candidates."""
+    from ae_mlsys_gnn_amd._lib import check, lib, ptr, stream_ptr
+    gen = torch.Generator().manual_seed(w)
+    deg = {"short": torch.randint(0, 4, (5000,), generator=gen), "empty_runs": torch.randint(0, 9, (20000,), generator=gen) * (torch.arange(20000) % 300 == 7),
+           "hub": torch.cat([torch.randint(0, 3, (700,), generator=gen), torch.tensor([30000]), torch.zeros(500, dtype=torch.long), torch.ones(65, dtype=torch.long)]),
+           "one_row": torch.tensor([1000]), "long_rows": torch.where(torch.arange(900) % 3 == 0, 8200 // w + 1, 2)}[shape]
+    n, e = deg.numel(), int(deg.sum())
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.long), deg.cumsum(0)]).int()
+    dst = torch.repeat_interleave(torch.arange(n), deg)
+    idx = torch.randint(0, n, (e,), generator=gen)
+    a, b, g = torch.randn(n, w, generator=gen), torch.randn(n, w, generator=gen), torch.randn(e, w, generator=gen)
+    dp, di, da, db, dg = (t.to(DEV) for t in (row_ptr, idx.int(), a, b, g))
+    out, gr = torch.empty(e, w, device=DEV), torch.empty(n, w, device=DEV)
+    check(lib().fgnn_u_add_v(n, e, w, ptr(dp), ptr(di), ptr(da), ptr(db), ptr(out), stream_ptr()), "fgnn_u_add_v")
+    check(lib().fgnn_edge_rowsum(n, e, w, ptr(dp), ptr(dg), ptr(gr), stream_ptr()), "fgnn_edge_rowsum")
+    assert torch.equal(out.cpu(), a[dst] + b[idx])
+    want = torch.zeros(n, w, dtype=torch.float64).index_add_(0, dst, g.double())
+    assert_close_sum(gr, want, torch.zeros(n, w, dtype=torch.float64).index_add_(0, dst, g.double().abs()), "row sums")
