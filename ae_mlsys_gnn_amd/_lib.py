@@ -62,6 +62,9 @@ _SIGNATURES = {
     "fgnn_edgeconv_backward_blocked": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 4 + [c_size_t, c_void_p]),
     "fgnn_edgeconv_backward_blocked_static_max_elems": (c_size_t, []),
     "fgnn_edgeconv_backward_blocked_static": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 3 + [c_void_p]),
+    "fgnn_gat_fold_weights": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 6 + [c_void_p]),
+    "fgnn_gat_scores": (c_int, [c_int64, c_int, c_int] + [c_void_p] * 4 + [c_void_p]),
+    "fgnn_gat_unfold_grads": (c_int, [c_int] * 4 + [c_void_p] * 4 + [c_int, c_void_p, c_int] + [c_void_p] * 3 + [c_void_p]),
     "fgnn_knn_graph": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "fgnn_gmm_forward_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int]),
     "fgnn_gmm_forward": (c_int, [c_int, c_int64, c_int, c_int, c_int] + [c_void_p] * 9 + [c_int]

@@ -173,6 +173,65 @@ class gat_native:
         return out, gar
 
 
+class gat_dense_native:
+    """The dense side of a GAT layer around feat @ W (layers/gatconv_layer.py:50-55): scores are feat @ ((W * attn).sum(-1))."""
+
+    @staticmethod
+    def scores_supported(fin, h):
+        """Where `scores` is the faster form: up to 8 heads at any width, up to 32 where the input is narrow (100 k x 64, 32 heads: 24
+        against 39 us for the library product and its split; 30 k x 602, 16 heads: 37 against 32)."""
+        return h <= 8 or (h <= 32 and fin <= 256)
+
+    @staticmethod
+    def fold(W, attn_l, attn_r, pad, want_all):
+        """(score weights [2H, in], W with pad zero columns per head [in, H*(F+pad)], both side by side [in, H*(F+pad) + 2H] or None)."""
+        require_cuda(W, attn_l, attn_r)
+        W, attn_l, attn_r = as_f32(W), as_f32(attn_l), as_f32(attn_r)
+        _, h, f = attn_l.shape
+        fin = W.shape[0]
+        if W.shape != (fin, h * f) or attn_r.shape != attn_l.shape:
+            raise _lib.FgnnError("gat_fold: shape mismatch W %s attn_l %s attn_r %s" % (tuple(W.shape), tuple(attn_l.shape), tuple(attn_r.shape)))
+        new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=W.device)
+        score_wt, proj = new(2 * h, fin), new(fin, h * (f + pad)) if pad else None
+        both = new(fin, h * (f + pad) + 2 * h) if want_all else None
+        with torch.cuda.device(W.device):
+            check(lib().fgnn_gat_fold_weights(fin, h, f, pad, ptr(W), ptr(attn_l), ptr(attn_r), ptr(score_wt), ptr(proj), ptr(both), stream_ptr()),
+                  "fgnn_gat_fold_weights")
+        return score_wt, W if proj is None else proj, both
+
+    @staticmethod
+    def scores(feat, score_wt):
+        """attn_row [N, H], attn_col [N, H] of feat [N, in] @ score_wt^T."""
+        require_cuda(feat, score_wt)
+        feat, score_wt = as_f32(feat), as_f32(score_wt)
+        n, k = feat.shape
+        h = score_wt.shape[0] // 2
+        if score_wt.shape != (2 * h, k):
+            raise _lib.FgnnError("gat_scores: score weights %s do not fit feat %s" % (tuple(score_wt.shape), tuple(feat.shape)))
+        row = torch.empty((n, h), dtype=torch.float32, device=feat.device)
+        col = torch.empty_like(row)
+        with torch.cuda.device(feat.device):
+            check(lib().fgnn_gat_scores(n, k, h, ptr(feat), ptr(score_wt), ptr(row), ptr(col), stream_ptr()), "fgnn_gat_scores")
+        return row, col
+
+    @staticmethod
+    def unfold(W, attn_l, attn_r, pad, dproj, dscore):
+        """(dW, dattn_l, dattn_r); dproj [in, H*(F+pad)] and dscore [in, 2H] may be column slices of one matrix."""
+        require_cuda(W, attn_l, attn_r, dproj, dscore)
+        W, attn_l, attn_r = as_f32(W), as_f32(attn_l), as_f32(attn_r)
+        _, h, f = attn_l.shape
+        fin = W.shape[0]
+        if W.shape != (fin, h * f) or dproj.shape != (fin, h * (f + pad)) or dscore.shape != (fin, 2 * h):
+            raise _lib.FgnnError("gat_unfold: shape mismatch W %s dproj %s dscore %s" % (tuple(W.shape), tuple(dproj.shape), tuple(dscore.shape)))
+        rows = lambda t: t if t.dtype == torch.float32 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] else as_f32(t)
+        dproj, dscore = rows(dproj), rows(dscore)
+        dW, dl, dr = torch.empty_like(W), torch.empty_like(attn_l), torch.empty_like(attn_r)
+        with torch.cuda.device(W.device):
+            check(lib().fgnn_gat_unfold_grads(fin, h, f, pad, ptr(W), ptr(attn_l), ptr(attn_r), ptr(dproj), dproj.stride(0), ptr(dscore), dscore.stride(0),
+                                              ptr(dW), ptr(dl), ptr(dr), stream_ptr()), "fgnn_gat_unfold_grads")
+        return dW, dl, dr
+
+
 def fused_gat_fusescatter(attn_row, attn_col, row_ptr, col_ind, col_ptr, row_ind, negative_slope, in_feat, permute):
     return FusedGATFunction.apply(attn_row, attn_col, row_ptr, col_ind, col_ptr, row_ind, negative_slope, in_feat, permute)
 

@@ -269,6 +269,20 @@ size_t fgnn_edgeconv_backward_blocked_static_max_elems(void);
 int    fgnn_edgeconv_backward_blocked_static(int N, int n_src, int F, int block, const int32_t *argmax,
                                              const float *grad_out, float *grad_src, void *stream);
 
+/* The dense side of a GAT layer around feat @ W (layers/gatconv_layer.py:50-55 of the reference).  W [fin, H*F], attn_l / attn_r [H, F].
+ * fold: score_wt [2H, fin] = (W * attn_l).sum(-1), (W * attn_r).sum(-1), transposed; proj [fin, H*(F+pad)] (optional) = W with pad zero
+ * columns per head; all [fin, H*(F+pad) + 2H] (optional) = proj and the score weights side by side.
+ * scores: attn_row [n, H], attn_col [n, H] = feat [n, K] @ score_wt^T; H <= 32.
+ * unfold: dW, dattn_l, dattn_r from the gradients of the projection's weights (dproj, row stride ldp) and of the score weights
+ * (dscore [fin, 2H], row stride lds). */
+int fgnn_gat_fold_weights(int fin, int H, int F, int pad, const float *W, const float *attn_l, const float *attn_r,
+                          float *score_wt, float *proj, float *all, void *stream);
+int fgnn_gat_scores(int64_t n, int K, int H, const float *feat, const float *score_wt, float *attn_row, float *attn_col,
+                    void *stream);
+int fgnn_gat_unfold_grads(int fin, int H, int F, int pad, const float *W, const float *attn_l, const float *attn_r,
+                          const float *dproj, int ldp, const float *dscore, int lds, float *dW, float *dattn_l,
+                          float *dattn_r, void *stream);
+
 /* k-nearest-neighbour graph of batched point clouds, the input of fgnn_edgeconv_forward: points
  * [n_clouds*P, D]; src_ind [n_clouds*P*k] gets, for every point, the global ids of the k nearest
  * points of its own cloud (itself included), nearest first, ties to the smaller id; 1 <= k <= min(P,

@@ -1399,3 +1399,34 @@ def test_u_add_v_row_search_and_row_sums(w, shape):
     assert torch.equal(out.cpu(), a[dst] + b[idx])
     want = torch.zeros(n, w, dtype=torch.float64).index_add_(0, dst, g.double())
     assert_close_sum(gr, want, torch.zeros(n, w, dtype=torch.float64).index_add_(0, dst, g.double().abs()), "row sums")
+
+
+@pytest.mark.parametrize("n,fin,h,f,pad", [(1, 1, 1, 1, 3), (15, 3, 2, 5, 3), (17, 16, 8, 8, 0), (40, 63, 9, 3, 1), (33, 64, 16, 4, 0), (70, 65, 17, 2, 2),
+                                           (48, 100, 32, 8, 0), (66000, 20, 8, 4, 0), (66001, 67, 3, 6, 2), (300, 1433, 1, 128, 0), (0, 8, 2, 4, 0)])
+def test_gat_dense_kernels(n, fin, h, f, pad):
+    """Folded weights, node scores and unfolded gradients against float64, around the tiles of 16 nodes, 16 scores and 16 dimensions,
+    with dimensions split over waves and not, and with the gradients as column slices of one matrix."""
+    from ae_mlsys_gnn_amd.operators.fused_gat import gat_dense_native as gd
+    gen = torch.Generator().manual_seed(n + fin)
+    W, al, ar, x = torch.randn(fin, h * f, generator=gen), torch.randn(1, h, f, generator=gen), torch.randn(1, h, f, generator=gen), torch.randn(n, fin, generator=gen)
+    wt, proj, both = gd.fold(W.to(DEV), al.to(DEV), ar.to(DEV), pad, True)
+    wv = W.double().view(fin, h, f)
+    want_w = torch.cat([(wv * al.double()).sum(-1), (wv * ar.double()).sum(-1)], 1)
+    abs_w = torch.cat([(wv * al.double()).abs().sum(-1), (wv * ar.double()).abs().sum(-1)], 1)
+    padded = torch.nn.functional.pad(W.view(fin, h, f), (0, pad)).view(fin, -1)
+    assert torch.equal(proj.cpu(), padded) and torch.equal(both[:, :h * (f + pad)].cpu(), padded)
+    assert_close_sum(wt, want_w.t(), abs_w.t(), "score weights")
+    assert torch.equal(both[:, h * (f + pad):], wt.t())
+    row, col = gd.scores(x.to(DEV), wt)
+    w64 = wt.cpu().double()
+    want, scale = x.double() @ w64.t(), x.double().abs() @ w64.abs().t()
+    assert_close_sum(torch.cat([row, col], 1), want, scale, "scores")
+    d = torch.randn(fin, h * (f + pad) + 2 * h, generator=gen)
+    dd = d.to(DEV)
+    dW, dl, dr = gd.unfold(W.to(DEV), al.to(DEV), ar.to(DEV), pad, dd[:, :h * (f + pad)], dd[:, h * (f + pad):])
+    d = d.double()
+    p, sl, sr = d[:, :h * (f + pad)].view(fin, h, f + pad)[:, :, :f], d[:, h * (f + pad):h * (f + pad) + h].unsqueeze(-1), d[:, h * (f + pad) + h:].unsqueeze(-1)
+    terms = [p, sl * al.double(), sr * ar.double()]
+    assert_close_sum(dW, sum(terms).reshape(fin, -1), sum(t.abs() for t in terms).reshape(fin, -1), "dW")
+    for got, s in ((dl, sl), (dr, sr)):
+        assert_close_sum(got, (wv * s).sum(0, keepdim=True), (wv * s).abs().sum(0, keepdim=True), "dattn")
