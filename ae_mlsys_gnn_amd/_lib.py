@@ -143,8 +143,15 @@ def ptr(t):
     return c_void_p(t.data_ptr())
 
 
+def device_guard(device):
+    """Makes a tensor's device the current one: torch.cuda.device without its parsing of the argument."""
+    return torch.cuda._DeviceGuard(device.index)
+
+
 def stream_ptr():
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device.  Asked for as a raw handle: building a torch Stream object around it took 10 us a
+    call, five times a layer step."""
+    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def require_cuda(*tensors):
@@ -175,7 +182,7 @@ class Schedule:
         self.idx_tensor = None if idx_tensor is None else as_i32(idx_tensor)
         self.n_rows = self.ptr_tensor.numel() - 1
         handle = c_void_p()
-        with torch.cuda.device(self.ptr_tensor.device):
+        with device_guard(self.ptr_tensor.device):
             if self.idx_tensor is not None and os.environ.get("FGNN_VALIDATE", "0") not in ("0", ""):
                 # opt-in: range-check the graph once, when its work list is built, before any gather kernel runs.  The ids
                 # index another array than the pointer array's rows (mhspmm / csrspmm: the gathered matrix), so the bound is
@@ -204,7 +211,7 @@ class Schedule:
         n_split = lib().fgnn_schedule_num_splits(self.handle)
         items = torch.empty((self.n_items, 4), dtype=torch.int32, device=dev)
         splits = torch.empty((n_split, 4), dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             check(lib().fgnn_schedule_export(self.handle, ptr(items), ptr(splits), stream_ptr()), "fgnn_schedule_export")
         return items, splits
 
@@ -216,7 +223,7 @@ class Schedule:
         """int32 [E]: caller's edge position of every entry in the schedule's own order.  The schedule gives
         up its copy; operators called with it afterwards take per-edge tensors in that order."""
         out = torch.empty(self.n_edges, dtype=torch.int32, device=self.ptr_tensor.device)
-        with torch.cuda.device(self.ptr_tensor.device):
+        with device_guard(self.ptr_tensor.device):
             check(lib().fgnn_schedule_take_positions(self.handle, ptr(out), stream_ptr()), "fgnn_schedule_take_positions")
         self.own_order = True
         return out
@@ -273,7 +280,7 @@ def xcd_buckets_enabled(ptr_tensor, idx_numel=None) -> bool:
     hit = _bucket_rule_cache.get(key)
     if hit is None:
         stats = (ctypes.c_int64 * 2)()
-        with torch.cuda.device(ptr_tensor.device):
+        with device_guard(ptr_tensor.device):
             check(lib().fgnn_row_length_stats(ptr(ptr_tensor), n_rows, BUCKET_ROW_LEN, ctypes.cast(stats, c_void_p), stream_ptr()),
                   "fgnn_row_length_stats")
         n_long, longest = int(stats[0]), int(stats[1])
@@ -365,7 +372,7 @@ class ColsumPlan:
         self.n_cols = int(n_cols)
         self.width = int(width)
         handle = c_void_p()
-        with torch.cuda.device(self.ptr_tensor.device):
+        with device_guard(self.ptr_tensor.device):
             check(lib().fgnn_colsum_plan_create(ptr(self.ptr_tensor), ptr(self.idx_tensor), self.n_rows, self.n_cols, self.idx_tensor.numel(),
                                                 self.width, int(lds_bytes), int(task_len), stream_ptr(), ctypes.byref(handle)),
                   "fgnn_colsum_plan_create")
@@ -385,7 +392,7 @@ class ColsumPlan:
             raise FgnnError("colsum: the array has %d rows, the plan %d entries" % (g.shape[0], e))
         w = g.numel() // max(e, 1) if e else int(torch.tensor(g.shape[1:]).prod()) if g.dim() > 1 else 1
         out = torch.empty((self.n_cols,) + tuple(g.shape[1:]), dtype=torch.float32, device=g.device)
-        with torch.cuda.device(g.device):
+        with device_guard(g.device):
             ws, wsb = workspace(lib().fgnn_colsum_workspace_bytes(self.handle, w), g.device)
             check(lib().fgnn_edge_colsum(self.handle, w, ptr(g), ptr(out), ptr(ws), wsb, stream_ptr()), "fgnn_edge_colsum")
         return out
@@ -432,7 +439,7 @@ def _gather_i32(src, index):
     """src[index] for int32 device vectors, by the library's row-gather kernel (the words move as they are)."""
     out = torch.empty_like(index)
     if index.numel():
-        with torch.cuda.device(src.device):
+        with device_guard(src.device):
             check(lib().fgnn_gather_rows(index.numel(), 1, ptr(index), ptr(src), ptr(out), stream_ptr()), "fgnn_gather_rows")
     return out
 

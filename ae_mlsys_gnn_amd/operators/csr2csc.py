@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_i32, check, lib, ptr, require_cuda, stream_ptr, workspace
+from .._lib import as_i32, check, device_guard, lib, ptr, require_cuda, stream_ptr, workspace
 
 
 def csr2csc(rowptr, colind, n_cols=None):
@@ -18,7 +18,7 @@ def csr2csc(rowptr, colind, n_cols=None):
     col_ptr = torch.empty(nc + 1, dtype=torch.int32, device=dev)
     row_ind = torch.empty(e, dtype=torch.int32, device=dev)
     permute = torch.empty(e, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         ws, wsb = workspace(lib().fgnn_csr2csc_workspace_bytes(n, nc, e), dev)
         check(lib().fgnn_csr2csc(n, nc, e, ptr(rowptr), ptr(colind), ptr(col_ptr), ptr(row_ind), ptr(permute), ptr(ws), wsb,
                                  stream_ptr()), "fgnn_csr2csc")
@@ -44,7 +44,7 @@ def coo2csr(dst, src, n_rows, n_cols=None, dedupe=True, return_edge_pos=False):
     col_ind = torch.empty(e, dtype=torch.int32, device=dev)
     n_out = torch.zeros(1, dtype=torch.int64, device=dev)
     edge_pos = torch.empty(e, dtype=torch.int32, device=dev) if return_edge_pos else None
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         ws, wsb = workspace(lib().fgnn_coo2csr_workspace_bytes(n_rows, nc, e), dev)
         check(lib().fgnn_coo2csr(n_rows, nc, e, ptr(dst), ptr(src), int(bool(dedupe)), ptr(row_ptr), ptr(col_ind), ptr(n_out),
                                  ptr(edge_pos), ptr(ws), wsb, stream_ptr()), "fgnn_coo2csr")

@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_f32, check, lib, ptr, require_cuda, stream_ptr, workspace
+from .._lib import as_f32, check, device_guard, lib, ptr, require_cuda, stream_ptr, workspace
 
 MAX_OUT = 4
 
@@ -19,7 +19,7 @@ class EdgeLinearTanhFunction(torch.autograd.Function):
         x, w, b = as_f32(x), as_f32(weight), as_f32(bias)
         e, d = x.shape[0], w.shape[0]
         y = torch.empty((e, d), dtype=torch.float32, device=x.device)
-        with torch.cuda.device(x.device):
+        with device_guard(x.device):
             check(lib().fgnn_edge_linear_tanh(e, d, ptr(x), ptr(w), ptr(b), ptr(y), stream_ptr()), "fgnn_edge_linear_tanh")
         ctx.save_for_backward(x, y)
         return y
@@ -32,7 +32,7 @@ class EdgeLinearTanhFunction(torch.autograd.Function):
         grad_w = torch.empty((d, 2), dtype=torch.float32, device=x.device)
         grad_b = torch.empty((d,), dtype=torch.float32, device=x.device)
         ws, ws_bytes = workspace(lib().fgnn_edge_linear_tanh_backward_workspace_bytes(e, d), x.device)
-        with torch.cuda.device(x.device):
+        with device_guard(x.device):
             check(lib().fgnn_edge_linear_tanh_backward(e, d, ptr(x), ptr(y), ptr(g), ptr(grad_w), ptr(grad_b), ptr(ws), ws_bytes, stream_ptr()),
                   "fgnn_edge_linear_tanh_backward")
         return None, grad_w, grad_b

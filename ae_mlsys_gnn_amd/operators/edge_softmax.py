@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_f32, as_i32, check, lib, ptr, require_cuda, stream_ptr
+from .._lib import as_f32, as_i32, check, device_guard, lib, ptr, require_cuda, stream_ptr
 
 
 class edge_softmax_native:
@@ -13,7 +13,7 @@ class edge_softmax_native:
         rowptr, h = as_i32(rowptr), as_f32(h)
         hh = h.view(h.shape[0], -1)
         out = torch.empty_like(hh)
-        with torch.cuda.device(h.device):
+        with device_guard(h.device):
             check(lib().fgnn_edge_softmax(rowptr.numel() - 1, hh.shape[0], hh.shape[1], ptr(rowptr), ptr(hh), ptr(out), stream_ptr()),
                   "fgnn_edge_softmax")
         return out.view_as(h)
@@ -24,7 +24,7 @@ class edge_softmax_native:
         rowptr, out, grad_out = as_i32(rowptr), as_f32(out), as_f32(grad_out)
         oo = out.view(out.shape[0], -1)
         gin = torch.empty_like(oo)
-        with torch.cuda.device(out.device):
+        with device_guard(out.device):
             check(lib().fgnn_edge_softmax_backward(rowptr.numel() - 1, oo.shape[0], oo.shape[1], ptr(rowptr), ptr(oo),
                                                    ptr(grad_out.view_as(oo)), ptr(gin), stream_ptr()), "fgnn_edge_softmax_backward")
         return gin.view_as(out)

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import FgnnError, as_f32, as_i32, check, lib, ptr, require_cuda, stream_ptr, workspace
+from .._lib import FgnnError, as_f32, as_i32, check, device_guard, lib, ptr, require_cuda, stream_ptr, workspace
 
 
 class edgeconv_native:
@@ -20,7 +20,7 @@ class edgeconv_native:
                 src_ind.numel(), n, int(k), h_src.shape[1], f))
         out = torch.empty_like(h_dst)
         max_idx = torch.empty((n, f), dtype=torch.int32, device=h_dst.device)
-        with torch.cuda.device(h_dst.device):
+        with device_guard(h_dst.device):
             if out_slope is None:
                 check(lib().fgnn_edgeconv_forward(n, h_src.shape[0], f, int(k), ptr(src_ind), ptr(h_src), ptr(h_dst), ptr(out),
                                                   ptr(max_idx), stream_ptr()), "fgnn_edgeconv_forward")
@@ -40,7 +40,7 @@ class edgeconv_native:
         n_src = n if n_src is None else n_src
         grad_src = torch.empty((n_src, f), dtype=torch.float32, device=grad_out.device)
         grad_dst = torch.empty_like(grad_out)
-        with torch.cuda.device(grad_out.device):
+        with device_guard(grad_out.device):
             ws, wsb = workspace(lib().fgnn_edgeconv_backward_blocked_workspace_bytes(n, f), grad_out.device) if block else (None, 0)
             check(lib().fgnn_edgeconv_backward_lrelu(n, n_src, f, int(block or 0), ptr(max_idx), ptr(out), float(out_slope), ptr(grad_out),
                                                      ptr(grad_src), ptr(grad_dst), ptr(ws), wsb, stream_ptr()), "fgnn_edgeconv_backward_lrelu")
@@ -55,7 +55,7 @@ class edgeconv_native:
         n, f = grad_out.shape
         n_src = n if n_src is None else n_src
         grad_src = torch.empty((n_src, f), dtype=torch.float32, device=grad_out.device)
-        with torch.cuda.device(grad_out.device):
+        with device_guard(grad_out.device):
             if block:
                 ws, wsb = workspace(lib().fgnn_edgeconv_backward_blocked_workspace_bytes(n, f), grad_out.device)
                 check(lib().fgnn_edgeconv_backward_blocked(n, n_src, f, int(block), ptr(max_idx), ptr(grad_out), ptr(grad_src), ptr(ws), wsb,
@@ -122,7 +122,7 @@ class FusedEdgeConvPairFunction(torch.autograd.Function):
         out = torch.empty((n, f), dtype=torch.float32, device=h.device)
         need = ctx.needs_input_grad[2]
         max_idx = torch.empty((n, f), dtype=torch.int32, device=h.device) if need else None
-        with torch.cuda.device(h.device):
+        with device_guard(h.device):
             check(lib().fgnn_edgeconv_pair_forward(n, f, int(k), ptr(src_ind), ptr(h), 1.0 if negative_slope_out is None else float(negative_slope_out),
                                                    ptr(out), ptr(max_idx), stream_ptr()), "fgnn_edgeconv_pair_forward")
         ctx.block, ctx.slope = block, negative_slope_out
@@ -136,7 +136,7 @@ class FusedEdgeConvPairFunction(torch.autograd.Function):
         grad_out = as_f32(grad_out)
         n, f = grad_out.shape
         grad_h = torch.empty((n, 2 * f), dtype=torch.float32, device=grad_out.device)
-        with torch.cuda.device(grad_out.device):
+        with device_guard(grad_out.device):
             ws, wsb = workspace(lib().fgnn_edgeconv_backward_blocked_workspace_bytes(n, f), grad_out.device) if ctx.block else (None, 0)
             check(lib().fgnn_edgeconv_pair_backward(n, f, int(ctx.block or 0), ptr(max_idx), ptr(out), 1.0 if ctx.slope is None else float(ctx.slope),
                                                     ptr(grad_out), ptr(grad_h), ptr(ws), wsb, stream_ptr()), "fgnn_edgeconv_pair_backward")

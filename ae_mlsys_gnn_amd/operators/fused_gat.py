@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .._lib import as_f32, as_i32, check, colsum_plan_for, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace
+from .._lib import as_f32, as_i32, check, colsum_plan_for, device_guard, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace
 
 
 class gat_native:
@@ -44,7 +44,7 @@ class gat_native:
         e_soft = torch.empty((e, h), dtype=torch.float32, device=dev) if stash else None
         sched = schedule_for(row_ptr, idx_tensor=col_ind, need_positions=False, n_cols=n) if use_schedule else None
         sh = sched.handle if sched is not None else None
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             ws, wsb = workspace(lib().fgnn_gat_forward_workspace_bytes(sh, h, f), dev)
             check(lib().fgnn_gat_forward(n, e, h, f, ptr(attn_row), ptr(attn_col), ptr(row_ptr), ptr(col_ind),
                                          float(negative_slope), ptr(in_feat), ptr(out), ptr(edge_max), ptr(edge_sum),
@@ -98,7 +98,7 @@ class gat_native:
         sched_csr = schedule_for(row_ptr, idx_tensor=col_ind, need_positions=False, n_cols=n) if (use_schedule and recompute) else None
         hc = sched_csc.handle if sched_csc is not None else None
         hr = sched_csr.handle if sched_csr is not None else None
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             ws, wsb = workspace(lib().fgnn_gat_backward_workspace_bytes(n, h, f, hc, hr, int(recompute) | (2 if e_soft is not None else 0)), dev)
             saved = (None if recompute else ptr(out_feat), None if recompute else ptr(out2), None if recompute else ptr(cc))
             if own:
@@ -129,7 +129,7 @@ class gat_native:
             raise _lib.FgnnError("gat_stash_own_order: shape mismatch for N=%d H=%d" % (n, h))
         out = torch.empty((e, h), dtype=torch.float32, device=attn_row.device)
         sched = schedule_for(col_ptr, idx_tensor=row_ind, need_positions=False, n_cols=n) if use_schedule else None
-        with torch.cuda.device(attn_row.device):
+        with device_guard(attn_row.device):
             check(lib().fgnn_gat_stash_own_order(n, e, h, float(negative_slope), ptr(col_ptr), ptr(row_ind), ptr(attn_row), ptr(attn_col),
                                                  ptr(edge_max), ptr(edge_sum), ptr(out), sched.handle if sched is not None else None,
                                                  stream_ptr()), "fgnn_gat_stash_own_order")
@@ -148,7 +148,7 @@ class gat_native:
             raise _lib.FgnnError("gat_scatter: shape mismatch for N=%d H=%d" % (n, h))
         e_soft = torch.empty((e, h), dtype=torch.float32, device=attn_row.device)
         e_lrelu = torch.empty((e, h), dtype=torch.float32, device=attn_row.device) if want_lrelu else None
-        with torch.cuda.device(attn_row.device):
+        with device_guard(attn_row.device):
             check(lib().fgnn_gat_scatter(n, e, h, ptr(row_ptr), ptr(col_ind), ptr(attn_row), ptr(attn_col), float(negative_slope),
                                          ptr(e_lrelu), ptr(e_soft), stream_ptr()), "fgnn_gat_scatter")
         return e_lrelu, e_soft
@@ -166,7 +166,7 @@ class gat_native:
             raise _lib.FgnnError("gat_gather_row: shape mismatch for N=%d E=%d H=%d" % (n, e, h))
         out = grad_edge if inplace else torch.empty_like(grad_edge)
         gar = torch.empty((n, h), dtype=torch.float32, device=attn_row.device)
-        with torch.cuda.device(attn_row.device):
+        with device_guard(attn_row.device):
             check(lib().fgnn_gat_gather_row(n, e, h, ptr(row_ptr), ptr(col_ind), ptr(attn_row), ptr(attn_col), ptr(e_lrelu),
                                             float(negative_slope), ptr(e_soft), ptr(grad_edge), ptr(out), ptr(gar), stream_ptr()),
                   "fgnn_gat_gather_row")
@@ -194,7 +194,7 @@ class gat_dense_native:
         new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=W.device)
         score_wt, proj = new(2 * h, fin), new(fin, h * (f + pad)) if pad else None
         both = new(fin, h * (f + pad) + 2 * h) if want_all else None
-        with torch.cuda.device(W.device):
+        with device_guard(W.device):
             check(lib().fgnn_gat_fold_weights(fin, h, f, pad, ptr(W), ptr(attn_l), ptr(attn_r), ptr(score_wt), ptr(proj), ptr(both), stream_ptr()),
                   "fgnn_gat_fold_weights")
         return score_wt, W if proj is None else proj, both
@@ -210,7 +210,7 @@ class gat_dense_native:
             raise _lib.FgnnError("gat_scores: score weights %s do not fit feat %s" % (tuple(score_wt.shape), tuple(feat.shape)))
         row = torch.empty((n, h), dtype=torch.float32, device=feat.device)
         col = torch.empty_like(row)
-        with torch.cuda.device(feat.device):
+        with device_guard(feat.device):
             check(lib().fgnn_gat_scores(n, k, h, ptr(feat), ptr(score_wt), ptr(row), ptr(col), stream_ptr()), "fgnn_gat_scores")
         return row, col
 
@@ -226,7 +226,7 @@ class gat_dense_native:
         rows = lambda t: t if t.dtype == torch.float32 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] else as_f32(t)
         dproj, dscore = rows(dproj), rows(dscore)
         dW, dl, dr = torch.empty_like(W), torch.empty_like(attn_l), torch.empty_like(attn_r)
-        with torch.cuda.device(W.device):
+        with device_guard(W.device):
             check(lib().fgnn_gat_unfold_grads(fin, h, f, pad, ptr(W), ptr(attn_l), ptr(attn_r), ptr(dproj), dproj.stride(0), ptr(dscore), dscore.stride(0),
                                               ptr(dW), ptr(dl), ptr(dr), stream_ptr()), "fgnn_gat_unfold_grads")
         return dW, dl, dr

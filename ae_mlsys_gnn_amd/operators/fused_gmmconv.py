@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import FgnnError, as_f32, as_i32, check, edge_positions, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace
+from .._lib import FgnnError, as_f32, as_i32, check, device_guard, edge_positions, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace
 
 
 def _plain_list_for_summed_backward(n, e):
@@ -45,7 +45,7 @@ class gmm_native:
             residual = None if residual is None else as_f32(residual)
             if (bias is not None and tuple(bias.shape) != (f,)) or (residual is not None and tuple(residual.shape) != (n, f)):
                 raise FgnnError("gmmconv: bias must be [%d] and residual [%d, %d]" % (f, n, f))
-        with torch.cuda.device(node_feat.device):
+        with device_guard(node_feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), node_feat.device)
             if epilogue:
                 check(lib().fgnn_gmm_forward_epilogue(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(node_feat), ptr(pseudo),
@@ -81,7 +81,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # own_order: pseudo, grad_pseudo (and permute) are indexed by the schedule's entry order (gmm_edge_positions(colptr, rowind, True))
         sched = schedule_for(colptr, idx_tensor=None if (sum_kernels and _plain_list_for_summed_backward(n, e)) else rowind, own_order=own_order, n_cols=n)
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             ws, wsb = workspace(lib().fgnn_gmm_backward_workspace_bytes(sched.handle, k, dim, f), dev)
             check(lib().fgnn_gmm_backward(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(node_feat), ptr(pseudo),
                                           ptr(mu), ptr(sigma), ptr(grad_out), int(sum_kernels), ptr(grad_feat), ptr(grad_pseudo), ptr(grad_mu),
@@ -111,7 +111,7 @@ class gmm_native:
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), e))
         out = torch.empty((n, k, f), dtype=torch.float32, device=feat.device)
         sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n)
-        with torch.cuda.device(feat.device):
+        with device_guard(feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), feat.device)
             check(lib().fgnn_gmm_forward(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(feat), ptr(pseudo),
                                          ptr(mu), ptr(sigma), ptr(out), None, 2, sched.handle, ptr(ws), wsb, stream_ptr()),
@@ -142,7 +142,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # same work list as the summed backward, so that one CSC-side copy of own-order edge data serves both kinds of layer
         sched = schedule_for(colptr, idx_tensor=None if _plain_list_for_summed_backward(n, e) else rowind, own_order=own_order, n_cols=n)
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             ws, wsb = workspace(lib().fgnn_gmm_backward_workspace_bytes(sched.handle, k, dim, f), dev)
             check(lib().fgnn_gmm_backward(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(feat), ptr(pseudo),
                                           ptr(mu), ptr(sigma), ptr(grad_out), 2, ptr(parts), ptr(grad_pseudo), ptr(grad_mu),
@@ -156,7 +156,7 @@ class gmm_native:
         e, dim = pseudo.shape
         k = mu.shape[0]
         out = torch.empty((e, k), dtype=torch.float32, device=pseudo.device)
-        with torch.cuda.device(pseudo.device):
+        with device_guard(pseudo.device):
             check(lib().fgnn_gaussian(e, k, dim, ptr(pseudo), ptr(mu), ptr(sigma), ptr(out), stream_ptr()), "fgnn_gaussian")
         return out
 
@@ -169,7 +169,7 @@ class gmm_native:
         gp = torch.empty_like(pseudo)
         gm = torch.empty_like(mu)
         gs = torch.empty_like(sigma)
-        with torch.cuda.device(pseudo.device):
+        with device_guard(pseudo.device):
             ws, wsb = workspace(lib().fgnn_gaussian_backward_workspace_bytes(e, k, dim), pseudo.device)
             check(lib().fgnn_gaussian_backward(e, k, dim, ptr(pseudo), ptr(mu), ptr(sigma), ptr(grad_out), ptr(gp), ptr(gm),
                                                ptr(gs), ptr(ws), wsb, stream_ptr()), "fgnn_gaussian_backward")

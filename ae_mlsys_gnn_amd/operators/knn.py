@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import FgnnError, as_f32, check, lib, ptr, require_cuda, stream_ptr
+from .._lib import FgnnError, as_f32, check, device_guard, lib, ptr, require_cuda, stream_ptr
 
 
 def knn_graph(points, k):
@@ -17,6 +17,6 @@ def knn_graph(points, k):
         raise FgnnError("knn_graph expects points of shape [clouds, points, dims], got %s" % (tuple(points.shape),))
     b, p, d = points.shape
     out = torch.empty(b * p * int(k), dtype=torch.int32, device=points.device)
-    with torch.cuda.device(points.device):
+    with device_guard(points.device):
         check(lib().fgnn_knn_graph(b, p, d, int(k), ptr(points), ptr(out), stream_ptr()), "fgnn_knn_graph")
     return out

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import FgnnError, check, lib, ptr, require_cuda, stream_ptr
+from .._lib import FgnnError, check, device_guard, lib, ptr, require_cuda, stream_ptr
 
 
 class CrossEntropyRows(torch.autograd.Function):
@@ -29,7 +29,7 @@ class CrossEntropyRows(torch.autograd.Function):
             raise FgnnError("cross entropy: overlapping logits rows (stride %d < %d)" % (ld, width))
         lse = torch.empty(n, dtype=torch.float32, device=logits.device)
         row_loss = torch.empty(n, dtype=torch.float32, device=logits.device)
-        with torch.cuda.device(logits.device):
+        with device_guard(logits.device):
             check(lib().fgnn_cross_entropy_forward(n, c, ld, ptr(logits), ptr(labels), ptr(lse), ptr(row_loss), stream_ptr()),
                   "fgnn_cross_entropy_forward")
         ctx.save_for_backward(logits, labels, lse)
@@ -42,7 +42,7 @@ class CrossEntropyRows(torch.autograd.Function):
         n, width = logits.shape
         grad = torch.empty((n, width), dtype=torch.float32, device=logits.device)
         up = grad_rows.contiguous()
-        with torch.cuda.device(logits.device):
+        with device_guard(logits.device):
             check(lib().fgnn_cross_entropy_backward(n, ctx.c, ctx.ld, width, ptr(logits), ptr(labels), ptr(lse), ptr(up), ptr(grad),
                                                     stream_ptr()), "fgnn_cross_entropy_backward")
         return grad, None, None

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import FgnnError, as_f32, as_i32, check, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace, xcd_buckets_enabled
+from .._lib import FgnnError, as_f32, as_i32, check, device_guard, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace, xcd_buckets_enabled
 
 
 def mhspmm(ptr_arr, idx, attention, feat, pos_map=None, own_order=False):
@@ -24,7 +24,7 @@ def mhspmm(ptr_arr, idx, attention, feat, pos_map=None, own_order=False):
         raise FgnnError("mhspmm: attention is %s, expected (%d, %d)" % (tuple(attention.shape), e, h))
     out = torch.empty((ptr_arr.numel() - 1, h, f), dtype=torch.float32, device=feat.device)
     sched = schedule_for(ptr_arr, idx_tensor=idx, n_cols=n, own_order=own_order)          # the ids index the rows of feat
-    with torch.cuda.device(feat.device):
+    with device_guard(feat.device):
         # unweighted: only the partial results of split rows (the same figure as the GMMConv forward's)
         need = (lib().fgnn_mhspmm_workspace_bytes if attention is not None else lib().fgnn_gmm_forward_workspace_bytes)(sched.handle, h, f)
         ws, wsb = workspace(need, feat.device)
@@ -44,7 +44,7 @@ def mhsddmm(rowptr, colind, grad, feat, own_order=False):
     # a skewed graph is walked under its XCD-aware work list (each XCD then gathers from one eighth of the feature
     # rows); otherwise the kernel cuts the entry array into equal chunks itself and needs no list
     sched = schedule_for(rowptr, idx_tensor=colind, n_cols=n, own_order=own_order) if e and xcd_buckets_enabled(rowptr, e) else None
-    with torch.cuda.device(feat.device):
+    with device_guard(feat.device):
         if sched is not None:
             check(lib().fgnn_mhsddmm_scheduled(rowptr.numel() - 1, e, h, f, ptr(rowptr), ptr(colind), ptr(grad), ptr(feat), ptr(out),
                                                sched.handle, stream_ptr()), "fgnn_mhsddmm_scheduled")
@@ -61,7 +61,7 @@ def mhtranspose(permute, attention):
     e = permute.numel()
     w = attention.numel() // max(e, 1) if e else (attention.shape[1] if attention.dim() > 1 else 1)
     out = torch.empty_like(attention)
-    with torch.cuda.device(attention.device):
+    with device_guard(attention.device):
         check(lib().fgnn_gather_rows(e, max(w, 1), ptr(permute), ptr(attention), ptr(out), stream_ptr()), "fgnn_gather_rows")
     return out
 

@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_f32, as_i32, check, lib, ptr, require_cuda, stream_ptr
+from .._lib import as_f32, as_i32, check, device_guard, lib, ptr, require_cuda, stream_ptr
 from .mhspmm import mhsddmm
 
 
@@ -24,7 +24,7 @@ def coo_sddmm(rowind, colind, D1, D2):
     b = D2 if heads else D2.unsqueeze(1)
     e, (_, h, f) = rowind.numel(), a.shape
     out = torch.empty(e, h, dtype=torch.float32, device=a.device)
-    with torch.cuda.device(a.device):
+    with device_guard(a.device):
         check(lib().fgnn_sddmm_coo(e, a.shape[0], b.shape[0], h, f, ptr(rowind), ptr(colind), ptr(a), ptr(b), ptr(out), stream_ptr()),
               "fgnn_sddmm_coo")
     return out if heads else out.squeeze(1)

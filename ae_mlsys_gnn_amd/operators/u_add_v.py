@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_f32, as_i32, check, colsum_plan_for, lib, ptr, require_cuda, stream_ptr, workspace
+from .._lib import as_f32, as_i32, check, colsum_plan_for, device_guard, lib, ptr, require_cuda, stream_ptr, workspace
 
 
 class u_add_v_native:
@@ -15,7 +15,7 @@ class u_add_v_native:
         w = row_val.numel() // max(n, 1)
         e = col_ind.numel()
         out = torch.empty((e,) + tuple(row_val.shape[1:]), dtype=torch.float32, device=row_val.device)
-        with torch.cuda.device(row_val.device):
+        with device_guard(row_val.device):
             check(lib().fgnn_u_add_v(n, e, w, ptr(row_ptr), ptr(col_ind), ptr(row_val), ptr(col_val), ptr(out), stream_ptr()), "fgnn_u_add_v")
         return out
 
@@ -33,7 +33,7 @@ class u_add_v_native:
         grad_row = torch.empty(shape, dtype=torch.float32, device=grad_out.device)
         grad_col = torch.empty(shape, dtype=torch.float32, device=grad_out.device)
         planned = not atomics and e > 0 and (w <= 64 or (w % 4 == 0 and w <= 256))
-        with torch.cuda.device(grad_out.device):
+        with device_guard(grad_out.device):
             if planned:
                 plan = colsum_plan_for(row_ptr, col_ind, n, w)
                 ws, wsb = workspace(lib().fgnn_colsum_workspace_bytes(plan.handle, w), grad_out.device)
