@@ -1458,17 +1458,38 @@ extern "C" int fgnn_u_add_v_backward_planned(int N, int64_t E, int W, const int3
 // reduction over all E edges, done here with per-thread partial sums, a fixed-order workgroup
 // reduction and a fixed-order sum over the workgroups (deterministic).
 #define ELT_BLOCKS 1024
-template <int D>
+// V = 4: a thread takes four consecutive edges, two 128-bit loads and D 128-bit stores (x and y on 16 bytes); V = 1: any alignment.
+// 115 M edges, D = 1: V = 1 283, V = 4 264 us (D = 3, a third of the edges: 208 and 180); bound by memory, 1.38 GB.
+template <int D, int V>
 __global__ __launch_bounds__(256) void edge_linear_tanh_kernel(int64_t E, const float2 *__restrict__ x, const float *__restrict__ W,
                                                                const float *__restrict__ b, float *__restrict__ y)
 {
     float w0[D], w1[D], bb[D];
 #pragma unroll
     for (int o = 0; o < D; ++o) { w0[o] = W[2 * o]; w1[o] = W[2 * o + 1]; bb[o] = b[o]; }
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < E; e += (int64_t)gridDim.x * 256) {
-        const float2 v = x[e];
+    auto one = [&](float2 v, int o) { return tanhf(fmaf(v.y, w1[o], fmaf(v.x, w0[o], bb[o]))); };
+    const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256, groups = E / V;
+    for (int64_t t = t0; t < groups; t += step) {
+        if constexpr (V == 4) {
+            const float4 lo = reinterpret_cast<const float4 *>(x)[2 * t], hi = reinterpret_cast<const float4 *>(x)[2 * t + 1];
+            const float2 v[4] = {make_float2(lo.x, lo.y), make_float2(lo.z, lo.w), make_float2(hi.x, hi.y), make_float2(hi.z, hi.w)};
+            float r[4 * D];
 #pragma unroll
-        for (int o = 0; o < D; ++o) y[e * D + o] = tanhf(fmaf(v.y, w1[o], fmaf(v.x, w0[o], bb[o])));
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int o = 0; o < D; ++o) r[u * D + o] = one(v[u], o);
+#pragma unroll
+            for (int o = 0; o < D; ++o) reinterpret_cast<float4 *>(y)[t * D + o] = make_float4(r[4 * o], r[4 * o + 1], r[4 * o + 2], r[4 * o + 3]);
+        } else {
+            const float2 v = x[t];
+#pragma unroll
+            for (int o = 0; o < D; ++o) y[t * D + o] = one(v, o);
+        }
+    }
+    if (t0 < E - groups * V) {                   // the last E mod V edges
+        const int64_t e = groups * V + t0;
+#pragma unroll
+        for (int o = 0; o < D; ++o) y[e * D + o] = one(x[e], o);
     }
 }
 
@@ -1503,13 +1524,20 @@ __global__ __launch_bounds__(256) void edge_linear_tanh_bwd_kernel(int64_t E, co
         part[(size_t)blockIdx.x * 3 * D + threadIdx.x] = (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
 }
 
-__global__ __launch_bounds__(64) void edge_linear_tanh_finish_kernel(int nblk, int D, const float *__restrict__ part, float *__restrict__ gW,
-                                                                     float *__restrict__ gb)
+// One workgroup per sum; 256 threads add the workgroups' shares in strides, then in a tree (one thread's chain of 1024 dependent
+// loads and adds took 76 us).
+__global__ __launch_bounds__(256) void edge_linear_tanh_finish_kernel(int nblk, int D, const float *__restrict__ part, float *__restrict__ gW,
+                                                                      float *__restrict__ gb)
 {
-    const int i = (int)threadIdx.x;
-    if (i >= 3 * D) return;
+    __shared__ float sh[4];
+    const int i = (int)blockIdx.x;              // 0 .. 3 D - 1
     float s = 0.f;
-    for (int k = 0; k < nblk; ++k) s += part[(size_t)k * 3 * D + i];
+    for (int k = (int)threadIdx.x; k < nblk; k += 256) s += part[(size_t)k * 3 * D + i];
+    s = fg_wave_sum(s);
+    if (fg_lane() == 0) sh[fg_wave()] = s;
+    __syncthreads();
+    if (threadIdx.x) return;
+    s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
     const int o = i / 3, c = i - 3 * o;
     if (c < 2) gW[2 * o + c] = s; else gb[o] = s;
 }
@@ -1524,12 +1552,17 @@ extern "C" int fgnn_edge_linear_tanh(int64_t E, int D, const float *x, const flo
     FGNN_REQUIRE(x && W && b && y, FGNN_ERR_NULL, "fgnn_edge_linear_tanh: NULL argument");
     FGNN_REQUIRE((((uintptr_t)x) & 7u) == 0, FGNN_ERR_ALIGN, "fgnn_edge_linear_tanh: x not 8-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)std::min<int64_t>(8192, (E + 255) / 256));
+    const bool v4 = fgnn_aligned16(x) && fgnn_aligned16(y);
+    const dim3 grid((unsigned)std::min<int64_t>(8192, (E / (v4 ? 4 : 1) + 256) / 256));
+    auto go = [&]<int DD>() {
+        if (v4) hipLaunchKernelGGL((edge_linear_tanh_kernel<DD, 4>), grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y);
+        else hipLaunchKernelGGL((edge_linear_tanh_kernel<DD, 1>), grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y);
+    };
     switch (D) {
-    case 1: hipLaunchKernelGGL(edge_linear_tanh_kernel<1>, grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y); break;
-    case 2: hipLaunchKernelGGL(edge_linear_tanh_kernel<2>, grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y); break;
-    case 3: hipLaunchKernelGGL(edge_linear_tanh_kernel<3>, grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y); break;
-    default: hipLaunchKernelGGL(edge_linear_tanh_kernel<4>, grid, dim3(256), 0, st, E, (const float2 *)x, W, b, y); break;
+    case 1: go.template operator()<1>(); break;
+    case 2: go.template operator()<2>(); break;
+    case 3: go.template operator()<3>(); break;
+    default: go.template operator()<4>(); break;
     }
     return fgnn_launch_status("edge_linear_tanh_kernel");
 }
@@ -1564,6 +1597,6 @@ extern "C" int fgnn_edge_linear_tanh_backward(int64_t E, int D, const float *x, 
     }
     int rc = fgnn_launch_status("edge_linear_tanh_bwd_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(edge_linear_tanh_finish_kernel, dim3(1), dim3(64), 0, st, nblk, D, part, grad_W, grad_b);
+    hipLaunchKernelGGL(edge_linear_tanh_finish_kernel, dim3((unsigned)(3 * D)), dim3(256), 0, st, nblk, D, part, grad_W, grad_b);
     return fgnn_launch_status("edge_linear_tanh_finish_kernel");
 }

@@ -1430,3 +1430,17 @@ def test_gat_dense_kernels(n, fin, h, f, pad):
     assert_close_sum(dW, sum(terms).reshape(fin, -1), sum(t.abs() for t in terms).reshape(fin, -1), "dW")
     for got, s in ((dl, sl), (dr, sr)):
         assert_close_sum(got, (wv * s).sum(0, keepdim=True), (wv * s).abs().sum(0, keepdim=True), "dattn")
+
+
+@pytest.mark.parametrize("e", [1, 3, 4, 5, 1023, 300001])
+@pytest.mark.parametrize("d", [1, 2, 3, 4])
+def test_edge_linear_tanh_alignment(e, d):
+    """Four edges per thread and one per thread (coordinates that start on 8 bytes only) give the same bits, remainders included."""
+    from ae_mlsys_gnn_amd.operators import edge_proj
+    gen = torch.Generator().manual_seed(e)
+    x, w, b = torch.randn(e + 1, 2, generator=gen).to(DEV), torch.randn(d, 2, generator=gen).to(DEV), torch.randn(d, generator=gen).to(DEV)
+    shifted = edge_proj.edge_linear_tanh(x[1:], w, b)
+    assert torch.equal(shifted, edge_proj.edge_linear_tanh(x[1:].clone(), w, b))
+    want = torch.tanh(x[1:].double() @ w.double().t() + b.double())
+    # three roundings of the argument (|x w| <= 30 here) and tanh's own error
+    assert float((shifted.double() - want).abs().max()) < 3 * 30 * 2.0 ** -24 + 1e-6
