@@ -10,8 +10,9 @@ typedef float gd_f4u __attribute__((ext_vector_type(4), aligned(4)));        // 
 
 // One workgroup per input feature i.  score_wt [2H, fin] gets sum_f W[i,h,f] * attn_l[h,f], then the same for attn_r (transposed, so that
 // the score kernel reads four consecutive k of a column at once); proj [fin, H*Fp] (NULL: not wanted) W with `pad` zero columns per
-// head; all [fin, H*Fp + 2H] (NULL) the two side by side, the operand of the input's gradient.  Bound by its launch: W is a few
-// hundred kilobytes.
+// head; all [fin, H*Fp + 2H] (NULL) the two side by side, the operand of the input's gradient.  Bound by its launch (W is a few
+// hundred kilobytes), so the sums are free to run in 64 bits: whatever the order, they are no further off than a reduction
+// of the products.
 __global__ __launch_bounds__(256) void gat_fold_kernel(int fin, int H, int F, int pad, const float *__restrict__ W, const float *__restrict__ al,
                                                        const float *__restrict__ ar, float *__restrict__ score_wt, float *__restrict__ proj,
                                                        float *__restrict__ all)
@@ -25,15 +26,16 @@ __global__ __launch_bounds__(256) void gat_fold_kernel(int fin, int H, int F, in
         if (all) all[(size_t)i * lda + c] = v;
     }
     for (int h = fg_wave(); h < H; h += 4) {
-        float l = 0.f, r = 0.f;
+        double dl = 0., dr = 0.;
         for (int f = fg_lane(); f < F; f += 64) {
-            const float v = w[h * F + f];
-            l = fmaf(v, al[h * F + f], l);
-            r = fmaf(v, ar[h * F + f], r);
+            const double v = w[h * F + f];
+            dl = fma(v, (double)al[h * F + f], dl);
+            dr = fma(v, (double)ar[h * F + f], dr);
         }
-        l = fg_wave_sum(l);
-        r = fg_wave_sum(r);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) { dl += __shfl_xor(dl, off); dr += __shfl_xor(dr, off); }
         if (fg_lane() == 0) {
+            const float l = (float)dl, r = (float)dr;
             score_wt[(size_t)h * fin + i] = l;
             score_wt[(size_t)(H + h) * fin + i] = r;
             if (all) { all[(size_t)i * lda + H * Fp + h] = l; all[(size_t)i * lda + H * Fp + H + h] = r; }
@@ -59,6 +61,8 @@ extern "C" int fgnn_gat_fold_weights(int fin, int H, int F, int pad, const float
 // nodes alone would leave compute units idle, else 1.  Against the library product and the two copies
 // that split it: 2.45 M nodes x 100, 8 heads 430 -> 310 us (196 us to read feat at 5 TB/s); 233 k x 602 217 -> 174; 2708 x 1433, 1 head 32 -> 14;
 // with more than 8 heads the weights' loads weigh in: 100 k x 64, 32 heads 39 -> 24, 30 k x 602, 16 heads 32 -> 37 us.
+// Every 64 dimensions form a sum of their own: one chain over all of them was up to twice as far from the float64 scores as
+// the library product (100 k x 602, 8 heads: 4.4e-7 against 2.2e-7; 1433, 2 heads: 6.8e-7 against 3.4e-7).
 template <int NT, int KS>
 __global__ __launch_bounds__(256) void gat_score_kernel(int64_t n, int K, int H, const float *__restrict__ feat, const float *__restrict__ wt,
                                                         float *__restrict__ arow, float *__restrict__ acol)
@@ -93,12 +97,17 @@ __global__ __launch_bounds__(256) void gat_score_kernel(int64_t n, int K, int H,
                 const int col = t * 16 + r16;
                 b[u][t] = frag(wt + (size_t)(col < 2 * H ? col : 0) * K, c0 + 16 * KS * u + 4 * kq, col < 2 * H);
             }
+        gd_f4 sum[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) sum[t] = gd_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][e], b[u][t][e], acc[t], 0, 0, 0);
+                for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][e], b[u][t][e], sum[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] += sum[t];
     }
     if constexpr (KS > 1) {
         if (wave) {
@@ -150,14 +159,15 @@ extern "C" int fgnn_gat_scores(int64_t n, int K, int H, const float *feat, const
 // (dscore [fin, 2H], rows lds apart):
 //   dW[i,h,f] = dproj[i,h,f] + dscore[i,h] * attn_l[h,f] + dscore[i,H+h] * attn_r[h,f],   dattn_l[h,f] = sum_i W[i,h,f] * dscore[i,h]  (r alike).
 // One launch: the first row_blocks workgroups write dW, each of the others sums 64 columns over the rows, 16 waves side by side in a
-// fixed order.
+// fixed order and in 64 bits: in 32, the chain of fin / 16 terms was further from the float64 sums than the reduction that it
+// replaced (fin = 1433: 1.8e-7 against 0.9e-7, 3703: 2.7e-7 against 1.0e-7), and nothing here waits for the arithmetic.
 #define GU_TPB 1024
 __global__ __launch_bounds__(GU_TPB) void gat_unfold_kernel(int fin, int H, int F, int pad, int row_blocks, const float *__restrict__ W, const float *__restrict__ al,
                                                             const float *__restrict__ ar, const float *__restrict__ dproj, int ldp,
                                                             const float *__restrict__ dscore, int lds, float *__restrict__ dW, float *__restrict__ dal,
                                                             float *__restrict__ dar)
 {
-    __shared__ float sl[GU_TPB], sr[GU_TPB];
+    __shared__ double sl[GU_TPB], sr[GU_TPB];
     const int HF = H * F, Fp = F + pad;
     if ((int)blockIdx.x < row_blocks) {
         const int64_t total = (int64_t)fin * HF;
@@ -170,13 +180,13 @@ __global__ __launch_bounds__(GU_TPB) void gat_unfold_kernel(int fin, int H, int 
     }
     const int lane = fg_lane(), wave = fg_wave(), c = ((int)blockIdx.x - row_blocks) * 64 + lane;
     const int h = c < HF ? c / F : 0;
-    float l = 0.f, r = 0.f;
+    double l = 0., r = 0.;
     if (c < HF) {
 #pragma unroll 4
         for (int i = wave; i < fin; i += GU_TPB / 64) {
-            const float w = W[(size_t)i * HF + c];
-            l = fmaf(w, dscore[(size_t)i * lds + h], l);
-            r = fmaf(w, dscore[(size_t)i * lds + H + h], r);
+            const double w = W[(size_t)i * HF + c];
+            l = fma(w, (double)dscore[(size_t)i * lds + h], l);
+            r = fma(w, (double)dscore[(size_t)i * lds + H + h], r);
         }
     }
     sl[wave * 64 + lane] = l;
@@ -184,8 +194,8 @@ __global__ __launch_bounds__(GU_TPB) void gat_unfold_kernel(int fin, int H, int 
     __syncthreads();
     if (wave || c >= HF) return;
     for (int w = 1; w < GU_TPB / 64; ++w) { l += sl[w * 64 + lane]; r += sr[w * 64 + lane]; }
-    dal[c] = l;
-    dar[c] = r;
+    dal[c] = (float)l;
+    dar[c] = (float)r;
 }
 
 extern "C" int fgnn_gat_unfold_grads(int fin, int H, int F, int pad, const float *W, const float *attn_l, const float *attn_r, const float *dproj, int ldp,

@@ -1432,6 +1432,28 @@ def test_gat_dense_kernels(n, fin, h, f, pad):
         assert_close_sum(got, (wv * s).sum(0, keepdim=True), (wv * s).abs().sum(0, keepdim=True), "dattn")
 
 
+@pytest.mark.parametrize("n,fin,h,f", [(70000, 602, 8, 8), (2708, 1433, 1, 128), (70000, 1433, 2, 30)])
+def test_gat_dense_precision(n, fin, h, f):
+    """How far the sums are from float64, in the 2-norm.  The folded weights and the attention vectors' gradients are summed in 64 bits:
+    one rounding, at most 2^-24 of each value.  A score is a sum of sums of 64 products: with roundings uniform in one unit in the last
+    place and random partial sums, the relative error is 2^-24 / sqrt(3) * sqrt(64 / 2 + fin / (2 * 64)); one chain over all of
+    them would have 2^-24 / sqrt(3) * sqrt(fin / 2)."""
+    from ae_mlsys_gnn_amd.operators.fused_gat import gat_dense_native as gd
+    gen = torch.Generator(device=DEV).manual_seed(fin)
+    new = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    W, al, ar, x = new(fin, h * f), new(1, h, f), new(1, h, f), new(n, fin)
+    rel = lambda got, want: float((got.double() - want).norm() / want.norm())
+    wv = W.double().view(fin, h, f)
+    wt, _, _ = gd.fold(W, al, ar, 0, False)
+    assert rel(wt, torch.cat([(wv * al.double()).sum(-1), (wv * ar.double()).sum(-1)], 1).t()) <= 1.001 * 2.0 ** -24
+    row, col = gd.scores(x, wt)
+    assert rel(torch.cat([row, col], 1), x.double() @ wt.double().t()) <= 2.0 ** -24 / 3 ** 0.5 * (32 + fin / 128) ** 0.5
+    dscore = new(fin, 2 * h)
+    _, dl, dr = gd.unfold(W, al, ar, 0, new(fin, h * f), dscore)
+    for got, d in ((dl, dscore[:, :h]), (dr, dscore[:, h:])):
+        assert rel(got, (wv * d.double().unsqueeze(-1)).sum(0, keepdim=True)) <= 1.001 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("e", [1, 3, 4, 5, 1023, 300001])
 @pytest.mark.parametrize("d", [1, 2, 3, 4])
 def test_edge_linear_tanh_alignment(e, d):
