@@ -56,13 +56,13 @@ class _ProjectScores(torch.autograd.Function):
     def forward(ctx, feat, W, attn_l, attn_r, pad):
         _, hh, ff = attn_l.shape
         score_wt, w_proj, w_all = gat_dense_native.fold(W, attn_l, attn_r, pad, ctx.needs_input_grad[0])
-        feat = feat.contiguous()
         h = torch.matmul(feat, w_proj)
         if gat_dense_native.scores_supported(feat.shape[1], hh):
             row, col = gat_dense_native.scores(feat, score_wt)
         else:
             score = torch.matmul(feat, score_wt.t())
             row, col = score[:, :hh].contiguous(), score[:, hh:].contiguous()
+        # the argument itself: a copy made here (of a strided input) would have no history under create_graph
         ctx.save_for_backward(feat, W, attn_l, attn_r, w_all)
         ctx.pad = pad
         return h.view(-1, hh, ff + pad), row, col
