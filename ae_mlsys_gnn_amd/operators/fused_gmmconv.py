@@ -338,8 +338,11 @@ def project_in_backward(k, fin, fout, input_grad):
     fout floats (rounded up to 4) of the layer's own gradient, for the price of projecting the input again (and of one more
     product for the input's gradient).  Layer steps, gathering K x fin / fout floats: 169 k nodes, 2.3 M edges, 384 / 64 floats 1.69 ->
     1.01 ms (1.16 with the input's gradient), 128 / 64 0.76 -> 0.68 (0.74), 96 / 44 0.66 -> 0.66 (0.69), 128 / 84 0.78 -> 0.89 ms (0.99);
-    300 k nodes, 0.9 M edges, 256 / 100 floats 1.53 -> 1.49 (1.70): the lines lie at ratios of 2 and 3."""
-    return k * fin >= (3 if input_grad else 2) * ((fout + 3) // 4 * 4)
+    300 k nodes, 0.9 M edges, 256 / 100 floats 1.53 -> 1.49 (1.70): the lines lie at ratios of 2 and 3.
+    The summed backward takes rows of at most 1024 floats over all kernels, and keeps the kernels in registers up to 256 each;
+    wider outputs gather the aggregate's gradient, which has no such limit on them."""
+    row = (fout + 3) // 4 * 4
+    return row <= 256 and k * row <= 1024 and k * fin >= (3 if input_grad else 2) * row
 
 
 def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order=False):

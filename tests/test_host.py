@@ -171,6 +171,21 @@ def test_more_argument_errors_without_gpu():
     l.fgnn_schedule_destroy(None)                                                  # no-op on NULL
 
 
+def test_gmm_backward_rule_stays_within_the_operator():
+    """Every layer that the rule sends to the backward with the layer's own gradient is one that the library takes."""
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import gmm_native, project_in_backward
+    l = _lib.lib()
+    for k in range(1, 6):
+        for fin in (4, 64, 96, 128, 252, 256):
+            if not gmm_native.shared_supported(k, fin):
+                continue
+            for fout in list(range(1, 70)) + [85, 86, 100, 127, 128, 129, 200, 255, 256, 257, 258, 300, 340, 341, 344, 352, 384, 512, 513]:
+                for input_grad in (False, True):
+                    if project_in_backward(k, fin, fout, input_grad):
+                        # pointers are missing, sizes are not refused
+                        assert l.fgnn_gmm_backward(8, 8, k, 2, (fout + 3) // 4 * 4, *[None] * 8, 1, *[None] * 6, 0, None) == -1, (k, fin, fout)
+
+
 def test_xcd_mapping_rule_without_gpu():
     """The rule behind the XCD-aware work lists: only a gfx950 device that shows all 256 compute units (eight XCDs of 32)
     is known to spread workgroups round-robin over eight XCDs; a partition of the part or another part gets plain lists."""

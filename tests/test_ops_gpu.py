@@ -373,6 +373,35 @@ def test_gmm_aggregate_linear(fin, fout, k, dim, form, input_grad):
         assert_close_sum(got.grad, want.grad, s[key], "grad " + name, c=c)
 
 
+@pytest.mark.parametrize("fin,fout,k", [(256, 256, 4), (256, 257, 4), (256, 512, 4), (256, 256, 3), (256, 340, 3), (256, 352, 3), (256, 260, 1)])
+@pytest.mark.parametrize("input_grad", [False, True])
+def test_gmm_layer_wide_outputs(fin, fout, k, input_grad):
+    """Layers on either side of the widths that the backward with the layer's own gradient takes (256 floats a row, 1024 over all kernels)
+    train, and their gradients are those of the float64 composed layer."""
+    from ae_mlsys_gnn_amd.layers import GMMConv
+    torch.manual_seed(fout)
+    g = graphs.add_csc_torch(graphs.rmat_graph(200, 2500, seed=4))
+    gd = g.to(DEV)
+    m = GMMConv(fin, fout, 2, k).to(DEV)
+    x, pseudo, go = torch.randn(g.n, fin), torch.rand(g.n_edges, 2), torch.randn(g.n, fout)
+    xd, pd = x.to(DEV).requires_grad_(input_grad), pseudo.to(DEV).requires_grad_(True)
+    out = m(gd.row_ptr, gd.col_ind, gd.col_ptr, gd.row_ind, gd.permute, xd, pd)
+    out.backward(go.to(DEV))
+    params = [m.fc.weight, m.mu, m.inv_sigma, m.bias]
+    leaves = [t.detach().cpu().double().requires_grad_(True) for t in params + [x, pseudo]]
+    ref = orc.gmm_layer_dgl(*leaves[:4], g.row_ptr, g.col_ind, leaves[4], leaves[5], torch.zeros(fout, fin, dtype=torch.float64))
+    ref.backward(go.double())
+    d = [t.detach() for t in leaves]
+    s = orc.gmm_layer_abs_sums(*d[:4], g.row_ptr, g.col_ind, d[4], d[5], torch.zeros(fout, fin, dtype=torch.float64), go.double())
+    c = _gmm_c(d[5], d[1], d[2])
+    assert_close_sum(out, ref.detach(), s["out"], "out", c=c)
+    assert_close_sum(pd.grad, leaves[5].grad, s["grad_pseudo"], "grad pseudo", c=c)
+    if input_grad:
+        assert_close_sum(xd.grad, leaves[4].grad, s["grad_feat"], "grad feat", c=c)
+    for got, want, key in zip(params, leaves, ("grad_fc", "grad_mu", "grad_sigma", "grad_bias")):
+        assert_close_sum(got.grad, want.grad, s[key], key, c=c)
+
+
 # ------------------------------------------------------------------ GAT layer vs the DGL-composed layer
 @pytest.mark.parametrize("fin,f,h,variant", [(64, 16, 4, "our"), (30, 47, 1, "our"), (30, 47, 1, "stash"), (20, 6, 3, "fusescatter"),
                                              (12, 128, 1, "our")])
