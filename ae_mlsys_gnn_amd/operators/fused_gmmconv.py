@@ -349,9 +349,25 @@ def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, ps
     """sum_k (sum_p w[p,k] * feat[colind[p],:]) @ W_k for feat [N, in] and the fc weight [K*out, in]: [N, out].  The forward aggregates the
     input (an edge gathers `in` floats); the backward takes the other order of the two linear steps, so an edge gathers the `out`
     floats of the gradient: T[j,k,:] = sum_p w[p,k] * g[row(p),:] is the gradient of feat @ W_k^T, the derivatives of the Gaussian weights
-    need <g[row(p),:], (feat @ W_k^T)[j,:]>, and the projection is formed again.  Nothing as wide as K x in is kept.
+    need <g[row(p),:], (feat @ W_k^T)[j,:]>, and the projection is formed again.  With one copy of the coordinates nothing as wide as K x in
+    is kept.
     pseudo_csc, own_order: as GmmConvFuseSumTwoOrders; pseudo_csc None: one copy, through permute."""
     return GmmAggregateLinearFunction.apply(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order)
+
+
+class _AggregateHistory(torch.autograd.Function):
+    """An aggregate that is there already, as the result of GmmAggregate / GmmAggregateTwoOrders: the value of `agg`, their backward."""
+
+    @staticmethod
+    def forward(ctx, agg, colptr, rowind, permute, feat, pseudo, mu, sigma, own_order):
+        ctx.save_for_backward(colptr, rowind, permute, feat, pseudo, mu, sigma)
+        ctx.own_order = own_order
+        return agg.view_as(agg)
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        grads = gmm_native.gmmconv_shared_backward(*ctx.saved_tensors, grad_out.contiguous(), own_order=ctx.own_order)
+        return (None, None, None, None) + grads + (None,)
 
 
 class GmmAggregateLinearFunction(torch.autograd.Function):
@@ -362,15 +378,31 @@ class GmmAggregateLinearFunction(torch.autograd.Function):
         agg = gmm_native.gmmconv_shared(rowptr, colind, feat, pseudo, mu, sigma, own_order=own_order)
         w = weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)
         ctx.two_orders, ctx.own_order = pseudo_csc is not None, own_order
-        ctx.save_for_backward(colptr, rowind, None if ctx.two_orders else permute, feat, pseudo_csc if ctx.two_orders else pseudo, mu, sigma, weight)
+        # for a graph of the gradients: the arrays to aggregate again, or, where the CSR copy of the coordinates is the caller's to reuse
+        # after the forward, the aggregate
+        ctx.save_for_backward(colptr, rowind, None if ctx.two_orders else permute, feat, pseudo_csc if ctx.two_orders else pseudo, mu, sigma, weight,
+                              rowptr, colind, agg if ctx.two_orders else None)
         return torch.matmul(agg.view(-1, k * fin), w.t())
 
     @staticmethod
     def backward(ctx, grad_out):
         from ..layers.dense import reduce_over_rows
-        colptr, rowind, permute, feat, pseudo, mu, sigma, weight = ctx.saved_tensors
+        colptr, rowind, permute, feat, pseudo, mu, sigma, weight, rowptr, colind, agg = ctx.saved_tensors
         k, fin = mu.shape[0], feat.shape[1]
         fout = weight.shape[0] // k
+        if torch.is_grad_enabled():
+            # a graph of the gradients is wanted: the weight's gradient from the aggregate, by operations that record one, as in the
+            # layer composed of GmmAggregate and a product (the other gradients come out of the library without history either way)
+            if agg is None:
+                agg = gmm_native.gmmconv_shared(rowptr, colind, feat, pseudo, mu, sigma, own_order=ctx.own_order)
+            agg = _AggregateHistory.apply(agg.detach(), colptr, rowind, permute, feat, pseudo, mu, sigma, ctx.own_order).view(-1, k * fin)
+            g = grad_out.contiguous()
+            grad_w = reduce_over_rows(g, agg).view(fout, k, fin).permute(1, 0, 2).reshape(k * fout, fin)
+            grad_agg = torch.matmul(g, weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)).view(-1, k, fin)
+            grad_feat, grad_pseudo, grad_mu, grad_sigma = gmm_native.gmmconv_shared_backward(colptr, rowind, permute, feat, pseudo, mu, sigma, grad_agg,
+                                                                                             own_order=ctx.own_order)
+            gp = (None, grad_pseudo) if ctx.two_orders else (grad_pseudo, None)
+            return (None, None, None, None, None, grad_feat) + gp + (grad_mu, grad_sigma, grad_w, None)
         pad = (-fout) % 4
         if pad:         # zero columns up to a multiple of 4: the operator then takes its 128-bit row layout
             weight = torch.nn.functional.pad(weight.view(k, fout, fin), (0, 0, 0, pad)).view(-1, fin)
