@@ -106,7 +106,11 @@ class _GMMBase(nn.Module):
             if own_order and pseudo_csc is None and th.is_grad_enabled() and (feat.requires_grad or pseudo.requires_grad):
                 raise ValueError("own_order without pseudo_csc is forward-only")
         two = pseudo_csc is not None
-        if th.is_grad_enabled() and (two or not own_order) and project_in_backward(k, fin, fout, feat.requires_grad):
+        # without a gradient for what is aggregated (frozen Gaussians, constant coordinates and input) the weight's is one product with the
+        # aggregate, and no pass over the edges
+        through_edges = any(t.requires_grad for t in (feat, pseudo_csc if two else pseudo, self.mu, self.inv_sigma))
+        if (th.is_grad_enabled() and through_edges and (two or not own_order)
+                and project_in_backward(k, fin, fout, feat.requires_grad)):
             return GmmAggregateLinear(rowptr, colind, colptr, rowind, None if two else permute, feat, pseudo.detach() if two else pseudo, pseudo_csc,
                                       self.mu, self.inv_sigma, self.fc.weight, own_order=own_order)
         if two or own_order:

@@ -1,5 +1,5 @@
-"""Gradients of gradients (create_graph=True) through the layers, on the CPU: the library calls are replaced by the same computation in
-torch, so what is tested is which operations the backward passes record.  Gradient penalties train on these."""
+"""The layers' backward passes on the CPU, the library calls replaced by the same computation in torch: what is tested is which operations
+they record (gradients of gradients, on which gradient penalties train) and which passes over the edges they run."""
 import pytest
 import torch
 
@@ -128,3 +128,19 @@ def test_gmm_gradient_penalty_on_the_weight(gmm_on_cpu, fin, fout, k, two, input
         result.append((gw,) + _grads((gw * gw).sum(), wrt))
     for got, want in zip(*result):
         assert torch.allclose(got, want, rtol=1e-9, atol=1e-9 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("frozen", [False, True])
+def test_gmm_frozen_gaussians_need_no_pass_over_the_edges(gmm_on_cpu, two, frozen):
+    """With constant coordinates and input, the backward walks the edges for mu and inv_sigma only."""
+    m, x, ps, run, composed = _gmm_case(24, 9, 3, two, False)
+    ps.requires_grad_(False)
+    m.mu.requires_grad_(not frozen)
+    m.inv_sigma.requires_grad_(not frozen)
+    run().sum().backward()
+    assert gmm_on_cpu == (["shared"] if frozen else ["shared", "backward"])
+    got = m.fc.weight.grad.clone()
+    m.fc.weight.grad = None
+    composed().sum().backward()
+    assert torch.allclose(got, m.fc.weight.grad, rtol=1e-9, atol=1e-9)
