@@ -110,7 +110,7 @@ class _GMMBase(nn.Module):
         # aggregate, and no pass over the edges
         through_edges = any(t.requires_grad for t in (feat, pseudo_csc if two else pseudo, self.mu, self.inv_sigma))
         if (th.is_grad_enabled() and through_edges and (two or not own_order)
-                and project_in_backward(k, fin, fout, feat.requires_grad)):
+                and project_in_backward(k, fin, fout, feat.requires_grad, feat.shape[0], colind.numel())):
             return GmmAggregateLinear(rowptr, colind, colptr, rowind, None if two else permute, feat, pseudo.detach() if two else pseudo, pseudo_csc,
                                       self.mu, self.inv_sigma, self.fc.weight, own_order=own_order)
         if two or own_order:

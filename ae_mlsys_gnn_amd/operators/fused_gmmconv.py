@@ -333,16 +333,24 @@ class GmmAggregateTwoOrdersFunction(torch.autograd.Function):
         return None, None, None, None, grad_feat, None, grad_pseudo_csc, grad_mu, grad_sigma, None
 
 
-def project_in_backward(k, fin, fout, input_grad):
-    """Which rows the backward of an aggregate-first layer gathers per edge: K x fin floats, the gradient of the aggregate, or the
-    fout floats (rounded up to 4) of the layer's own gradient, for the price of projecting the input again (and of one more
+def project_in_backward(k, fin, fout, input_grad, n, e):
+    """Which rows the backward of an aggregate-first layer (n nodes, e edges) gathers per edge: K x fin floats, the gradient of the aggregate,
+    or the fout floats (rounded up to 4) of the layer's own gradient, for the price of projecting the input again (and of one more
     product for the input's gradient).  Layer steps, gathering K x fin / fout floats: 169 k nodes, 2.3 M edges, 384 / 64 floats 1.69 ->
     1.01 ms (1.16 with the input's gradient), 128 / 64 0.76 -> 0.68 (0.74), 96 / 44 0.66 -> 0.66 (0.69), 128 / 84 0.78 -> 0.89 ms (0.99);
     300 k nodes, 0.9 M edges, 256 / 100 floats 1.53 -> 1.49 (1.70): the lines lie at ratios of 2 and 3.
+    With the input's gradient and few edges the product's n fin K fout multiply-adds outweigh the gathers, at 50 of them for every float that an
+    edge no longer gathers: 300 k nodes, 1024 / 256 floats: 5.59 -> 6.31 ms at 3 edges a node, 7.17 -> 6.81 at 9; 384 / 128: 1.85 ->
+    2.02 and 2.27 -> 2.18; 1024 / 128: 3.95 -> 3.64 at 3.  On dense graphs rows of up to two cache lines cost what rows of one do: 32 / 16
+    floats 0.95 -> 0.90 ms at 51 edges a node, 0.84 -> 0.87 at 200; 64 / 32 0.86 -> 0.89 there and 5.94 -> 6.00 at 258.
     The summed backward takes rows of at most 1024 floats over all kernels, and keeps the kernels in registers up to 256 each;
     wider outputs gather the aggregate's gradient, which has no such limit on them."""
     row = (fout + 3) // 4 * 4
-    return row <= 256 and k * row <= 1024 and k * fin >= (3 if input_grad else 2) * row
+    if row > 256 or k * row > 1024 or (k * fin <= 64 and e >= 128 * n):
+        return False
+    if not input_grad:
+        return k * fin >= 2 * row
+    return k * fin >= 3 * row and n * fin * k * fout <= 50 * e * (k * fin - row)
 
 
 def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order=False):

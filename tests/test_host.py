@@ -181,9 +181,19 @@ def test_gmm_backward_rule_stays_within_the_operator():
                 continue
             for fout in list(range(1, 70)) + [85, 86, 100, 127, 128, 129, 200, 255, 256, 257, 258, 300, 340, 341, 344, 352, 384, 512, 513]:
                 for input_grad in (False, True):
-                    if project_in_backward(k, fin, fout, input_grad):
+                    if project_in_backward(k, fin, fout, input_grad, 10, 1000):
                         # pointers are missing, sizes are not refused
                         assert l.fgnn_gmm_backward(8, 8, k, 2, (fout + 3) // 4 * 4, *[None] * 8, 1, *[None] * 6, 0, None) == -1, (k, fin, fout)
+
+
+@pytest.mark.parametrize("k,fin,fout,input_grad,degree,want", [
+    (4, 256, 256, True, 3, False), (4, 256, 256, True, 9, True), (4, 256, 256, False, 3, True), (3, 128, 128, True, 3, False),
+    (3, 128, 128, True, 9, True), (4, 256, 128, True, 3, True), (3, 128, 64, True, 4, True), (2, 16, 16, False, 50, True),
+    (2, 16, 16, False, 200, False), (2, 32, 32, False, 260, False), (3, 32, 32, False, 260, True)])
+def test_gmm_backward_rule_follows_the_degree(k, fin, fout, input_grad, degree, want):
+    """Both sides of the lines that the degree draws (layer steps measured on either side)."""
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import project_in_backward
+    assert project_in_backward(k, fin, fout, input_grad, 100000, 100000 * degree) is want
 
 
 def test_xcd_mapping_rule_without_gpu():
