@@ -133,6 +133,10 @@ class FusedEdgeConvPairFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         max_idx, out = ctx.saved_tensors
+        if torch.is_grad_enabled():             # a graph of the gradients is wanted: the same in operations that record one
+            g = grad_out if ctx.slope is None else grad_out * torch.where(out > 0, 1.0, float(ctx.slope))
+            src = torch.zeros_like(g).scatter_add(0, max_idx.long(), g)
+            return None, None, torch.cat([src - g, g], 1), None, None
         grad_out = as_f32(grad_out)
         n, f = grad_out.shape
         grad_h = torch.empty((n, 2 * f), dtype=torch.float32, device=grad_out.device)

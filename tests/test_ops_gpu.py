@@ -725,6 +725,32 @@ def test_knn_graph_ties_are_ordered_by_id():
         knn_graph(torch.zeros(1, 200, 3, device=DEV), 129)
 
 
+@pytest.mark.parametrize("slope", [None, 0.2])
+@pytest.mark.parametrize("block", [None, 32])
+def test_edgeconv_layer_gradient_penalty(slope, block):
+    """Penalties on the layer's gradients (create_graph=True) against the composed layer: the values, and what they pass on to both
+    weights and the input."""
+    from ae_mlsys_gnn_amd.layers import EdgeConv
+    torch.manual_seed(4)
+    n, k = 96, 5
+    m = EdgeConv(6, 7).to(DEV)
+    nb = (torch.randint(0, 32, (n, k)) + 32 * torch.arange(3).repeat_interleave(32).unsqueeze(1)).to(DEV)
+    x = torch.randn(n, 6, device=DEV, requires_grad=True)
+    params = [m.theta.weight, m.phi.weight, x]
+
+    def composed():
+        h = x @ torch.cat([m.theta.weight, m.phi.weight]).t()
+        best = ((h[:, 7:] - h[:, :7]).unsqueeze(1) + h[:, :7][nb]).amax(1)
+        return best if slope is None else torch.nn.functional.leaky_relu(best, slope)
+
+    result = []
+    for run in (lambda: m(k, nb.view(-1).int(), x, block=block, negative_slope_out=slope), composed):
+        grads = torch.autograd.grad((run() ** 3).sum(), params, create_graph=True)
+        result.append(grads + torch.autograd.grad(sum((g * g).sum() for g in grads), params))
+    for got, want in zip(*result):          # float32 sums of up to 96 x 7 terms, three products deep: a few hundred roundings of the largest
+        assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("b,p,f,k,block", [(3, 100, 8, 5, 100), (3, 100, 8, 5, None), (2, 65, 3, 1, 65), (2, 300, 130, 9, 64), (2, 40, 12, 7, 5000),
                                            (9, 128, 64, 20, 128), (1, 2049, 5, 3, 2049)])
 @pytest.mark.parametrize("slope", [None, 0.2])
