@@ -411,7 +411,6 @@ extern "C" int fgnn_edgeconv_pair_backward(int N, int F, int block, const int32_
     FGNN_REQUIRE(N >= 0 && F >= 1 && F <= (1 << 28), FGNN_ERR_SHAPE, "fgnn_edgeconv_pair_backward: bad sizes N=%d F=%d", N, F);
     FGNN_REQUIRE(argmax && grad_out && grad_h, FGNN_ERR_NULL, "fgnn_edgeconv_pair_backward: NULL argument");
     FGNN_REQUIRE(out_slope > 0.f, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_backward: out_slope=%g must be positive", (double)out_slope);
-    FGNN_REQUIRE((int64_t)N * F <= 2147483647LL, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_backward: N*F exceeds int32");
     if (N == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     const int fs = block > 0 ? ec_blocked_fs(block) : 0;
@@ -422,6 +421,8 @@ extern "C" int fgnn_edgeconv_pair_backward(int N, int F, int block, const int32_
         hipLaunchKernelGGL(edgeconv_bwd_kernel, dim3(grid), dim3(256), 0, st, total, F, argmax, grad_out, out, out_slope, grad_h, nullptr, 2 * F);
         return fgnn_launch_status("edgeconv_bwd_kernel");
     }
+    // the blocked form keeps element numbers in 32 bits; the plain scatter above has no such limit
+    FGNN_REQUIRE((int64_t)N * F <= 2147483647LL, FGNN_ERR_LIMIT, "fgnn_edgeconv_pair_backward: N*F exceeds int32");
     const size_t need = fgnn_edgeconv_backward_blocked_workspace_bytes(N, F);
     FGNN_REQUIRE(workspace && workspace_bytes >= need, FGNN_ERR_WORKSPACE, "fgnn_edgeconv_pair_backward: workspace %zu < %zu bytes", workspace_bytes, need);
     return edgeconv_backward_blocked_run(N, F, block, fs, argmax, grad_out, grad_h, (int *)workspace, st, out, out_slope, grad_h + F, 2 * F, 1);

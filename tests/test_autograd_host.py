@@ -127,7 +127,7 @@ def test_gmm_gradient_penalty_on_the_weight(gmm_on_cpu, fin, fout, k, two, input
         gw = _grads(loss, [m.fc.weight], create_graph=True)[0]
         result.append((gw,) + _grads((gw * gw).sum(), wrt))
     for got, want in zip(*result):
-        assert torch.allclose(got, want, rtol=1e-9, atol=1e-9 * float(want.abs().max()))
+        assert torch.allclose(got, want, rtol=1e-9, atol=1e-9 * float(want.detach().abs().max()))
 
 
 @pytest.mark.parametrize("two", [False, True])

@@ -725,6 +725,24 @@ def test_knn_graph_ties_are_ordered_by_id():
         knn_graph(torch.zeros(1, 200, 3, device=DEV), 129)
 
 
+def test_edgeconv_pair_more_than_2_31_elements():
+    """The plain form has no 32-bit element numbers in either pass (2^31 + 1024 elements; 60 GB)."""
+    from ae_mlsys_gnn_amd.operators import fused_edgeconv as fe
+    n, f = (1 << 21) + 1, 1024
+    src = torch.roll(torch.arange(n, dtype=torch.int32, device=DEV), 1)           # the row before, the last one for row 0
+    v = (torch.arange(n, device=DEV) % 7).float()
+    h = torch.empty(n, 2 * f, device=DEV)
+    h[:, :f] = v.unsqueeze(1)                                                     # theta; phi = 1
+    h[:, f:] = 1
+    h.requires_grad_(True)
+    out = fe.fused_edgeconv_pair_op(1, src, h)
+    prev = torch.roll(v, 1)
+    assert bool((out == (1 - v + prev).unsqueeze(1)).all())
+    out.backward(v.unsqueeze(1).expand(n, f).contiguous())
+    nxt = torch.roll(v, -1)
+    assert bool((h.grad[:, :f] == (nxt - v).unsqueeze(1)).all()) and bool((h.grad[:, f:] == v.unsqueeze(1)).all())
+
+
 @pytest.mark.parametrize("slope", [None, 0.2])
 @pytest.mark.parametrize("block", [None, 32])
 def test_edgeconv_layer_gradient_penalty(slope, block):
@@ -748,7 +766,7 @@ def test_edgeconv_layer_gradient_penalty(slope, block):
         grads = torch.autograd.grad((run() ** 3).sum(), params, create_graph=True)
         result.append(grads + torch.autograd.grad(sum((g * g).sum() for g in grads), params))
     for got, want in zip(*result):          # float32 sums of up to 96 x 7 terms, three products deep: a few hundred roundings of the largest
-        assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max())
+        assert float((got - want).detach().abs().max()) <= 1e-4 * float(want.detach().abs().max())
 
 
 @pytest.mark.parametrize("b,p,f,k,block", [(3, 100, 8, 5, 100), (3, 100, 8, 5, None), (2, 65, 3, 1, 65), (2, 300, 130, 9, 64), (2, 40, 12, 7, 5000),
