@@ -582,7 +582,9 @@ extern "C" int fgnn_knn_graph(int n_clouds, int P, int D, int k, const float *po
     // The matrix form costs less per dimension (64 clouds: 1.4 against 4 us at 1024 points, 0.5 against 0.8 at 512) and more per query
     // (140 against 115 us, 44 against 30): equal at 10 to 16 and at 45 dimensions.  At 256 points it loses up to 128 dimensions
     // (46 against 44 us; 34 against 29 at 64).
-    if (k <= 64 && ((rg == 4 && D >= 16) || (rg == 2 && D >= 48))) {
+    // A launch holds fewer than 2^32 threads in one dimension: 2^23 workgroups of the matrix form, whose grid has only one.
+    const bool fits = (int64_t)n_clouds * ((P + KNN_MQ - 1) / KNN_MQ) <= (1 << 23) - FGNN_NUM_XCD;
+    if (k <= 64 && fits && ((rg == 4 && D >= 16) || (rg == 2 && D >= 48))) {
         if (rg == 2) knn_mfma_launch<2>(n_clouds, P, D, k, points, src_ind, st);
         else knn_mfma_launch<4>(n_clouds, P, D, k, points, src_ind, st);
     } else if (k <= 64) {

@@ -686,6 +686,15 @@ def test_coo_and_csr_sddmm(h, f):
     assert sddmm.coo_sddmm(rows[:0].to(DEV), cols[:0].to(DEV), a.float().to(DEV), b.float().to(DEV)).shape == (0, h)
 
 
+def test_knn_graph_of_very_many_points():
+    """More queries than the matrix-core form's grid holds (2^23 workgroups of 32): every point is its own nearest neighbour."""
+    from ae_mlsys_gnn_amd.operators.knn import knn_graph
+    b, p = 65535, 4100
+    points = torch.rand(b, p, 16, device=DEV)
+    out = knn_graph(points, 1)
+    assert torch.equal(out, torch.arange(b * p, dtype=torch.int32, device=DEV))
+
+
 # ------------------------------------------------------------------ kNN graph builder
 @pytest.mark.parametrize("b,p,d,k", [(3, 100, 3, 5), (2, 1024, 3, 20), (2, 300, 64, 20), (1, 64, 7, 64), (4, 65, 2, 1),
                                      (2, 2500, 5, 70), (1, 1025, 9, 128), (2, 257, 11, 65), (3, 513, 1, 8)])
