@@ -127,6 +127,11 @@ struct rs_args {
 // hint[k] = row of position min(k << CSC_HINT_SHIFT, n - 1): a coarse inverse of row_ptr.  128 = the records a wave of a small
 // tile owns, so that every wave of RS_CSR finds the row of its first record there.
 #define CSC_HINT_SHIFT 7
+// Up to this many rows per position of a tile their starts are scanned for the positions' rows; beyond, the positions are searched
+// for.  Scanning costs one workgroup 1 us per thousand rows (100 M empty rows between two halves of 1 M entries: 16 ms, searched 0.08);
+// where all tiles span such runs the two meet at about 10 rows per entry (8 M entries: scanned 365 us at 10 and 458 at 14, searched
+// 423 at 18).
+#define CSC_SCAN_ROWS 8
 static int csc_num_hints(int64_t E) { return E > 0 ? (int)((E - 1) >> CSC_HINT_SHIFT) + 2 : 0; }
 __global__ __launch_bounds__(256) void csc_row_hint_kernel(int64_t n, int n_rows, int n_hint, const int *__restrict__ row_ptr, int *__restrict__ hint)
 {
@@ -136,7 +141,7 @@ __global__ __launch_bounds__(256) void csc_row_hint_kernel(int64_t n, int n_rows
     if (p > n - 1) p = n - 1;
     int lo = 0, hi = n_rows;                    // the last r with row_ptr[r] <= p
     while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
+        const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
         if (row_ptr[mid] <= (int)p) lo = mid; else hi = mid;
     }
     hint[k] = lo;
@@ -182,37 +187,51 @@ __global__ __launch_bounds__(RS_TPB, 8) void rs_scatter_kernel(rs_args A, int64_
         rec[it] = r;
     }
     if constexpr (IN == RS_CSR) {
-        // row of every position of the tile: the starts of the non-empty rows leave their number in LDS (several rows that
-        // start at one position are empty but for the last, the largest number), then a running maximum over the positions
-        int *mark = reinterpret_cast<int *>(buf);
-        for (int i = tid; i < TILE; i += RS_TPB) mark[i] = 0;
-        __syncthreads();
         const int64_t last = tile0 + TILE < n ? tile0 + TILE : n - 1;      // rows up to the one that holds the next tile's first position
         const int r0 = A.hint[tile0 >> CSC_HINT_SHIFT], r1 = A.hint[(last + (1 << CSC_HINT_SHIFT) - 1) >> CSC_HINT_SHIFT];
-        for (int r = r0 + 1 + tid; r <= r1; r += RS_TPB) {
-            const int64_t o = (int64_t)A.row_ptr[r] - tile0;
-            if (o >= 0 && o < TILE) atomicMax(&mark[o], r);
+        if (r1 - r0 > CSC_SCAN_ROWS * TILE) {
+            // the tile spans a long run of empty rows: each position is searched for between the two hints around it
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) {
+                const int p = (int)(tile0 + min(wave * SUB + it * 64 + lane, count - 1));
+                int lo = A.hint[p >> CSC_HINT_SHIFT], hi = A.hint[(p >> CSC_HINT_SHIFT) + 1] + 1;
+                while (hi - lo > 1) {
+                    const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
+                    if (A.row_ptr[mid] <= p) lo = mid; else hi = mid;
+                }
+                rec[it].y = lo;
+            }
+        } else {
+            // row of every position of the tile: the starts of the non-empty rows leave their number in LDS (several rows that
+            // start at one position are empty but for the last, the largest number), then a running maximum over the positions
+            int *mark = reinterpret_cast<int *>(buf);
+            for (int i = tid; i < TILE; i += RS_TPB) mark[i] = 0;
+            __syncthreads();
+            for (int64_t r = (int64_t)r0 + 1 + tid; r <= r1; r += RS_TPB) {
+                const int64_t o = (int64_t)A.row_ptr[r] - tile0;
+                if (o >= 0 && o < TILE) atomicMax(&mark[o], (int)r);
+            }
+            __syncthreads();
+            // a lane takes ITEMS consecutive positions, the lanes of a wave the wave's SUB positions
+            int m[ITEMS];
+            int *own = mark + wave * SUB + lane * ITEMS;
+            int top = 0;
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) { m[it] = own[it]; top = max(top, m[it]); m[it] = top; }
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int t = __shfl_up(top, off);
+                if (lane >= off) top = max(top, t);
+            }
+            int run = __shfl_up(top, 1);
+            run = max(lane == 0 ? 0 : run, first < n ? A.hint[first >> CSC_HINT_SHIFT] : 0);
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) own[it] = max(m[it], run);
+            fg_wave_lds_sync();
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) rec[it].y = mark[wave * SUB + it * 64 + lane];
+            __syncthreads();
         }
-        __syncthreads();
-        // a lane takes ITEMS consecutive positions, the lanes of a wave the wave's SUB positions
-        int m[ITEMS];
-        int *own = mark + wave * SUB + lane * ITEMS;
-        int top = 0;
-#pragma unroll
-        for (int it = 0; it < ITEMS; ++it) { m[it] = own[it]; top = max(top, m[it]); m[it] = top; }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(top, off);
-            if (lane >= off) top = max(top, t);
-        }
-        int run = __shfl_up(top, 1);
-        run = max(lane == 0 ? 0 : run, first < n ? A.hint[first >> CSC_HINT_SHIFT] : 0);
-#pragma unroll
-        for (int it = 0; it < ITEMS; ++it) own[it] = max(m[it], run);
-        fg_wave_lds_sync();
-#pragma unroll
-        for (int it = 0; it < ITEMS; ++it) rec[it].y = mark[wave * SUB + it * 64 + lane];
-        __syncthreads();
     }
     for (int d = tid; d < RS_WAVES * RS_MAX_DIGITS / 2; d += RS_TPB) reinterpret_cast<int *>(buf)[d] = 0;
     __syncthreads();

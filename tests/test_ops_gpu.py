@@ -46,6 +46,25 @@ def test_csr2csc_duplicates_unsorted_and_empty():
     assert torch.equal(out.cpu(), torch.from_numpy(pm).float() * 0.5)
 
 
+@pytest.mark.parametrize("e", [2, 2048, 2049, 100000, 4300000])
+@pytest.mark.parametrize("gap", [0, 16383, 16384, 16385, 70000, 3000000])
+def test_csr2csc_long_runs_of_empty_rows(e, gap):
+    """Runs of empty rows in front of, between and behind the entries, on either side of the lengths (8 rows per position of a tile of 2048
+    or 8192) beyond which a position's row is searched for, not scanned for."""
+    from ae_mlsys_gnn_amd.operators import csr2csc as op
+    gen = torch.Generator(device=DEV).manual_seed(e)
+    used = 3000
+    r = torch.sort(torch.randint(0, used, (e,), generator=gen, device=DEV)).values
+    r = gap + r + torch.where(r >= used // 2, gap, 0)
+    n = used + 3 * gap
+    row_ptr = torch.searchsorted(r, torch.arange(n + 1, device=DEV)).int()
+    col = torch.randint(0, 500, (e,), generator=gen, device=DEV).int()
+    col_ptr, row_ind, permute = op.csr2csc(row_ptr, col, 500)
+    order = torch.sort(col, stable=True).indices
+    assert torch.equal(permute.long(), order) and torch.equal(row_ind.long(), r[order])
+    assert torch.equal(col_ptr.long(), torch.searchsorted(col[order].long(), torch.arange(501, device=DEV)))
+
+
 def test_csr2csc_round_trip_large():
     # transpose of the transpose is the original (columns sorted inside rows): size-independent property
     from ae_mlsys_gnn_amd.operators import csr2csc as op
