@@ -632,6 +632,19 @@ __global__ __launch_bounds__(256) void coo_count_kernel(int64_t n, const int *__
     if (threadIdx.x == 0) sums[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
+// row_ptr[from .. to] = v for every lane of a wave (all of them call it; to < from: nothing).  Runs of more than a few rows are written by
+// the whole wave: one lane's stores to 10 M empty rows took half a second.
+__device__ __forceinline__ void coo_fill_rows(int *__restrict__ row_ptr, int from, int to, int v)
+{
+    const bool big = (int64_t)to - from >= 16;
+    if (!big)
+        for (int i = from; i <= to; ++i) row_ptr[i] = v;
+    for (unsigned long long m = __ballot(big); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m), a = __builtin_amdgcn_readlane(from, l), b = __builtin_amdgcn_readlane(to, l), x = __builtin_amdgcn_readlane(v, l);
+        for (int64_t i = (int64_t)a + fg_lane(); i <= b; i += 64) row_ptr[i] = x;
+    }
+}
+
 // The CSR from the sorted records: the first record of every group writes its source at the group's position and, where its
 // destination is a new one, the row pointers up to it; every input edge learns the position of its group.  sums: exclusive
 // tile offsets (NULL: no merging, record q is entry q).
@@ -672,17 +685,14 @@ __global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, c
         for (int w = 0; w < wave; ++w) ofs += wave_cnt[k][w];
         const int pos = ofs + before[k] - 1;
         run += (wave_cnt[k][0] + wave_cnt[k][1]) + (wave_cnt[k][2] + wave_cnt[k][3]);
+        const bool head = (fl >> k) & 1, end = q == n - 1;
         if (q < n) {
-            if ((fl >> k) & 1) {
-                col_ind[pos] = r[k].y;
-                for (int i = prev_dst[k] + 1; i <= r[k].x; ++i) row_ptr[i] = pos;
-            }
-            if (q == n - 1) {
-                for (int i = r[k].x + 1; i <= n_rows; ++i) row_ptr[i] = pos + 1;
-                *n_out = pos + 1;
-            }
+            if (head) col_ind[pos] = r[k].y;
+            if (end) *n_out = pos + 1;
             if constexpr (TRIPLE) edge_pos[rec[q].y] = pos;
         }
+        coo_fill_rows(row_ptr, prev_dst[k] + 1, head ? r[k].x : prev_dst[k], pos);
+        if (base + SC_TILE >= n) coo_fill_rows(row_ptr, r[k].x + 1, end ? n_rows : r[k].x, pos + 1);      // uniform: the last tile
     }
 }
 

@@ -46,6 +46,27 @@ def test_csr2csc_duplicates_unsorted_and_empty():
     assert torch.equal(out.cpu(), torch.from_numpy(pm).float() * 0.5)
 
 
+@pytest.mark.parametrize("gap", [0, 1, 14, 15, 16, 17, 63, 64, 65, 100000])
+@pytest.mark.parametrize("e", [1, 3, 64, 5000])
+@pytest.mark.parametrize("dedupe", [False, True])
+def test_coo2csr_runs_of_empty_rows(e, gap, dedupe):
+    """Runs of empty rows in front of, between and behind the used ones: written by one lane up to 16 rows, by the wave beyond."""
+    from ae_mlsys_gnn_amd.operators import csr2csc as op
+    gen = torch.Generator(device=DEV).manual_seed(e + gap)
+    dst = torch.randint(0, 40, (e,), generator=gen, device=DEV) * (gap + 1) + gap
+    src = torch.randint(0, 50, (e,), generator=gen, device=DEV)
+    n = 42 * (gap + 1) + gap
+    row_ptr, col_ind, pos = op.coo2csr(dst.int(), src.int(), n, 50, dedupe=dedupe, return_edge_pos=True)
+    keys = dst * 50 + src
+    keys, inverse = torch.unique(keys, return_inverse=True) if dedupe else (torch.sort(keys).values, None)
+    assert torch.equal(row_ptr.long(), torch.searchsorted(keys // 50, torch.arange(n + 1, device=DEV)))
+    assert torch.equal(col_ind.long(), keys % 50)
+    if dedupe:
+        assert torch.equal(pos.long(), inverse)
+    else:
+        assert torch.equal(torch.sort(pos).values.long(), torch.arange(e, device=DEV)) and torch.equal(col_ind[pos.long()].long(), src)
+
+
 @pytest.mark.parametrize("e", [2, 2048, 2049, 100000, 4300000])
 @pytest.mark.parametrize("gap", [0, 16383, 16384, 16385, 70000, 3000000])
 def test_csr2csc_long_runs_of_empty_rows(e, gap):
