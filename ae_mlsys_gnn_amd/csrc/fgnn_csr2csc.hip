@@ -189,22 +189,24 @@ __global__ __launch_bounds__(RS_TPB, 8) void rs_scatter_kernel(rs_args A, int64_
     if constexpr (IN == RS_CSR) {
         const int64_t last = tile0 + TILE < n ? tile0 + TILE : n - 1;      // rows up to the one that holds the next tile's first position
         const int r0 = A.hint[tile0 >> CSC_HINT_SHIFT], r1 = A.hint[(last + (1 << CSC_HINT_SHIFT) - 1) >> CSC_HINT_SHIFT];
+        // row of every position of the tile, in LDS
+        int *mark = reinterpret_cast<int *>(buf);
         if (r1 - r0 > CSC_SCAN_ROWS * TILE) {
             // the tile spans a long run of empty rows: each position is searched for between the two hints around it
-#pragma unroll
-            for (int it = 0; it < ITEMS; ++it) {
-                const int p = (int)(tile0 + min(wave * SUB + it * 64 + lane, count - 1));
+#pragma unroll 1
+            for (int i = tid; i < count; i += RS_TPB) {
+                const int p = (int)(tile0 + i);
                 int lo = A.hint[p >> CSC_HINT_SHIFT], hi = A.hint[(p >> CSC_HINT_SHIFT) + 1] + 1;
                 while (hi - lo > 1) {
                     const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
                     if (A.row_ptr[mid] <= p) lo = mid; else hi = mid;
                 }
-                rec[it].y = lo;
+                mark[i] = lo;
             }
+            __syncthreads();
         } else {
-            // row of every position of the tile: the starts of the non-empty rows leave their number in LDS (several rows that
-            // start at one position are empty but for the last, the largest number), then a running maximum over the positions
-            int *mark = reinterpret_cast<int *>(buf);
+            // the starts of the non-empty rows leave their number (several rows that start at one position are empty but for the
+            // last, the largest number), then a running maximum over the positions
             for (int i = tid; i < TILE; i += RS_TPB) mark[i] = 0;
             __syncthreads();
             for (int64_t r = (int64_t)r0 + 1 + tid; r <= r1; r += RS_TPB) {
@@ -228,10 +230,10 @@ __global__ __launch_bounds__(RS_TPB, 8) void rs_scatter_kernel(rs_args A, int64_
 #pragma unroll
             for (int it = 0; it < ITEMS; ++it) own[it] = max(m[it], run);
             fg_wave_lds_sync();
-#pragma unroll
-            for (int it = 0; it < ITEMS; ++it) rec[it].y = mark[wave * SUB + it * 64 + lane];
-            __syncthreads();
         }
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) rec[it].y = mark[wave * SUB + it * 64 + lane];
+        __syncthreads();
     }
     for (int d = tid; d < RS_WAVES * RS_MAX_DIGITS / 2; d += RS_TPB) reinterpret_cast<int *>(buf)[d] = 0;
     __syncthreads();
