@@ -634,13 +634,15 @@ __global__ __launch_bounds__(256) void coo_count_kernel(int64_t n, const int *__
     if (threadIdx.x == 0) sums[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// row_ptr[from .. to] = v for every lane of a wave (all of them call it; to < from: nothing).  Runs of more than a few rows are written by
-// the whole wave: one lane's stores to 10 M empty rows took half a second.
-__device__ __forceinline__ void coo_fill_rows(int *__restrict__ row_ptr, int from, int to, int v)
+// row_ptr[from .. to] = v for every lane of a wave (all of them call it; to < from: nothing).  Runs of COO_LONG_RUN rows and more are
+// written by the whole wave: one lane's stores to 10 M empty rows took half a second.  any_long (uniform): there may be such runs.
+#define COO_LONG_RUN 16
+__device__ __forceinline__ void coo_fill_rows(int *__restrict__ row_ptr, int from, int to, int v, bool any_long)
 {
-    const bool big = (int64_t)to - from >= 16;
+    const bool big = any_long && (int64_t)to - from >= COO_LONG_RUN;
     if (!big)
         for (int i = from; i <= to; ++i) row_ptr[i] = v;
+    if (!any_long) return;
     for (unsigned long long m = __ballot(big); m; m &= m - 1) {
         const int l = __builtin_ctzll(m), a = __builtin_amdgcn_readlane(from, l), b = __builtin_amdgcn_readlane(to, l), x = __builtin_amdgcn_readlane(v, l);
         for (int64_t i = (int64_t)a + fg_lane(); i <= b; i += 64) row_ptr[i] = x;
@@ -662,6 +664,7 @@ __global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, c
     int2 r[SC_ITEMS];
     int before[SC_ITEMS], prev_dst[SC_ITEMS];       // groups started in the wave's 64 records up to and with this one
     unsigned fl = 0;
+    int jump = 0;                                   // rows from record to record (never negative), or-ed: below COO_LONG_RUN where all are
 #pragma unroll
     for (int k = 0; k < SC_ITEMS; ++k) {
         const int64_t q = base + k * 256 + (int)threadIdx.x;
@@ -673,12 +676,14 @@ __global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, c
         }
         const bool f = q < n && (!sums || r[k].x != b.x || r[k].y != b.y);
         prev_dst[k] = b.x;
+        jump |= r[k].x - b.x;
         fl |= (unsigned)f << k;
         const unsigned long long m = __ballot(f);
         before[k] = __popcll(m & le);
         if (lane == 0) wave_cnt[k][wave] = __popcll(m);
     }
     __syncthreads();
+    const bool any_long = __ballot(jump >= COO_LONG_RUN) != 0;
     int run = sums ? sums[blockIdx.x] : (int)base;
 #pragma unroll
     for (int k = 0; k < SC_ITEMS; ++k) {
@@ -693,8 +698,8 @@ __global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, c
             if (end) *n_out = pos + 1;
             if constexpr (TRIPLE) edge_pos[rec[q].y] = pos;
         }
-        coo_fill_rows(row_ptr, prev_dst[k] + 1, head ? r[k].x : prev_dst[k], pos);
-        if (base + SC_TILE >= n) coo_fill_rows(row_ptr, r[k].x + 1, end ? n_rows : r[k].x, pos + 1);      // uniform: the last tile
+        coo_fill_rows(row_ptr, prev_dst[k] + 1, head ? r[k].x : prev_dst[k], pos, any_long);
+        if (base + SC_TILE >= n) coo_fill_rows(row_ptr, r[k].x + 1, end ? n_rows : r[k].x, pos + 1, true);      // uniform: the last tile
     }
 }
 
