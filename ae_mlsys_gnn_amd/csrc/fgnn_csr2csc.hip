@@ -24,8 +24,9 @@
 #define RS_MAX_DIGITS (1 << RS_MAX_BITS)
 #define RS_DPT (RS_MAX_DIGITS / RS_TPB)      // digits per thread in the per-tile scans
 // Records per thread: tiles of 8192 keep the per-tile digit runs long; small inputs take tiles of 2048 so that they
-// spread over the chip (1 M records: 512 workgroups instead of 128).
-#define RS_SMALL_N (4 << 20)
+// spread over the chip (1 M records: 512 workgroups instead of 128).  From 2 M records on the runs count for more: CSR -> CSC of 2.1 M
+// entries in 2000 columns 57 us with the large tiles and 81 with the small ones, of 4 M in 131 k columns 86 and 126.
+#define RS_SMALL_N (2 << 20)
 static inline int rs_items(int64_t n) { return n < RS_SMALL_N ? 2 : 8; }
 static inline int rs_num_tiles(int64_t n) { const int64_t t = (int64_t)RS_TPB * rs_items(n); return (int)((n + t - 1) / t); }
 static __host__ __device__ inline int rs_hist_ld(int ntiles) { return (ntiles + 7) & ~7; }     // ints per digit of the count array

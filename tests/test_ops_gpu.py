@@ -98,9 +98,9 @@ def test_csr2csc_round_trip_large():
 
 
 @pytest.mark.parametrize("n,e", [(2048, 2047), (2048, 2048), (2049, 2049), (5, 8192), (4194304, 300001), (4194305, 300000), (700, 4194303),
-                                 (300000, 4194304), (300000, 4202497), (16777217, 4200000)])
+                                 (300000, 4194304), (300000, 4202497), (16777217, 4200000), (700, 2097151), (300000, 2097152)])
 def test_coo2csr_and_csr2csc_at_the_edges_of_the_radix_passes(n, e):
-    # either side of a tile (2048 and 8192 records), of the switch between the two tile sizes (4 Mi) and of one, two and three
+    # either side of a tile (2048 and 8192 records), of the switch between the two tile sizes (2 Mi) and of one, two and three
     # passes (11 and 22 bits), against torch's stable sort; one hub row longer than a tile, many empty rows
     from ae_mlsys_gnn_amd.operators import csr2csc as op
     gen = torch.Generator(device=DEV).manual_seed(n + e)
