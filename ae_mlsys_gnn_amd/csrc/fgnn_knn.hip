@@ -15,7 +15,8 @@
 //
 // Selection (k <= 64): a threshold that at least k candidates pass, the k-th smallest of lane minima; the candidates under it
 // (usually k to 1.3 k of the 1024) are compacted into LDS with ballots and ordered by a merge sort over the wave, whose exchanges
-// stay on the vector ALU.  When more than 128 pass (many equal distances) and for 64 < k <= 128 the selection runs k extraction rounds
+// stay on the vector ALU.  When more than 128 pass, mostly candidates at equal distances, the list takes those below the threshold and the
+// k smallest ids of those at it.  Where even that is too long, and for 64 < k <= 128, the selection runs k extraction rounds
 // instead: wave-wide minimum (DPP butterfly), holder with the smallest node id by ballots, retire it.  Either way the order is
 // total (smaller distance first, smaller node id on equal distance), so the result is deterministic.  Clouds with more points than
 // one tile keep the best k of the tiles seen so far in registers and run them through the next tile's selection, where they win ties
@@ -179,9 +180,9 @@ __device__ __forceinline__ void knn_order(const float2 *list, int cnt, int lane,
 }
 
 // The k best of {prior list, tile} for k <= 64: (1) a threshold that at least k candidates pass; (2) the candidates under it
-// (usually k to 2k) are compacted into wave-private LDS with ballots; (3) a merge sort over the wave orders them.  More than KNN_CAP
-// candidates under the threshold (many equal distances, or fewer than k groups with a candidate) fall back to the extraction
-// rounds.  list: KNN_CAP entries of LDS owned by this wave.
+// (usually k to 1.3 k) are compacted into wave-private LDS with ballots; (3) a merge sort over the wave orders them.  More than KNN_CAP
+// candidates under the threshold are thinned to those below it and the k smallest ids at it; more than KNN_CAP - 64 below it, or fewer
+// than k groups with a candidate, fall back to the extraction rounds.  list: KNN_CAP entries of LDS owned by this wave.
 template <int NR>
 __device__ __forceinline__ void knn_select(float (&dist)[NR], int tile0, float (&pd)[1], int (&pi)[1], int k, int lane, int fallback_id, float2 *list)
 {
@@ -201,6 +202,37 @@ __device__ __forceinline__ void knn_select(float (&dist)[NR], int tile0, float (
     if (tile0) put(pd[0] <= tau, pd[0], pi[0]);
 #pragma unroll
     for (int r = 0; r < NR; ++r) put(dist[r] <= tau, dist[r], tile0 + (r / 4) * 256 + lane * 4 + (r % 4));
+    if (cnt > KNN_CAP && tau < INFINITY) {
+        // mostly equal distances: whoever is below tau, and of those at tau the k smallest ids (the prior list's first, which are smaller
+        // than the tile's and in order; then by group of 256, lane and register)
+        fg_wave_lds_sync();
+        cnt = 0;
+        if (tile0) put(pd[0] < tau, pd[0], pi[0]);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) put(dist[r] < tau, dist[r], tile0 + (r / 4) * 256 + lane * 4 + (r % 4));
+        if (cnt <= KNN_CAP - 64) {
+            const int end = cnt + k;
+            if (tile0) put(pd[0] == tau, pd[0], pi[0]);
+            const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+            for (int g = 0; g < NR / 4; ++g) {
+                int pos = cnt;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const unsigned long long m = __ballot(dist[4 * g + u] == tau);
+                    pos += __popcll(m & below);
+                    cnt += __popcll(m);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (dist[4 * g + u] == tau) {
+                        if (pos < end) list[pos] = make_float2(tau, __int_as_float(tile0 + g * 256 + lane * 4 + u));
+                        ++pos;
+                    }
+            }
+            cnt = min(cnt, end);
+        } else cnt = KNN_CAP + 1;
+    }
     if (cnt > KNN_CAP || !(tau < INFINITY)) {
         knn_select_rounds<NR, 1>(dist, tile0, pd, pi, k, lane, fallback_id);
         return;
@@ -321,7 +353,8 @@ __global__ __launch_bounds__(KNN_WAVES * 64) void knn_kernel(int P, int D, int k
 // A workgroup of 8 waves takes 32 queries; wave w multiplies its eighth of the tile's candidates (16 x 16 x 4 products, rows =
 // candidates, columns = queries) straight out of global memory: lane (r, q) reads 4 consecutive floats of row r, and the 4
 // products of a chunk take the first, second, third and fourth of them, a permutation of the dimensions that both operands share.
-// The row of the workgroup's first query is taken off all points, so a common offset costs no precision.
+// The median, dimension by dimension, of three of the workgroup's queries is taken off all points, so a common offset costs no
+// precision and one far point among the three does no harm.
 // |c - q|^2 = |c|^2 - 2 c.q + |q|^2 then goes through LDS, 16 queries at a time, to the wave that selects.
 //
 // With u = 2^-24, S = |q|^2 + max |c|^2 (of the shifted points) the product form is within u S (2 D + 11) of the true distance and the
@@ -331,8 +364,13 @@ __global__ __launch_bounds__(KNN_WAVES * 64) void knn_kernel(int P, int D, int k
 // neighbours in the list more than 2 E apart are in order; those closer are computed by the exact path's operations in the
 // exact path's order, and the list is sorted once more.  (All 47 candidates of a query at k = 40 cost 24 KB of gathered rows, and
 // the L2 rate was the bound.)  With more candidates than lanes, or more points than a tile, all candidates are computed.  The graph is
-// bit for bit the one of the kernel above.  More than KNN_CAP candidates, or norms that overflow or are no numbers, send the query to
-// the exact path's selection over the exact distances of what passed.
+// bit for bit the one of the kernel above.
+//
+// E holds for the farthest point of the tile.  Where more than KNN_CAP candidates pass because a few points are far out, the query
+// is tried again with every candidate's own bound, E(c) = 2 u (|q|^2 + |c|^2) (4 D + 32): the k-th smallest of approximation + E(c) bounds
+// the k-th smallest exact distance, and whoever's approximation - E(c) is not above it stays.  What is still open then (hundreds of points
+// at one place, norms that overflow or are no numbers) takes the direct kernel's way: the workgroup streams the tile through LDS
+// and the waves with open queries form all their distances.
 //
 // Bound by the fp32 matrix rate (1.4 us per dimension of 64 clouds x 1024 points, 95 TFLOP/s) and the selection, 140 us there.
 // Before and after at k = 40: 64 dimensions 634 (379 with the present selection) -> 243 us, 128 dimensions 904 (642) -> 344 us.
@@ -359,7 +397,80 @@ __device__ __forceinline__ float knn_exact(const float *cp, int D, int q, int c,
     return fminf(acc, FLT_MAX);
 }
 
-template <int RG, bool WHOLE>
+// The open queries of a workgroup (bits of `any`; of the wave: `open`) against one tile, by the direct kernel's operations in their order: the
+// tile streams through LDS (cs, KNN_DC x TILE floats) and the waves with open queries form all their distances, 2 x 8 waves at a time.
+struct knn_best { float d[4]; int i[4]; };
+template <int RG>
+__device__ __forceinline__ knn_best knn_exact_tile(int P, int D, int k, int rows_aligned, const float *cp, int q0, int tile0, unsigned any, unsigned open,
+                                                   float *cs, float2 *list, knn_best best)
+{
+    constexpr int NR = 4 * RG, TILE = 256 * RG;
+    const int lane = fg_lane(), wave = fg_uni(fg_wave());
+#pragma unroll 1
+    for (int gq = 0; gq < 2; ++gq) {
+        if (!((any >> (2 * gq)) & 3)) continue;         // uniform over the workgroup
+        const unsigned mine = (open >> (2 * gq)) & 3;
+        const int q = q0 + gq * 16 + 2 * wave, qa = min(q, P - 1), qb = min(q + 1, P - 1);
+        float ex[2][NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) ex[0][r] = ex[1][r] = 0.f;
+        for (int d0 = 0; d0 < D; d0 += KNN_DC) {
+            const int dn = min(KNN_DC, D - d0);
+            __syncthreads();                            // the previous slice has been consumed
+            for (int c = (int)threadIdx.x; c < TILE; c += KNN_MW * 64) {
+                const bool ok = tile0 + c < P;
+                const float *src = cp + (size_t)(ok ? tile0 + c : 0) * D + d0;
+                if (dn == KNN_DC && rows_aligned) {
+                    const knn_f4 lo = *reinterpret_cast<const knn_f4 *>(src), hi = *reinterpret_cast<const knn_f4 *>(src + 4);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) { cs[u * TILE + c] = ok ? lo[u] : 0.f; cs[(4 + u) * TILE + c] = ok ? hi[u] : 0.f; }
+                } else {
+                    for (int dd = 0; dd < dn; ++dd) cs[dd * TILE + c] = ok ? src[dd] : 0.f;
+                }
+            }
+            __syncthreads();
+            if (mine) {
+#pragma unroll 2
+                for (int dd = 0; dd < dn; ++dd) {
+                    const float v0 = cp[(size_t)qa * D + d0 + dd], v1 = cp[(size_t)qb * D + d0 + dd];
+#pragma unroll
+                    for (int g = 0; g < RG; ++g) {
+                        const knn_f4 c4 = *reinterpret_cast<const knn_f4 *>(&cs[dd * TILE + g * 256 + lane * 4]);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const float f0 = v0 - c4[u], f1 = v1 - c4[u];
+                            ex[0][4 * g + u] = fmaf(f0, f0, ex[0][4 * g + u]);
+                            ex[1][4 * g + u] = fmaf(f1, f1, ex[1][4 * g + u]);
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll 1
+        for (int j = 0; j < 2; ++j) {
+            if (!((mine >> j) & 1)) continue;           // uniform over the wave
+            float dist[NR];
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+                dist[r] = tile0 + (r / 4) * 256 + lane * 4 + (r % 4) < P ? fminf(j ? ex[1][r] : ex[0][r], FLT_MAX) : INFINITY;
+            float hd[1] = {gq ? (j ? best.d[3] : best.d[2]) : (j ? best.d[1] : best.d[0])};
+            int hi[1] = {gq ? (j ? best.i[3] : best.i[2]) : (j ? best.i[1] : best.i[0])};
+            knn_select<NR>(dist, tile0, hd, hi, k, lane, j ? qb : qa, list);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) if (a == 2 * gq + j) { best.d[a] = hd[0]; best.i[a] = hi[0]; }
+        }
+    }
+    __syncthreads();                                    // the last slice has been read
+    return best;
+}
+template <int RG>
+__device__ __attribute__((noinline)) knn_best knn_exact_tile_call(int P, int D, int k, int rows_aligned, const float *cp, int q0, int tile0, unsigned any, unsigned open,
+                                                                  float *cs, float2 *list, knn_best best)
+{
+    return knn_exact_tile<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, cs, list, best);
+}
+
+template <int RG, bool MULTI>
 __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, int k, int rows_aligned, unsigned per_xcd, unsigned q_blocks, unsigned n_blocks,
                                                                   const float *__restrict__ pts, int *__restrict__ out)
 {
@@ -368,34 +479,40 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
     __shared__ __attribute__((aligned(16))) float cn[TILE];
     __shared__ float2 lists[KNN_MW * KNN_CAP];
     __shared__ float wmax[KNN_MW];
+    __shared__ unsigned open_of[KNN_MW];
     const unsigned b = per_xcd ? (blockIdx.x % FGNN_NUM_XCD) * per_xcd + blockIdx.x / FGNN_NUM_XCD : blockIdx.x;
     if (b >= n_blocks) return;                  // the whole workgroup
     const int cloud = (int)(b / q_blocks), q0 = (int)(b % q_blocks) * KNN_MQ;
     const float *cp = pts + (size_t)cloud * P * D;
     const int lane = fg_lane(), wave = fg_uni(fg_wave()), r16 = lane & 15, kq = lane >> 4;
     float2 *list = lists + wave * KNN_CAP;
-    float pd[4];                                // the lists of the wave's queries q0 + 16 (a / 2) + 2 wave + a % 2
+    // MULTI (more points than a tile): the best of the tiles seen so far, for the wave's queries q0 + 16 (a / 2) + 2 wave + a % 2
+    float pd[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
     int pi[4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) { pd[a] = INFINITY; pi[a] = min(q0 + (a / 2) * 16 + 2 * wave + a % 2, P - 1); }
+    for (int a = 0; a < 4; ++a) pi[a] = min(q0 + (a / 2) * 16 + 2 * wave + a % 2, P - 1);
+    auto finish = [&](int q, int i) { if (q < P && lane < k) out[((size_t)cloud * P + q) * k + lane] = cloud * P + i; };
 
-    // 4 floats of a row from dimension d0 + 4 kq on, zero past the end.  WHOLE: D is a multiple of 16 and rows start on 16 bytes; one
-    // bounds-checked load (rows past the cloud read as zero) then needs no test of its own.
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(cp), 0, WHOLE ? P * D * 4 : 0, 0x00027000);
-    const int lane_off = (r16 * D + 4 * kq) * 4;
-    auto frag = [&](int row0, bool one_row, int d0) {          // row row0 + r16, or row row0 in all lanes
-        if constexpr (WHOLE) {
-            return __builtin_bit_cast(knn_f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (one_row ? 16 * kq : lane_off) + (row0 * D + d0) * 4, 0, 0));
-        } else {
-            const int d = d0 + 4 * kq;
-            const float *src = cp + (size_t)min(row0 + (one_row ? 0 : r16), P - 1) * D + d;
-            knn_f4 v = {0.f, 0.f, 0.f, 0.f};
+    // 4 floats of a row from dimension d0 + 4 kq on: one load that checks the cloud's bounds (rows past its end read as zero).  TAIL, the last
+    // chunk where D is no multiple of 16: zero past the row's end, too, and floats one by one where four could straddle the cloud's.
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(cp), 0, P * D * 4, 0x00027000);
+    const unsigned lane_off = (unsigned)(r16 * D + 4 * kq) * 4u;
+    auto frag = [&](int row0, bool one_row, int d0, auto tail) {          // row row0 + r16, or row row0 in all lanes
+        const int off = (int)((one_row ? 16u * kq : lane_off) + ((unsigned)row0 * D + d0) * 4u);
+        knn_f4 v;
+        if constexpr (!decltype(tail)::value) v = __builtin_bit_cast(knn_f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+        else {
+            if (D % 4 == 0) v = __builtin_bit_cast(knn_f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+            else {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) if (d + u < D) v[u] = src[u];
-            return v;
+                for (int u = 0; u < 4; ++u) v[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off + 4 * u, 0, 0));
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = d0 + 4 * kq + u < D ? v[u] : 0.f;
         }
+        return v;
     };
-    for (int tile0 = 0; tile0 < P; tile0 += TILE) {
+    for (int tile0 = 0; tile0 < (MULTI ? P : 1); tile0 += TILE) {
         knn_f4 acc[NT][2];
         float nrm[NT], qn[2] = {0.f, 0.f};
         const int crow = tile0 + wave * NT * 16;
@@ -404,15 +521,19 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
             acc[t][0] = acc[t][1] = knn_f4{0.f, 0.f, 0.f, 0.f};
             nrm[t] = 0.f;
         }
-        for (int d0 = 0; d0 < D; d0 += 16) {
-            const knn_f4 m = frag(q0, true, d0), b0 = frag(q0, false, d0) - m, b1 = frag(q0 + 16, false, d0) - m;
+        auto chunk = [&](int d0, auto tail) {
+            const knn_f4 m0 = frag(q0, true, d0, tail), m1 = frag(q0 + 10, true, d0, tail), m2 = frag(q0 + 21, true, d0, tail);
+            knn_f4 m;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) m[u] = __builtin_amdgcn_fmed3f(m0[u], m1[u], m2[u]);
+            const knn_f4 b0 = frag(q0, false, d0, tail) - m, b1 = frag(q0 + 16, false, d0, tail) - m;
 #pragma unroll
             for (int u = 0; u < 4; ++u) { qn[0] = fmaf(b0[u], b0[u], qn[0]); qn[1] = fmaf(b1[u], b1[u], qn[1]); }
 #pragma unroll
             for (int h = 0; h < NT; h += NH) {          // at most 4 tiles of operands in registers
                 knn_f4 a[NH];
 #pragma unroll
-                for (int t = 0; t < NH; ++t) a[t] = frag(crow + (h + t) * 16, false, d0);
+                for (int t = 0; t < NH; ++t) a[t] = frag(crow + (h + t) * 16, false, d0, tail);
 #pragma unroll
                 for (int t = 0; t < NH; ++t) {
                     a[t] -= m;
@@ -427,7 +548,10 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
                         acc[h + t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][u], b1[u], acc[h + t][1], 0, 0, 0);
                     }
             }
-        }
+        };
+        int d0 = 0;
+        for (; d0 + 16 <= D; d0 += 16) chunk(d0, std::false_type());
+        if (d0 < D) chunk(d0, std::true_type());
         // lane (r, q) holds a quarter of the norms of row r: add the quarters up
         auto quarters = [&](float v) {
             v += __uint_as_float(knn_xor<16>(__float_as_uint(v), lane));
@@ -445,6 +569,7 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
         }
         mx = fg_wave_max(mx);
         if (lane == 0) wmax[wave] = mx;
+        unsigned open = 0;                      // the wave's queries that the filter leaves open, bit a as in pd[a] (uniform)
         fg_wave_lds_sync();                     // a wave reads only the norms that it wrote
         auto select16 = [&](auto group) {
             constexpr int gq = decltype(group)::value;
@@ -462,8 +587,9 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
 #pragma unroll 1
             for (int j = 0; j < 2; ++j) {
                 const int ql = 2 * wave + j, q = min(q0 + gq * 16 + ql, P - 1);
-                float hd[1] = {j ? pd[2 * gq + 1] : pd[2 * gq]};
-                int hi[1] = {j ? pi[2 * gq + 1] : pi[2 * gq]};
+                float hd = INFINITY;
+                int hi = q;
+                if constexpr (MULTI) { hd = j ? pd[2 * gq + 1] : pd[2 * gq]; hi = j ? pi[2 * gq + 1] : pi[2 * gq]; }
                 float *row = &buf[ql * ROW + lane * 4];
                 float dist[NR];
                 auto fetch = [&]() {
@@ -475,15 +601,14 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
                     }
                 };
                 fetch();
-                const float S = sane(fg_readlane(qg, ql)) + cmax;
-                const float E = (float)(4 * D + 32) * 0x1p-23f * S + (float)(D + 1) * 1e-36f;
-                const float tau = knn_threshold<NR>(hd[0], k, lane, [&](int from, int to) {
+                const float qn2 = sane(fg_readlane(qg, ql)), rel = (float)(4 * D + 32) * 0x1p-23f, tiny = (float)(D + 1) * 1e-36f;
+                float E = rel * (qn2 + cmax) + tiny;
+                auto least = [&](int from, int to) {
                     float m = dist[from];
 #pragma unroll
                     for (int r = 0; r < NR; ++r) if (r > from && r < to) m = fminf(m, dist[r]);
                     return m;
-                });
-                const float lim = tau + 2.f * E;
+                };
                 int cnt = 0;
                 auto put = [&](bool in, float d, int i) {
                     const unsigned long long m = __ballot(in);
@@ -491,11 +616,45 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
                     if (in && pos < KNN_CAP) list[pos] = make_float2(d, __int_as_float(i));
                     cnt += __popcll(m);
                 };
-                if (tile0) put(hd[0] <= lim, hd[0], hi[0]);
+                const float lim = knn_threshold<NR>(hd, k, lane, least) + 2.f * E;
+                bool bounded = lim < INFINITY;              // false, too, where E is infinite or the threshold no number
+                if (MULTI && tile0) put(hd <= lim, hd, hi);
 #pragma unroll
                 for (int r = 0; r < NR; ++r) put(dist[r] <= lim, dist[r], tile0 + (r / 4) * 256 + lane * 4 + (r % 4));
+                // once more with every candidate's own bound, where half of a sample have a good deal less than the farthest
+                if (bounded && cnt > KNN_CAP && __popcll(__ballot(16.f * cn[lane * 4] < cmax)) >= 32) {
+                    fg_wave_lds_sync();
+                    auto own = [&](int g) {                 // E(c) of the lane's four candidates of group g
+                        knn_f4 e = *reinterpret_cast<const knn_f4 *>(&cn[g * 256 + lane * 4]);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) e[u] = rel * (qn2 + e[u]) + tiny;
+                        return e;
+                    };
+#pragma unroll
+                    for (int g = 0; g < RG; ++g) {
+                        const knn_f4 e = own(g);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) dist[4 * g + u] = dist[4 * g + u] < INFINITY ? dist[4 * g + u] + e[u] : INFINITY;
+                    }
+                    const float tau = knn_threshold<NR>(hd, k, lane, least);
+                    bounded = tau < INFINITY;
+                    cnt = 0;
+                    E = 0.f;                                // the largest bound of those that stay
+                    if (MULTI && tile0) put(hd <= tau, hd, hi);
+#pragma unroll
+                    for (int g = 0; g < RG; ++g) {
+                        const knn_f4 e = own(g);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const bool in = dist[4 * g + u] - 2.f * e[u] <= tau && dist[4 * g + u] < INFINITY;
+                            if (in) E = fmaxf(E, e[u]);
+                            put(in, dist[4 * g + u] - e[u], tile0 + g * 256 + lane * 4 + u);
+                        }
+                    }
+                    E = fg_wave_max(E);
+                }
                 fg_wave_lds_sync();
-                if (lim < INFINITY && cnt <= 64 && P <= TILE) {
+                if (bounded && cnt <= 64 && !MULTI) {
                     const float2 e = lane < cnt ? list[lane] : make_float2(INFINITY, __int_as_float(0x7fffffff));
                     float cd = e.x;
                     int ci = __float_as_int(e.y);
@@ -506,43 +665,57 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
                         if (near) cd = knn_exact(cp, D, q, ci, rows_aligned);
                         KNN_SORT_64(cd, ci, lane);
                     }
-                    hd[0] = lane < k ? cd : INFINITY;
-                    hi[0] = lane < k ? ci : q;
-                } else if (lim < INFINITY && cnt <= KNN_CAP) {
+                    hd = lane < k ? cd : INFINITY;
+                    hi = lane < k ? ci : q;
+                } else if (bounded && cnt <= KNN_CAP) {
                     for (int e = lane; e < cnt; e += 64) list[e].x = knn_exact(cp, D, q, __float_as_int(list[e].y), rows_aligned);
                     fg_wave_lds_sync();
                     float cd;
                     int ci;
                     knn_order(list, cnt, lane, cd, ci);
-                    hd[0] = lane < k ? cd : INFINITY;
-                    hi[0] = lane < k ? ci : q;
+                    hd = lane < k ? cd : INFINITY;
+                    hi = lane < k ? ci : q;
                 } else {
-                    _Pragma("unroll 1") for (int r = 0; r < NR; ++r) {
-                        const int c = tile0 + (r / 4) * 256 + lane * 4 + (r % 4);
-                        float &v = row[(r / 4) * 256 + r % 4];
-                        v = c < P && !(v > lim) ? knn_exact(cp, D, q, c, rows_aligned) : INFINITY;
-                    }
-                    fg_wave_lds_sync();
-                    fetch();
-                    knn_select<NR>(dist, tile0, hd, hi, k, lane, q, list);
+                    open |= 1u << (2 * gq + j);
                 }
-                if (j) { pd[2 * gq + 1] = hd[0]; pi[2 * gq + 1] = hi[0]; }
-                else { pd[2 * gq] = hd[0]; pi[2 * gq] = hi[0]; }
+                if constexpr (MULTI) {
+                    if (j) { pd[2 * gq + 1] = hd; pi[2 * gq + 1] = hi; }
+                    else { pd[2 * gq] = hd; pi[2 * gq] = hi; }
+                } else if (!((open >> (2 * gq + j)) & 1)) finish(q0 + gq * 16 + ql, hi);
                 fg_wave_lds_sync();
             }
             __syncthreads();                    // the rows have been read
         };
         select16(std::integral_constant<int, 0>());
         select16(std::integral_constant<int, 1>());
-    }
+
+        // the queries that are still open (the rows of buf have been read)
+        if (lane == 0) open_of[wave] = open;
+        __syncthreads();
+        unsigned any = 0;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int q = q0 + (a / 2) * 16 + 2 * wave + a % 2;
-        if (q < P && lane < k) out[((size_t)cloud * P + q) * k + lane] = cloud * P + pi[a];
+        for (int w = 0; w < KNN_MW; ++w) any |= open_of[w];
+        static_assert(KNN_DC * TILE <= 16 * ROW, "the slices go where the approximations were");
+        if (any) {
+            knn_best best;
+#pragma unroll
+            for (int a = 0; a < 4; ++a) { best.d[a] = pd[a]; best.i[a] = pi[a]; }
+            if constexpr (MULTI) best = knn_exact_tile_call<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, buf, list, best);
+            else best = knn_exact_tile<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, buf, list, best);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                if constexpr (MULTI) { pd[a] = best.d[a]; pi[a] = best.i[a]; }
+                else if ((open >> a) & 1) finish(q0 + (a / 2) * 16 + 2 * wave + a % 2, best.i[a]);
+            }
+        }
+    }
+    if constexpr (MULTI) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) finish(q0 + (a / 2) * 16 + 2 * wave + a % 2, pi[a]);
     }
 }
 
-template <int RG>
+template <int RG, bool MULTI>
 static void knn_mfma_launch(int n_clouds, int P, int D, int k, const float *points, int32_t *src_ind, hipStream_t st)
 {
     const unsigned q_blocks = (unsigned)((P + KNN_MQ - 1) / KNN_MQ), n_blocks = q_blocks * (unsigned)n_clouds;
@@ -551,12 +724,8 @@ static void knn_mfma_launch(int n_clouds, int P, int D, int k, const float *poin
         per_xcd = (grid + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD;
         grid = per_xcd * FGNN_NUM_XCD;
     }
-    const int rows_aligned = D % 4 == 0 && fgnn_aligned16(points) ? 1 : 0;
-    if (rows_aligned && D % 16 == 0 && (int64_t)P * D * 4 <= 0x7fffffff)
-        hipLaunchKernelGGL((knn_mfma_kernel<RG, true>), dim3(grid), dim3(KNN_MW * 64), 0, st, P, D, k, 1, per_xcd, q_blocks, n_blocks, points, src_ind);
-    else
-        hipLaunchKernelGGL((knn_mfma_kernel<RG, false>), dim3(grid), dim3(KNN_MW * 64), 0, st, P, D, k, rows_aligned, per_xcd, q_blocks, n_blocks, points,
-                           src_ind);
+    hipLaunchKernelGGL((knn_mfma_kernel<RG, MULTI>), dim3(grid), dim3(KNN_MW * 64), 0, st, P, D, k, D % 4 == 0 && fgnn_aligned16(points) ? 1 : 0, per_xcd,
+                       q_blocks, n_blocks, points, src_ind);
 }
 
 template <int RG, int KR>
@@ -579,14 +748,19 @@ extern "C" int fgnn_knn_graph(int n_clouds, int P, int D, int k, const float *po
     if (n_clouds == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     const int rg = P <= 256 ? 1 : P <= 512 ? 2 : 4;     // tile = 256 * rg candidate points
-    // The matrix form costs less per dimension (64 clouds: 1.4 against 4 us at 1024 points, 0.5 against 0.8 at 512) and more per query
-    // (140 against 115 us, 44 against 30): equal at 10 to 16 and at 45 dimensions.  At 256 points it loses up to 128 dimensions
-    // (46 against 44 us; 34 against 29 at 64).
     // A launch holds fewer than 2^32 threads in one dimension: 2^23 workgroups of the matrix form, whose grid has only one.
-    const bool fits = (int64_t)n_clouds * ((P + KNN_MQ - 1) / KNN_MQ) <= (1 << 23) - FGNN_NUM_XCD;
-    if (k <= 64 && fits && ((rg == 4 && D >= 16) || (rg == 2 && D >= 48))) {
-        if (rg == 2) knn_mfma_launch<2>(n_clouds, P, D, k, points, src_ind, st);
-        else knn_mfma_launch<4>(n_clouds, P, D, k, points, src_ind, st);
+    // A cloud's bytes are counted in 31 bits by the loads that check its bounds.
+    const int64_t blocks = (int64_t)n_clouds * ((P + KNN_MQ - 1) / KNN_MQ);
+    const bool fits = blocks <= (1 << 23) - FGNN_NUM_XCD && (int64_t)P * D * 4 <= 0x7fffffff;
+    // The matrix form costs less per dimension (64 clouds: 1.5 against 4.2 us at 1024 points, 0.5 against 0.85 at 512) and at 512 points more
+    // per query, where the two meet at 48 dimensions (67 against 66 us; 32: 55 against 59).  With more points it wins from 16 on where
+    // its 32 queries a workgroup still fill the chip twice (64 x 1024: 158 against 117 us at 16; 8 x 2048: 80 against 68); with
+    // fewer workgroups the meeting point moves up (8 x 1024: 22 against 26 at 16, 40 against 34 at 48; 1 x 1024: 32 against 33 at 48).  At
+    // 256 points it loses up to 128 dimensions (46 against 44 us; 34 against 29 at 64).
+    if (k <= 64 && fits && rg >= 2 && D >= (rg == 4 && blocks >= 512 ? 16 : 48)) {
+        if (rg == 2) knn_mfma_launch<2, false>(n_clouds, P, D, k, points, src_ind, st);
+        else if (P <= 1024) knn_mfma_launch<4, false>(n_clouds, P, D, k, points, src_ind, st);
+        else knn_mfma_launch<4, true>(n_clouds, P, D, k, points, src_ind, st);
     } else if (k <= 64) {
         if (rg == 1) knn_launch<1, 1>(n_clouds, P, D, k, points, src_ind, st);
         else if (rg == 2) knn_launch<2, 1>(n_clouds, P, D, k, points, src_ind, st);
