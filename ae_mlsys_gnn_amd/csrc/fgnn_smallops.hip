@@ -441,17 +441,20 @@ extern "C" int fgnn_gather_rows(int64_t E, int W, const int32_t *permute, const 
 // load is a contiguous run of S0 floats.  Rows of up to SO_LONG_ELEMS floats are taken by one wave
 // each, longer ones by a whole workgroup each: a 100 k-entry hub row is then a few hundred trips of a
 // workgroup instead of tens of thousands of trips of one wave.  Both kinds run in ONE launch: its first
-// workgroups each look at 16 or 64 candidate rows (the first wave reads their lengths, a ballot names the
+// workgroups each look at 16 to 64 candidate rows (the first wave reads their lengths, a ballot names the
 // long ones, the workgroup takes those one after the other), the workgroups behind them give one short
 // row to each of their waves and fill the machine while the last long rows finish.  (On a 233 k-row
 // power-law graph 31 k rows are long and hold 83 % of the entries; a workgroup per row would start
 // 233 k workgroups of which seven in eight leave at once.)
 #define SO_LONG_ELEMS 8192
 // Candidate rows per workgroup of a long-row launch: 16 where a good part of the rows is long (the workgroup takes its long rows one
-// after the other), 64 where the mean row is short and most of these workgroups leave at once (169 k rows of 15 entries, 8 heads: row sums 59 -> 43 us, with the loads
-// in flight below).
+// after the other), 64 where the mean row is short and most of these workgroups leave at once (169 k rows of 15 entries, 8 heads: row
+// sums 59 -> 43 us, with the loads in flight below), 32 in between (softmax of 60 M entries in 233 k rows, 2 and 3 heads: 360 and 543 us
+// with 64, 323 and 486 with 32 or 16; row sums there 151 and 187, 151 and 184, 157 and 187).
 #define SO_CAND_DENSE 16
+#define SO_CAND_MEDIUM 32
 #define SO_CAND_SPARSE 64
+#define SO_SPARSE_ROW_FLOATS 256          // mean floats per row up to which a launch looks at SO_CAND_SPARSE rows
 // Registers a row-reduction kernel spends on a row: CACHE groups of VEC floats per lane kept over both phases by a wave on a short
 // row, CLONG by the workgroup on a long row, STREAM loads in flight per lane in the part of a row that is streamed.  The numbers
 // set the kernel's register count and with it the waves resident per SIMD: rows that mostly fit one trip of a wave want a small
@@ -496,7 +499,7 @@ static inline int so_pick_lanes(int N, int64_t elems, int vec, int W)
 // 3.29 / 2.77 / 2.48, the scatter kernel 3.93 / 3.60 / 4.43, gather-row 4.03 / 4.06 / 4.83, row sums 1.08 / 0.79 / 0.66.
 static inline unsigned so_grid(int N, int64_t elems, int tpb, unsigned *n_long, int lanes_per_row = 64)
 {
-    const int cand = so_dense_rows(N, elems) ? SO_CAND_DENSE : SO_CAND_SPARSE;
+    const int cand = so_dense_rows(N, elems) ? SO_CAND_DENSE : elems >= (int64_t)SO_SPARSE_ROW_FLOATS * N ? SO_CAND_MEDIUM : SO_CAND_SPARSE;
     *n_long = elems > SO_LONG_ELEMS ? (unsigned)((N + cand - 1) / cand) : 0u;      // otherwise no row can be long
     const int rows_per_block = (tpb / 64) * (64 / lanes_per_row);
     return *n_long + (unsigned)((N + rows_per_block - 1) / rows_per_block);

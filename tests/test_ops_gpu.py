@@ -1528,15 +1528,17 @@ def test_mhspmm_and_mhsddmm_rows_wider_than_1024_floats(h, f, monkeypatch):
 
 
 @pytest.mark.parametrize("w", [1, 3, 4, 8, 64])
-@pytest.mark.parametrize("shape", ["short", "empty_runs", "hub", "one_row", "long_rows"])
+@pytest.mark.parametrize("shape", ["short", "empty_runs", "hub", "one_row", "long_rows", "some_long_rows", "few_long_rows"])
 def test_u_add_v_row_search_and_row_sums(w, shape):
     """Rows found by the wave-wide search and inside the window of 64 row ends: runs of empty rows longer than the window, a row that
-    spans many waves, a single row, and enough long rows that a workgroup finds several among its candidates."""
+    spans many waves, a single row, and enough long rows that a workgroup finds several among its 16, 32 or 64 candidates."""
     from ae_mlsys_gnn_amd._lib import check, lib, ptr, stream_ptr
     gen = torch.Generator().manual_seed(w)
     deg = {"short": torch.randint(0, 4, (5000,), generator=gen), "empty_runs": torch.randint(0, 9, (20000,), generator=gen) * (torch.arange(20000) % 300 == 7),
            "hub": torch.cat([torch.randint(0, 3, (700,), generator=gen), torch.tensor([30000]), torch.zeros(500, dtype=torch.long), torch.ones(65, dtype=torch.long)]),
-           "one_row": torch.tensor([1000]), "long_rows": torch.where(torch.arange(900) % 3 == 0, 8200 // w + 1, 2)}[shape]
+           "one_row": torch.tensor([1000]), "long_rows": torch.where(torch.arange(900) % 3 == 0, 8200 // w + 1, 2),
+           "some_long_rows": torch.where(torch.arange(900) % 12 == 0, 8200 // w + 1, 1),
+           "few_long_rows": torch.where(torch.arange(2000) % 50 == 0, 8200 // w + 1, 0)}[shape]
     n, e = deg.numel(), int(deg.sum())
     row_ptr = torch.cat([torch.zeros(1, dtype=torch.long), deg.cumsum(0)]).int()
     dst = torch.repeat_interleave(torch.arange(n), deg)
