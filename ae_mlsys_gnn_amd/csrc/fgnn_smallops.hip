@@ -1174,8 +1174,9 @@ __device__ __forceinline__ int so_wave_row_of(const int *__restrict__ ptr, int l
 // out[p,w] = row_val[row(p),w] + col_val[col_ind[p],w]  (src/u_add_v/u_add_v.cu:4-26).  W <= 64: one thread per
 // element of out, a wave takes `chunks` x 64 consecutive ones.  The row of the wave's first edge is found by a wave-wide search of
 // row_ptr; from there on the 64 row ends that follow sit in a register, and a lane bisects them by lane exchange.  Only
-// where 512 elements span more than 64 rows is row_ptr itself bisected.  (2.5 M entries in 169 k rows, 8 heads: 85 -> 30 us, 64 M entries 1.09 -> 1.06 ms;
-// before, two searches of 18 dependent loads per wave, 7 more per 512 elements, and 2424 waves.)
+// where 512 elements span more than 64 rows is row_ptr itself bisected.  2.5 M entries in 169 k rows, 8 heads: 85 -> 31 us repeated by
+// itself, its arrays in the caches, and 48 us among other kernels; 64 M entries 1.09 -> 1.06 ms.  Before, two searches of 18
+// dependent loads per wave, 7 more per 512 elements, and 2424 waves.
 #define UAV_UJ 8                // chunks in flight; divides the chunks of a wave
 // VEC = 4: an element is four consecutive columns (W % 4 == 0, 16-byte aligned arrays), W counts such groups.
 template <int VEC>
@@ -1363,9 +1364,10 @@ extern "C" int fgnn_u_add_v(int N, int64_t E, int W, const int32_t *row_ptr, con
     }
     FGNN_REQUIRE(E <= 2147483647LL, FGNN_ERR_LIMIT, "fgnn_u_add_v: E=%lld exceeds the 32-bit row_ptr", (long long)E);
     const bool vec4 = W % 4 == 0 && fgnn_aligned16(row_val) && fgnn_aligned16(col_val) && fgnn_aligned16(out);
-    // 2048 elements per wave where that gives every compute unit 32 waves four times over, else 512
+    // 2048 elements per wave where that gives every compute unit 32 waves twice over, else 512 (60 M entries in 233 k rows, 1 head: 223
+    // and 247 us; 20 M in 100 k rows, 2 heads: 91 and 101; below that the waves run out: 24 M groups of four in 1 M rows, 201 and 190)
     const int64_t elems = E * (vec4 ? W / 4 : W);
-    const int chunks = elems >= (int64_t)2048 * 32768 ? 32 : 8;
+    const int chunks = elems >= (int64_t)2048 * 16384 ? 32 : 8;
     const int64_t per_block = (int64_t)FGNN_WPB * 64 * chunks;
     const unsigned blocks = (unsigned)((elems + per_block - 1) / per_block);
     if (vec4) hipLaunchKernelGGL(u_add_v_kernel<4>, dim3(blocks), dim3(FGNN_TPB), 0, st, N, E, W / 4, chunks, row_ptr, col_ind, row_val, col_val, out);

@@ -1553,6 +1553,20 @@ def test_u_add_v_row_search_and_row_sums(w, shape):
     assert_close_sum(gr, want, torch.zeros(n, w, dtype=torch.float64).index_add_(0, dst, g.double().abs()), "row sums")
 
 
+@pytest.mark.parametrize("e,w", [((1 << 25) - 1, 1), ((1 << 25) + 1, 1), ((1 << 25) + 3, 4), (17000000, 2), (11200001, 3)])
+def test_u_add_v_split(e, w):
+    """Either side of the size (2^25 elements or groups of four) from which a wave takes 2048 of them."""
+    from ae_mlsys_gnn_amd.operators.u_add_v import u_add_v_native
+    gen = torch.Generator(device=DEV).manual_seed(w)
+    n = 90001
+    dst = torch.sort(torch.randint(0, n, (e,), generator=gen, device=DEV)).values
+    row_ptr = torch.searchsorted(dst, torch.arange(n + 1, device=DEV)).int()
+    idx = torch.randint(0, n, (e,), generator=gen, device=DEV)
+    a, b = torch.randn(n, w, generator=gen, device=DEV), torch.randn(n, w, generator=gen, device=DEV)
+    out = u_add_v_native.u_add_v_forward(row_ptr, idx.int(), a, b)
+    assert torch.equal(out.view(e, w), a[dst] + b[idx])
+
+
 @pytest.mark.parametrize("n,fin,h,f,pad", [(1, 1, 1, 1, 3), (15, 3, 2, 5, 3), (17, 16, 8, 8, 0), (40, 63, 9, 3, 1), (33, 64, 16, 4, 0), (70, 65, 17, 2, 2),
                                            (48, 100, 32, 8, 0), (66000, 20, 8, 4, 0), (66001, 67, 3, 6, 2), (300, 1433, 1, 128, 0), (0, 8, 2, 4, 0)])
 def test_gat_dense_kernels(n, fin, h, f, pad):
