@@ -339,10 +339,11 @@ def project_in_backward(k, fin, fout, input_grad, n, e):
     product for the input's gradient).  Layer steps, gathering K x fin / fout floats: 169 k nodes, 2.3 M edges, 384 / 64 floats 1.69 ->
     1.01 ms (1.16 with the input's gradient), 128 / 64 0.76 -> 0.68 (0.74), 96 / 44 0.66 -> 0.66 (0.69), 128 / 84 0.78 -> 0.89 ms (0.99);
     300 k nodes, 0.9 M edges, 256 / 100 floats 1.53 -> 1.49 (1.70): the lines lie at ratios of 2 and 3.
-    With the input's gradient and few edges the product's n fin K fout multiply-adds outweigh the gathers, at 50 of them for every float that an
-    edge no longer gathers: 300 k nodes, 1024 / 256 floats: 5.59 -> 6.31 ms at 3 edges a node, 7.17 -> 6.81 at 9; 384 / 128: 1.85 ->
-    2.02 and 2.27 -> 2.18; 1024 / 128: 3.95 -> 3.64 at 3.  On dense graphs rows of up to two cache lines cost what rows of one do: 32 / 16
-    floats 0.95 -> 0.90 ms at 51 edges a node, 0.84 -> 0.87 at 200; 64 / 32 0.86 -> 0.89 there and 5.94 -> 6.00 at 258.
+    With the input's gradient and few edges the products, n fin K fout multiply-adds more, outweigh the gathers, at about 20 of them for
+    every float that an edge no longer gathers: 169 k nodes of 15 edges, 1024 / 256 floats 5.47 -> 5.56 ms, 1024 / 128 4.47 -> 3.16;
+    300 k nodes of 4 edges, 1024 / 128 4.21 -> 4.20, 384 / 64 1.54 -> 1.46.  On dense graphs rows of up to two cache lines cost what
+    rows of one do: 32 / 16 floats 0.95 -> 0.90 ms at 51 edges a node, 0.84 -> 0.87 at 200; 64 / 32 0.86 -> 0.89 there and 5.94 -> 6.00 at
+    258.
     The summed backward takes rows of at most 1024 floats over all kernels, and keeps the kernels in registers up to 256 each;
     wider outputs gather the aggregate's gradient, which has no such limit on them."""
     row = (fout + 3) // 4 * 4
@@ -350,7 +351,7 @@ def project_in_backward(k, fin, fout, input_grad, n, e):
         return False
     if not input_grad:
         return k * fin >= 2 * row
-    return k * fin >= 3 * row and n * fin * k * fout <= 50 * e * (k * fin - row)
+    return k * fin >= 3 * row and n * fin * k * fout <= 20 * e * (k * fin - row)
 
 
 def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order=False):
@@ -361,6 +362,19 @@ def GmmAggregateLinear(rowptr, colind, colptr, rowind, permute, feat, pseudo, ps
     is kept.
     pseudo_csc, own_order: as GmmConvFuseSumTwoOrders; pseudo_csc None: one copy, through permute."""
     return GmmAggregateLinearFunction.apply(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, mu, sigma, weight, own_order)
+
+
+def _matmul_in_parts(a, b, part):
+    """a @ b, the inner dimension summed in parts.  The backward below takes the two linear steps in the other order, with the longer inner
+    dimension in the product: as one chain its gradients of the coordinates and of the input were further from float64 than in the
+    order of the forward (169 k nodes, 128 -> 64 with 3 kernels: 2.2e-7 against 1.7e-7; 300 k, 256 -> 128 with 4: 3.0e-7 and 4.1e-7 against
+    2.3e-7 and 2.1e-7).  In parts of the layer's outputs they are as near (1.7e-7; 2.3e-7 and 2.1e-7), for a pass over the result
+    per part: layer steps 1.01 -> 1.03 and 3.07 -> 3.24 ms."""
+    part = max(32, part // 16 * 16)
+    out = torch.matmul(a[:, :part], b[:part])
+    for c in range(part, a.shape[1], part):
+        out.addmm_(a[:, c:c + part], b[c:c + part])
+    return out
 
 
 class _AggregateHistory(torch.autograd.Function):
@@ -415,11 +429,11 @@ class GmmAggregateLinearFunction(torch.autograd.Function):
         if pad:         # zero columns up to a multiple of 4: the operator then takes its 128-bit row layout
             weight = torch.nn.functional.pad(weight.view(k, fout, fin), (0, 0, 0, pad)).view(-1, fin)
             grad_out = torch.nn.functional.pad(grad_out, (0, pad))
-        proj = torch.matmul(feat, weight.t()).view(-1, k, fout + pad)
+        proj = _matmul_in_parts(feat, weight.t(), fout).view(-1, k, fout + pad)
         t, grad_pseudo, grad_mu, grad_sigma = gmm_native.gmmconv_backward(colptr, rowind, permute, proj, pseudo, mu, sigma, grad_out.contiguous(),
                                                                           sum_kernels=True, own_order=ctx.own_order)
         t = t.view(-1, k * (fout + pad))
-        grad_feat = torch.matmul(t, weight) if ctx.needs_input_grad[5] else None
+        grad_feat = _matmul_in_parts(t, weight, fout) if ctx.needs_input_grad[5] else None
         grad_w = reduce_over_rows(t, feat) if ctx.needs_input_grad[10] else None
         if pad and grad_w is not None:
             grad_w = grad_w.view(k, fout + pad, fin)[:, :fout].reshape(-1, fin)

@@ -187,9 +187,9 @@ def test_gmm_backward_rule_stays_within_the_operator():
 
 
 @pytest.mark.parametrize("k,fin,fout,input_grad,degree,want", [
-    (4, 256, 256, True, 3, False), (4, 256, 256, True, 9, True), (4, 256, 256, False, 3, True), (3, 128, 128, True, 3, False),
-    (3, 128, 128, True, 9, True), (4, 256, 128, True, 3, True), (3, 128, 64, True, 4, True), (2, 16, 16, False, 50, True),
-    (2, 16, 16, False, 200, False), (2, 32, 32, False, 260, False), (3, 32, 32, False, 260, True)])
+    (4, 256, 256, True, 15, False), (4, 256, 256, True, 20, True), (4, 256, 256, False, 3, True), (3, 128, 128, True, 9, False),
+    (3, 128, 128, True, 15, True), (4, 256, 128, True, 4, False), (4, 256, 128, True, 9, True), (3, 128, 64, True, 4, True),
+    (2, 16, 16, False, 50, True), (2, 16, 16, False, 200, False), (2, 32, 32, False, 260, False), (3, 32, 32, False, 260, True)])
 def test_gmm_backward_rule_follows_the_degree(k, fin, fout, input_grad, degree, want):
     """Both sides of the lines that the degree draws (layer steps measured on either side)."""
     from ae_mlsys_gnn_amd.operators.fused_gmmconv import project_in_backward

@@ -413,6 +413,31 @@ def test_gmm_aggregate_linear(fin, fout, k, dim, form, input_grad):
         assert_close_sum(got.grad, want.grad, s[key], "grad " + name, c=c)
 
 
+@pytest.mark.parametrize("fin,fout,k", [(256, 64, 4), (256, 100, 3)])
+def test_gmm_aggregate_linear_precision(fin, fout, k):
+    """The coordinates' gradient is <g_i, (x @ W_k^T)_j> per edge and kernel.  Its error in the 2-norm comes from the product's chain of
+    additions: with the chain in parts of `fout` terms (at least 32, a multiple of 16) and the parts added up, 2^-24 / sqrt(3) *
+    sqrt(part / 2 + parts / 2) of the random sums, where one chain over the inputs has 2^-24 / sqrt(3) * sqrt(fin / 2).  What the dot
+    product and the Gaussian add is less than what the matrix cores, which round less often than once a term, leave of that."""
+    from ae_mlsys_gnn_amd.operators import fused_gmmconv as fg
+    gen = torch.Generator(device=DEV).manual_seed(fin + fout)
+    new = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    g = graphs.uniform_graph(20000, 60000, seed=3).to(DEV)
+    g = graphs.add_csc_torch(g)
+    x, w, go = new(g.n, fin), new(k * fout, fin), new(g.n, fout)
+    ps, mu, sg = torch.rand(g.n_edges, 1, generator=gen, device=DEV).requires_grad_(True), torch.rand(k, 1, generator=gen, device=DEV), 1 + torch.rand(k, 1, generator=gen, device=DEV)
+    fg.GmmAggregateLinear(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, x, ps, None, mu, sg, w).backward(go)
+    row = torch.repeat_interleave(torch.arange(g.n, device=DEV), (g.row_ptr[1:] - g.row_ptr[:-1]).long())
+    h = (x.double() @ w.double().t()).view(g.n, k, fout)
+    dot = torch.stack([(h[:, i][g.col_ind.long()] * go.double()[row]).sum(-1) for i in range(k)], 1)
+    t = (ps.detach().double() - mu.double().t()) * sg.double().t()
+    want = -(dot * torch.exp(-0.5 * t * t) * t * sg.double().t()).sum(1, keepdim=True)
+    part = max(32, fout // 16 * 16)
+    bound = 2.0 ** -24 / 3 ** 0.5 * (part / 2 + -(-fin // part) / 2) ** 0.5
+    err = float((ps.grad.double() - want).norm() / want.norm())
+    assert err <= bound, (err, bound)
+
+
 @pytest.mark.parametrize("fin,fout,k", [(256, 256, 4), (256, 257, 4), (256, 512, 4), (256, 256, 3), (256, 340, 3), (256, 352, 3), (256, 260, 1)])
 @pytest.mark.parametrize("input_grad", [False, True])
 def test_gmm_layer_wide_outputs(fin, fout, k, input_grad):
