@@ -122,7 +122,6 @@ struct rs_args {
     const int *key; const int2 *rec;
     int *a_out, *b_out, *key_out; int2 *rec_out;
     const int *row_ptr, *hint;      // RS_CSR
-    int n_rows, n_hint;
 };
 
 // hint[k] = row of position min(k << CSC_HINT_SHIFT, n - 1): a coarse inverse of row_ptr.  128 = the records a wave of a small
@@ -488,7 +487,7 @@ extern "C" int fgnn_csr2csc(int n_rows, int n_cols, int64_t E, const int32_t *ro
     for (int i = 0; i < p.passes && !rc; ++i) {
         const bool last = i == p.passes - 1;
         rs_args A = {};
-        A.a = col_ind; A.row_ptr = row_ptr; A.hint = hint; A.n_rows = n_rows; A.n_hint = n_hint;
+        A.a = col_ind; A.row_ptr = row_ptr; A.hint = hint;
         if (i > 0) { A.key = key[(i - 1) & 1]; A.rec = rec[(i - 1) & 1]; }
         A.key_out = last ? sorted : key[i & 1];
         A.rec_out = last ? nullptr : rec[i & 1];
