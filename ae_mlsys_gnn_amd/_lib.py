@@ -143,15 +143,20 @@ def ptr(t):
     return c_void_p(t.data_ptr())
 
 
+# torch's own names for the two below are private: where a torch does not have them, the public forms do the same, more slowly.
+_DeviceGuard = getattr(torch.cuda, "_DeviceGuard", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def device_guard(device):
     """Makes a tensor's device the current one: torch.cuda.device without its parsing of the argument."""
-    return torch.cuda._DeviceGuard(device.index)
+    return torch.cuda.device(device) if _DeviceGuard is None else _DeviceGuard(device.index)
 
 
 def stream_ptr():
     """The current stream of the current device.  Asked for as a raw handle: building a torch Stream object around it took 10 us a
     call, five times a layer step."""
-    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    return c_void_p(torch.cuda.current_stream().cuda_stream if _raw_stream is None else _raw_stream(torch.cuda.current_device()))
 
 
 def require_cuda(*tensors):

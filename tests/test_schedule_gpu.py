@@ -157,3 +157,19 @@ def test_own_order_view_of_a_graph(monkeypatch):
     idx_p, perm_p = _lib.own_order_view(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute)
     assert idx_p.data_ptr() == g.col_ind.data_ptr() and perm_p.data_ptr() == g.permute.data_ptr()
     _lib.clear_schedule_cache()
+
+
+@pytest.mark.parametrize("private_names", [True, False])
+def test_native_calls_follow_the_current_stream(monkeypatch, private_names):
+    """The stream handed to the library is the current one of the tensors' device, with torch's private names and without them."""
+    from ae_mlsys_gnn_amd import _lib
+    if not private_names:
+        monkeypatch.setattr(_lib, "_raw_stream", None)
+        monkeypatch.setattr(_lib, "_DeviceGuard", None)
+    dev = torch.device("cuda", torch.cuda.current_device())
+    side = torch.cuda.Stream()
+    with _lib.device_guard(dev):
+        assert (_lib.stream_ptr().value or 0) == torch.cuda.current_stream().cuda_stream
+        with torch.cuda.stream(side):
+            assert _lib.stream_ptr().value == side.cuda_stream
+    assert torch.cuda.current_device() == dev.index
