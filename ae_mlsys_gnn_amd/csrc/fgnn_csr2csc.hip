@@ -446,7 +446,8 @@ static int rs_sort_pairs(const int *keys_in, const int *pay_in, int64_t n, int k
     return 0;
 }
 
-// Up to two buffers of (key, two words), the sorted columns, the digit counts, the row hints.
+// Up to two buffers of (key, two words), the sorted columns, the digit counts, the row hints: 16 bytes per entry up to 22 bits of column
+// ids (4 M columns) and 28 above, where the passes through an index payload held 12.
 extern "C" size_t fgnn_csr2csc_workspace_bytes(int n_rows, int n_cols, int64_t E)
 {
     (void)n_rows;
@@ -703,7 +704,8 @@ __global__ __launch_bounds__(256) void coo_write_kernel(int64_t n, int n_rows, c
     }
 }
 
-// With positions: two buffers of (key, two words); without: two of pairs.  The caller's edge_pos is not known here: room for both.
+// With positions: two buffers of (key, two words); without: two of pairs.  The caller's edge_pos is not known here: room for both, 24 bytes
+// per edge (through index payloads, 36).
 extern "C" size_t fgnn_coo2csr_workspace_bytes(int n_rows, int n_cols, int64_t E)
 {
     const rs_plan ps = rs_plan_of(rs_key_bits(n_cols)), pd = rs_plan_of(rs_key_bits(n_rows));

@@ -473,7 +473,7 @@ int    fgnn_cross_entropy_backward(int64_t N, int C, int64_t ld, int64_t ld_grad
  * Replaces csrtocsc.csr2csc (src/csr2csc/csr2csc.cc; csr2csc.cu:7-43, a cuSPARSE
  * cusparseCsr2cscEx2 call).  Stable: entries of a column keep ascending CSR position.
  * Outputs col_ptr [n_cols+1], row_ind [E], permute [E] (int32 positions; the reference carries
- * them as float values). */
+ * them as float values).  The workspace holds 16 bytes per entry for up to 2^22 columns, 28 above. */
 size_t fgnn_csr2csc_workspace_bytes(int n_rows, int n_cols, int64_t E);
 int    fgnn_csr2csc(int n_rows, int n_cols, int64_t E, const int32_t *row_ptr, const int32_t *col_ind,
                     int32_t *col_ptr, int32_t *row_ind, int32_t *permute,
@@ -484,7 +484,8 @@ int    fgnn_csr2csc(int n_rows, int n_cols, int64_t E, const int32_t *row_ptr, c
  * dedupe != 0 duplicate (dst, src) pairs are merged.  Replaces the host-side scipy csr_matrix call of
  * the reference's drivers (script/train/train_gatconv_our.py:87-91).  Outputs: row_ptr [n_rows+1],
  * col_ind (first *n_out entries valid; capacity E), n_out (device int64: number of CSR entries),
- * edge_pos [E] optional: CSR position of every input edge (to carry per-edge data along). */
+ * edge_pos [E] optional: CSR position of every input edge (to carry per-edge data along).  The workspace
+ * holds 24 bytes per edge. */
 size_t fgnn_coo2csr_workspace_bytes(int n_rows, int n_cols, int64_t E);
 int    fgnn_coo2csr(int n_rows, int n_cols, int64_t E, const int32_t *dst, const int32_t *src, int dedupe,
                     int32_t *row_ptr, int32_t *col_ind, int64_t *n_out, int32_t *edge_pos,
