@@ -463,11 +463,16 @@ __device__ __forceinline__ knn_best knn_exact_tile(int P, int D, int k, int rows
     __syncthreads();                                    // the last slice has been read
     return best;
 }
+// The same as a function of its own.  Its pointers name their memory: plain ones would be accessed by flat instructions, of which the
+// ordering that fg_wave_lds_sync counts on (LDS instructions of a wave execute in order) is not known.
+typedef __attribute__((address_space(3))) float *knn_lds_floats;
+typedef __attribute__((address_space(3))) float2 *knn_lds_pairs;
+typedef const __attribute__((address_space(1))) float *knn_global_floats;
 template <int RG>
-__device__ __attribute__((noinline)) knn_best knn_exact_tile_call(int P, int D, int k, int rows_aligned, const float *cp, int q0, int tile0, unsigned any, unsigned open,
-                                                                  float *cs, float2 *list, knn_best best)
+__device__ __attribute__((noinline)) knn_best knn_exact_tile_call(int P, int D, int k, int rows_aligned, knn_global_floats cp, int q0, int tile0, unsigned any,
+                                                                  unsigned open, knn_lds_floats cs, knn_lds_pairs list, knn_best best)
 {
-    return knn_exact_tile<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, cs, list, best);
+    return knn_exact_tile<RG>(P, D, k, rows_aligned, (const float *)cp, q0, tile0, any, open, (float *)cs, (float2 *)list, best);
 }
 
 template <int RG, bool MULTI>
@@ -700,7 +705,7 @@ __global__ __launch_bounds__(KNN_MW * 64, 4) void knn_mfma_kernel(int P, int D, 
             knn_best best;
 #pragma unroll
             for (int a = 0; a < 4; ++a) { best.d[a] = pd[a]; best.i[a] = pi[a]; }
-            if constexpr (MULTI) best = knn_exact_tile_call<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, buf, list, best);
+            if constexpr (MULTI) best = knn_exact_tile_call<RG>(P, D, k, rows_aligned, (knn_global_floats)cp, q0, tile0, any, open, (knn_lds_floats)buf, (knn_lds_pairs)list, best);
             else best = knn_exact_tile<RG>(P, D, k, rows_aligned, cp, q0, tile0, any, open, buf, list, best);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
