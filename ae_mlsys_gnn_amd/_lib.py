@@ -143,9 +143,10 @@ def ptr(t):
     return c_void_p(t.data_ptr())
 
 
-# torch's own names for the two below are private: where a torch does not have them, the public forms do the same, more slowly.
+# torch's own names for what the two below need are private: where a torch does not have them, the public forms do the same, more slowly.
 _DeviceGuard = getattr(torch.cuda, "_DeviceGuard", None)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def device_guard(device):
@@ -156,7 +157,7 @@ def device_guard(device):
 def stream_ptr():
     """The current stream of the current device.  Asked for as a raw handle: building a torch Stream object around it took 10 us a
     call, five times a layer step."""
-    return c_void_p(torch.cuda.current_stream().cuda_stream if _raw_stream is None else _raw_stream(torch.cuda.current_device()))
+    return c_void_p(torch.cuda.current_stream().cuda_stream if _raw_stream is None else _raw_stream(_current_device()))
 
 
 def require_cuda(*tensors):
