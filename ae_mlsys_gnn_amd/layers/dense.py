@@ -8,9 +8,13 @@ from __future__ import annotations
 
 import torch
 
+from ..operators.tall import product_wanted, reduce_wanted, tall_product, tall_reduce
+
 
 def reduce_over_rows(x, g):
     """x^T @ g for tall x [N, a], g [N, b]."""
+    if not torch.is_grad_enabled() and reduce_wanted(x, g):        # (a graph of the result is recorded by the operations below)
+        return tall_reduce(x, g)
     n = x.shape[0]
     chunks = min(256, n // 2048)
     if chunks < 2:
@@ -58,6 +62,8 @@ class _TallLinear(torch.autograd.Function):
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
+        if product_wanted(x, weight, x.shape[1], weight.shape[0]) and (bias is None or (bias.is_cuda and bias.dtype == torch.float32)):
+            return tall_product(x, weight, transposed=True, bias=bias)
         y = torch.matmul(x, weight.t())
         return y if bias is None else y.add_(bias)
 
@@ -65,8 +71,13 @@ class _TallLinear(torch.autograd.Function):
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
         g = g.contiguous()
-        gx = torch.matmul(g, weight) if ctx.needs_input_grad[0] else None
-        gw = reduce_over_rows(g, x) if ctx.needs_input_grad[1] else None
+        gx = gw = None
+        if ctx.needs_input_grad[0]:
+            # where a graph of the gradients is wanted, the operation that records one
+            own = not torch.is_grad_enabled() and product_wanted(g, weight, *weight.shape)
+            gx = tall_product(g, weight) if own else torch.matmul(g, weight)
+        if ctx.needs_input_grad[1]:
+            gw = reduce_over_rows(g, x)
         gb = column_sum(g) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return gx, gw, gb
 

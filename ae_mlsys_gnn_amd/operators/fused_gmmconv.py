@@ -7,6 +7,7 @@ from __future__ import annotations
 import torch
 
 from .._lib import FgnnError, as_f32, as_i32, check, device_guard, edge_positions, lib, ptr, require_cuda, schedule_for, stream_ptr, workspace
+from .tall import product_wanted, tall_product
 
 
 def _plain_list_for_summed_backward(n, e):
@@ -404,7 +405,8 @@ class GmmAggregateLinearFunction(torch.autograd.Function):
         # after the forward, the aggregate
         ctx.save_for_backward(colptr, rowind, None if ctx.two_orders else permute, feat, pseudo_csc if ctx.two_orders else pseudo, mu, sigma, weight,
                               rowptr, colind, agg if ctx.two_orders else None)
-        return torch.matmul(agg.view(-1, k * fin), w.t())
+        agg = agg.view(-1, k * fin)
+        return tall_product(agg, w, transposed=True) if product_wanted(agg, w, k * fin, fout) else torch.matmul(agg, w.t())
 
     @staticmethod
     def backward(ctx, grad_out):

@@ -283,6 +283,20 @@ int fgnn_gat_unfold_grads(int fin, int H, int F, int pad, const float *W, const 
                           const float *dproj, int ldp, const float *dscore, int lds, float *dW, float *dattn_l,
                           float *dattn_r, void *stream);
 
+/* Dense products over very many rows, in fp32 on the matrix instructions.
+ * fgnn_tall_product: y [n, m] = x [n, k] @ B [k, m] (+ bias [m]); B[r][c] at b[r*ldb + c], or at b[c*ldb + r] when b_transposed.
+ * With hin > 0, xe0 and xe1 [n, hin] are the input columns k .. k+2*hin; with hout > 0, ye0 and ye1 [n, hout] receive the output
+ * columns m .. m+2*hout (B has those rows and columns too).  At most 18 tiles of 16 output columns, the extra ones a
+ * tile of their own; hin, hout <= 8; y 16-byte aligned when ldy is a multiple of 4.
+ * fgnn_tall_reduce: c [ka, kb + 2h] = x [n, ka]^T @ [g [n, kb] | ge0 [n, h] | ge1 [n, h]], deterministic; workspace_bytes is 0 for
+ * shapes it does not take. */
+int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_t ldx, const float *b, int64_t ldb, int b_transposed,
+                      const float *bias, float *y, int64_t ldy, int hin, const float *xe0, const float *xe1, int hout,
+                      float *ye0, float *ye1, void *stream);
+size_t fgnn_tall_reduce_workspace_bytes(int64_t n, int ka, int kb, int h);
+int fgnn_tall_reduce(int64_t n, int ka, int kb, const float *x, int64_t ldx, const float *g, int64_t ldg, int h,
+                     const float *ge0, const float *ge1, float *c, void *workspace, size_t workspace_bytes, void *stream);
+
 /* k-nearest-neighbour graph of batched point clouds, the input of fgnn_edgeconv_forward: points
  * [n_clouds*P, D]; src_ind [n_clouds*P*k] gets, for every point, the global ids of the k nearest
  * points of its own cloud (itself included), nearest first, ties to the smaller id; 1 <= k <= min(P,

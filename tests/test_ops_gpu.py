@@ -1657,3 +1657,59 @@ def test_edge_linear_tanh_alignment(e, d):
     want = torch.tanh(x[1:].double() @ w.double().t() + b.double())
     # three roundings of the argument (|x w| <= 30 here) and tanh's own error
     assert float((shifted.double() - want).abs().max()) < 3 * 30 * 2.0 ** -24 + 1e-6
+
+
+# ---------------------------------------------------------------- dense products over many rows
+
+def _bound(a, b, chain):
+    """Largest error of a sum of products in fp32: one rounding per step of the longest chain, on the sum of absolute products."""
+    return (chain + 2) * 2.0 ** -24 * (a.abs().double() @ b.abs().double()) + 1e-30
+
+
+# rows below, at and past a tile of 16 and a workgroup's 256; input columns around a chunk of 16 and a group of 64, in rows of every alignment;
+# output columns around a tile, a column range of LDS and the kernels' numbers of tiles
+@pytest.mark.parametrize("n,k,m,h_in,h_out", [(1, 1, 1, 0, 0), (15, 3, 17, 0, 0), (16, 16, 16, 0, 1), (17, 20, 15, 8, 0), (257, 64, 48, 1, 0), (300, 63, 100, 0, 8),
+                                              (1000, 65, 256, 0, 3), (777, 41, 23, 0, 0), (515, 602, 32, 0, 0), (260, 256, 256, 0, 8), (270, 256, 100, 8, 0),
+                                              (64, 1024, 33, 2, 0), (129, 130, 280, 0, 5), (40, 12, 512, 0, 0), (5000, 48, 64, 3, 0)])
+def test_tall_product(n, k, m, h_in, h_out):
+    from ae_mlsys_gnn_amd.operators.tall import tall_product
+    gen = torch.Generator().manual_seed(n * 131 + k)
+    rnd = lambda *s: torch.randn(*s, generator=gen)
+    x, b, bias, extra = rnd(n, k), rnd(k + 2 * h_in, m + 2 * h_out), rnd(m), [rnd(n, h_in), rnd(n, h_in)] if h_in else None
+    full = torch.cat([x] + (extra or []), 1)
+    ref, tol = full.double() @ b.double(), _bound(full, b, full.shape[1])
+    dx, db, de = x.cuda(), b.cuda(), [t.cuda() for t in extra] if h_in else None
+    strided = torch.full((n, k + 4), float("nan"), device="cuda")       # rows further apart than they are long, NaN between them
+    strided[:, :k] = dx
+    for xx, bb, tr in ((dx, db, False), (strided[:, :k], db.t().contiguous(), True)):
+        out = tall_product(xx, bb, transposed=tr, extra_in=de, extra_out=h_out)
+        got = torch.cat(list(out), 1) if h_out else out
+        assert got.shape == ref.shape and bool(((got.cpu().double() - ref).abs() <= tol).all())
+    if not h_out:
+        got = tall_product(dx, db, extra_in=de, bias=bias.cuda())
+        assert bool(((got.cpu().double() - ref - bias.double()).abs() <= tol + 2.0 ** -23 * (ref + bias.double()).abs() + 1e-30).all())
+    # a row of infinities stays its own
+    if n > 1:
+        dx[0, 0] = float("inf")
+        got = tall_product(dx, db, extra_in=de, extra_out=h_out)
+        got = torch.cat(list(got), 1) if h_out else got
+        assert bool(torch.isinf(got[0]).all()) and bool(((got[1:].cpu().double() - ref[1:]).abs() <= tol[1:]).all())
+
+
+# results of one tile to the most tiles a wave takes (and one tile row per wave), rows around a staged block and around a workgroup's share
+@pytest.mark.parametrize("n,a,b,h", [(1, 1, 1, 0), (31, 16, 16, 0), (33, 17, 15, 1), (255, 64, 64, 4), (257, 100, 256, 8), (1025, 256, 48, 1), (4100, 41, 23, 0),
+                                     (600, 602, 32, 0), (513, 256, 256, 8), (70000, 20, 4, 0), (300, 48, 200, 0), (90, 4, 512, 2), (2000, 144, 160, 3)])
+def test_tall_reduce(n, a, b, h):
+    from ae_mlsys_gnn_amd.operators.tall import tall_reduce
+    gen = torch.Generator().manual_seed(n * 17 + a)
+    rnd = lambda *s: torch.randn(*s, generator=gen)
+    x, g, extra = rnd(n, a), rnd(n, b), [rnd(n, h), rnd(n, h)] if h else None
+    full = torch.cat([g] + (extra or []), 1)
+    ref, tol = x.double().t() @ full.double(), _bound(x.t(), full, n)
+    dx, dg, de = x.cuda(), g.cuda(), [t.cuda() for t in extra] if h else None
+    wide = torch.full((n, b + 3), float("nan"), device="cuda")
+    wide[:, :b] = dg
+    one = tall_reduce(dx, dg, de)
+    for got in (one, tall_reduce(dx, wide[:, :b], de)):
+        assert got.shape == ref.shape and bool(((got.cpu().double() - ref).abs() <= tol).all())
+    assert torch.equal(one, tall_reduce(dx, dg, de))                     # fixed order of summation
