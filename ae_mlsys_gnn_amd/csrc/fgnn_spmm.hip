@@ -39,6 +39,38 @@ __device__ __forceinline__ float gmm_weight(const float (&pv)[GMM_PV], const flo
     return __expf(-0.5f * acc);
 }
 
+// A mixture whose pseudo-coordinates are tanh(raw @ W^T + b) of two constant numbers per edge (the projection in front of every layer of
+// the MoNet drivers): the kernels' PJ forms read the raw pair and form the coordinates where they need them.
+struct GmmProj { const float2 *raw; const float *W; const float *b; };
+
+// mu | inv_sigma | W | b into LDS, by n threads
+template <bool PJ>
+__device__ __forceinline__ void gmm_stage(float *shared, int tid, int n, int K, int dim, const float *mu, const float *isg, const GmmProj &pj)
+{
+    const int KD = K * dim;
+    for (int i = tid; i < KD; i += n) { shared[i] = mu[i]; shared[KD + i] = isg[i]; }
+    if constexpr (PJ) {
+        for (int i = tid; i < 3 * dim; i += n) shared[2 * KD + i] = i < 2 * dim ? pj.W[i] : pj.b[i - 2 * dim];
+    }
+}
+// The coordinates of the edge at `pos` (the first GMM_PV of them; ps: all of them, where they are given) and, projected, its raw pair.
+template <bool PJ>
+__device__ __forceinline__ const float *gmm_coordinates(const float *pseudo, const GmmProj &pj, const float *shared, size_t pos, int K, int dim,
+                                                        float (&pv)[GMM_PV], float2 &rv)
+{
+    if constexpr (PJ) {
+        rv = pj.raw[pos];
+        const float *w = shared + 2 * K * dim;
+#pragma unroll
+        for (int d = 0; d < GMM_PV; ++d) pv[d] = d < dim ? tanhf(fmaf(rv.y, w[2 * d + 1], fmaf(rv.x, w[2 * d], w[2 * dim + d]))) : 0.f;
+        return nullptr;                             // dim <= GMM_PV
+    } else {
+        const float *ps = pseudo + pos * dim;
+        gmm_load_pseudo(ps, dim, pv);
+        return ps;
+    }
+}
+
 // Final store of an accumulated row: either the [H,F] row itself or, with sum_h, its sum over heads.
 // scr: wave-private LDS of HF floats (only touched with sum_h).
 template <int VEC, int R, bool FULL>
@@ -89,18 +121,16 @@ struct WAtt {
         for (int h = 0; h < H; ++h) wl[h * 64 + lane] = ok ? (att ? att[pos * ld + h] : 1.f) : 0.f;
     }
 };
+template <bool PJ>
 struct WGauss {
-    const float *pseudo; const float *mu; const float *isg; float *gauss_out; int dim;
-    // stage mu / inv_sigma [K,dim] into workgroup LDS
-    __device__ __forceinline__ void prepare(float *shared, int tid, int K) const
-    {
-        for (int i = tid; i < K * dim; i += FGNN_TPB) { shared[i] = mu[i]; shared[K * dim + i] = isg[i]; }
-    }
+    const float *pseudo; const float *mu; const float *isg; float *gauss_out; int dim; GmmProj pj;
+    // stage mu / inv_sigma [K,dim] (and the projection) into workgroup LDS
+    __device__ __forceinline__ void prepare(float *shared, int tid, int K) const { gmm_stage<PJ>(shared, tid, FGNN_TPB, K, dim, mu, isg, pj); }
     __device__ __forceinline__ void fill(float *wl, const float *shared, int lane, size_t pos, bool ok, int K) const
     {
-        const float *ps = pseudo + pos * dim;
         float pv[GMM_PV];
-        gmm_load_pseudo(ps, dim, pv);
+        float2 rv;
+        const float *ps = gmm_coordinates<PJ>(pseudo, pj, shared, pos, K, dim, pv, rv);
         for (int k = 0; k < K; ++k) {
             float w = gmm_weight(pv, ps, shared + k * dim, shared + K * dim + k * dim, dim);
             wl[k * 64 + lane] = ok ? w : 0.f;
@@ -563,31 +593,62 @@ extern "C" size_t fgnn_gmm_forward_workspace_bytes(const fgnn_schedule_t *sched,
 }
 
 static int gmm_forward_shared(int N, int K, int dim, int F, const int32_t *ptr, const int32_t *idx, const int32_t *pos_map, const float *feat,
-                              const float *pseudo, const float *mu, const float *isg, float *out, const fgnn_schedule_t *sched,
+                              const float *pseudo, const GmmProj &pj, const float *mu, const float *isg, float *out, const fgnn_schedule_t *sched,
                               void *workspace, size_t workspace_bytes, hipStream_t st);
+
+// Limits of a projection: the coordinates fit the registers of gmm_coordinates, a lane's sums the LDS of a workgroup.
+#define GMM_PROJ_K 4
+static int gmm_checks(const char *fn, int N, int64_t E, int K, int dim, int F, const int32_t *ptr, const int32_t *idx, const float *pseudo, const GmmProj *pj,
+                      const fgnn_schedule_t *sched)
+{
+    int rc = spmm_checks(fn, N, E, K, F, sched, ptr, idx);
+    if (rc) return rc;
+    FGNN_REQUIRE((int64_t)K * F <= 1024, FGNN_ERR_LIMIT, "%s: K*F=%lld > 1024 unsupported", fn, (long long)K * F);
+    FGNN_REQUIRE(dim >= 1 && dim <= 64 && K * dim <= 1024, FGNN_ERR_LIMIT, "%s: dim=%d K*dim=%d unsupported", fn, dim, K * dim);
+    if (pj) {
+        FGNN_REQUIRE(dim <= GMM_PV && K <= GMM_PROJ_K, FGNN_ERR_LIMIT, "%s: at most %d projected coordinates and %d kernels (dim=%d, K=%d)", fn, GMM_PV,
+                     GMM_PROJ_K, dim, K);
+        FGNN_REQUIRE(pj->raw || E == 0, FGNN_ERR_NULL, "%s: NULL argument", fn);
+        FGNN_REQUIRE(pj->W && pj->b, FGNN_ERR_NULL, "%s: NULL argument", fn);
+        FGNN_REQUIRE((((uintptr_t)pj->raw) & 7u) == 0, FGNN_ERR_ALIGN, "%s: raw pairs not 8-byte aligned", fn);
+    } else FGNN_REQUIRE(pseudo || E == 0, FGNN_ERR_NULL, "%s: NULL argument", fn);
+    return 0;
+}
+
+static int gmm_forward_impl(const char *fn, int N, int64_t E, int K, int dim, int F, const int32_t *ptr, const int32_t *idx, const int32_t *pos_map,
+                            const float *node_feat, const float *pseudo, const GmmProj *proj, const float *mu, const float *inv_sigma, const float *bias,
+                            const float *residual, float *out, float *gauss_out, int sum_kernels, const fgnn_schedule_t *sched, void *workspace,
+                            size_t workspace_bytes, void *stream)
+{
+    int rc = gmm_checks(fn, N, E, K, dim, F, ptr, idx, pseudo, proj, sched);
+    if (rc) return rc;
+    FGNN_REQUIRE(ptr && (idx || E == 0) && node_feat && mu && inv_sigma && out, FGNN_ERR_NULL, "%s: NULL argument", fn);
+    FGNN_REQUIRE(sum_kernels >= 0 && sum_kernels <= 2, FGNN_ERR_SHAPE, "%s: sum_kernels=%d (0, 1 or 2)", fn, sum_kernels);
+    FGNN_REQUIRE(sum_kernels == 1 || (!bias && !residual), FGNN_ERR_SHAPE, "%s: bias and residual are added to the sum over the kernels", fn);
+    const GmmProj pj = proj && E > 0 ? *proj : GmmProj{nullptr, nullptr, nullptr};
+    if (sum_kernels == 2) {
+        FGNN_REQUIRE(!gauss_out, FGNN_ERR_SHAPE, "%s: gauss_out is not available with shared node features", fn);
+        return gmm_forward_shared(N, K, dim, F, ptr, idx, pos_map, node_feat, pseudo, pj, mu, inv_sigma, out, sched, workspace, workspace_bytes,
+                                  (hipStream_t)stream);
+    }
+    SpmmP p{};
+    p.ptr = ptr; p.idx = idx; p.pos_map = pos_map; p.feat = node_feat; p.out = out; p.N = N; p.H = K; p.F = F; p.HF = K * F;
+    p.sum_h = sum_kernels; p.bias = bias; p.res = residual;
+    const bool aligned = fgnn_aligned16(node_feat) && fgnn_aligned16(out) && (!bias || fgnn_aligned16(bias)) && (!residual || fgnn_aligned16(residual));
+    if (pj.raw)
+        return spmm_launch(fn, p, WGauss<true>{pseudo, mu, inv_sigma, gauss_out, dim, pj}, 2 * K * dim + 3 * dim, sched, aligned, workspace, workspace_bytes,
+                           (hipStream_t)stream);
+    return spmm_launch(fn, p, WGauss<false>{pseudo, mu, inv_sigma, gauss_out, dim, pj}, 2 * K * dim, sched, aligned, workspace, workspace_bytes,
+                       (hipStream_t)stream);
+}
 
 extern "C" int fgnn_gmm_forward(int N, int64_t E, int K, int dim, int F, const int32_t *ptr, const int32_t *idx,
                                 const int32_t *pos_map, const float *node_feat, const float *pseudo, const float *mu,
                                 const float *inv_sigma, float *out, float *gauss_out, int sum_kernels,
                                 const fgnn_schedule_t *sched, void *workspace, size_t workspace_bytes, void *stream)
 {
-    int rc = spmm_checks("fgnn_gmm_forward", N, E, K, F, sched, ptr, idx);
-    if (rc) return rc;
-    FGNN_REQUIRE((int64_t)K * F <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_forward: K*F=%lld > 1024 unsupported", (long long)K * F);
-    FGNN_REQUIRE(dim >= 1 && dim <= 64 && K * dim <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_forward: dim=%d K*dim=%d unsupported", dim, K * dim);
-    FGNN_REQUIRE(ptr && (idx || E == 0) && node_feat && (pseudo || E == 0) && mu && inv_sigma && out, FGNN_ERR_NULL, "fgnn_gmm_forward: NULL argument");
-    FGNN_REQUIRE(sum_kernels >= 0 && sum_kernels <= 2, FGNN_ERR_SHAPE, "fgnn_gmm_forward: sum_kernels=%d (0, 1 or 2)", sum_kernels);
-    if (sum_kernels == 2) {
-        FGNN_REQUIRE(!gauss_out, FGNN_ERR_SHAPE, "fgnn_gmm_forward: gauss_out is not available with shared node features");
-        return gmm_forward_shared(N, K, dim, F, ptr, idx, pos_map, node_feat, pseudo, mu, inv_sigma, out, sched, workspace, workspace_bytes,
-                                  (hipStream_t)stream);
-    }
-    SpmmP p{};
-    p.ptr = ptr; p.idx = idx; p.pos_map = pos_map; p.feat = node_feat; p.out = out; p.N = N; p.H = K; p.F = F; p.HF = K * F;
-    p.sum_h = sum_kernels;
-    WGauss wf{pseudo, mu, inv_sigma, gauss_out, dim};
-    return spmm_launch("fgnn_gmm_forward", p, wf, 2 * K * dim, sched, fgnn_aligned16(node_feat) && fgnn_aligned16(out), workspace,
-                       workspace_bytes, (hipStream_t)stream);
+    return gmm_forward_impl("fgnn_gmm_forward", N, E, K, dim, F, ptr, idx, pos_map, node_feat, pseudo, nullptr, mu, inv_sigma, nullptr, nullptr, out, gauss_out,
+                            sum_kernels, sched, workspace, workspace_bytes, stream);
 }
 
 // fgnn_gmm_forward with sum_kernels == 1 and the rest of the layer's forward in the store: out[i,:] = sum_k sum_p ... +
@@ -597,18 +658,19 @@ extern "C" int fgnn_gmm_forward_epilogue(int N, int64_t E, int K, int dim, int F
                                          const float *inv_sigma, const float *bias, const float *residual, float *out, float *gauss_out,
                                          const fgnn_schedule_t *sched, void *workspace, size_t workspace_bytes, void *stream)
 {
-    int rc = spmm_checks("fgnn_gmm_forward_epilogue", N, E, K, F, sched, ptr, idx);
-    if (rc) return rc;
-    FGNN_REQUIRE((int64_t)K * F <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_forward_epilogue: K*F=%lld > 1024 unsupported", (long long)K * F);
-    FGNN_REQUIRE(dim >= 1 && dim <= 64 && K * dim <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_forward_epilogue: dim=%d K*dim=%d unsupported", dim, K * dim);
-    FGNN_REQUIRE(ptr && (idx || E == 0) && node_feat && (pseudo || E == 0) && mu && inv_sigma && out, FGNN_ERR_NULL,
-                 "fgnn_gmm_forward_epilogue: NULL argument");
-    SpmmP p{};
-    p.ptr = ptr; p.idx = idx; p.pos_map = pos_map; p.feat = node_feat; p.out = out; p.N = N; p.H = K; p.F = F; p.HF = K * F;
-    p.sum_h = 1; p.bias = bias; p.res = residual;
-    WGauss wf{pseudo, mu, inv_sigma, gauss_out, dim};
-    const bool aligned = fgnn_aligned16(node_feat) && fgnn_aligned16(out) && (!bias || fgnn_aligned16(bias)) && (!residual || fgnn_aligned16(residual));
-    return spmm_launch("fgnn_gmm_forward_epilogue", p, wf, 2 * K * dim, sched, aligned, workspace, workspace_bytes, (hipStream_t)stream);
+    return gmm_forward_impl("fgnn_gmm_forward_epilogue", N, E, K, dim, F, ptr, idx, pos_map, node_feat, pseudo, nullptr, mu, inv_sigma, bias, residual, out,
+                            gauss_out, 1, sched, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fgnn_gmm_forward_projected(int N, int64_t E, int K, int dim, int F, const int32_t *ptr, const int32_t *idx,
+                                          const int32_t *pos_map, const float *node_feat, const float *raw, const float *proj_W, const float *proj_b,
+                                          const float *mu, const float *inv_sigma, const float *bias, const float *residual, float *out,
+                                          float *gauss_out, int sum_kernels, const fgnn_schedule_t *sched, void *workspace, size_t workspace_bytes,
+                                          void *stream)
+{
+    const GmmProj pj{(const float2 *)raw, proj_W, proj_b};
+    return gmm_forward_impl("fgnn_gmm_forward_projected", N, E, K, dim, F, ptr, idx, pos_map, node_feat, nullptr, &pj, mu, inv_sigma, bias, residual, out,
+                            gauss_out, sum_kernels, sched, workspace, workspace_bytes, stream);
 }
 
 // ------------------------------------------------------------------------------- GMM backward
@@ -621,25 +683,86 @@ struct GmmBwdP {
     int g_stride;   // floats per grad_out row: HF, or F when grad_out is the gradient of the sum over kernels
     int x_stride;   // floats per node_feat row: HF, or F when all mixture kernels share one [N,F] feature matrix
     int lphp;       // > 0: head-aligned lane map with this many lanes per mixture kernel
+    GmmProj pj;
+    float *acc;     // projected coordinates: per wave of the launch the sums of GmmAcc, in place of gww
 };
+
+// The derivatives of a projected mixture are sums over all edges (of mu, inv_sigma, and the projection's W and b): formed where gw * w
+// is, instead of storing gw * w per edge and kernel and reading it back with the coordinates in two more passes over the edges.
+// Each lane takes the entry of the chunk whose weights it formed, with sums of its own in LDS (2 K dim + 3 dim of
+// them; registers would cost the gather a wave per SIMD), which a wave adds up at its end.
+//   mu | inv_sigma [K, dim] each | W [dim, 2] | b [dim]
+__host__ __device__ static inline int gmm_n_acc(int K, int dim) { return 2 * K * dim + 3 * dim; }
+struct GmmAcc {
+    float *sums;        // [n][64]
+    int n;
+    __device__ __forceinline__ void init(float *lds, int K, int dim, int lane)
+    {
+        sums = lds + lane; n = gmm_n_acc(K, dim);
+#pragma unroll 1
+        for (int i = 0; i < n; ++i) sums[i * 64] = 0.f;
+    }
+    // gww: the lane's gw * w of kernel 0, kernels 64 floats apart (0 for a lane without an entry)
+    __device__ __forceinline__ void add(const float *gww, const float *shared, int K, int dim, const float (&pv)[GMM_PV], float2 rv)
+    {
+        const int KD = K * dim;
+#pragma unroll 1                                    // (a few dozen instructions per 64 entries; unrolled they cost registers over the whole pass)
+        for (int d = 0; d < dim; ++d) {
+            const float pd = d == 0 ? pv[0] : d == 1 ? pv[1] : d == 2 ? pv[2] : pv[3];
+            float gp = 0.f;
+#pragma unroll 1
+            for (int k = 0; k < K; ++k) {
+                const float g = gww[k * 64], sg = shared[KD + k * dim + d], diff = pd - shared[k * dim + d];
+                const float a = g * diff * sg;
+                sums[(k * dim + d) * 64] += a * sg;
+                sums[(KD + k * dim + d) * 64] -= a * diff;
+                gp = fmaf(-g * diff, sg * sg, gp);
+            }
+            const float gt = gp * (1.f - pd * pd);
+            float *w = sums + 2 * KD * 64;
+            w[(2 * d) * 64] = fmaf(gt, rv.x, w[(2 * d) * 64]);
+            w[(2 * d + 1) * 64] = fmaf(gt, rv.y, w[(2 * d + 1) * 64]);
+            w[(2 * dim + d) * 64] += gt;
+        }
+    }
+    __device__ __forceinline__ void finish(float *out, int lane)
+    {
+#pragma unroll 1
+        for (int i = 0; i < n; ++i) {
+            const float v = fg_wave_sum(sums[i * 64]);
+            if (lane == 0) out[i] = v;
+        }
+    }
+};
+// This wave's sums; a wave without work leaves zeros.
+__device__ __forceinline__ float *gmm_acc_out(const GmmBwdP &p) { return p.acc + ((size_t)blockIdx.x * FGNN_WPB + fg_wave()) * gmm_n_acc(p.K, p.dim); }
+template <bool ACC>
+__device__ __forceinline__ void gmm_acc_none(const GmmBwdP &p)
+{
+    if constexpr (ACC)
+        for (int i = fg_lane(); i < gmm_n_acc(p.K, p.dim); i += 64) gmm_acc_out(p)[i] = 0.f;
+}
 
 // One pass over CSC column j (x[j] stays in registers): per in-edge gather grad_out[i], accumulate
 // w * grad_out[i] into grad_feat[j] and form gw = <grad_out[i,k,:], x[j,k,:]> per mixture kernel
 // (DPP butterflies inside head groups).  gw*w is written once per edge at its CSR position; the
 // Gaussian derivatives are finished by gauss_grad_kernel below.
-template <int VEC, int R, bool FULL, int LPH>
+template <int VEC, int R, bool FULL, int LPH, bool PJ>
 __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_kernel(GmmBwdP p)
 {
     extern __shared__ float lds[];
     const int K = p.K, dim = p.dim, KD = K * dim;
-    const int per_wave = K * 64 + 64 * R;
+    constexpr bool ACC = PJ;              // sums of the derivatives, in place of gw * w per edge
+    const int n_acc = ACC ? gmm_n_acc(K, dim) : 0, per_wave = K * 64 + 64 * R + n_acc * 64;
     float *shared = lds + FGNN_WPB * per_wave;          // mu | inv_sigma
-    for (int i = (int)threadIdx.x; i < KD; i += FGNN_TPB) { shared[i] = p.mu[i]; shared[KD + i] = p.isg[i]; }
+    gmm_stage<PJ>(shared, (int)threadIdx.x, FGNN_TPB, K, dim, p.mu, p.isg, p.pj);
     __syncthreads();
     int col, b, e, slot;
-    if (!fg_get_item(p.items, p.n_items, p.ptr, col, b, e, slot)) return;
+    if (!fg_get_item(p.items, p.n_items, p.ptr, col, b, e, slot)) { gmm_acc_none<ACC>(p); return; }
     const int lane = fg_lane();
     float *wl = lds + fg_wave() * per_wave;
+    GmmAcc ga;
+    if constexpr (ACC) ga.init(wl + per_wave - n_acc * 64, K, dim, lane);
     float *scr = wl + K * 64;
     fg_lanemap<VEC, R> lm;
     if (p.lphp) lm.init_padded(lane, p.K, p.F, p.lphp); else lm.init(lane, p.HF, p.F);
@@ -673,10 +796,10 @@ __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_kernel(GmmBwdP p)
             }
         };
         request(0);
-        const float *ps = p.pseudo + (size_t)(unsigned)posv * dim;
-        float pv[GMM_PV];
-        gmm_load_pseudo(ps, dim, pv);
-        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(pv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
+        float cv[GMM_PV];
+        float2 rv;
+        const float *ps = gmm_coordinates<PJ>(p.pseudo, p.pj, shared, (size_t)(unsigned)posv, K, dim, cv, rv);
+        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(cv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
         fg_wave_lds_sync();
         for (int t = 0; t < cnt; t += UG) {
             if (t > 0) request(t);
@@ -695,17 +818,24 @@ __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_kernel(GmmBwdP p)
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
                         float sum = fg_group_sum<LPH>(dpart[r]);
-                        if ((FULL || lm.ok[r]) && lm.eoff[r] % p.F == 0) __builtin_nontemporal_store(sum * w[r], gdst + lm.hd[r]);
+                        if ((FULL || lm.ok[r]) && lm.eoff[r] % p.F == 0) {
+                            if constexpr (ACC) wl[lm.hd[r] * 64 + t + u] = sum * w[r]; else __builtin_nontemporal_store(sum * w[r], gdst + lm.hd[r]);
+                        }
                     }
                 } else {
                     float sum = K <= FGNN_FEW_HEADS ? fg_head_reduce_few<VEC, R>(dpart, lm, lane, K)
                                                     : fg_head_reduce<VEC, R>(scr, dpart, lm, lane, K, p.F);
-                    if (lane < K) __builtin_nontemporal_store(sum * wl[lane * 64 + t + u], gdst + lane);
+                    if (lane < K) {
+                        const float v = sum * wl[lane * 64 + t + u];
+                        if constexpr (ACC) wl[lane * 64 + t + u] = v; else __builtin_nontemporal_store(v, gdst + lane);
+                    }
                 }
             }
         }
         fg_wave_lds_sync();
+        if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
     }
+    if constexpr (ACC) ga.finish(gmm_acc_out(p), lane);
     float *dst = slot < 0 ? p.gfeat + (size_t)col * p.HF : p.part + (size_t)slot * spmm_pw(p.HF);
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -714,18 +844,21 @@ __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_kernel(GmmBwdP p)
 
 // The same pass for rows narrower than a wave, G column entries per load instruction (see
 // spmm_packed_kernel).  Needs F/4 lanes per mixture kernel to be a power of two (LPH > 0).
-template <int G, int LPH>
+template <int G, int LPH, bool PJ>
 __device__ __forceinline__ void gmm_bwd_packed_item(const GmmBwdP &p, int n_head, float *lds)
 {
     const int K = p.K, dim = p.dim, KD = K * dim;
-    const int per_wave = K * 64 + 64;
+    constexpr bool ACC = PJ;              // sums of the derivatives, in place of gw * w per edge
+    const int n_acc = ACC ? gmm_n_acc(K, dim) : 0, per_wave = K * 64 + 64 + n_acc * 64;
     float *shared = lds + FGNN_WPB * per_wave;          // mu | inv_sigma
-    for (int i = (int)threadIdx.x; i < KD; i += FGNN_TPB) { shared[i] = p.mu[i]; shared[KD + i] = p.isg[i]; }
+    gmm_stage<PJ>(shared, (int)threadIdx.x, FGNN_TPB, K, dim, p.mu, p.isg, p.pj);
     __syncthreads();
     int col, b, e, slot;
-    if (!fg_get_item(p.items, n_head, p.ptr, col, b, e, slot)) return;
+    if (!fg_get_item(p.items, n_head, p.ptr, col, b, e, slot)) { gmm_acc_none<ACC>(p); return; }
     const int lane = fg_lane();
     float *wl = lds + fg_wave() * per_wave;
+    GmmAcc ga;
+    if constexpr (ACC) ga.init(wl + per_wave - n_acc * 64, K, dim, lane);
     fg_packmap<G> pm;
     if (p.lphp) pm.init_padded(lane, p.K, p.F, p.lphp); else pm.init(lane, p.HF, p.F);
     fg_vec<4> T, xr;
@@ -742,10 +875,10 @@ __device__ __forceinline__ void gmm_bwd_packed_item(const GmmBwdP &p, int n_head
         int id = p.idx[qq];
         int posv = p.pos ? p.pos[qq] : qq;
         if (p.permute) posv = p.permute[posv];      // NULL: pseudo and gww are in this pass's own (CSC) order
-        const float *ps = p.pseudo + (size_t)(unsigned)posv * dim;
-        float pv[GMM_PV];
-        gmm_load_pseudo(ps, dim, pv);
-        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(pv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
+        float cv[GMM_PV];
+        float2 rv;
+        const float *ps = gmm_coordinates<PJ>(p.pseudo, p.pj, shared, (size_t)(unsigned)posv, K, dim, cv, rv);
+        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(cv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
         fg_wave_lds_sync();
         for (int t = 0; t < cnt; t += U * G) {
             fg_vec<4> ld[U];
@@ -765,25 +898,30 @@ __device__ __forceinline__ void gmm_bwd_packed_item(const GmmBwdP &p, int n_head
                 const float w = live ? wl[pm.hd * 64 + ei] : 0.f;
                 T.fma(w, ld[u]);
                 const float sum = fg_group_sum<LPH>(ld[u].dot(xr));
-                if (live && writer) __builtin_nontemporal_store(sum * w, p.gww + (size_t)(unsigned)pv[u] * K + pm.hd);
+                if (live && writer) {
+                    if constexpr (ACC) wl[pm.hd * 64 + ei] = sum * w; else __builtin_nontemporal_store(sum * w, p.gww + (size_t)(unsigned)pv[u] * K + pm.hd);
+                }
             }
         }
         fg_wave_lds_sync();
+        if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
     }
+    if constexpr (ACC) ga.finish(gmm_acc_out(p), lane);
     fg_pack_reduce<G>(T, lane);
     float *dst = slot < 0 ? p.gfeat + (size_t)col * p.HF : p.part + (size_t)slot * spmm_pw(p.HF);
     if (pm.ok && pm.grp == 0) T.store_nt(dst + pm.eoff);
 }
 
 // The same with the lane groups on different work items (see spmm_packed_group_items).
-template <int G, int LPH>
+template <int G, int LPH, bool PJ>
 __device__ __forceinline__ void gmm_bwd_packed_group_items(const GmmBwdP &p, int bucketed, int first, int w, float *lds)
 {
     constexpr int LPR = 64 / G, U = 4;
     const int K = p.K, dim = p.dim, KD = K * dim;
-    const int per_wave = K * 64 + 64;
+    constexpr bool ACC = PJ;              // sums of the derivatives, in place of gw * w per edge
+    const int n_acc = ACC ? gmm_n_acc(K, dim) : 0, per_wave = K * 64 + 64 + n_acc * 64;
     float *shared = lds + FGNN_WPB * per_wave;          // mu | inv_sigma
-    for (int i = (int)threadIdx.x; i < KD; i += FGNN_TPB) { shared[i] = p.mu[i]; shared[KD + i] = p.isg[i]; }
+    gmm_stage<PJ>(shared, (int)threadIdx.x, FGNN_TPB, K, dim, p.mu, p.isg, p.pj);
     __syncthreads();
     const int lane = fg_lane();
     float *wl = lds + fg_wave() * per_wave;
@@ -797,7 +935,9 @@ __device__ __forceinline__ void gmm_bwd_packed_group_items(const GmmBwdP &p, int
         else { col = it; b = p.ptr[it]; e = p.ptr[it + 1]; }
     }
     if (col < 0) { b = 0; e = 0; }                      // padding item or past the list: nothing to walk or store
-    if (__builtin_amdgcn_ballot_w64(col >= 0) == 0ull) return;
+    if (__builtin_amdgcn_ballot_w64(col >= 0) == 0ull) { gmm_acc_none<ACC>(p); return; }
+    GmmAcc ga;
+    if constexpr (ACC) ga.init(wl + per_wave - n_acc * 64, K, dim, lane);
     const bool mine = pm.ok && col >= 0;
     fg_vec<4> T, xr;
     T.zero();
@@ -814,11 +954,11 @@ __device__ __forceinline__ void gmm_bwd_packed_group_items(const GmmBwdP &p, int
             posv = p.pos ? p.pos[qq] : qq;
             if (p.permute) posv = p.permute[posv];
         }
+        float cv[GMM_PV] = {};
+        float2 rv = make_float2(0.f, 0.f);
         if (ok) {
-            const float *ps = p.pseudo + (size_t)(unsigned)posv * dim;
-            float pv[GMM_PV];
-            gmm_load_pseudo(ps, dim, pv);
-            for (int k = 0; k < K; ++k) wl[k * 64 + lane] = gmm_weight(pv, ps, shared + k * dim, shared + KD + k * dim, dim);
+            const float *ps = gmm_coordinates<PJ>(p.pseudo, p.pj, shared, (size_t)(unsigned)posv, K, dim, cv, rv);
+            for (int k = 0; k < K; ++k) wl[k * 64 + lane] = gmm_weight(cv, ps, shared + k * dim, shared + KD + k * dim, dim);
         } else {
             for (int k = 0; k < K; ++k) wl[k * 64 + lane] = 0.f;
         }
@@ -841,28 +981,33 @@ __device__ __forceinline__ void gmm_bwd_packed_group_items(const GmmBwdP &p, int
                 const float wv = live ? wl[pm.hd * 64 + gbase + (ei & (LPR - 1))] : 0.f;
                 T.fma(wv, ld[u]);
                 const float sum = fg_group_sum<LPH>(ld[u].dot(xr));
-                if (live && writer) __builtin_nontemporal_store(sum * wv, p.gww + (size_t)(unsigned)pe[u] * K + pm.hd);
+                if (live && writer) {
+                    if constexpr (ACC) wl[pm.hd * 64 + gbase + (ei & (LPR - 1))] = sum * wv;
+                    else __builtin_nontemporal_store(sum * wv, p.gww + (size_t)(unsigned)pe[u] * K + pm.hd);
+                }
             }
         }
         fg_wave_lds_sync();
+        if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
     }
+    if constexpr (ACC) ga.finish(gmm_acc_out(p), lane);
     if (!mine) return;
     float *dst = slot < 0 ? p.gfeat + (size_t)col * p.HF : p.part + (size_t)slot * spmm_pw(p.HF);
     T.store_nt(dst + pm.eoff);
 }
 
-template <int G, int LPH>
+template <int G, int LPH, bool PJ>
 __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_packed_kernel(GmmBwdP p)
 {
     extern __shared__ float lds[];
-    gmm_bwd_packed_item<G, LPH>(p, p.n_items, lds);
+    gmm_bwd_packed_item<G, LPH, PJ>(p, p.n_items, lds);
 }
-template <int G, int LPH>
+template <int G, int LPH, bool PJ>
 __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_packed_mixed_kernel(GmmBwdP p, int bucketed, int first, unsigned head_blocks)
 {
     extern __shared__ float lds[];
-    if (blockIdx.x < head_blocks) gmm_bwd_packed_item<G, LPH>(p, first, lds);
-    else gmm_bwd_packed_group_items<G, LPH>(p, bucketed, first, (int)(blockIdx.x - head_blocks), lds);
+    if (blockIdx.x < head_blocks) gmm_bwd_packed_item<G, LPH, PJ>(p, first, lds);
+    else gmm_bwd_packed_group_items<G, LPH, PJ>(p, bucketed, first, (int)(blockIdx.x - head_blocks), lds);
 }
 
 // The column pass when grad_out is the gradient of the SUM over the mixture kernels ([N, F], the
@@ -874,20 +1019,23 @@ __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_packed_mixed_kernel(GmmBwdP 
 // feature matrix (aggregate first, transform afterwards): out[i,k,:] = sum_p w[p,k] * g[idx[p],:], nothing
 // per edge is written and x is not read.
 #define GMM_SUMK_MAX 4
-template <int LPF, bool GWW>
+template <int LPF, bool GWW, bool PJ>
 __device__ __forceinline__ void gmm_bwd_sum_item(const GmmBwdP &p, int n_head, float *lds)
 {
     constexpr int G = 64 / LPF;         // rows per load instruction
     constexpr int U = G > 8 ? 64 / G : 8;       // load instructions in flight; U * G divides 64
     const int K = p.K, dim = p.dim, KD = K * dim, F = p.F;
-    const int per_wave = K * 64;
+    constexpr bool ACC = PJ && GWW;              // sums of the derivatives, in place of gw * w per edge
+    const int n_acc = ACC ? gmm_n_acc(K, dim) : 0, per_wave = K * 64 + n_acc * 64;
     float *shared = lds + FGNN_WPB * per_wave;          // mu | inv_sigma
-    for (int i = (int)threadIdx.x; i < KD; i += FGNN_TPB) { shared[i] = p.mu[i]; shared[KD + i] = p.isg[i]; }
+    gmm_stage<PJ>(shared, (int)threadIdx.x, FGNN_TPB, K, dim, p.mu, p.isg, p.pj);
     __syncthreads();
     int col, b, e, slot;
-    if (!fg_get_item(p.items, n_head, p.ptr, col, b, e, slot)) return;
+    if (!fg_get_item(p.items, n_head, p.ptr, col, b, e, slot)) { gmm_acc_none<ACC>(p); return; }
     const int lane = fg_lane();
     float *wl = lds + fg_wave() * per_wave;
+    GmmAcc ga;
+    if constexpr (ACC) ga.init(wl + per_wave - n_acc * 64, K, dim, lane);
     const int grp = lane / LPF, sub = lane % LPF;
     const bool fok = sub * 4 < F;
     const int foff = fok ? sub * 4 : 0;
@@ -905,10 +1053,10 @@ __device__ __forceinline__ void gmm_bwd_sum_item(const GmmBwdP &p, int n_head, f
         int id = p.idx[qq];
         int posv = p.pos ? p.pos[qq] : qq;
         if (p.permute) posv = p.permute[posv];      // NULL: pseudo and gww are in this pass's own (CSC) order
-        const float *ps = p.pseudo + (size_t)(unsigned)posv * dim;
-        float pv[GMM_PV];
-        gmm_load_pseudo(ps, dim, pv);
-        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(pv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
+        float cv[GMM_PV];
+        float2 rv;
+        const float *ps = gmm_coordinates<PJ>(p.pseudo, p.pj, shared, (size_t)(unsigned)posv, K, dim, cv, rv);
+        for (int k = 0; k < K; ++k) wl[k * 64 + lane] = ok ? gmm_weight(cv, ps, shared + k * dim, shared + KD + k * dim, dim) : 0.f;
         fg_wave_lds_sync();
         for (int t = 0; t < cnt; t += U * G) {
             fg_vec<4> ld[U];
@@ -933,16 +1081,20 @@ __device__ __forceinline__ void gmm_bwd_sum_item(const GmmBwdP &p, int n_head, f
                         if constexpr (GWW) {
                             const float sum = fg_group_sum<LPF>(ld[u].dot(xr[k]));
                             if constexpr (LPF >= GMM_SUMK_MAX) mine = sub == k ? sum * w : mine;
-                            else if (ei < cnt && sub == 0) __builtin_nontemporal_store(sum * w, gdst + k);
+                            else if (ei < cnt && sub == 0) { if constexpr (ACC) wl[k * 64 + ei] = sum * w; else __builtin_nontemporal_store(sum * w, gdst + k); }
                         }
                     }
                 }
                 // the K values of an edge leave with one store instruction, K adjacent lanes writing K adjacent floats
-                if constexpr (GWW && LPF >= GMM_SUMK_MAX) { if (ei < cnt && sub < K) __builtin_nontemporal_store(mine, gdst + sub); }
+                if constexpr (GWW && LPF >= GMM_SUMK_MAX) {
+                    if (ei < cnt && sub < K) { if constexpr (ACC) wl[sub * 64 + ei] = mine; else __builtin_nontemporal_store(mine, gdst + sub); }
+                }
             }
         }
         fg_wave_lds_sync();
+        if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
     }
+    if constexpr (ACC) ga.finish(gmm_acc_out(p), lane);
     float *dst = slot < 0 ? p.gfeat + (size_t)col * p.HF : p.part + (size_t)slot * spmm_pw(p.HF);
 #pragma unroll
     for (int k = 0; k < GMM_SUMK_MAX; ++k) {
@@ -956,15 +1108,16 @@ __device__ __forceinline__ void gmm_bwd_sum_item(const GmmBwdP &p, int n_head, f
 // The same pass with the lane groups on different work items (fg_group_slot): group g walks its own item LPF entries at a
 // time (its LPF lanes compute the weights of LPF entries), min(4, LPF) gathered rows of the group in flight, and writes its
 // own result; no butterfly over the groups.
-template <int LPF, bool GWW>
+template <int LPF, bool GWW, bool PJ>
 __device__ __forceinline__ void gmm_bwd_sum_group_items(const GmmBwdP &p, int bucketed, int first, int w, float *lds)
 {
     constexpr int G = 64 / LPF;
     constexpr int U = LPF < 4 ? LPF : 4;
     const int K = p.K, dim = p.dim, KD = K * dim, F = p.F;
-    const int per_wave = K * 64;
+    constexpr bool ACC = PJ && GWW;              // sums of the derivatives, in place of gw * w per edge
+    const int n_acc = ACC ? gmm_n_acc(K, dim) : 0, per_wave = K * 64 + n_acc * 64;
     float *shared = lds + FGNN_WPB * per_wave;          // mu | inv_sigma
-    for (int i = (int)threadIdx.x; i < KD; i += FGNN_TPB) { shared[i] = p.mu[i]; shared[KD + i] = p.isg[i]; }
+    gmm_stage<PJ>(shared, (int)threadIdx.x, FGNN_TPB, K, dim, p.mu, p.isg, p.pj);
     __syncthreads();
     const int lane = fg_lane();
     const int grp = lane / LPF, sub = lane % LPF, gbase = lane - sub;
@@ -975,8 +1128,10 @@ __device__ __forceinline__ void gmm_bwd_sum_group_items(const GmmBwdP &p, int bu
         else { col = it; b = p.ptr[it]; e = p.ptr[it + 1]; }
     }
     if (col < 0) { b = 0; e = 0; }                      // padding item or past the list: nothing to walk or store
-    if (__builtin_amdgcn_ballot_w64(col >= 0) == 0ull) return;
+    if (__builtin_amdgcn_ballot_w64(col >= 0) == 0ull) { gmm_acc_none<ACC>(p); return; }
     float *wl = lds + fg_wave() * per_wave;
+    GmmAcc ga;
+    if constexpr (ACC) ga.init(wl + per_wave - n_acc * 64, K, dim, lane);
     const bool fok = sub * 4 < F;
     const int foff = fok ? sub * 4 : 0;
     fg_vec<4> T[GMM_SUMK_MAX], xr[GMM_SUMK_MAX];
@@ -995,11 +1150,11 @@ __device__ __forceinline__ void gmm_bwd_sum_group_items(const GmmBwdP &p, int bu
             posv = p.pos ? p.pos[qq] : qq;
             if (p.permute) posv = p.permute[posv];
         }
+        float cv[GMM_PV] = {};
+        float2 rv = make_float2(0.f, 0.f);
         if (ok) {
-            const float *ps = p.pseudo + (size_t)(unsigned)posv * dim;
-            float pv[GMM_PV];
-            gmm_load_pseudo(ps, dim, pv);
-            for (int k = 0; k < K; ++k) wl[k * 64 + lane] = gmm_weight(pv, ps, shared + k * dim, shared + KD + k * dim, dim);
+            const float *ps = gmm_coordinates<PJ>(p.pseudo, p.pj, shared, (size_t)(unsigned)posv, K, dim, cv, rv);
+            for (int k = 0; k < K; ++k) wl[k * 64 + lane] = gmm_weight(cv, ps, shared + k * dim, shared + KD + k * dim, dim);
         } else {
             for (int k = 0; k < K; ++k) wl[k * 64 + lane] = 0.f;
         }
@@ -1028,15 +1183,19 @@ __device__ __forceinline__ void gmm_bwd_sum_group_items(const GmmBwdP &p, int bu
                         if constexpr (GWW) {
                             const float sum = fg_group_sum<LPF>(ld[u].dot(xr[k]));
                             if constexpr (LPF >= GMM_SUMK_MAX) mine = sub == k ? sum * w : mine;
-                            else if (live && sub == 0) __builtin_nontemporal_store(sum * w, gdst + k);
+                            else if (live && sub == 0) { if constexpr (ACC) wl[k * 64 + gbase + (ei & (LPF - 1))] = sum * w; else __builtin_nontemporal_store(sum * w, gdst + k); }
                         }
                     }
                 }
-                if constexpr (GWW && LPF >= GMM_SUMK_MAX) { if (live && sub < K) __builtin_nontemporal_store(mine, gdst + sub); }
+                if constexpr (GWW && LPF >= GMM_SUMK_MAX) {
+                    if (live && sub < K) { if constexpr (ACC) wl[sub * 64 + gbase + (ei & (LPF - 1))] = mine; else __builtin_nontemporal_store(mine, gdst + sub); }
+                }
             }
         }
         fg_wave_lds_sync();
+        if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
     }
+    if constexpr (ACC) ga.finish(gmm_acc_out(p), lane);
     if (col < 0 || !fok) return;
     float *dst = slot < 0 ? p.gfeat + (size_t)col * p.HF : p.part + (size_t)slot * spmm_pw(p.HF);
 #pragma unroll
@@ -1044,20 +1203,20 @@ __device__ __forceinline__ void gmm_bwd_sum_group_items(const GmmBwdP &p, int bu
         if (k < K) T[k].store_nt(dst + k * F + foff);
 }
 
-template <int LPF, bool GWW = true>
+template <int LPF, bool GWW, bool PJ>
 __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_sum_kernel(GmmBwdP p)
 {
     extern __shared__ float lds[];
-    gmm_bwd_sum_item<LPF, GWW>(p, p.n_items, lds);
+    gmm_bwd_sum_item<LPF, GWW, PJ>(p, p.n_items, lds);
 }
 // One launch for a list with a long head: the first head_blocks workgroups put a wave on each of the `first` leading items,
 // the others give every lane group an item of the rest; the long items then run beside the short ones.
-template <int LPF, bool GWW = true>
+template <int LPF, bool GWW, bool PJ>
 __global__ __launch_bounds__(FGNN_TPB) void gmm_bwd_sum_mixed_kernel(GmmBwdP p, int bucketed, int first, unsigned head_blocks)
 {
     extern __shared__ float lds[];
-    if (blockIdx.x < head_blocks) gmm_bwd_sum_item<LPF, GWW>(p, first, lds);
-    else gmm_bwd_sum_group_items<LPF, GWW>(p, bucketed, first, (int)(blockIdx.x - head_blocks), lds);
+    if (blockIdx.x < head_blocks) gmm_bwd_sum_item<LPF, GWW, PJ>(p, first, lds);
+    else gmm_bwd_sum_group_items<LPF, GWW, PJ>(p, bucketed, first, (int)(blockIdx.x - head_blocks), lds);
 }
 
 // Where the lane-group part of a launch starts (-1: a wave per item throughout).  Groups of at most 16 lanes (F <= 64) on
@@ -1071,37 +1230,38 @@ static inline int gmm_group_items_first(const fgnn_schedule_t *sched, int lpf)
     return sched->n_wave_slots;
 }
 
-template <bool GWW>
-static void gmm_sum_launch(int lpf, unsigned grid, size_t shm, hipStream_t st, const GmmBwdP &p, int first = -1, int bucketed = 0)
+template <bool GWW, bool PJ>
+static unsigned gmm_sum_launch(int lpf, unsigned grid, size_t shm, hipStream_t st, const GmmBwdP &p, int first = -1, int bucketed = 0)
 {
     // first >= 0: the items from slot `first` on are short and go 64/lpf to a wave (gmm_bwd_sum_group_items)
     if (first >= 0 && first < p.n_items && lpf <= 32) {
         const unsigned hb = (unsigned)((first + FGNN_WPB - 1) / FGNN_WPB);
         const unsigned g2 = hb + fgnn_group_item_grid(p.n_items - first, 64 / lpf, bucketed != 0);
         switch (lpf) {
-        case 1: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<1, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
-        case 2: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<2, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
-        case 4: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<4, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
-        case 8: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<8, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
-        case 16: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<16, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
-        default: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<32, GWW>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        case 1: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<1, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        case 2: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<2, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        case 4: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<4, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        case 8: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<8, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        case 16: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<16, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
+        default: hipLaunchKernelGGL((gmm_bwd_sum_mixed_kernel<32, GWW, PJ>), dim3(g2), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); break;
         }
-        return;
+        return g2;
     }
     switch (lpf) {
-    case 1: hipLaunchKernelGGL((gmm_bwd_sum_kernel<1, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    case 2: hipLaunchKernelGGL((gmm_bwd_sum_kernel<2, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    case 4: hipLaunchKernelGGL((gmm_bwd_sum_kernel<4, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    case 8: hipLaunchKernelGGL((gmm_bwd_sum_kernel<8, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    case 16: hipLaunchKernelGGL((gmm_bwd_sum_kernel<16, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    case 32: hipLaunchKernelGGL((gmm_bwd_sum_kernel<32, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
-    default: hipLaunchKernelGGL((gmm_bwd_sum_kernel<64, GWW>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 1: hipLaunchKernelGGL((gmm_bwd_sum_kernel<1, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 2: hipLaunchKernelGGL((gmm_bwd_sum_kernel<2, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 4: hipLaunchKernelGGL((gmm_bwd_sum_kernel<4, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 8: hipLaunchKernelGGL((gmm_bwd_sum_kernel<8, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 16: hipLaunchKernelGGL((gmm_bwd_sum_kernel<16, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    case 32: hipLaunchKernelGGL((gmm_bwd_sum_kernel<32, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
+    default: hipLaunchKernelGGL((gmm_bwd_sum_kernel<64, GWW, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); break;
     }
+    return grid;
 }
 
 // Forward with one [N,F] feature matrix shared by the K mixture kernels: out[i,k,:] = sum_p w[p,k] * feat[idx[p],:].
 static int gmm_forward_shared(int N, int K, int dim, int F, const int32_t *ptr, const int32_t *idx, const int32_t *pos_map, const float *feat,
-                              const float *pseudo, const float *mu, const float *isg, float *out, const fgnn_schedule_t *sched,
+                              const float *pseudo, const GmmProj &pj, const float *mu, const float *isg, float *out, const fgnn_schedule_t *sched,
                               void *workspace, size_t workspace_bytes, hipStream_t st)
 {
     const int HF = K * F, KD = K * dim;
@@ -1117,14 +1277,16 @@ static int gmm_forward_shared(int N, int K, int dim, int F, const int32_t *ptr, 
     p.items = sched ? sched->items_dev : nullptr; p.n_items = sched ? sched->n_items : N;
     if (p.n_items == 0) return 0;
     p.ptr = ptr; p.idx = fgnn_sched_idx(sched, idx); p.pos = fgnn_sched_pos(sched); p.permute = pos_map;
-    p.g = feat; p.pseudo = pseudo; p.mu = mu; p.isg = isg; p.gfeat = out; p.part = (float *)workspace;
+    p.g = feat; p.pseudo = pseudo; p.pj = pj; p.mu = mu; p.isg = isg; p.gfeat = out; p.part = (float *)workspace;
     p.N = N; p.K = K; p.dim = dim; p.F = F; p.HF = HF; p.g_stride = F; p.x_stride = HF;
     int lpf = 1;
     while (lpf * 4 < F) lpf *= 2;
-    const size_t shm = ((size_t)FGNN_WPB * K * 64 + 2 * KD) * sizeof(float);
+    const size_t shm = ((size_t)FGNN_WPB * K * 64 + 2 * KD + (pj.raw ? 3 * dim : 0)) * sizeof(float);
     FGNN_REQUIRE(shm <= 64 * 1024, FGNN_ERR_LIMIT, "fgnn_gmm_forward: K=%d, dim=%d need %zu bytes of LDS per workgroup (limit 64 KiB)", K, dim, shm);
     const unsigned grid = (unsigned)((p.n_items + FGNN_WPB - 1) / FGNN_WPB);
-    gmm_sum_launch<false>(lpf, grid, shm, st, p, gmm_group_items_first(sched, lpf), sched && sched->n_buckets > 0);
+    const int first = gmm_group_items_first(sched, lpf), bucketed = sched && sched->n_buckets > 0;
+    if (pj.raw) gmm_sum_launch<false, true>(lpf, grid, shm, st, p, first, bucketed);
+    else gmm_sum_launch<false, false>(lpf, grid, shm, st, p, first, bucketed);
     int rc = fgnn_launch_status("gmm_bwd_sum_kernel (forward, shared features)");
     if (rc) return rc;
     if (sched && sched->n_split > 0) {
@@ -1345,6 +1507,45 @@ static int gauss_grad_launch(int64_t E, int K, int dim, const float *pseudo, con
     return fgnn_launch_status("colsum_level2");
 }
 
+// Sums of the waves' GmmAcc records, [waves][n_acc]: GMM_SUM_BLOCKS workgroups, each thread one of the n_acc sums (so that a workgroup reads
+// consecutive floats), then one workgroup; in 64 bits and in a fixed order.
+#define GMM_SUM_BLOCKS 256
+__global__ __launch_bounds__(256) void gmm_acc_sum1_kernel(int64_t waves, int n_acc, const float *__restrict__ acc, double *__restrict__ part)
+{
+    __shared__ double sh[256];
+    const int per = 256 / n_acc, r = (int)threadIdx.x / n_acc, c = (int)threadIdx.x - r * n_acc;
+    double v = 0.;
+    if (r < per) {
+#pragma unroll 4
+        for (int64_t i = (int64_t)blockIdx.x * per + r; i < waves; i += (int64_t)GMM_SUM_BLOCKS * per) v += (double)acc[i * n_acc + c];
+    }
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    if ((int)threadIdx.x >= n_acc) return;
+    for (int i = 1; i < per; ++i) v += sh[i * n_acc + c];
+    part[(size_t)blockIdx.x * n_acc + c] = v;
+}
+__global__ __launch_bounds__(256) void gmm_acc_sum2_kernel(int KD, int dim, const double *__restrict__ part, float *__restrict__ gmu, float *__restrict__ gsig,
+                                                           float *__restrict__ gW, float *__restrict__ gb)
+{
+    __shared__ double sh[256];
+    const int n_acc = 2 * KD + 3 * dim, per = 256 / n_acc, r = (int)threadIdx.x / n_acc, c = (int)threadIdx.x - r * n_acc;
+    double v = 0.;
+    if (r < per)
+        for (int i = r; i < GMM_SUM_BLOCKS; i += per) v += part[(size_t)i * n_acc + c];
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    if ((int)threadIdx.x >= n_acc) return;
+    for (int i = 1; i < per; ++i) v += sh[i * n_acc + c];
+    const float f = (float)v;
+    if (c < KD) gmu[c] = f;
+    else if (c < 2 * KD) gsig[c - KD] = f;
+    else if (c < 2 * KD + 2 * dim) gW[c - 2 * KD] = f;
+    else gb[c - 2 * KD - 2 * dim] = f;
+}
+// Most waves that a launch over the list has (its lane-group part is rounded up to whole rounds over the XCDs).
+static inline size_t gmm_waves(const fgnn_schedule_t *s) { return (size_t)FGNN_WPB * ((size_t)(s->n_items + FGNN_WPB - 1) / FGNN_WPB + 2 * FGNN_NUM_XCD); }
+
 extern "C" size_t fgnn_gmm_backward_workspace_bytes(const fgnn_schedule_t *sched_csc, int K, int dim, int F)
 {
     // partials | gw*w [E,K] | reduction scratch
@@ -1354,31 +1555,39 @@ extern "C" size_t fgnn_gmm_backward_workspace_bytes(const fgnn_schedule_t *sched
     b += gauss_grad_workspace(sched_csc->n_edges, K, dim);
     return b;
 }
-
-extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const int32_t *col_ptr, const int32_t *row_ind,
-                                 const int32_t *permute, const float *node_feat, const float *pseudo, const float *mu,
-                                 const float *inv_sigma, const float *grad_out, int sum_kernels, float *grad_feat, float *grad_pseudo,
-                                 float *grad_mu, float *grad_sigma, const fgnn_schedule_t *sched_csc, void *workspace,
-                                 size_t workspace_bytes, void *stream)
+extern "C" size_t fgnn_gmm_backward_projected_workspace_bytes(const fgnn_schedule_t *sched_csc, int K, int dim, int F)
 {
-    int rc = spmm_checks("fgnn_gmm_backward", N, E, K, F, sched_csc, col_ptr, row_ind);
+    // partials | sums of the waves | sums of the workgroups that add them up
+    if (!sched_csc) return 0;
+    return fgnn_align256((size_t)sched_csc->n_partials * spmm_pw(K * F) * sizeof(float)) + fgnn_align256(gmm_waves(sched_csc) * gmm_n_acc(K, dim) * sizeof(float))
+        + fgnn_align256((size_t)GMM_SUM_BLOCKS * gmm_n_acc(K, dim) * sizeof(double));
+}
+
+static int gmm_backward_impl(const char *fn, int N, int64_t E, int K, int dim, int F, const int32_t *col_ptr, const int32_t *row_ind,
+                             const int32_t *permute, const float *node_feat, const float *pseudo, const GmmProj *proj, const float *mu,
+                             const float *inv_sigma, const float *grad_out, int sum_kernels, float *grad_feat, float *grad_pseudo, float *grad_W, float *grad_b,
+                             float *grad_mu, float *grad_sigma, const fgnn_schedule_t *sched_csc, void *workspace, size_t workspace_bytes, void *stream)
+{
+    int rc = gmm_checks(fn, N, E, K, dim, F, col_ptr, row_ind, pseudo, proj, sched_csc);
     if (rc) return rc;
-    FGNN_REQUIRE((int64_t)K * F <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_backward: K*F=%lld > 1024 unsupported", (long long)K * F);
-    FGNN_REQUIRE(dim >= 1 && dim <= 64 && K * dim <= 1024, FGNN_ERR_LIMIT, "fgnn_gmm_backward: dim=%d K*dim=%d unsupported", dim, K * dim);
-    FGNN_REQUIRE(col_ptr && (row_ind || E == 0) && node_feat && (pseudo || E == 0) && mu && inv_sigma &&
-                     grad_out && grad_feat && (grad_pseudo || E == 0) && grad_mu && grad_sigma,
-                 FGNN_ERR_NULL, "fgnn_gmm_backward: NULL argument");
-    FGNN_REQUIRE(sched_csc, FGNN_ERR_SCHEDULE, "fgnn_gmm_backward: a schedule of col_ptr is required");
-    FGNN_REQUIRE(sum_kernels >= 0 && sum_kernels <= 2, FGNN_ERR_SHAPE, "fgnn_gmm_backward: sum_kernels=%d (0, 1 or 2)", sum_kernels);
-    size_t need = fgnn_gmm_backward_workspace_bytes(sched_csc, K, dim, F);
+    FGNN_REQUIRE(col_ptr && (row_ind || E == 0) && node_feat && mu && inv_sigma && grad_out && grad_feat && grad_mu && grad_sigma &&
+                     (proj ? grad_W && grad_b : grad_pseudo || E == 0), FGNN_ERR_NULL, "%s: NULL argument", fn);
+    FGNN_REQUIRE(sched_csc, FGNN_ERR_SCHEDULE, "%s: a schedule of col_ptr is required", fn);
+    FGNN_REQUIRE(sum_kernels >= 0 && sum_kernels <= 2, FGNN_ERR_SHAPE, "%s: sum_kernels=%d (0, 1 or 2)", fn, sum_kernels);
+    size_t need = proj ? fgnn_gmm_backward_projected_workspace_bytes(sched_csc, K, dim, F) : fgnn_gmm_backward_workspace_bytes(sched_csc, K, dim, F);
     FGNN_REQUIRE(workspace && workspace_bytes >= need && fgnn_aligned16(workspace), FGNN_ERR_WORKSPACE,
-                 "fgnn_gmm_backward: workspace %zu < %zu bytes (or unaligned)", workspace_bytes, need);
+                 "%s: workspace %zu < %zu bytes (or unaligned)", fn, workspace_bytes, need);
     hipStream_t st = (hipStream_t)stream;
     const int HF = K * F, KD = K * dim;
     char *w = (char *)workspace;
     float *part = (float *)w; w += fgnn_align256((size_t)sched_csc->n_partials * spmm_pw(HF) * sizeof(float));
-    float *gww = (float *)w; w += fgnn_align256((size_t)E * K * sizeof(float));
+    float *gww = proj ? nullptr : (float *)w;
+    float *acc = proj ? (float *)w : nullptr;
+    w += fgnn_align256(proj ? gmm_waves(sched_csc) * gmm_n_acc(K, dim) * sizeof(float) : (size_t)E * K * sizeof(float));
     void *gws = w;
+    // LDS floats per wave for the sums of a projected mixture, and the projection behind mu and inv_sigma
+    const int acc_floats = proj ? gmm_n_acc(K, dim) * 64 : 0, pj_floats = proj ? 3 * dim : 0;
+    unsigned blocks = 0;                                    // of the launch, where its waves leave sums
     if (sched_csc->n_items > 0) {
         bool aligned = fgnn_aligned16(node_feat) && fgnn_aligned16(grad_out) && fgnn_aligned16(grad_feat);
         fgnn_rowcfg cfg;
@@ -1386,7 +1595,8 @@ extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const 
         GmmBwdP p{};
         p.items = sched_csc->items_dev; p.n_items = sched_csc->n_items; p.ptr = col_ptr; p.idx = fgnn_sched_idx(sched_csc, row_ind);
         p.pos = fgnn_sched_pos(sched_csc); p.permute = permute;
-        p.x = node_feat; p.g = grad_out; p.pseudo = pseudo; p.mu = mu; p.isg = inv_sigma; p.gfeat = grad_feat; p.gww = gww;
+        p.x = node_feat; p.g = grad_out; p.pseudo = pseudo; p.mu = mu; p.isg = inv_sigma; p.gfeat = grad_feat; p.gww = gww; p.acc = acc;
+        if (proj) p.pj = *proj;
         p.part = part; p.N = N; p.K = K; p.dim = dim; p.F = F; p.HF = HF;
         p.g_stride = sum_kernels == 1 ? F : HF;
         p.x_stride = sum_kernels == 2 ? F : HF;
@@ -1407,10 +1617,11 @@ extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const 
             // lanes over F only, the K mixture kernels in registers (see gmm_bwd_sum_kernel)
             int lpf = 1;
             while (lpf * 4 < F) lpf *= 2;
-            const size_t shm = ((size_t)FGNN_WPB * K * 64 + 2 * KD) * sizeof(float);
+            const size_t shm = ((size_t)FGNN_WPB * (K * 64 + acc_floats) + 2 * KD + pj_floats) * sizeof(float);
             FGNN_REQUIRE(shm <= 64 * 1024, FGNN_ERR_LIMIT, "fgnn_gmm_backward: K=%d, dim=%d need %zu bytes of LDS per workgroup (limit 64 KiB)", K, dim, shm);
             p.lphp = 0;
-            gmm_sum_launch<true>(lpf, grid, shm, st, p, gmm_group_items_first(sched_csc, lpf), sched_csc->n_buckets > 0);
+            const int first = gmm_group_items_first(sched_csc, lpf), bucketed = sched_csc->n_buckets > 0;
+            blocks = proj ? gmm_sum_launch<true, true>(lpf, grid, shm, st, p, first, bucketed) : gmm_sum_launch<true, false>(lpf, grid, shm, st, p, first, bucketed);
             rc = fgnn_launch_status("gmm_bwd_sum_kernel");
             if (rc) return rc;
             if (sched_csc->n_split > 0) {
@@ -1425,10 +1636,10 @@ extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const 
             }
         }
         if (!sumk) rc = fgnn_dispatch_rowcfg(cfg, [&]<int VEC, int R, bool FULL>() -> int {
-            size_t shm = ((size_t)FGNN_WPB * (K * 64 + 64 * R) + 2 * KD) * sizeof(float);
+            size_t shm = ((size_t)FGNN_WPB * (K * 64 + 64 * R + acc_floats) + 2 * KD + pj_floats) * sizeof(float);
             FGNN_REQUIRE(shm <= 64 * 1024, FGNN_ERR_LIMIT, "fgnn_gmm_backward: K=%d, dim=%d need %zu bytes of LDS per workgroup (limit 64 KiB)", K, dim, shm);
             const int pack = lph > 0 ? fgnn_pick_pack(cfg.vec, lanes_hf) : 1;
-            int rc2 = fgnn_dispatch_lph(VEC == 4 ? lph : 0, [&]<int LPH>() -> int {
+            auto go = [&]<int LPH, bool PJ>() -> int {
                 if constexpr (VEC == 4 && R == 1 && LPH > 0 && LPH <= 32) {
                     // a mixture kernel's LPH lanes must fit inside one group of 64/pack lanes
                     // graphs of short rows: the items behind the long head of the list go `pack` to a wave (gmm_bwd_packed_group_items;
@@ -1437,14 +1648,20 @@ extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const 
                     const int bucketed = sched_csc->n_buckets > 0;
                     const unsigned hb = (unsigned)((first + FGNN_WPB - 1) / FGNN_WPB);
                     const unsigned gm = hb + fgnn_group_item_grid(p.n_items - first, pack, bucketed);
-                    if (pack == 8 && LPH <= 8 && first < p.n_items) { hipLaunchKernelGGL((gmm_bwd_packed_mixed_kernel<8, (LPH <= 8 ? LPH : 1)>), dim3(gm), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); return fgnn_launch_status("gmm_bwd_packed_mixed_kernel"); }
-                    if (pack == 4 && LPH <= 16 && first < p.n_items) { hipLaunchKernelGGL((gmm_bwd_packed_mixed_kernel<4, (LPH <= 16 ? LPH : 1)>), dim3(gm), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); return fgnn_launch_status("gmm_bwd_packed_mixed_kernel"); }
-                    if (pack == 8 && LPH <= 8) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<8, (LPH <= 8 ? LPH : 1)>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
-                    if (pack == 4 && LPH <= 16) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<4, (LPH <= 16 ? LPH : 1)>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
-                    if (pack == 2 && LPH <= 32) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<2, LPH>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
+                    blocks = gm;
+                    if (pack == 8 && LPH <= 8 && first < p.n_items) { hipLaunchKernelGGL((gmm_bwd_packed_mixed_kernel<8, (LPH <= 8 ? LPH : 1), PJ>), dim3(gm), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); return fgnn_launch_status("gmm_bwd_packed_mixed_kernel"); }
+                    if (pack == 4 && LPH <= 16 && first < p.n_items) { hipLaunchKernelGGL((gmm_bwd_packed_mixed_kernel<4, (LPH <= 16 ? LPH : 1), PJ>), dim3(gm), dim3(FGNN_TPB), shm, st, p, bucketed, first, hb); return fgnn_launch_status("gmm_bwd_packed_mixed_kernel"); }
+                    blocks = grid;
+                    if (pack == 8 && LPH <= 8) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<8, (LPH <= 8 ? LPH : 1), PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
+                    if (pack == 4 && LPH <= 16) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<4, (LPH <= 16 ? LPH : 1), PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
+                    if (pack == 2 && LPH <= 32) { hipLaunchKernelGGL((gmm_bwd_packed_kernel<2, LPH, PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p); return fgnn_launch_status("gmm_bwd_packed_kernel"); }
                 }
-                hipLaunchKernelGGL((gmm_bwd_kernel<VEC, R, FULL, (VEC == 4 ? LPH : 0)>), dim3(grid), dim3(FGNN_TPB), shm, st, p);
+                blocks = grid;
+                hipLaunchKernelGGL((gmm_bwd_kernel<VEC, R, FULL, (VEC == 4 ? LPH : 0), PJ>), dim3(grid), dim3(FGNN_TPB), shm, st, p);
                 return fgnn_launch_status("gmm_bwd_kernel");
+            };
+            int rc2 = fgnn_dispatch_lph(VEC == 4 ? lph : 0, [&]<int LPH>() -> int {
+                return proj ? go.template operator()<LPH, true>() : go.template operator()<LPH, false>();
             });
             if (rc2) return rc2;
             if (sched_csc->n_split > 0) {
@@ -1458,7 +1675,35 @@ extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const 
         });
         if (rc) return rc;
     }
+    if (proj) {
+        hipLaunchKernelGGL(gmm_acc_sum1_kernel, dim3(GMM_SUM_BLOCKS), dim3(256), 0, st, (int64_t)blocks * FGNN_WPB, gmm_n_acc(K, dim), acc, (double *)gws);
+        rc = fgnn_launch_status("gmm_acc_sum1_kernel");
+        if (rc) return rc;
+        hipLaunchKernelGGL(gmm_acc_sum2_kernel, dim3(1), dim3(256), 0, st, KD, dim, (const double *)gws, grad_mu, grad_sigma, grad_W, grad_b);
+        return fgnn_launch_status("gmm_acc_sum2_kernel");
+    }
     return gauss_grad_launch(E, K, dim, pseudo, mu, inv_sigma, gww, 1, grad_pseudo, grad_mu, grad_sigma, gws, st);
+}
+
+extern "C" int fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F, const int32_t *col_ptr, const int32_t *row_ind,
+                                 const int32_t *permute, const float *node_feat, const float *pseudo, const float *mu,
+                                 const float *inv_sigma, const float *grad_out, int sum_kernels, float *grad_feat, float *grad_pseudo,
+                                 float *grad_mu, float *grad_sigma, const fgnn_schedule_t *sched_csc, void *workspace,
+                                 size_t workspace_bytes, void *stream)
+{
+    return gmm_backward_impl("fgnn_gmm_backward", N, E, K, dim, F, col_ptr, row_ind, permute, node_feat, pseudo, nullptr, mu, inv_sigma, grad_out, sum_kernels,
+                             grad_feat, grad_pseudo, nullptr, nullptr, grad_mu, grad_sigma, sched_csc, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fgnn_gmm_backward_projected(int N, int64_t E, int K, int dim, int F, const int32_t *col_ptr, const int32_t *row_ind,
+                                           const int32_t *permute, const float *node_feat, const float *raw, const float *proj_W, const float *proj_b,
+                                           const float *mu, const float *inv_sigma, const float *grad_out, int sum_kernels, float *grad_feat,
+                                           float *grad_W, float *grad_b, float *grad_mu, float *grad_sigma, const fgnn_schedule_t *sched_csc,
+                                           void *workspace, size_t workspace_bytes, void *stream)
+{
+    const GmmProj pj{(const float2 *)raw, proj_W, proj_b};
+    return gmm_backward_impl("fgnn_gmm_backward_projected", N, E, K, dim, F, col_ptr, row_ind, permute, node_feat, nullptr, &pj, mu, inv_sigma, grad_out,
+                             sum_kernels, grad_feat, nullptr, grad_W, grad_b, grad_mu, grad_sigma, sched_csc, workspace, workspace_bytes, stream);
 }
 
 // ------------------------------------------------------------------------------- standalone Gaussian

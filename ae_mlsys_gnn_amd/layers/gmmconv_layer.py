@@ -6,8 +6,9 @@ import torch as th
 from torch import nn
 from torch.nn import init
 
+from ..operators.edge_proj import edge_linear_tanh
 from ..operators.fused_gmmconv import (GmmAggregate, GmmAggregateLinear, GmmAggregateTwoOrders, GmmConvFuseSum, GmmConvFuseSumTwoOrders, GmmConvStash,
-                                        GmmConvStashSumTwoOrders, gmm_native, project_in_backward)
+                                        GmmConvStashSumTwoOrders, GmmProjectedTwoOrders, gmm_native, project_in_backward)
 from .dense import add_bias, tall_linear
 
 
@@ -50,14 +51,25 @@ class _GMMBase(nn.Module):
     def set_allow_zero_in_degree(self, set_value):
         self._allow_zero_in_degree = set_value
 
-    def forward(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc=None, own_order=False):
+    def forward(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc=None, own_order=False, proj=None):
         """pseudo_csc: the same pseudo-coordinates in CSC order, pseudo[permute], built by
         the caller from its own CSC-ordered edge data.  The backward then works in CSC order throughout
         and the gradient of the pseudo-coordinates flows through pseudo_csc instead of pseudo.
         own_order: pseudo and pseudo_csc are in the entry order of the operators' schedules
-        (operators.fused_gmmconv.gmm_edge_positions); without pseudo_csc the layer is forward-only."""
+        (operators.fused_gmmconv.gmm_edge_positions); without pseudo_csc the layer is forward-only.
+        proj: a Linear(2, dim) whose tanh gives the coordinates; pseudo and pseudo_csc are then raw [E, 2] pairs (constant data), and where the
+        operators can, they project them on the way."""
+        if proj is not None and not self._projects(feat, pseudo, pseudo_csc, proj, colind):
+            apply = lambda t: edge_linear_tanh(t, proj.weight, proj.bias)
+            if pseudo_csc is not None:
+                with th.no_grad():
+                    pseudo = apply(pseudo)
+                pseudo_csc = apply(pseudo_csc)
+            else:
+                pseudo = apply(pseudo)
+            proj = None
         if self._aggregate_first(feat):
-            return self._finish(self._forward_aggregate_first(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order), feat)
+            return self._finish(self._forward_aggregate_first(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj), feat)
         node_feat = tall_linear(feat, self.fc.weight).view(-1, self._n_kernels, self._out_feats)    # = self.fc(feat)
         pad = (-self._out_feats) % 4
         if pad:         # zero columns up to a multiple of 4: the operator then takes its 128-bit row layout
@@ -69,6 +81,11 @@ class _GMMBase(nn.Module):
         if pseudo_csc is not None or own_order:
             if own_order and pseudo_csc is None and th.is_grad_enabled() and (node_feat.requires_grad or pseudo.requires_grad):
                 raise ValueError("own_order without pseudo_csc is forward-only")
+            if proj is not None:
+                t = tail()
+                rst = GmmProjectedTwoOrders(rowptr, colind, colptr, rowind, node_feat, pseudo, pseudo_csc, proj.weight, proj.bias, self.mu, self.inv_sigma,
+                                            own_order, type(self)._op is not GmmConvFuseSum, t.get("bias"), t.get("residual"))
+                return rst if fuse_tail else self._finish(rst[..., :self._out_feats], feat)
             two_orders = GmmConvFuseSumTwoOrders if (type(self)._op is GmmConvFuseSum or pseudo_csc is None) else GmmConvStashSumTwoOrders
             rst = two_orders(rowptr, colind, colptr, rowind, node_feat, pseudo.detach(), pseudo_csc, self.mu, self.inv_sigma,
                              own_order=own_order, **tail())
@@ -82,6 +99,15 @@ class _GMMBase(nn.Module):
         if pad:
             rst = rst[..., :self._out_feats]
         return self._finish(rst, feat)
+
+    def _projects(self, feat, raw, raw_csc, proj, colind):
+        """Whether this call leaves the projection to the operators: two orders of constant fp32 pairs, few kernels and coordinates, and not the
+        form of the layer whose backward takes the coordinates' gradient through a projection of the input."""
+        k, fin = self._n_kernels, feat.shape[1]
+        if (raw_csc is None or not gmm_native.projection_supported(k, self._dim) or raw.requires_grad or raw_csc.requires_grad
+                or any(t.dtype != th.float32 or not t.is_cuda for t in (raw, raw_csc, proj.weight, proj.bias))):
+            return False
+        return not (self._aggregate_first(feat) and project_in_backward(k, fin, self._out_feats, feat.requires_grad, feat.shape[0], colind.numel()))
 
     def _finish(self, rst, feat):
         if self.res_fc is not None:
@@ -97,7 +123,7 @@ class _GMMBase(nn.Module):
         return (type(self)._op is GmmConvFuseSum and feat.dim() == 2 and fin < k * self._out_feats
                 and gmm_native.shared_supported(k, fin))
 
-    def _forward_aggregate_first(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order):
+    def _forward_aggregate_first(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj=None):
         """sum_k (sum_p w[p,k] feat[col(p),:]) @ W_k: the reference's sum over k of the aggregated fc(feat)[:,k,:]
         (layers/gmmconv_layer.py:67-69) with the two linear steps exchanged."""
         k, fin, fout = self._n_kernels, feat.shape[1], self._out_feats
@@ -106,6 +132,10 @@ class _GMMBase(nn.Module):
             if own_order and pseudo_csc is None and th.is_grad_enabled() and (feat.requires_grad or pseudo.requires_grad):
                 raise ValueError("own_order without pseudo_csc is forward-only")
         two = pseudo_csc is not None
+        w = lambda: self.fc.weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)       # [out, K*in]: rst = agg.view(N, K*in) @ w^T
+        if proj is not None:
+            agg = GmmProjectedTwoOrders(rowptr, colind, colptr, rowind, feat, pseudo, pseudo_csc, proj.weight, proj.bias, self.mu, self.inv_sigma, own_order)
+            return tall_linear(agg.view(-1, k * fin), w())
         # without a gradient for what is aggregated (frozen Gaussians, constant coordinates and input) the weight's is one product with the
         # aggregate, and no pass over the edges
         through_edges = any(t.requires_grad for t in (feat, pseudo_csc if two else pseudo, self.mu, self.inv_sigma))
@@ -118,8 +148,7 @@ class _GMMBase(nn.Module):
                                         own_order=own_order)
         else:
             agg = GmmAggregate(rowptr, colind, colptr, rowind, permute, feat, pseudo, self.mu, self.inv_sigma)
-        w = self.fc.weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)       # [out, K*in]: rst = agg.view(N, K*in) @ w^T
-        return tall_linear(agg.view(-1, k * fin), w)
+        return tall_linear(agg.view(-1, k * fin), w())
 
 
 class GMMConv(_GMMBase):

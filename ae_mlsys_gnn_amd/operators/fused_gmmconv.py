@@ -20,9 +20,24 @@ class gmm_native:
     """gmmconv.gmmconv / gmmconvstash / Gaussian / GaussianBp (src/fused_gmmconv/gmmconv.cc:36-94)."""
 
     @staticmethod
+    def projection(proj, pseudo, k, dim, e):
+        """(weight, bias) of a projection for pseudo [E, 2], checked; the operators form tanh(pseudo @ weight^T + bias) themselves."""
+        weight, bias = as_f32(proj[0]), as_f32(proj[1])
+        require_cuda(weight, bias)
+        if tuple(weight.shape) != (dim, 2) or tuple(bias.shape) != (dim,) or tuple(pseudo.shape) != (e, 2) or not gmm_native.projection_supported(k, dim):
+            raise FgnnError("gmmconv: projection weight %s, bias %s do not fit pseudo %s for K=%d dim=%d (at most 4 of each) E=%d" % (
+                tuple(weight.shape), tuple(bias.shape), tuple(pseudo.shape), k, dim, e))
+        return weight, bias
+
+    @staticmethod
+    def projection_supported(k, dim):
+        return 0 < k <= 4 and 0 < dim <= 4
+
+    @staticmethod
     def gmmconv(rowptr, colind, node_feat, pseudo, mu, sigma, *, pos_map=None, want_gauss=False, sum_kernels=False, own_order=False,
-                bias=None, residual=None):
-        """bias [F] / residual [N,F] (with sum_kernels only): added to the summed output inside the operator's store."""
+                bias=None, residual=None, proj=None):
+        """bias [F] / residual [N,F] (with sum_kernels only): added to the summed output inside the operator's store.
+        proj: (weight [dim,2], bias [dim]); pseudo is then [E,2] and the coordinates are tanh(pseudo @ weight^T + bias)."""
         require_cuda(rowptr, colind, node_feat, pseudo, mu, sigma, bias, residual)
         rowptr, colind = as_i32(rowptr), as_i32(colind)
         node_feat, pseudo, mu, sigma = as_f32(node_feat), as_f32(pseudo), as_f32(mu), as_f32(sigma)
@@ -31,7 +46,8 @@ class gmm_native:
         n, k, f = node_feat.shape
         e = colind.numel()
         dim = mu.shape[1]
-        if mu.shape != (k, dim) or sigma.shape != (k, dim) or pseudo.shape != (e, dim) or rowptr.numel() != n + 1:
+        pw, pb = (None, None) if proj is None else gmm_native.projection(proj, pseudo, k, dim, e)
+        if mu.shape != (k, dim) or sigma.shape != (k, dim) or (proj is None and pseudo.shape != (e, dim)) or rowptr.numel() != n + 1:
             raise FgnnError("gmmconv: shape mismatch mu %s sigma %s pseudo %s for K=%d E=%d" % (
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), k, e))
         out = torch.empty((n, f), dtype=torch.float32, device=node_feat.device) if sum_kernels else torch.empty_like(node_feat)
@@ -48,7 +64,11 @@ class gmm_native:
                 raise FgnnError("gmmconv: bias must be [%d] and residual [%d, %d]" % (f, n, f))
         with device_guard(node_feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), node_feat.device)
-            if epilogue:
+            if proj is not None:
+                check(lib().fgnn_gmm_forward_projected(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(node_feat), ptr(pseudo), ptr(pw), ptr(pb),
+                                                       ptr(mu), ptr(sigma), ptr(bias), ptr(residual), ptr(out), ptr(gauss), int(sum_kernels), sched.handle,
+                                                       ptr(ws), wsb, stream_ptr()), "fgnn_gmm_forward_projected")
+            elif epilogue:
                 check(lib().fgnn_gmm_forward_epilogue(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(node_feat), ptr(pseudo),
                                                       ptr(mu), ptr(sigma), ptr(bias), ptr(residual), ptr(out), ptr(gauss), sched.handle,
                                                       ptr(ws), wsb, stream_ptr()), "fgnn_gmm_forward_epilogue")
@@ -59,7 +79,9 @@ class gmm_native:
         return (out, gauss) if want_gauss else out
 
     @staticmethod
-    def gmmconv_backward(colptr, rowind, permute, node_feat, pseudo, mu, sigma, grad_out, sum_kernels=False, own_order=False):
+    def gmmconv_backward(colptr, rowind, permute, node_feat, pseudo, mu, sigma, grad_out, sum_kernels=False, own_order=False, proj=None):
+        """(grad_feat, grad_pseudo, grad_mu, grad_sigma); with proj (see gmmconv) the gradients of its weight and bias in the place of
+        grad_pseudo, and nothing is written per edge."""
         require_cuda(colptr, rowind, permute, node_feat, pseudo, mu, sigma, grad_out)
         colptr, rowind = as_i32(colptr), as_i32(rowind)
         permute = None if permute is None else as_i32(permute)      # None: pseudo / grad_pseudo in CSC order
@@ -72,22 +94,35 @@ class gmm_native:
         dim = mu.shape[1]
         dev = node_feat.device
         want_go = (n, f) if sum_kernels else (n, k, f)
-        if (mu.shape != (k, dim) or sigma.shape != (k, dim) or pseudo.shape != (e, dim) or colptr.numel() != n + 1
+        pw, pb = (None, None) if proj is None else gmm_native.projection(proj, pseudo, k, dim, e)
+        if (mu.shape != (k, dim) or sigma.shape != (k, dim) or (proj is None and pseudo.shape != (e, dim)) or colptr.numel() != n + 1
                 or tuple(grad_out.shape) != want_go or (permute is not None and permute.numel() != e)):
             raise FgnnError("gmmconv_backward: shape mismatch mu %s sigma %s pseudo %s grad_out %s col_ptr %d for N=%d K=%d F=%d E=%d" % (
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), tuple(grad_out.shape), colptr.numel(), n, k, f, e))
         grad_feat = torch.empty_like(node_feat)
-        grad_pseudo = torch.empty((e, dim), dtype=torch.float32, device=dev)
+        grad_pseudo = torch.empty((e, dim), dtype=torch.float32, device=dev) if proj is None else (torch.empty_like(pw), torch.empty_like(pb))
         grad_mu = torch.empty_like(mu)
         grad_sigma = torch.empty_like(sigma)
         # own_order: pseudo, grad_pseudo (and permute) are indexed by the schedule's entry order (gmm_edge_positions(colptr, rowind, True))
         sched = schedule_for(colptr, idx_tensor=None if (sum_kernels and _plain_list_for_summed_backward(n, e)) else rowind, own_order=own_order, n_cols=n)
-        with device_guard(dev):
-            ws, wsb = workspace(lib().fgnn_gmm_backward_workspace_bytes(sched.handle, k, dim, f), dev)
-            check(lib().fgnn_gmm_backward(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(node_feat), ptr(pseudo),
-                                          ptr(mu), ptr(sigma), ptr(grad_out), int(sum_kernels), ptr(grad_feat), ptr(grad_pseudo), ptr(grad_mu),
-                                          ptr(grad_sigma), sched.handle, ptr(ws), wsb, stream_ptr()), "fgnn_gmm_backward")
+        gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, node_feat, pseudo, (pw, pb), mu, sigma, grad_out, int(sum_kernels), grad_feat, grad_pseudo,
+                             grad_mu, grad_sigma, sched, dev)
         return grad_feat, grad_pseudo, grad_mu, grad_sigma
+
+    @staticmethod
+    def _backward(n, e, k, dim, f, colptr, rowind, permute, feat, pseudo, proj, mu, sigma, grad_out, sum_kernels, grad_feat, grad_pseudo, grad_mu, grad_sigma, sched,
+                  dev):
+        with device_guard(dev):
+            if proj[0] is None:
+                ws, wsb = workspace(lib().fgnn_gmm_backward_workspace_bytes(sched.handle, k, dim, f), dev)
+                check(lib().fgnn_gmm_backward(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(feat), ptr(pseudo),
+                                              ptr(mu), ptr(sigma), ptr(grad_out), sum_kernels, ptr(grad_feat), ptr(grad_pseudo), ptr(grad_mu),
+                                              ptr(grad_sigma), sched.handle, ptr(ws), wsb, stream_ptr()), "fgnn_gmm_backward")
+                return
+            ws, wsb = workspace(lib().fgnn_gmm_backward_projected_workspace_bytes(sched.handle, k, dim, f), dev)
+            check(lib().fgnn_gmm_backward_projected(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(feat), ptr(pseudo), ptr(proj[0]), ptr(proj[1]),
+                                                    ptr(mu), ptr(sigma), ptr(grad_out), sum_kernels, ptr(grad_feat), ptr(grad_pseudo[0]), ptr(grad_pseudo[1]),
+                                                    ptr(grad_mu), ptr(grad_sigma), sched.handle, ptr(ws), wsb, stream_ptr()), "fgnn_gmm_backward_projected")
 
     @staticmethod
     def shared_supported(k, f):
@@ -96,7 +131,7 @@ class gmm_native:
         return f % 4 == 0 and 0 < f <= 256 and 0 < k <= 4
 
     @staticmethod
-    def gmmconv_shared(rowptr, colind, feat, pseudo, mu, sigma, *, pos_map=None, own_order=False):
+    def gmmconv_shared(rowptr, colind, feat, pseudo, mu, sigma, *, pos_map=None, own_order=False, proj=None):
         """out[i,k,:] = sum_p w[p,k] * feat[colind[p],:] for one [N,F] feature matrix shared by the K mixture
         kernels (the reference's gmmconv with node_feat[:,k,:] == feat for every k).  Returns [N,K,F]."""
         require_cuda(rowptr, colind, feat, pseudo, mu, sigma)
@@ -107,21 +142,27 @@ class gmm_native:
         n, f = feat.shape
         k, dim = mu.shape
         e = colind.numel()
-        if sigma.shape != (k, dim) or pseudo.shape != (e, dim) or rowptr.numel() != n + 1:
+        pw, pb = (None, None) if proj is None else gmm_native.projection(proj, pseudo, k, dim, e)
+        if sigma.shape != (k, dim) or (proj is None and pseudo.shape != (e, dim)) or rowptr.numel() != n + 1:
             raise FgnnError("gmmconv_shared: shape mismatch mu %s sigma %s pseudo %s for E=%d" % (
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), e))
         out = torch.empty((n, k, f), dtype=torch.float32, device=feat.device)
         sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n)
         with device_guard(feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), feat.device)
+            if proj is not None:
+                check(lib().fgnn_gmm_forward_projected(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(feat), ptr(pseudo), ptr(pw), ptr(pb), ptr(mu),
+                                                       ptr(sigma), None, None, ptr(out), None, 2, sched.handle, ptr(ws), wsb, stream_ptr()),
+                      "fgnn_gmm_forward_projected (shared features)")
+                return out
             check(lib().fgnn_gmm_forward(n, e, k, dim, f, ptr(rowptr), ptr(colind), ptr(pos_map), ptr(feat), ptr(pseudo),
                                          ptr(mu), ptr(sigma), ptr(out), None, 2, sched.handle, ptr(ws), wsb, stream_ptr()),
                   "fgnn_gmm_forward (shared features)")
         return out
 
     @staticmethod
-    def gmmconv_shared_backward(colptr, rowind, permute, feat, pseudo, mu, sigma, grad_out, own_order=False):
-        """Backward of gmmconv_shared for grad_out [N,K,F]: (grad_feat [N,F], grad_pseudo, grad_mu, grad_sigma)."""
+    def gmmconv_shared_backward(colptr, rowind, permute, feat, pseudo, mu, sigma, grad_out, own_order=False, proj=None):
+        """Backward of gmmconv_shared for grad_out [N,K,F]: (grad_feat [N,F], grad_pseudo (see gmmconv_backward), grad_mu, grad_sigma)."""
         require_cuda(colptr, rowind, permute, feat, pseudo, mu, sigma, grad_out)
         colptr, rowind = as_i32(colptr), as_i32(rowind)
         permute = None if permute is None else as_i32(permute)
@@ -134,20 +175,18 @@ class gmm_native:
         dev = feat.device
         if grad_out.shape != (n, k, f):
             raise FgnnError("gmmconv_shared_backward: grad_out is %s, expected (%d, %d, %d)" % (tuple(grad_out.shape), n, k, f))
-        if sigma.shape != (k, dim) or pseudo.shape != (e, dim) or colptr.numel() != n + 1 or (permute is not None and permute.numel() != e):
+        pw, pb = (None, None) if proj is None else gmm_native.projection(proj, pseudo, k, dim, e)
+        if sigma.shape != (k, dim) or (proj is None and pseudo.shape != (e, dim)) or colptr.numel() != n + 1 or (permute is not None and permute.numel() != e):
             raise FgnnError("gmmconv_shared_backward: shape mismatch sigma %s pseudo %s col_ptr %d for N=%d K=%d E=%d" % (
                 tuple(sigma.shape), tuple(pseudo.shape), colptr.numel(), n, k, e))
         parts = torch.empty((n, k, f), dtype=torch.float32, device=dev)      # kernel k's share of grad_feat
-        grad_pseudo = torch.empty((e, dim), dtype=torch.float32, device=dev)
+        grad_pseudo = torch.empty((e, dim), dtype=torch.float32, device=dev) if proj is None else (torch.empty_like(pw), torch.empty_like(pb))
         grad_mu = torch.empty_like(mu)
         grad_sigma = torch.empty_like(sigma)
         # same work list as the summed backward, so that one CSC-side copy of own-order edge data serves both kinds of layer
         sched = schedule_for(colptr, idx_tensor=None if _plain_list_for_summed_backward(n, e) else rowind, own_order=own_order, n_cols=n)
-        with device_guard(dev):
-            ws, wsb = workspace(lib().fgnn_gmm_backward_workspace_bytes(sched.handle, k, dim, f), dev)
-            check(lib().fgnn_gmm_backward(n, e, k, dim, f, ptr(colptr), ptr(rowind), ptr(permute), ptr(feat), ptr(pseudo),
-                                          ptr(mu), ptr(sigma), ptr(grad_out), 2, ptr(parts), ptr(grad_pseudo), ptr(grad_mu),
-                                          ptr(grad_sigma), sched.handle, ptr(ws), wsb, stream_ptr()), "fgnn_gmm_backward (shared features)")
+        gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, feat, pseudo, (pw, pb), mu, sigma, grad_out, 2, parts, grad_pseudo, grad_mu, grad_sigma, sched,
+                             dev)
         return parts.sum(1), grad_pseudo, grad_mu, grad_sigma
 
     @staticmethod
@@ -332,6 +371,44 @@ class GmmAggregateTwoOrdersFunction(torch.autograd.Function):
         grad_feat, grad_pseudo_csc, grad_mu, grad_sigma = gmm_native.gmmconv_shared_backward(
             colptr, rowind, None, feat, pseudo_csc, mu, sigma, grad_out.contiguous(), own_order=ctx.own_order)
         return None, None, None, None, grad_feat, None, grad_pseudo_csc, grad_mu, grad_sigma, None
+
+
+def GmmProjectedTwoOrders(rowptr, colind, colptr, rowind, node_feat, raw_csr, raw_csc, weight, bias, mu, sigma, own_order=False, keep_gauss=False,
+                          out_bias=None, residual=None):
+    """GmmConvFuseSumTwoOrders (node_feat [N,K,F]; keep_gauss: GmmConvStashSumTwoOrders) or GmmAggregateTwoOrders (node_feat [N,F]) on the
+    coordinates tanh(raw @ weight^T + bias) of constant raw [E,2] edge data, in both edge orders: the passes over the edges form them
+    themselves, and the backward sums the gradients of weight, bias, mu and sigma where it forms the derivatives of the mixture weights.
+    Instead of 4 E dim floats of coordinates and their gradients and E K of derivatives, written and read back, an edge costs 8 bytes
+    a pass (115 M edges, 2 kernels of 1 coordinate, two layers: MoNet step 8.96 -> 7.64 ms)."""
+    return GmmProjectedTwoOrdersFunction.apply(rowptr, colind, colptr, rowind, node_feat, raw_csr, raw_csc, weight, bias, mu, sigma, own_order, keep_gauss,
+                                               out_bias, residual)
+
+
+class GmmProjectedTwoOrdersFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, rowptr, colind, colptr, rowind, node_feat, raw_csr, raw_csc, weight, bias, mu, sigma, own_order, keep_gauss, out_bias=None, residual=None):
+        gauss = None
+        if node_feat.dim() == 2:
+            out = gmm_native.gmmconv_shared(rowptr, colind, node_feat, raw_csr, mu, sigma, own_order=own_order, proj=(weight, bias))
+        else:
+            out = gmm_native.gmmconv(rowptr, colind, node_feat, raw_csr, mu, sigma, want_gauss=keep_gauss, sum_kernels=True, own_order=own_order, bias=out_bias,
+                                     residual=residual, proj=(weight, bias))
+            out, gauss = out if keep_gauss else (out, None)
+        ctx.save_for_backward(colptr, rowind, node_feat, raw_csc, weight, bias, mu, sigma, gauss)
+        ctx.own_order = own_order
+        ctx.has_bias, ctx.has_res = out_bias is not None, residual is not None
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        colptr, rowind, node_feat, raw_csc, weight, bias, mu, sigma, _gauss = ctx.saved_tensors
+        args = (colptr, rowind, None, node_feat, raw_csc, mu, sigma, grad_out.contiguous())
+        if node_feat.dim() == 2:
+            grads = gmm_native.gmmconv_shared_backward(*args, own_order=ctx.own_order, proj=(weight, bias))
+        else:
+            grads = gmm_native.gmmconv_backward(*args, sum_kernels=True, own_order=ctx.own_order, proj=(weight, bias))
+        grad_feat, (grad_w, grad_b), grad_mu, grad_sigma = grads
+        return (None, None, None, None, grad_feat, None, None, grad_w, grad_b, grad_mu, grad_sigma, None, None) + _epilogue_grads(ctx, grad_out.contiguous(), 13)
 
 
 def project_in_backward(k, fin, fout, input_grad, n, e):

@@ -38,6 +38,13 @@ class PseudoProj(nn.Linear):
         return torch.tanh(out + self.bias)
 
 
+    def plain(self, *pseudo):
+        """Whether a layer may apply the projection's parameters itself: the fused form's shapes, and nobody hooked to the module."""
+        hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
+        return (type(self) is PseudoProj and self.out_features <= edge_proj.MAX_OUT and self.bias is not None and not any(hooks)
+                and all(t.is_cuda and not t.requires_grad for t in pseudo))
+
+
 class MoNet(nn.Module):
     def __init__(self, conv, in_feats, n_hidden, out_feats, n_layers, dim, n_kernels, dropout):
         super().__init__()
@@ -55,7 +62,9 @@ class MoNet(nn.Module):
         for i, (layer, proj) in enumerate(zip(self.layers, self.pseudo_proj)):
             if i:
                 h = self.dropout(h)
-            if pseudo_csc is not None and torch.is_grad_enabled():
+            if pseudo_csc is not None and torch.is_grad_enabled() and proj.plain(pseudo, pseudo_csc):
+                h = layer(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, h, pseudo, pseudo_csc=pseudo_csc, own_order=own_order, proj=proj)
+            elif pseudo_csc is not None and torch.is_grad_enabled():
                 with torch.no_grad():
                     ps = proj(pseudo)
                 h = layer(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, h, ps, pseudo_csc=proj(pseudo_csc), own_order=own_order)

@@ -361,6 +361,26 @@ int    fgnn_gmm_backward(int N, int64_t E, int K, int dim, int F,
                          const fgnn_schedule_t *sched_csc, void *workspace, size_t workspace_bytes,
                          void *stream);
 
+/* The same passes on projected coordinates: pseudo[p,:] = tanh(raw[p,:] @ proj_W^T + proj_b) of constant pairs raw [E,2] (8-byte aligned),
+ * proj_W [dim,2], proj_b [dim], dim <= 4, K <= 4 (the projection in front of every layer of the MoNet drivers,
+ * script/train/train_gmmconv_our.py:46-57).  Forward: bias and residual as in fgnn_gmm_forward_epilogue, with sum_kernels == 1 only (else
+ * NULL).  Backward: the gradients of proj_W and proj_b in the place of grad_pseudo; nothing is kept per edge, all sums in a fixed
+ * order. */
+int    fgnn_gmm_forward_projected(int N, int64_t E, int K, int dim, int F,
+                                  const int32_t *ptr, const int32_t *idx, const int32_t *pos_map,
+                                  const float *node_feat, const float *raw, const float *proj_W, const float *proj_b,
+                                  const float *mu, const float *inv_sigma, const float *bias, const float *residual,
+                                  float *out, float *gauss_out, int sum_kernels, const fgnn_schedule_t *sched,
+                                  void *workspace, size_t workspace_bytes, void *stream);
+size_t fgnn_gmm_backward_projected_workspace_bytes(const fgnn_schedule_t *sched_csc, int K, int dim, int F);
+int    fgnn_gmm_backward_projected(int N, int64_t E, int K, int dim, int F,
+                                   const int32_t *col_ptr, const int32_t *row_ind, const int32_t *permute,
+                                   const float *node_feat, const float *raw, const float *proj_W, const float *proj_b,
+                                   const float *mu, const float *inv_sigma, const float *grad_out, int sum_kernels,
+                                   float *grad_feat, float *grad_W, float *grad_b, float *grad_mu, float *grad_sigma,
+                                   const fgnn_schedule_t *sched_csc, void *workspace, size_t workspace_bytes,
+                                   void *stream);
+
 /* gmmconv.Gaussian / gmmconv.GaussianBp (gmmconv.cc:36-41,80-86; gmmconv.cu:187-199,265-285).
  * The backward implements the closed-form derivatives of the Gaussian weight; grad_mu and
  * grad_sigma are reduced in a fixed order (bit-reproducible). */

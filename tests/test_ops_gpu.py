@@ -1713,3 +1713,69 @@ def test_tall_reduce(n, a, b, h):
     for got in (one, tall_reduce(dx, wide[:, :b], de)):
         assert got.shape == ref.shape and bool(((got.cpu().double() - ref).abs() <= tol).all())
     assert torch.equal(one, tall_reduce(dx, dg, de))                     # fixed order of summation
+
+
+# ---------------------------------------------------------------- GMMConv on projected coordinates
+
+def _monet_layer_f64(g, feat, raw, layer, proj):
+    """The layer and its gradients' graph in float64 on the CPU, edge by edge (raw in CSR order)."""
+    dst = torch.repeat_interleave(torch.arange(g.n), (g.row_ptr[1:] - g.row_ptr[:-1]).long())
+    ps = torch.tanh(raw @ proj.weight.t() + proj.bias)
+    w = torch.exp(-0.5 * (((ps[:, None, :] - layer.mu) * layer.inv_sigma) ** 2).sum(-1))                            # [E, K]
+    h = (feat @ layer.fc.weight.t()).view(g.n, layer.mu.shape[0], -1)
+    out = torch.zeros(g.n, h.shape[2], dtype=torch.float64)
+    out = out.index_add(0, dst, (w[:, :, None] * h[g.col_ind.long()]).sum(1))
+    return out if layer.bias is None else out + layer.bias
+
+
+# every pass that has a projected form: the summed column pass on lane groups of 1 to 64 lanes, packed and wide rows, shared features
+# (aggregate first), whole items and short items in lane groups (low and high degree), split rows; padded widths; the stash variant
+@pytest.mark.parametrize("n,e,fin,fout,k,dim,stash", [(300, 1200, 40, 16, 2, 1, False), (300, 1200, 16, 41, 2, 1, False), (500, 60000, 8, 44, 4, 4, False),
+                                                      (200, 3000, 64, 4, 3, 2, True), (400, 2000, 200, 64, 3, 3, True), (150, 20000, 300, 100, 1, 2, False),
+                                                      (600, 90000, 32, 64, 2, 3, False), (90, 200, 12, 7, 1, 1, True), (700, 9000, 24, 100, 3, 2, False),
+                                                      (260, 2000, 30, 250, 4, 2, True), (40, 0, 8, 8, 2, 2, False)])
+@pytest.mark.parametrize("own_order", [False, True])
+def test_gmm_projected_coordinates(n, e, fin, fout, k, dim, stash, own_order):
+    import copy
+    from ae_mlsys_gnn_amd.layers import GMMConv, GMMConv_stash
+    from ae_mlsys_gnn_amd.operators.csr2csc import csr2csc
+    from ae_mlsys_gnn_amd.train import train_gmmconv
+    torch.manual_seed(n + e)
+    g = graphs.rmat_graph(n, e, seed=1) if e else custom_graph([[]] * n)
+    gd = g.to(DEV)
+    gd.col_ptr, gd.row_ind, gd.permute = csr2csc(gd.row_ptr, gd.col_ind)
+    layer = (GMMConv_stash if stash else GMMConv)(fin, fout, dim, k)
+    torch.nn.init.normal_(layer.bias)
+    torch.nn.init.uniform_(layer.inv_sigma, 0.5, 1.5)
+    proj = train_gmmconv.PseudoProj(2, dim)
+    feat, raw, go = torch.randn(n, fin), torch.rand(g.n_edges, 2), torch.randn(n, fout)
+    ref_layer, ref_proj = copy.deepcopy(layer).double(), copy.deepcopy(proj).double()
+    ref_feat = feat.double().requires_grad_(True)
+    out = _monet_layer_f64(g, ref_feat, raw.double(), ref_layer, ref_proj)
+    out.backward(go.double())
+    want = [out.detach(), ref_feat.grad] + [p.grad for p in list(ref_layer.parameters()) + list(ref_proj.parameters())]
+
+    layer, proj = layer.to(DEV), proj.to(DEV)
+    rd = raw.to(DEV)
+    fwd, bwd = train_gmmconv.schedule_order_copies(gd, rd) if own_order else (rd, rd[gd.permute.long()].contiguous())
+    results = []
+    for projected in (True, False, True):
+        x = feat.to(DEV).requires_grad_(True)
+        for p in list(layer.parameters()) + list(proj.parameters()):
+            p.grad = None
+        if projected:
+            y = layer(gd.row_ptr, gd.col_ind, gd.col_ptr, gd.row_ind, gd.permute, x, fwd, pseudo_csc=bwd, own_order=own_order, proj=proj)
+        else:
+            with torch.no_grad():
+                ps = proj(fwd)
+            y = layer(gd.row_ptr, gd.col_ind, gd.col_ptr, gd.row_ind, gd.permute, x, ps, pseudo_csc=proj(bwd), own_order=own_order)
+        y.backward(go.to(DEV))
+        zero = lambda t, p: torch.zeros_like(p) if t is None else t
+        results.append([y.detach(), x.grad] + [zero(p.grad, p) for p in list(layer.parameters()) + list(proj.parameters())])
+    assert all(torch.equal(a, b) for a, b in zip(results[0], results[2]))                 # sums in a fixed order
+    for i, (got, comp, ref) in enumerate(zip(results[0], results[1], want)):
+        scale = ref.norm() + 1e-12
+        err, old = float((got.cpu().double() - ref).norm() / scale), float((comp.cpu().double() - ref).norm() / scale)
+        # 2-norm of the error: a few roundings (2^-24 each) of every product and sum; a parameter's gradient is a cancelling sum over the
+        # edges, and the composed passes are the measure of it
+        assert err <= max(2.0 ** -20, 2 * old + 2.0 ** -22), (i, err, old)
