@@ -27,6 +27,7 @@ _SIGNATURES = {
     "fgnn_last_error": (ctypes.c_char_p, []),
     "fgnn_schedule_create": (c_int, [c_void_p, c_int, c_int, c_void_p, ctypes.POINTER(c_void_p)]),
     "fgnn_schedule_create_bucketed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, ctypes.POINTER(c_void_p)]),
+    "fgnn_schedule_create_flat": (c_int, [c_void_p, c_int, c_void_p, ctypes.POINTER(c_void_p)]),
     "fgnn_schedule_take_positions": (c_int, [c_void_p, c_void_p, c_void_p]),
     "fgnn_schedule_destroy": (None, [c_void_p]),
     "fgnn_schedule_num_items": (c_int, [c_void_p]),
@@ -190,9 +191,11 @@ class Schedule:
     """Degree-binned work list of one pointer array (row_ptr or col_ptr).  With `idx_tensor` it is
     the XCD-aware form: long rows are cut by source bucket and each XCD gets one bucket."""
 
-    def __init__(self, ptr_tensor, seg_len=0, idx_tensor=None, min_deg=0, with_positions=True, n_cols=None):
+    def __init__(self, ptr_tensor, seg_len=0, idx_tensor=None, min_deg=0, with_positions=True, n_cols=None, flat_of=None):
+        """flat_of: an XCD-aware Schedule of the same arrays; the list is then the plain one over its entry order."""
         require_cuda(ptr_tensor)
         self.ptr_tensor = as_i32(ptr_tensor)      # keeps the device memory alive
+        self.flat_of = flat_of                    # ...and the index copy it walks
         self.idx_tensor = None if idx_tensor is None else as_i32(idx_tensor)
         self.n_rows = self.ptr_tensor.numel() - 1
         handle = c_void_p()
@@ -204,7 +207,9 @@ class Schedule:
                 bound = int(n_cols) if n_cols is not None else 2147483647
                 check(lib().fgnn_validate_graph(ptr(self.ptr_tensor), ptr(self.idx_tensor), self.n_rows, bound,
                                                 self.idx_tensor.numel(), stream_ptr()), "fgnn_validate_graph")
-            if self.idx_tensor is None:
+            if flat_of is not None:
+                check(lib().fgnn_schedule_create_flat(flat_of.handle, int(seg_len), stream_ptr(), ctypes.byref(handle)), "fgnn_schedule_create_flat")
+            elif self.idx_tensor is None:
                 check(lib().fgnn_schedule_create(ptr(self.ptr_tensor), self.n_rows, int(seg_len), stream_ptr(),
                                                  ctypes.byref(handle)), "fgnn_schedule_create")
             else:
@@ -217,7 +222,7 @@ class Schedule:
         self.n_partials = lib().fgnn_schedule_num_partials(handle)
         self.n_wave_slots = lib().fgnn_schedule_num_wave_slots(handle)   # items from this slot on have at most 64 entries
         self.n_edges = lib().fgnn_schedule_num_edges(handle)
-        self.own_order = False
+        self.own_order = flat_of is not None and flat_of.own_order
 
     def export(self):
         """(items int32 [n_items, 4], splits int32 [n_split, 4]) on the device: the work list itself."""
@@ -308,7 +313,7 @@ def xcd_buckets_enabled(ptr_tensor, idx_numel=None) -> bool:
 
 
 @_locked
-def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True, own_order=False, n_cols=None) -> Schedule:
+def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True, own_order=False, n_cols=None, flat=False) -> Schedule:
     """Cached schedule of a pointer array.  The cache entry holds the tensors, so their device
     addresses cannot be reused while the entry lives; in-place edits bump `_version`.
     idx_tensor: the index array, for operators that may use an XCD-aware schedule.
@@ -316,9 +321,13 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
     the caller's position of every entry, 4*E bytes more); a schedule with positions serves both.
     n_cols: rows of the array the ids index, for the opt-in FGNN_VALIDATE check (None: only ids >= 0 is checked).
     own_order: a schedule of its own (never shared with the other kinds) whose position map was taken
-    out (`edge_positions`): operators called with it take per-edge tensors in the schedule's order."""
+    out (`edge_positions`): operators called with it take per-edge tensors in the schedule's order.
+    flat: the plain list in any case (rows too narrow for the cut by source bucket to pay), over the own-order entry order where the
+    per-edge tensors are in that."""
     if seg_len is None:
         seg_len = default_seg_len()
+    if flat and not own_order:
+        idx_tensor = None
     if idx_tensor is not None and not xcd_buckets_enabled(ptr_tensor, idx_tensor.numel()):
         idx_tensor = None
     min_deg = int(os.environ.get("FGNN_BUCKET_MIN_DEG", "0"))
@@ -333,6 +342,15 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
             raise FgnnError("no own-order schedule for these arrays: call edge_positions(ptr, idx) first and pass per-edge "
                             "tensors permuted by its result")
         _sched_cache.move_to_end(k)
+        if flat and s.n_buckets > 0:
+            kf = k + ("flat",)
+            f = _sched_cache.get(kf)
+            if f is None or f.flat_of is not s:
+                f = _sched_cache[kf] = Schedule(ptr_tensor, seg_len, flat_of=s)
+                while len(_sched_cache) > _SCHED_CACHE_MAX:
+                    _sched_cache.popitem(last=False)
+            _sched_cache.move_to_end(kf)
+            return f
         return s
     k = key(True)
     s = _sched_cache.get(k)

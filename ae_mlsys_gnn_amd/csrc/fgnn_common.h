@@ -76,6 +76,10 @@ struct fgnn_schedule {
     int32_t *bidx_dev;
     int32_t *bpos_dev;      // original position of every bucket-ordered entry (for per-edge arrays)
     int own_order;          // the position map was handed to the caller: per-edge arrays come in the schedule's entry order
+    // A flat list (fgnn_schedule_create_flat): plain items (n_buckets 0) over the entry order of an XCD-aware schedule, whose index
+    // array and position map it uses; that schedule has to outlive it.
+    int borrows;
+    int lent;               // there are flat lists over this schedule: its position map stays
     // Every item at a slot >= n_wave_slots has at most FGNN_GROUP_ITEM_MAX entries (the lists are sorted longest first, so the
     // long items are a prefix).  A multiple of 64 slots per source bucket, or n_items.  Kernels that give each lane group of a
     // wave its own item start there; the prefix goes to the kernels that put a whole wave on an item.
@@ -84,10 +88,10 @@ struct fgnn_schedule {
 #define FGNN_GROUP_ITEM_MAX 64
 // The index array a kernel walks under schedule `s`, and the map from its positions back to the
 // caller's edge positions (NULL = identity).
-static inline const int32_t *fgnn_sched_idx(const fgnn_schedule *s, const int32_t *idx) { return (s && s->n_buckets > 0) ? s->bidx_dev : idx; }
-static inline const int32_t *fgnn_sched_pos(const fgnn_schedule *s) { return (s && s->n_buckets > 0) ? s->bpos_dev : nullptr; }
+static inline const int32_t *fgnn_sched_idx(const fgnn_schedule *s, const int32_t *idx) { return (s && s->bidx_dev) ? s->bidx_dev : idx; }
+static inline const int32_t *fgnn_sched_pos(const fgnn_schedule *s) { return (s && s->bidx_dev) ? s->bpos_dev : nullptr; }
 // false for an XCD-aware schedule built without the position map: operators with per-edge tensors must refuse it
-static inline bool fgnn_sched_has_pos(const fgnn_schedule *s) { return !s || s->n_buckets == 0 || s->n_edges == 0 || s->bpos_dev != nullptr || s->own_order; }
+static inline bool fgnn_sched_has_pos(const fgnn_schedule *s) { return !s || !s->bidx_dev || s->bpos_dev != nullptr || s->own_order; }
 
 #define FGNN_NUM_XCD 8      // workgroup w of a dispatch runs on XCD w % 8 (gfx942 / gfx950, SPX mode)
 // Source bucket of a node id: the top 3 bits of a multiplicative hash, so hot ids spread evenly.

@@ -1318,7 +1318,7 @@ static int check_sched(const fgnn_schedule_t *s, const int32_t *ptr, const int32
     FGNN_REQUIRE(s->ptr_dev == ptr && s->n_rows == n && s->n_edges == E, FGNN_ERR_SCHEDULE,
                  "%s: schedule was built for another pointer array (n_rows %d vs %d, edges %lld vs %lld)", what,
                  s->n_rows, n, (long long)s->n_edges, (long long)E);
-    if (s->n_buckets > 0)
+    if (s->bidx_dev)
         FGNN_REQUIRE(s->idx_src_dev == idx, FGNN_ERR_SCHEDULE, "%s: XCD-aware schedule was built from another index array", what);
     return 0;
 }

@@ -164,7 +164,7 @@ static fgnn_schedule *new_schedule(const int32_t *ptr_dev, int n_rows, int64_t n
     s->n_rows = n_rows; s->n_edges = n_edges; s->seg_len = seg_len;
     s->n_items = s->n_partials = s->n_split = 0;
     s->items_dev = nullptr; s->split_dev = nullptr; s->ptr_dev = ptr_dev;
-    s->n_buckets = 0; s->idx_src_dev = nullptr; s->bidx_dev = nullptr; s->bpos_dev = nullptr; s->own_order = 0; s->n_wave_slots = 0;
+    s->n_buckets = 0; s->idx_src_dev = nullptr; s->bidx_dev = nullptr; s->bpos_dev = nullptr; s->own_order = 0; s->n_wave_slots = 0; s->borrows = s->lent = 0;
     (void)hipGetDevice(&s->device);
     return s;
 }
@@ -632,6 +632,23 @@ extern "C" int fgnn_schedule_create_bucketed(const int32_t *ptr_dev, const int32
     return 0;
 }
 
+// The plain list (rows cut only past seg_len entries) over the entry order of an XCD-aware schedule: for operators on rows so narrow that
+// the gathered matrix stays in the caches anyway, where cutting every row by source bucket only costs partial results, while
+// the caller's per-edge arrays are in that schedule's order.
+extern "C" int fgnn_schedule_create_flat(fgnn_schedule_t *base, int seg_len, void *stream, fgnn_schedule_t **out)
+{
+    FGNN_REQUIRE(base && out, FGNN_ERR_NULL, "fgnn_schedule_create_flat: NULL argument");
+    FGNN_REQUIRE(!base->borrows, FGNN_ERR_SCHEDULE, "fgnn_schedule_create_flat: the schedule is a flat list itself");
+    fgnn_schedule_t *s = nullptr;
+    int rc = fgnn_schedule_create(base->ptr_dev, base->n_rows, seg_len, stream, &s);
+    if (rc) return rc;
+    s->idx_src_dev = base->idx_src_dev; s->bidx_dev = base->bidx_dev; s->bpos_dev = base->bpos_dev; s->own_order = base->own_order;
+    s->borrows = 1;
+    base->lent = 1;
+    *out = s;
+    return 0;
+}
+
 // Copies the work items (4 ints each: row, begin, end, slot) and the split table (4 ints each: row, first slot,
 // segments, 0) to caller memory on the device; either pointer may be NULL.
 extern "C" int fgnn_schedule_export(const fgnn_schedule_t *s, int32_t *items_out, int32_t *splits_out, void *stream)
@@ -661,6 +678,7 @@ extern "C" int fgnn_schedule_take_positions(fgnn_schedule_t *s, int32_t *pos_out
 {
     FGNN_REQUIRE(s, FGNN_ERR_NULL, "fgnn_schedule_take_positions: NULL schedule");
     FGNN_REQUIRE(pos_out_dev || s->n_edges == 0, FGNN_ERR_NULL, "fgnn_schedule_take_positions: NULL output");
+    FGNN_REQUIRE(!s->borrows && !s->lent, FGNN_ERR_SCHEDULE, "fgnn_schedule_take_positions: the position map is shared with a flat list");
     FGNN_REQUIRE(!s->own_order, FGNN_ERR_SCHEDULE, "fgnn_schedule_take_positions: the positions of this schedule were taken before");
     FGNN_REQUIRE(fgnn_sched_has_pos(s), FGNN_ERR_SCHEDULE, "fgnn_schedule_take_positions: the schedule was built without edge positions");
     hipStream_t st = (hipStream_t)stream;
@@ -684,8 +702,8 @@ extern "C" void fgnn_schedule_destroy(fgnn_schedule_t *s)
     if (!s) return;
     if (s->items_dev) (void)hipFree(s->items_dev);
     if (s->split_dev) (void)hipFree(s->split_dev);
-    if (s->bidx_dev) (void)hipFree(s->bidx_dev);
-    if (s->bpos_dev) (void)hipFree(s->bpos_dev);
+    if (s->bidx_dev && !s->borrows) (void)hipFree(s->bidx_dev);
+    if (s->bpos_dev && !s->borrows) (void)hipFree(s->bpos_dev);
     delete s;
 }
 
@@ -693,8 +711,8 @@ extern "C" size_t fgnn_schedule_device_bytes(const fgnn_schedule_t *s)
 {
     if (!s) return 0;
     size_t b = (size_t)s->n_items * sizeof(fgnn_item) + (size_t)s->n_split * sizeof(fgnn_split);
-    if (s->bidx_dev) b += (size_t)s->n_edges * sizeof(int32_t);
-    if (s->bpos_dev) b += (size_t)s->n_edges * sizeof(int32_t);
+    if (s->bidx_dev && !s->borrows) b += (size_t)s->n_edges * sizeof(int32_t);
+    if (s->bpos_dev && !s->borrows) b += (size_t)s->n_edges * sizeof(int32_t);
     return b;
 }
 

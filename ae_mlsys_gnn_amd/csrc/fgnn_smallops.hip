@@ -224,7 +224,7 @@ static int mhsddmm_run(const char *fn, int N, int64_t E, int H, int F, const int
     if (sched) {
         FGNN_REQUIRE(sched->ptr_dev == row_ptr && sched->n_rows == N && sched->n_edges == E, FGNN_ERR_SCHEDULE,
                      "%s: schedule was built for another pointer array", fn);
-        FGNN_REQUIRE(sched->n_buckets == 0 || sched->idx_src_dev == col_ind, FGNN_ERR_SCHEDULE,
+        FGNN_REQUIRE(!sched->bidx_dev || sched->idx_src_dev == col_ind, FGNN_ERR_SCHEDULE,
                      "%s: XCD-aware schedule was built from another index array", fn);
         // a list whose position map was handed to the caller (fgnn_schedule_take_positions) stores in its own entry order
         FGNN_REQUIRE(fgnn_sched_has_pos(sched), FGNN_ERR_SCHEDULE,

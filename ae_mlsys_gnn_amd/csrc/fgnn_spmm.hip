@@ -287,8 +287,11 @@ __device__ __forceinline__ void spmm_packed_item(const SpmmP &p, const WF &wf, c
                 w[u] = live ? wl[pm.hd * 64 + ei] : 0.f;
                 if (live) ld[u].load(p.feat + (size_t)rid * (size_t)p.ld + pm.eoff); else ld[u].zero();
             }
+            fg_vec<4> S;            // the batch by itself: a chain of 8 in a row of any length
+            S.zero();
 #pragma unroll
-            for (int u = 0; u < U; ++u) T.fma(w[u], ld[u]);
+            for (int u = 0; u < U; ++u) S.fma(w[u], ld[u]);
+            T.add(S);
         }
         fg_wave_lds_sync();
     }
@@ -434,7 +437,7 @@ static int spmm_checks(const char *fn, int N, int64_t E, int H, int F, const fgn
     if (sched) {
         FGNN_REQUIRE(sched->ptr_dev == ptr && sched->n_rows == N && sched->n_edges == E, FGNN_ERR_SCHEDULE,
                      "%s: schedule was built for another pointer array", fn);
-        FGNN_REQUIRE(sched->n_buckets == 0 || sched->idx_src_dev == idx, FGNN_ERR_SCHEDULE,
+        FGNN_REQUIRE(!sched->bidx_dev || sched->idx_src_dev == idx, FGNN_ERR_SCHEDULE,
                      "%s: XCD-aware schedule was built from another index array", fn);
         FGNN_REQUIRE(fgnn_sched_has_pos(sched), FGNN_ERR_SCHEDULE, "%s: the schedule was built without edge positions", fn);
     }
@@ -891,17 +894,20 @@ __device__ __forceinline__ void gmm_bwd_packed_item(const GmmBwdP &p, int n_head
                 pv[u] = __builtin_amdgcn_ds_bpermute((ei & 63) << 2, posv);
                 if (live) ld[u].load(p.g + (size_t)rid * p.g_stride + goff); else ld[u].zero();
             }
+            fg_vec<4> S;            // as in spmm_packed_item
+            S.zero();
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int ei = t + u * G + pm.grp;
                 const bool live = ei < cnt && pm.ok;
                 const float w = live ? wl[pm.hd * 64 + ei] : 0.f;
-                T.fma(w, ld[u]);
+                S.fma(w, ld[u]);
                 const float sum = fg_group_sum<LPH>(ld[u].dot(xr));
                 if (live && writer) {
                     if constexpr (ACC) wl[pm.hd * 64 + ei] = sum * w; else __builtin_nontemporal_store(sum * w, p.gww + (size_t)(unsigned)pv[u] * K + pm.hd);
                 }
             }
+            T.add(S);
         }
         fg_wave_lds_sync();
         if constexpr (ACC) ga.add(wl + lane, shared, K, dim, cv, rv);
@@ -1069,25 +1075,33 @@ __device__ __forceinline__ void gmm_bwd_sum_item(const GmmBwdP &p, int n_head, f
                 if (ei < cnt && fok) ld[u].load(p.g + (size_t)rid * F + foff); else ld[u].zero();
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int ei = t + u * G + grp;
-                float *gdst = p.gww + (size_t)(unsigned)pe[u] * K;
-                float mine = 0.f;                                   // lane `sub` of a row keeps the value of kernel `sub`
+            for (int k = 0; k < GMM_SUMK_MAX; ++k) {
+                if (k < K) {
+                    fg_vec<4> S;                                    // the batch by itself: a chain of U in a row of any length
+                    S.zero();
 #pragma unroll
-                for (int k = 0; k < GMM_SUMK_MAX; ++k) {
-                    if (k < K) {
-                        const float w = wl[k * 64 + ei];            // 0 past the end of the chunk
-                        T[k].fma(w, ld[u]);
-                        if constexpr (GWW) {
-                            const float sum = fg_group_sum<LPF>(ld[u].dot(xr[k]));
-                            if constexpr (LPF >= GMM_SUMK_MAX) mine = sub == k ? sum * w : mine;
-                            else if (ei < cnt && sub == 0) { if constexpr (ACC) wl[k * 64 + ei] = sum * w; else __builtin_nontemporal_store(sum * w, gdst + k); }
+                    for (int u = 0; u < U; ++u) S.fma(wl[k * 64 + t + u * G + grp], ld[u]);         // weight 0 past the end of the chunk
+                    T[k].add(S);
+                }
+            }
+            if constexpr (GWW) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int ei = t + u * G + grp;
+                    float *gdst = p.gww + (size_t)(unsigned)pe[u] * K;
+                    float mine = 0.f;                               // lane `sub` of a row keeps the value of kernel `sub`
+#pragma unroll
+                    for (int k = 0; k < GMM_SUMK_MAX; ++k) {
+                        if (k < K) {
+                            const float v = fg_group_sum<LPF>(ld[u].dot(xr[k])) * wl[k * 64 + ei];
+                            if constexpr (LPF >= GMM_SUMK_MAX) mine = sub == k ? v : mine;
+                            else if (ei < cnt && sub == 0) { if constexpr (ACC) wl[k * 64 + ei] = v; else __builtin_nontemporal_store(v, gdst + k); }
                         }
                     }
-                }
-                // the K values of an edge leave with one store instruction, K adjacent lanes writing K adjacent floats
-                if constexpr (GWW && LPF >= GMM_SUMK_MAX) {
-                    if (ei < cnt && sub < K) { if constexpr (ACC) wl[sub * 64 + ei] = mine; else __builtin_nontemporal_store(mine, gdst + sub); }
+                    // the K values of an edge leave with one store instruction, K adjacent lanes writing K adjacent floats
+                    if constexpr (LPF >= GMM_SUMK_MAX) {
+                        if (ei < cnt && sub < K) { if constexpr (ACC) wl[sub * 64 + ei] = mine; else __builtin_nontemporal_store(mine, gdst + sub); }
+                    }
                 }
             }
         }

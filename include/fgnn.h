@@ -80,6 +80,10 @@ int     fgnn_schedule_create_bucketed(const int32_t *ptr_dev, const int32_t *idx
  * 114.8 M edges: backward 3.6 -> 2.5 ms).  Once per schedule; FGNN_ERR_SCHEDULE for an XCD-aware schedule
  * built without positions.  No counterpart in the reference.  Synchronises `stream`. */
 int     fgnn_schedule_take_positions(fgnn_schedule_t *s, int32_t *pos_out_dev, void *stream);
+/* A plain list over the entry order of an XCD-aware schedule `base`, which has to outlive it (its index copy and position map are used,
+ * and its positions can no longer be taken): for operators on rows so narrow that cutting by source bucket does not pay, with
+ * per-edge arrays in base's order. */
+int     fgnn_schedule_create_flat(fgnn_schedule_t *base, int seg_len, void *stream, fgnn_schedule_t **out);
 void    fgnn_schedule_destroy(fgnn_schedule_t *s);
 int     fgnn_schedule_num_items(const fgnn_schedule_t *s);
 int     fgnn_schedule_num_partials(const fgnn_schedule_t *s);   /* segments of split rows */

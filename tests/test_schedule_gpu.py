@@ -173,3 +173,35 @@ def test_native_calls_follow_the_current_stream(monkeypatch, private_names):
         with torch.cuda.stream(side):
             assert _lib.stream_ptr().value == side.cuda_stream
     assert torch.cuda.current_device() == dev.index
+
+
+def test_flat_list_over_bucketed_order():
+    """The plain list over an XCD-aware schedule's entry order: same operators, same per-edge order, its own cuts; positions stay put."""
+    from ae_mlsys_gnn_amd import _lib
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import gmm_native
+    g = graphs.rmat_graph(3000, 400000, seed=3).to("cuda:0")
+    base = _lib.Schedule(g.row_ptr, 0, g.col_ind, 0)
+    if base.n_buckets == 0:
+        pytest.skip("the device has no workgroup-to-XCD mapping: every list is plain")
+    flat = _lib.Schedule(g.row_ptr, 128, flat_of=base)
+    plain = _lib.Schedule(g.row_ptr, 128)
+    assert flat.n_buckets == 0 and all(torch.equal(a, b) for a, b in zip(flat.export(), plain.export()))
+    assert flat.device_bytes() == plain.device_bytes()
+    with pytest.raises(_lib.FgnnError):
+        base.take_positions()
+    with pytest.raises(_lib.FgnnError):
+        flat.take_positions()
+    with pytest.raises(_lib.FgnnError):
+        _lib.Schedule(g.row_ptr, 0, flat_of=flat)
+    # own order: the narrow passes take the flat list, the wide ones the cut one, from the same per-edge copies
+    pos = _lib.edge_positions(g.row_ptr, g.col_ind).long()
+    ps = torch.rand(g.n_edges, 2, device="cuda:0")
+    mu, sg = torch.zeros(2, 2, device="cuda:0"), torch.ones(2, 2, device="cuda:0")
+    dst = torch.repeat_interleave(torch.arange(g.n, device="cuda:0"), (g.row_ptr[1:] - g.row_ptr[:-1]).long())
+    w = torch.exp(-0.5 * (ps.double() ** 2).sum(1))
+    for f in (16, 64):
+        x = torch.randn(g.n, 2, f, device="cuda:0")
+        got = gmm_native.gmmconv(g.row_ptr, g.col_ind, x, ps[pos].contiguous(), mu, sg, sum_kernels=True, own_order=True)
+        ref = torch.zeros(g.n, f, dtype=torch.float64, device="cuda:0").index_add_(0, dst, w[:, None] * x.sum(1).double()[g.col_ind.long()])
+        mag = torch.zeros(g.n, f, dtype=torch.float64, device="cuda:0").index_add_(0, dst, w[:, None] * x.abs().sum(1).double()[g.col_ind.long()])
+        assert bool(((got.double() - ref).abs() <= 64 * 2.0 ** -24 * mag + 1e-30).all())      # chains of at most 64, exp's last bits
