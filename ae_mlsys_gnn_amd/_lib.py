@@ -273,6 +273,13 @@ def default_seg_len() -> int:
     return int(os.environ.get("FGNN_SEG_LEN", "0"))
 
 
+def flat_seg_len(n_edges) -> int:
+    """Entries at which the plain list of a skewed graph cuts a hub's row: one eight-thousandth of all (about a resident wave's share), between
+    256 and the usual 2048, so that no hub outlasts the rest (forward pass of 2 x 16 floats, 50 k nodes, 1 M entries: 71 us with 2048, 41
+    so; 169 k nodes, 2.3 M 88 / 62)."""
+    return max(256, min(2048, n_edges // 8192 // 64 * 64))
+
+
 _bucket_rule_cache: "collections.OrderedDict" = collections.OrderedDict()
 BUCKET_ROW_LEN = 64          # rows longer than this are the ones an XCD-aware schedule cuts by source bucket
 BUCKET_MIN_SHARE = 0.25      # ...and they must hold at least this share of the entries
@@ -322,12 +329,16 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
     n_cols: rows of the array the ids index, for the opt-in FGNN_VALIDATE check (None: only ids >= 0 is checked).
     own_order: a schedule of its own (never shared with the other kinds) whose position map was taken
     out (`edge_positions`): operators called with it take per-edge tensors in the schedule's order.
-    flat: the plain list in any case (rows too narrow for the cut by source bucket to pay), over the own-order entry order where the
-    per-edge tensors are in that."""
+    flat: the plain list on skewed graphs too (rows too narrow for the cut by source bucket to pay), over the own-order entry order
+    where the per-edge tensors are in that."""
     if seg_len is None:
         seg_len = default_seg_len()
-    if flat and not own_order:
-        idx_tensor = None
+    if flat and idx_tensor is not None and xcd_buckets_enabled(ptr_tensor, idx_tensor.numel()):
+        flat_len = seg_len or flat_seg_len(idx_tensor.numel())
+        if not own_order:
+            idx_tensor, seg_len = None, flat_len
+    else:
+        flat = False
     if idx_tensor is not None and not xcd_buckets_enabled(ptr_tensor, idx_tensor.numel()):
         idx_tensor = None
     min_deg = int(os.environ.get("FGNN_BUCKET_MIN_DEG", "0"))
@@ -343,10 +354,10 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
                             "tensors permuted by its result")
         _sched_cache.move_to_end(k)
         if flat and s.n_buckets > 0:
-            kf = k + ("flat",)
+            kf = k + ("flat", flat_len)
             f = _sched_cache.get(kf)
             if f is None or f.flat_of is not s:
-                f = _sched_cache[kf] = Schedule(ptr_tensor, seg_len, flat_of=s)
+                f = _sched_cache[kf] = Schedule(ptr_tensor, flat_len, flat_of=s)
                 while len(_sched_cache) > _SCHED_CACHE_MAX:
                     _sched_cache.popitem(last=False)
             _sched_cache.move_to_end(kf)

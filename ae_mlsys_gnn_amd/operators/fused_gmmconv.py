@@ -16,14 +16,15 @@ def _plain_list_for_summed_backward(n, e):
     return e < 64 * n
 
 
-def _flat_list(n, row, backward):
+def _flat_list(n, e, row, backward):
     """Whether a pass that gathers rows of `row` floats out of an [n, row] matrix takes the plain work list on skewed graphs too: rows
     narrower than a wave (which sums them batch by batch, so their length costs no precision) of a matrix that the eight L2s hold, or, in the
     backward, whose partial results are wider than what it gathers, twice that.  The cut by source bucket then has nothing to keep
     apart and only costs partial results (115 M edges, 233 k nodes, us, cut / plain: forward 16 x 2 floats, 30 MB 1590 / 1240, 48 floats, 45 MB
     2110 / 2280, 64 floats, 60 MB 2030 / 2430; backward of the sum, 16 floats 2630 / 1730, 64 floats, 60 MB 3750 / 2930; shared features, 32 floats
-    2880 / 1770, 88 floats, 82 MB 4120 / 4770)."""
-    return row <= 64 and row % 4 == 0 and 4 * n * row <= ((64 << 20) if backward else (32 << 20))
+    2880 / 1770, 88 floats, 82 MB 4120 / 4770; 500 k nodes, 7 M edges, 2 x 16 floats 140 / 127 and 217 / 205).  Under 4 M edges either is as
+    fast as often (169 k nodes, 2.3 M edges: 65 / 62, 68 / 78, 107 / 115)."""
+    return e >= (1 << 22) and row <= 64 and row % 4 == 0 and 4 * n * row <= ((64 << 20) if backward else (32 << 20))
 
 
 class gmm_native:
@@ -63,7 +64,7 @@ class gmm_native:
         out = torch.empty((n, f), dtype=torch.float32, device=node_feat.device) if sum_kernels else torch.empty_like(node_feat)
         gauss = torch.empty((e, k), dtype=torch.float32, device=node_feat.device) if want_gauss else None
         # own_order: pseudo (and gauss) are indexed by the schedule's entry order, pseudo_caller[edge_positions(rowptr, colind)]
-        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, k * f, False))
+        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, e, k * f, False))
         epilogue = bias is not None or residual is not None
         if epilogue:
             if not sum_kernels:
@@ -115,7 +116,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # own_order: pseudo, grad_pseudo (and permute) are indexed by the schedule's entry order (gmm_edge_positions(colptr, rowind, True))
         sched = schedule_for(colptr, idx_tensor=None if (sum_kernels and _plain_list_for_summed_backward(n, e)) else rowind, own_order=own_order, n_cols=n,
-                             flat=_flat_list(n, f if sum_kernels else k * f, True))
+                             flat=_flat_list(n, e, f if sum_kernels else k * f, True))
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, node_feat, pseudo, (pw, pb), mu, sigma, grad_out, int(sum_kernels), grad_feat, grad_pseudo,
                              grad_mu, grad_sigma, sched, dev)
         return grad_feat, grad_pseudo, grad_mu, grad_sigma
@@ -158,7 +159,7 @@ class gmm_native:
             raise FgnnError("gmmconv_shared: shape mismatch mu %s sigma %s pseudo %s for E=%d" % (
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), e))
         out = torch.empty((n, k, f), dtype=torch.float32, device=feat.device)
-        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, f, False))
+        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, e, f, False))
         with device_guard(feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), feat.device)
             if proj is not None:
@@ -196,7 +197,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # same work list as the summed backward, so that one CSC-side copy of own-order edge data serves both kinds of layer
         sched = schedule_for(colptr, idx_tensor=None if _plain_list_for_summed_backward(n, e) else rowind, own_order=own_order, n_cols=n,
-                             flat=_flat_list(n, k * f, True))
+                             flat=_flat_list(n, e, k * f, True))
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, feat, pseudo, (pw, pb), mu, sigma, grad_out, 2, parts, grad_pseudo, grad_mu, grad_sigma, sched,
                              dev)
         return parts.sum(1), grad_pseudo, grad_mu, grad_sigma

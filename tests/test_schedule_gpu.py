@@ -175,10 +175,12 @@ def test_native_calls_follow_the_current_stream(monkeypatch, private_names):
     assert torch.cuda.current_device() == dev.index
 
 
-def test_flat_list_over_bucketed_order():
+def test_flat_list_over_bucketed_order(monkeypatch):
     """The plain list over an XCD-aware schedule's entry order: same operators, same per-edge order, its own cuts; positions stay put."""
     from ae_mlsys_gnn_amd import _lib
-    from ae_mlsys_gnn_amd.operators.fused_gmmconv import gmm_native
+    from ae_mlsys_gnn_amd.operators import fused_gmmconv
+    gmm_native = fused_gmmconv.gmm_native
+    monkeypatch.setattr(fused_gmmconv, "_flat_list", lambda n, e, row, backward: row <= 64)         # the rule's sizes are too large for a test
     g = graphs.rmat_graph(3000, 400000, seed=3).to("cuda:0")
     base = _lib.Schedule(g.row_ptr, 0, g.col_ind, 0)
     if base.n_buckets == 0:
@@ -199,6 +201,8 @@ def test_flat_list_over_bucketed_order():
     mu, sg = torch.zeros(2, 2, device="cuda:0"), torch.ones(2, 2, device="cuda:0")
     dst = torch.repeat_interleave(torch.arange(g.n, device="cuda:0"), (g.row_ptr[1:] - g.row_ptr[:-1]).long())
     w = torch.exp(-0.5 * (ps.double() ** 2).sum(1))
+    assert _lib.schedule_for(g.row_ptr, idx_tensor=g.col_ind, own_order=True, flat=True).n_buckets == 0
+    assert _lib.schedule_for(g.row_ptr, idx_tensor=g.col_ind, own_order=True).n_buckets > 0
     for f in (16, 64):
         x = torch.randn(g.n, 2, f, device="cuda:0")
         got = gmm_native.gmmconv(g.row_ptr, g.col_ind, x, ps[pos].contiguous(), mu, sg, sum_kernels=True, own_order=True)
