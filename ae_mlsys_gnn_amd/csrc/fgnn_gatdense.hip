@@ -1,4 +1,5 @@
-// The dense side of a GAT layer around its one large product (feat @ W, which stays a library GEMM): the score weights folded out
+// The dense side of a GAT layer around its one large product (feat @ W: fgnn_tall.hip where the scores come out of it as columns, a
+// library product and gat_score_kernel elsewhere): the score weights folded out
 // of W and the attention vectors, the scores of all nodes, and the gradients unfolded again
 // (layers/gatconv_layer.py:50-55 of the reference: h = feat @ W, attn_row = (attn_l * h).sum(-1), attn_col = (attn_r * h).sum(-1)).
 // The scores are taken as feat @ ((W * attn).sum(-1)), the same sums in another order: `feat` is read instead of the

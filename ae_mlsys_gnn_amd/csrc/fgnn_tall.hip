@@ -44,6 +44,9 @@ __device__ __forceinline__ tl_f4 tl_load4(const float *__restrict__ q)
 // consecutive columns of one row (row lane % 16, columns 16 t + 4 (lane / 16) ..) and stores them as 128 bits; x goes
 // straight from memory to registers, four consecutive floats per lane, 64 columns ahead of their use.  Column ranges of the same rows
 // run side by side on one XCD, where the second finds x in the L2.
+// Bound by the matrix unit (155 TFLOP/s in these instructions alone; the operand reads and the x loads beside them leave 100-110).
+// us, library products and what stood around them / this kernel: 2.4 M x 100 -> 256 + 16 scores 1474 + 260 / 1285 (104 TFLOP/s), 256 -> 48 + 2
+// 698 + 590 / 746 (3.4 TB/s of x), 2.4 M gradients 48 + 2 -> 256 1061 + 210 / 835; 169 k x 128 -> 256 + 8 125 + 28 / 152, 384 -> 64 178 / 107.
 template <int NT, int VEC, bool HIN>
 __global__ __launch_bounds__(64 * TL_WAVES(NT)) void tall_product_kernel(TallP p)
 {
@@ -306,14 +309,18 @@ struct TallR {
 #define TR_WAVES 16
 #define TR_TPB (64 * TR_WAVES)
 #define TR_SLOTS 5
+#define TR_MAX_U 9                          // tiles a wave holds, a number that tl_tiles knows
 #define TR_TILE(R) ((R) * 16 + 16)          // floats an operand tile of R rows takes in LDS; the 16 spread the tiles' rows over the banks
 
 // A workgroup sums the whole result over a range of rows; its waves hold U 16 x 16 tiles of it each, dealt out one after the other, so
-// that 7 x 17 tiles keep 16 waves busy as well as 8 x 16 do (ROW: one tile of x and all U of g per wave).  R rows of both operands
+// that 7 x 17 tiles keep 16 waves busy as well as 8 x 16 do.  R rows of both operands
 // are staged in LDS tile by tile (read from memory once, 128 bits per thread where the rows allow it, one stage ahead): the operand of
 // four rows is then 64 consecutive floats, at an offset known when compiling, and an instruction costs two LDS reads and
 // no vector arithmetic, which would take its time from the matrix unit (a vector instruction beside every matrix instruction: 11 % less).
-template <int U, int R, bool ROW>
+// us, batched library product over chunks of rows, its sum and the stacked operand / this kernel and its sum: 2.4 M x 256, 48 + 2
+// 638 + 460 / 918 (bound by reading x: 3.2 TB/s), 169 k x 256, 40 + 2 82 + 30 / 76, 33 k x 64, 128 32 / 23.  A second stage of LDS, so that rows are stored
+// while the others are multiplied, spilled registers and was slower (2.4 M x 100, 272: 1.59 -> 1.65 to 2.2 ms).
+template <int U, int R>
 __global__ __launch_bounds__(TR_TPB) void tall_reduce_kernel(TallR p)
 {
     extern __shared__ float sm[];
@@ -366,16 +373,17 @@ __global__ __launch_bounds__(TR_TPB) void tall_reduce_kernel(TallR p)
         }
     };
     // operands of the wave's tiles (wave-uniform); past the last tile the last one again, results unused
-    const int t0 = ROW ? wave * p.tb : wave * U;
+    const int t0 = wave * U;
     int at[U], bt[U];
-    const float *ap[ROW ? 1 : U], *bp[ROW ? 1 : U];
+    const float *ap[U], *bp[U];
     tl_f4 acc[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int t = fg_uni(min(t0 + u, p.tiles - 1));
-        at[u] = ROW ? min(wave, p.ta - 1) : t / p.tb;
-        bt[u] = ROW ? u : t % p.tb;
-        if (!ROW || u == 0) { ap[u] = sm + at[u] * TR_TILE(R) + lane; bp[u] = gs + bt[u] * TR_TILE(R) + lane; }
+        at[u] = t / p.tb;
+        bt[u] = t % p.tb;
+        ap[u] = sm + at[u] * TR_TILE(R) + lane;
+        bp[u] = gs + bt[u] * TR_TILE(R) + lane;
         acc[u] = tl_f4{0.f, 0.f, 0.f, 0.f};
     }
     const bool busy = t0 < p.tiles;
@@ -402,15 +410,15 @@ __global__ __launch_bounds__(TR_TPB) void tall_reduce_kernel(TallR p)
 #pragma unroll
                 for (int u = 0; u < G; ++u) {
                     if (u0 + u >= U) continue;
-                    if (!ROW || u == 0) { const float *a = ap[ROW ? 0 : u0 + u]; xv[0][u] = a[64 * s]; xv[1][u] = a[64 * s + 64]; }
-                    const float *b = ROW ? bp[0] + (u0 + u) * TR_TILE(R) : bp[ROW ? 0 : u0 + u];
+                    const float *a = ap[u0 + u], *b = bp[u0 + u];
+                    xv[0][u] = a[64 * s]; xv[1][u] = a[64 * s + 64];
                     gv[0][u] = b[64 * s]; gv[1][u] = b[64 * s + 64];
                 }
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int u = 0; u < G; ++u)
-                        if (u0 + u < U) acc[u0 + u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[h][ROW ? 0 : u], gv[h][u], acc[u0 + u], 0, 0, 0);
+                        if (u0 + u < U) acc[u0 + u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[h][u], gv[h][u], acc[u0 + u], 0, 0, 0);
                 if (U > 4) __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -419,7 +427,7 @@ __global__ __launch_bounds__(TR_TPB) void tall_reduce_kernel(TallR p)
     float *out = p.part + (size_t)blockIdx.x * p.ka * kb2;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        if (t0 + u >= p.tiles || (ROW && u >= p.tb)) continue;
+        if (t0 + u >= p.tiles) continue;
         const bool extra = p.h > 0 && bt[u] == p.tb - 1;
         const int j = extra ? r16 : 16 * bt[u] + r16;
         if (extra ? j >= 2 * p.h : j >= p.kb) continue;
@@ -450,7 +458,7 @@ __global__ __launch_bounds__(256) void tall_reduce_sum_kernel(int64_t total, int
     c[i] = (float)s;
 }
 
-struct TallRPlan { int ta, tb, tiles, u, R, rpp, blocks; bool row; int64_t rows; size_t lds; };
+struct TallRPlan { int ta, tb, tiles, u, R, rpp, blocks; int64_t rows; size_t lds; };
 static bool tall_reduce_plan(int64_t n, int ka, int kb, int h, TallRPlan *pl)
 {
     const int cols = (ka + 3) / 4 + (kb + 3) / 4;
@@ -458,13 +466,11 @@ static bool tall_reduce_plan(int64_t n, int ka, int kb, int h, TallRPlan *pl)
     pl->ta = (ka + 15) / 16;
     pl->tb = (kb + 15) / 16 + (h ? 1 : 0);
     pl->tiles = pl->ta * pl->tb;
-    pl->row = pl->tiles > 9 * TR_WAVES;
-    if (pl->row && (pl->ta > TR_WAVES || pl->tb > 18)) return false;
-    pl->u = pl->row ? std::max(12, tl_tiles(pl->tb)) : tl_tiles((pl->tiles + TR_WAVES - 1) / TR_WAVES);
+    if (pl->tiles > TR_MAX_U * TR_WAVES) return false;
+    pl->u = tl_tiles((pl->tiles + TR_WAVES - 1) / TR_WAVES);
     pl->rpp = std::min(TR_TPB / cols, 32);                                   // at least 4: TR_SLOTS passes take R rows
     pl->R = pl->rpp * TR_SLOTS >= 32 ? 32 : 16;
-    // ROW waves read u tiles of g also where there are fewer
-    pl->lds = (size_t)(pl->ta + (pl->row ? pl->u : pl->tb)) * TR_TILE(pl->R) * sizeof(float);
+    pl->lds = (size_t)(pl->ta + pl->tb) * TR_TILE(pl->R) * sizeof(float);
     if (pl->lds > TL_LDS_MAX) return false;
     const int64_t want = std::min<int64_t>(256, (n + 255) / 256);
     const int64_t rows = (n + want - 1) / std::max<int64_t>(want, 1);
@@ -496,9 +502,10 @@ extern "C" int fgnn_tall_reduce(int64_t n, int ka, int kb, const float *x, int64
     p.ta = pl.ta; p.tb = pl.tb; p.tiles = pl.tiles; p.rpp = pl.rpp; p.part = (float *)workspace;
     hipStream_t st = (hipStream_t)stream;
     tl_dispatch_tiles(pl.u, [&]<int U>() {
-        constexpr bool ROW = U > 9;
-        if (pl.R == 32) hipLaunchKernelGGL((tall_reduce_kernel<U, 32, ROW>), dim3((unsigned)pl.blocks), dim3(TR_TPB), pl.lds, st, p);
-        else hipLaunchKernelGGL((tall_reduce_kernel<U, 16, ROW>), dim3((unsigned)pl.blocks), dim3(TR_TPB), pl.lds, st, p);
+        if constexpr (U <= TR_MAX_U) {
+            if (pl.R == 32) hipLaunchKernelGGL((tall_reduce_kernel<U, 32>), dim3((unsigned)pl.blocks), dim3(TR_TPB), pl.lds, st, p);
+            else hipLaunchKernelGGL((tall_reduce_kernel<U, 16>), dim3((unsigned)pl.blocks), dim3(TR_TPB), pl.lds, st, p);
+        }
     });
     int rc = fgnn_launch_status("tall_reduce_kernel");
     if (rc) return rc;

@@ -3,7 +3,7 @@
 The weight gradient of such a map, x^T @ g, reduces over the rows.  As one GEMM that reduction
 lands on the few workgroups the small output has tiles for (117 us for 32,768 rows, 64 x 64; 4.6 ms
 for 2.4 M rows, 100 x 272); cut into chunks of rows it is a batched matmul over all of them plus a
-small sum (26 us and 1.5 ms)."""
+small sum (26 us and 1.5 ms), or one kernel (operators/tall.py) where that is faster."""
 from __future__ import annotations
 
 import torch

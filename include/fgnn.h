@@ -290,10 +290,10 @@ int fgnn_gat_unfold_grads(int fin, int H, int F, int pad, const float *W, const 
 /* Dense products over very many rows, in fp32 on the matrix instructions.
  * fgnn_tall_product: y [n, m] = x [n, k] @ B [k, m] (+ bias [m]); B[r][c] at b[r*ldb + c], or at b[c*ldb + r] when b_transposed.
  * With hin > 0, xe0 and xe1 [n, hin] are the input columns k .. k+2*hin; with hout > 0, ye0 and ye1 [n, hout] receive the output
- * columns m .. m+2*hout (B has those rows and columns too).  At most 18 tiles of 16 output columns, the extra ones a
- * tile of their own; hin, hout <= 8; y 16-byte aligned when ldy is a multiple of 4.
- * fgnn_tall_reduce: c [ka, kb + 2h] = x [n, ka]^T @ [g [n, kb] | ge0 [n, h] | ge1 [n, h]], deterministic; workspace_bytes is 0 for
- * shapes it does not take. */
+ * columns m .. m+2*hout (B has those rows and columns too).  Sixteen columns of B have to fit the 160 KB of LDS: k up to 2560, 2544 with
+ * hin > 0; hin, hout <= 8; y 16-byte aligned when ldy is a multiple of 4.
+ * fgnn_tall_reduce: c [ka, kb + 2h] = x [n, ka]^T @ [g [n, kb] | ge0 [n, h] | ge1 [n, h]], deterministic; at most 144 tiles of 16 x 16
+ * in c (the extra columns take a row of tiles of their own) and 1024 columns of x and g; workspace_bytes is 0 for other shapes. */
 int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_t ldx, const float *b, int64_t ldb, int b_transposed,
                       const float *bias, float *y, int64_t ldy, int hin, const float *xe0, const float *xe1, int hout,
                       float *ye0, float *ye1, void *stream);
