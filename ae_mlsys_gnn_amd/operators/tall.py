@@ -14,30 +14,36 @@ def _plain(*ts):
 
 def product_wanted(x, b, k, m, h_in=0, h_out=0):
     """Where tall_product of x [n, k] with the [k + 2 h_in, m + 2 h_out] matrix b is the faster form (us, library / own).  It reads x and
-    writes the result once at 100-110 TFLOP/s; the library's products take 19 at least and reach 60-85 TFLOP/s on thin shapes, 150 on large
-    ones.  Up to 8192 weights: 4 k rows x 64 -> 64 20 / 9, 33 k x 64 -> 128 19 / 14, 170 k 62 / 44; beyond that on many rows
-    only (65 k x 64 -> 192 25 / 30, 128 -> 128 26 / 36; 170 k x 384 -> 64 181 / 108, 500 k x 128 -> 128 213 / 171), with more than 192
-    columns on more still (170 k x 64 -> 256 72 / 83, 1 M 423 / 360).  With extra columns the library needs a score kernel (10 to 600) or a
-    stacked operand besides: 8 k x 128 -> 144 20 + 10 / 17, 233 k x 256 -> 272 334 + 70 / 355, 2.4 M x 100 -> 272 1474 + 260 / 1310; 20 k rows of
-    gradients 272 -> 256 33 + 8 / 53, 2.4 M 50 -> 256 1030 + 250 / 840."""
+    writes the result once at 100-110 TFLOP/s, and every workgroup lays b out in LDS first, 5 to 30 us.  The library reaches 60-85 TFLOP/s on
+    thin shapes and more at the sizes it is tuned for, takes 19 of the host at least, and needs a score kernel (10 to 600) or a stacked
+    operand besides for extra columns.
+    No extra columns.  Up to 49 k rows both are within the library's host time: 4 k x 64 -> 64 19 / 8 (5 / 7 of the GPU), 33 k x 64 -> 128 19 / 14
+    (11 / 13), 33 k x 256 -> 128 22 / 31.  Up to 131 k rows: 65 k x 16 -> 64 11 / 8, 64 -> 64 12 / 13, 64 -> 128 18 / 22, 128 -> 128 25 / 31.  Above:
+    169 k x 64 -> 64 48 / 27, 64 -> 128 62 / 44, 128 -> 128 70 / 70, 384 -> 64 171 / 98, 64 -> 256 72 / 77, 128 -> 256 116 / 128; 500 k x 128 -> 128
+    213 / 178; 1 M x 64 -> 256 423 / 360 (at powers of two the library is the better one up to 524 k: 262 k x 128 -> 128 88 / 93).
+    With them, scores included: 16 k x 64 -> 64 + 8 9 / 8, 256 -> 48 + 2 15 / 17, 128 -> 256 + 8 20 / 35; 65 k 18 / 15, 34 / 30, 56 / 57; 169 k 60 / 33,
+    85 / 68, 142 / 138; 1 M 231 / 137, 521 / 323, 761 / 601.  Gradients, stacking included: 16 k x 64 + 8 -> 64 11 / 8, 48 + 2 -> 256 16 / 18, 256 + 8 ->
+    128 26 / 34; 65 k 26 / 17, 41 / 31, 72 / 65; 1 M 401 / 142, 628 / 348, 1216 / 598."""
     n = x.shape[0]
-    if h_out or (h_in and n >= 65536):
-        most = 73728
-    elif h_in:
-        most = 16384
+    if h_out or h_in:
+        most = 73728 if n >= 65536 else 20480 if h_out else 16384
+    elif n < 131072:
+        most = 8192 if n <= 49152 else 4096
     else:
-        most = 8192 if n < 131072 or (m > 192 and n < (1 << 19)) else 32768
+        most = 8192 if m > 192 and n < (1 << 19) else 32768
     return (n > 0 and k > 0 and m > 0 and max(h_in, h_out) <= 8 and (k + 2 * h_in) * (m + 2 * h_out) <= most
             and k <= 1024 and m <= 512 and _plain(x, b) and (not h_in or (k % 4 == 0 and x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0)))
 
 
 def reduce_wanted(x, g, h=0):
     """Where tall_reduce of x [n, a] and g [n, b] (and 2h extra columns) is the faster form: one launch and a small sum for a batched product
-    over chunks, a sum, a remainder, and a stacked operand where there are extra columns (us, library / own: 33 k x 64, 128 32 / 23; 169 k x
-    256, 42 98 + 30 / 80; 2.4 M x 256, 50 880 + 250 / 960; without extra columns, 233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116)."""
+    over chunks, a sum, a remainder, and a stacked operand where there are extra columns (us of the GPU, library / own).  33 k x 64, 128 32 / 23;
+    extra columns: 4 k x 64, 64 + 8 25 / 17, 256, 48 + 2 21 / 30, 128, 256 + 8 24 / 52; 65 k 32 / 21, 34 / 36, 86 / 63; 169 k 69 / 40, 100 / 73, 229 /
+    135; 1 M 341 / 184, 444 / 375, 1153 / 684.  On few rows the sum over the workgroups' results is what takes the time, so those are small
+    ones there.  Without extra columns 233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116."""
     n, a, b = x.shape[0], x.shape[1], g.shape[1]
     tiles = -(-a // 16) * (-(-b // 16) + (h > 0))
-    return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= 144 and (h > 0 or n <= 131072) and _plain(x, g)
+    return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= (144 if n > 49152 else 36) and (h > 0 or n <= 131072) and _plain(x, g)
             and all(t.shape[1] % 4 == 0 and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (x, g)))
 
 
