@@ -69,7 +69,13 @@ class _GMMBase(nn.Module):
                 pseudo = apply(pseudo)
             proj = None
         if self._aggregate_first(feat):
-            return self._finish(self._forward_aggregate_first(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj), feat)
+            # without a residual the bias is added in the store of the product behind the aggregation (autocast and other types: as a sum of
+            # its own, whose type is the wider one)
+            bias = self.bias
+            if bias is not None and (self.res_fc is not None or bias.dtype != th.float32 or th.is_autocast_enabled("cuda")):
+                bias = None
+            rst = self._forward_aggregate_first(rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj, bias)
+            return rst if bias is not None else self._finish(rst, feat)
         node_feat = tall_linear(feat, self.fc.weight).view(-1, self._n_kernels, self._out_feats)    # = self.fc(feat)
         pad = (-self._out_feats) % 4
         if pad:         # zero columns up to a multiple of 4: the operator then takes its 128-bit row layout
@@ -123,8 +129,8 @@ class _GMMBase(nn.Module):
         return (type(self)._op is GmmConvFuseSum and feat.dim() == 2 and fin < k * self._out_feats
                 and gmm_native.shared_supported(k, fin))
 
-    def _forward_aggregate_first(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj=None):
-        """sum_k (sum_p w[p,k] feat[col(p),:]) @ W_k: the reference's sum over k of the aggregated fc(feat)[:,k,:]
+    def _forward_aggregate_first(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc, own_order, proj=None, bias=None):
+        """sum_k (sum_p w[p,k] feat[col(p),:]) @ W_k (+ bias): the reference's sum over k of the aggregated fc(feat)[:,k,:]
         (layers/gmmconv_layer.py:67-69) with the two linear steps exchanged."""
         k, fin, fout = self._n_kernels, feat.shape[1], self._out_feats
         feat = feat.contiguous()
@@ -135,20 +141,20 @@ class _GMMBase(nn.Module):
         w = lambda: self.fc.weight.view(k, fout, fin).permute(1, 0, 2).reshape(fout, k * fin)       # [out, K*in]: rst = agg.view(N, K*in) @ w^T
         if proj is not None:
             agg = GmmProjectedTwoOrders(rowptr, colind, colptr, rowind, feat, pseudo, pseudo_csc, proj.weight, proj.bias, self.mu, self.inv_sigma, own_order)
-            return tall_linear(agg.view(-1, k * fin), w())
+            return tall_linear(agg.view(-1, k * fin), w(), bias)
         # without a gradient for what is aggregated (frozen Gaussians, constant coordinates and input) the weight's is one product with the
         # aggregate, and no pass over the edges
         through_edges = any(t.requires_grad for t in (feat, pseudo_csc if two else pseudo, self.mu, self.inv_sigma))
         if (th.is_grad_enabled() and through_edges and (two or not own_order)
                 and project_in_backward(k, fin, fout, feat.requires_grad, feat.shape[0], colind.numel())):
             return GmmAggregateLinear(rowptr, colind, colptr, rowind, None if two else permute, feat, pseudo.detach() if two else pseudo, pseudo_csc,
-                                      self.mu, self.inv_sigma, self.fc.weight, own_order=own_order)
+                                      self.mu, self.inv_sigma, self.fc.weight, own_order=own_order, bias=bias)
         if two or own_order:
             agg = GmmAggregateTwoOrders(rowptr, colind, colptr, rowind, feat, pseudo.detach(), pseudo_csc, self.mu, self.inv_sigma,
                                         own_order=own_order)
         else:
             agg = GmmAggregate(rowptr, colind, colptr, rowind, permute, feat, pseudo, self.mu, self.inv_sigma)
-        return tall_linear(agg.view(-1, k * fin), w())
+        return tall_linear(agg.view(-1, k * fin), w(), bias)
 
 
 class GMMConv(_GMMBase):

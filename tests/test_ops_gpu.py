@@ -413,6 +413,35 @@ def test_gmm_aggregate_linear(fin, fout, k, dim, form, input_grad):
         assert_close_sum(got.grad, want.grad, s[key], "grad " + name, c=c)
 
 
+# the product's own kernel and the library's (few rows, many weights), with and without the pass that projects in the backward, padded width
+@pytest.mark.parametrize("fin,fout,k,dim", [(16, 24, 2, 1), (64, 24, 3, 1), (128, 64, 3, 2), (48, 31, 3, 2)])
+@pytest.mark.parametrize("two_orders", [False, True])
+def test_gmm_layer_bias_in_the_product(fin, fout, k, dim, two_orders):
+    """Without a residual the bias is added where the product behind the aggregation is stored: bit for bit the sum afterwards, and the same
+    gradients; the bias' own is a column sum (n terms in chunks and chunk sums, at most n rounded additions)."""
+    from ae_mlsys_gnn_amd.layers import GMMConv
+    g = graphs.add_csc_torch(graphs.rmat_graph(700, 9000, seed=4)).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(fin + fout)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    layer = GMMConv(fin, fout, dim=dim, n_kernels=k, residual=False, bias=True).to(DEV)
+    feat, pseudo, go, bias = rnd(g.n, fin), rnd(g.n_edges, dim), rnd(g.n, fout), rnd(fout)
+    assert layer._aggregate_first(feat)
+
+    def run(b):
+        with torch.no_grad():
+            layer.bias.copy_(b)
+        layer.zero_grad()
+        x = feat.clone().requires_grad_(True)
+        extra = {"pseudo_csc": pseudo[g.permute.long()].contiguous().requires_grad_(True)} if two_orders else {}
+        out = layer(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, x, pseudo, **extra)
+        out.backward(go)
+        return out.detach(), [t.grad.clone() for t in (x, layer.fc.weight, layer.mu, layer.inv_sigma)], layer.bias.grad.clone()
+    base, grads, _ = run(torch.zeros_like(bias))
+    out, grads_b, gb = run(bias)
+    assert torch.equal(out, base + bias) and all(torch.equal(p, q) for p, q in zip(grads, grads_b))
+    assert bool(((gb.double() - go.double().sum(0)).abs() <= g.n * 2.0 ** -24 * go.double().abs().sum(0)).all())
+
+
 @pytest.mark.parametrize("fin,fout,k", [(256, 64, 4), (256, 100, 3)])
 def test_gmm_aggregate_linear_precision(fin, fout, k):
     """The coordinates' gradient is <g_i, (x @ W_k^T)_j> per edge and kernel.  Its error in the 2-norm comes from the product's chain of
