@@ -78,6 +78,8 @@ _SIGNATURES = {
     "fgnn_gmm_backward_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int, c_int]),
     "fgnn_gmm_backward": (c_int, [c_int, c_int64, c_int, c_int, c_int] + [c_void_p] * 8 + [c_int] + [c_void_p] * 4
                           + [c_void_p, c_void_p, c_size_t, c_void_p]),
+    "fgnn_column_sum_workspace_bytes": (c_size_t, [c_int64, c_int]),
+    "fgnn_column_sum": (c_int, [c_int64, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_size_t, c_void_p]),
     "fgnn_gmm_forward_projected": (c_int, [c_int, c_int64, c_int, c_int, c_int] + [c_void_p] * 13 + [c_int] + [c_void_p, c_void_p, c_size_t, c_void_p]),
     "fgnn_gmm_backward_projected_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int, c_int]),
     "fgnn_gmm_backward_projected": (c_int, [c_int, c_int64, c_int, c_int, c_int] + [c_void_p] * 10 + [c_int] + [c_void_p] * 5

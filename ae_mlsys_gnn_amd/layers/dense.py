@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import torch
 
-from ..operators.tall import product_wanted, reduce_wanted, tall_product, tall_reduce
+from ..operators.tall import product_wanted, reduce_wanted, sum_wanted, tall_product, tall_reduce, tall_sum
 
 
 def reduce_over_rows(x, g):
@@ -31,7 +31,10 @@ def column_sum(g):
     """g.sum(0) for tall g [N, c].  torch's reduction over the rows falls off a cliff when c is not a
     multiple of 4 (19 ms for 2.4 M x 47, 1.2 ms for 233 k x 41, against 40 us and 14 us for 16
     columns): the rows are cut into chunks that are summed side by side, then the chunk sums are added
-    (0.15 ms and 0.04 ms).  Narrow, aligned, moderately sized inputs keep the single reduction."""
+    (0.15 ms and 0.04 ms).  Narrow, aligned, moderately sized inputs keep the single reduction, large ones take a
+    kernel of their own (operators/tall.py)."""
+    if not torch.is_grad_enabled() and sum_wanted(g):
+        return tall_sum(g)
     n, c = g.shape
     chunks = min(256, n // 2048)
     if chunks < 2 or (c % 4 == 0 and n * c < (1 << 25)):

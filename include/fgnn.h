@@ -300,6 +300,10 @@ int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_t ldx, cons
 size_t fgnn_tall_reduce_workspace_bytes(int64_t n, int ka, int kb, int h);
 int fgnn_tall_reduce(int64_t n, int ka, int kb, const float *x, int64_t ldx, const float *g, int64_t ldg, int h,
                      const float *ge0, const float *ge1, float *c, void *workspace, size_t workspace_bytes, void *stream);
+/* out [c] = the column sums of x [n, c] (row stride ldx), c <= 1024, deterministic. */
+size_t fgnn_column_sum_workspace_bytes(int64_t n, int c);
+int fgnn_column_sum(int64_t n, int c, const float *x, int64_t ldx, float *out, void *workspace, size_t workspace_bytes,
+                    void *stream);
 
 /* k-nearest-neighbour graph of batched point clouds, the input of fgnn_edgeconv_forward: points
  * [n_clouds*P, D]; src_ind [n_clouds*P*k] gets, for every point, the global ids of the k nearest

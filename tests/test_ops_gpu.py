@@ -1744,6 +1744,24 @@ def test_tall_reduce(n, a, b, h):
     assert torch.equal(one, tall_reduce(dx, dg, de))                     # fixed order of summation
 
 
+# one column to one per thread, whole quads and odd widths, rows around a workgroup's share and a pass of its threads
+@pytest.mark.parametrize("n,c", [(1, 1), (255, 3), (257, 4), (300, 1024), (1023, 1023), (4097, 41), (70001, 64), (140000, 47), (131072, 7)])
+def test_tall_sum(n, c):
+    from ae_mlsys_gnn_amd.layers.dense import column_sum
+    from ae_mlsys_gnn_amd.operators.tall import tall_sum
+    x = torch.randn(n, c, generator=torch.Generator().manual_seed(n + c))
+    ref = x.double().sum(0)
+    tol = 2.0 ** -23 * x.double().abs().sum(0)          # summed in 64 bits; at most 256 partial sums and their total are rounded once each
+    dx = x.cuda()
+    wide = torch.full((n, c + 1), float("nan"), device="cuda")
+    wide[:, :c] = dx
+    for got in (tall_sum(dx), tall_sum(wide[:, :c]), column_sum(dx) if n >= 131072 else tall_sum(dx)):
+        assert got.shape == ref.shape and bool(((got.cpu().double() - ref).abs() <= tol).all())
+    dx[0, 0] = float("inf")
+    got = tall_sum(dx)
+    assert bool(torch.isinf(got[0])) and bool(((got[1:].cpu().double() - ref[1:]).abs() <= tol[1:]).all())
+
+
 # ---------------------------------------------------------------- GMMConv on projected coordinates
 
 def _monet_layer_f64(g, feat, raw, layer, proj):
