@@ -65,7 +65,7 @@ class _TallLinear(torch.autograd.Function):
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
-        if product_wanted(x, weight, x.shape[1], weight.shape[0]) and (bias is None or (bias.is_cuda and bias.dtype == torch.float32)):
+        if product_wanted(x, weight, transposed=True, bias=bias):
             return tall_product(x, weight, transposed=True, bias=bias)
         y = torch.matmul(x, weight.t())
         return y if bias is None else y.add_(bias)
@@ -77,7 +77,7 @@ class _TallLinear(torch.autograd.Function):
         gx = gw = None
         if ctx.needs_input_grad[0]:
             # where a graph of the gradients is wanted, the operation that records one
-            own = not torch.is_grad_enabled() and product_wanted(g, weight, *weight.shape)
+            own = not torch.is_grad_enabled() and product_wanted(g, weight)
             gx = tall_product(g, weight) if own else torch.matmul(g, weight)
         if ctx.needs_input_grad[1]:
             gw = reduce_over_rows(g, x)

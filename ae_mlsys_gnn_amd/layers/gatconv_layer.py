@@ -56,7 +56,7 @@ class _ProjectScores(torch.autograd.Function):
     @staticmethod
     def forward(ctx, feat, W, attn_l, attn_r, pad):
         _, hh, ff = attn_l.shape
-        own = product_wanted(feat, W, feat.shape[1], hh * (ff + pad), h_out=hh)
+        own = product_wanted(feat, W, h_out=hh, m=hh * (ff + pad))
         score_wt, w_proj, w_all = gat_dense_native.fold(W, attn_l, attn_r, pad, own or ctx.needs_input_grad[0])
         if own:                                 # the scores are columns of the same product
             h, row, col = tall_product(feat, w_all, extra_out=hh)
@@ -84,7 +84,7 @@ class _ProjectScores(torch.autograd.Function):
         if not recorded and dh is not None and drow is not None and dcol is not None and drow.dtype == dcol.dtype == torch.float32:
             dh2 = dh.reshape(n, hfp)
             if ctx.needs_input_grad[0]:
-                own = product_wanted(dh2, w_all, hfp, feat.shape[1], h_in=hh) and reduce_wanted(feat, dh2, hh)
+                own = product_wanted(dh2, w_all, transposed=True, h_in=hh) and reduce_wanted(feat, dh2, hh)
             else:       # on many rows two library reductions are as fast (2.4 M x 100, 256 + 16 columns: 1.45 / 1.55 ms)
                 own = n <= 262144 and reduce_wanted(feat, dh2, hh)
         if own:                                 # nothing is stacked

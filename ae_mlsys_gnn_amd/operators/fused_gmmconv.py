@@ -497,7 +497,7 @@ class GmmAggregateLinearFunction(torch.autograd.Function):
         ctx.save_for_backward(colptr, rowind, None if ctx.two_orders else permute, feat, pseudo_csc if ctx.two_orders else pseudo, mu, sigma, weight,
                               rowptr, colind, agg if ctx.two_orders else None)
         agg = agg.view(-1, k * fin)
-        if product_wanted(agg, w, k * fin, fout) and (bias is None or (bias.is_cuda and bias.dtype == torch.float32)):
+        if product_wanted(agg, w, transposed=True, bias=bias):
             return tall_product(agg, w, transposed=True, bias=bias)
         y = torch.matmul(agg, w.t())
         return y if bias is None else y + bias

@@ -3,17 +3,29 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import as_f32, check, device_guard, lib, ptr, stream_ptr, workspace
+from .._lib import FgnnError, as_f32, check, device_guard, lib, ptr, stream_ptr, workspace
+
+
+def _matrices(*ts):
+    """fp32 matrices on one GPU with unit column stride."""
+    return all(t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] for t in ts) \
+        and all(t.device == ts[0].device for t in ts)
 
 
 def _plain(*ts):
-    """fp32 matrices on one GPU with unit column stride, outside autocast (which asks for another precision)."""
-    return all(t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] for t in ts) \
-        and all(t.device == ts[0].device for t in ts) and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
+    """Such matrices outside autocast (which asks for another precision)."""
+    return _matrices(*ts) and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
 
 
-def product_wanted(x, b, k, m, h_in=0, h_out=0):
-    """Where tall_product of x [n, k] with the [k + 2 h_in, m + 2 h_out] matrix b is the faster form (us, library / own).  It reads x and
+def _fits(x, k, m, bias=None):
+    """Whether x has k columns and bias, where there is one, m floats beside x: the kernels read by these sizes alone."""
+    return x.dim() == 2 and x.shape[1] == k and (bias is None or (bias.shape == (m,) and bias.dtype == torch.float32 and bias.device == x.device))
+
+
+def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None):
+    """Whether tall_product takes x [n, k] and the [k + 2 h_in, m + 2 h_out] matrix b (its transpose when `transposed`) and is the faster
+    form; what does not fit goes to the library, which says so.  m: the columns, where b [k, .] is only what the matrix is laid out from.
+    (us, library / own.)  It reads x and
     writes the result once at 100-110 TFLOP/s, and every workgroup lays b out in LDS first, 5 to 30 us.  The library reaches 60-85 TFLOP/s on
     thin shapes and more at the sizes it is tuned for, takes 19 of the host at least, and needs a score kernel (10 to 600) or a stacked
     operand besides for extra columns.
@@ -24,6 +36,13 @@ def product_wanted(x, b, k, m, h_in=0, h_out=0):
     With them, scores included: 16 k x 64 -> 64 + 8 9 / 8, 256 -> 48 + 2 15 / 17, 128 -> 256 + 8 20 / 35; 65 k 18 / 15, 34 / 30, 56 / 57; 169 k 60 / 33,
     85 / 68, 142 / 138; 1 M 231 / 137, 521 / 323, 761 / 601.  Gradients, stacking included: 16 k x 64 + 8 -> 64 11 / 8, 48 + 2 -> 256 16 / 18, 256 + 8 ->
     128 26 / 34; 65 k 26 / 17, 41 / 31, 72 / 65; 1 M 401 / 142, 628 / 348, 1216 / 598."""
+    if b.dim() != 2:
+        return False
+    k = b.shape[1 if transposed else 0] - 2 * h_in
+    if m is None:
+        m = b.shape[0 if transposed else 1] - 2 * h_out
+    if not _fits(x, k, m, bias):
+        return False
     n = x.shape[0]
     if h_out or h_in:
         most = 73728 if n >= 65536 else 20480 if h_out else 16384
@@ -41,19 +60,30 @@ def reduce_wanted(x, g, h=0):
     extra columns: 4 k x 64, 64 + 8 25 / 17, 256, 48 + 2 21 / 30, 128, 256 + 8 24 / 52; 65 k 32 / 21, 34 / 36, 86 / 63; 169 k 69 / 40, 100 / 73, 229 /
     135; 1 M 341 / 184, 444 / 375, 1153 / 684.  On few rows the sum over the workgroups' results is what takes the time, so those are small
     ones there.  Without extra columns 233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116."""
+    if x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
+        return False
     n, a, b = x.shape[0], x.shape[1], g.shape[1]
     tiles = -(-a // 16) * (-(-b // 16) + (h > 0))
     return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= (144 if n > 49152 else 36) and (h > 0 or n <= 131072) and _plain(x, g)
             and all(t.shape[1] % 4 == 0 and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (x, g)))
 
 
+def _columns(x, extra):
+    """Whether extra is None or two contiguous [n, h] arrays beside x [n, .]."""
+    return extra is None or all(t.is_contiguous() and t.dtype == torch.float32 and t.device == x.device and t.shape == (x.shape[0], extra[0].shape[1])
+                                for t in extra)
+
+
 def tall_product(x, b, *, transposed=False, bias=None, extra_in=None, extra_out=0):
     """x [n, k] @ b (b^T when `transposed`) (+ bias).  extra_in: two [n, h] arrays that follow x's columns; extra_out: h, the last 2h
     columns of the result are returned as two [n, h] arrays of their own."""
     n, k = x.shape
-    bias = None if bias is None else as_f32(bias)
     hin = 0 if extra_in is None else extra_in[0].shape[1]
     m = b.shape[0 if transposed else 1] - 2 * extra_out
+    if not _matrices(x, b) or m < 1 or b.shape[1 if transposed else 0] != k + 2 * hin or not _fits(x, k, m, bias) or not _columns(x, extra_in):
+        raise FgnnError("tall_product: x %s, matrix %s%s, bias %s and %d + %d extra columns do not fit one another" % (
+            tuple(x.shape), tuple(b.shape), " (transposed)" if transposed else "", None if bias is None else tuple(bias.shape), hin, extra_out))
+    bias = None if bias is None else as_f32(bias)
     y = torch.empty((n, m), dtype=torch.float32, device=x.device)
     e0 = torch.empty((n, extra_out), dtype=torch.float32, device=x.device) if extra_out else None
     e1 = torch.empty_like(e0) if extra_out else None
@@ -69,6 +99,8 @@ def tall_reduce(x, g, extra=None):
     n, a = x.shape
     b = g.shape[1]
     h = 0 if extra is None else extra[0].shape[1]
+    if not _matrices(x, g) or g.shape[0] != n or not _columns(x, extra):
+        raise FgnnError("tall_reduce: x %s, g %s and 2 x %d extra columns do not fit one another" % (tuple(x.shape), tuple(g.shape), h))
     c = torch.empty((a, b + 2 * h), dtype=torch.float32, device=x.device)
     e0, e1 = extra if h else (None, None)
     with device_guard(x.device):
@@ -86,6 +118,8 @@ def sum_wanted(g):
 def tall_sum(g):
     """The column sums of g [n, c]."""
     n, c = g.shape
+    if not _matrices(g):
+        raise FgnnError("tall_sum: not an fp32 matrix on the GPU with unit column stride")
     out = torch.empty(c, dtype=torch.float32, device=g.device)
     with device_guard(g.device):
         ws, wsb = workspace(lib().fgnn_column_sum_workspace_bytes(n, c), g.device)

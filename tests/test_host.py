@@ -229,3 +229,49 @@ def test_column_sum_and_wide_row_argument_errors_without_gpu():
     narrow = l.fgnn_gat_backward_workspace_bytes(1000, 4, 256, None, None, 0)
     wide = l.fgnn_gat_backward_workspace_bytes(1000, 8, 256, None, None, 0)
     assert wide > narrow + 5 * 1000 * 1024 * 4
+
+
+# an input wider and narrower than the weights, a row or a column of them short, a bias that only broadcasts, one on another device
+@pytest.mark.parametrize("x,w,b", [((4096, 128), (64, 64), None), ((4096, 50), (64, 64), None), ((4096, 64), (64,), None), ((4096, 64), (64, 64), (1,)),
+                                   ((4096, 64), (64, 64), (63,)), ((4096, 64), (64, 64), (1, 64)), ((64,), (64, 64), None), ((4096, 64), (64, 64), "meta")])
+def test_products_over_many_rows_take_only_what_fits(monkeypatch, x, w, b):
+    """The kernels read by the sizes they are given: whatever does not fit stays with torch, which broadcasts or refuses it as it always did."""
+    from ae_mlsys_gnn_amd.layers import dense
+    from ae_mlsys_gnn_amd.operators import tall
+    def no_kernel():
+        raise AssertionError("a kernel was launched")
+    monkeypatch.setattr(tall, "_plain", lambda *ts: True)
+    monkeypatch.setattr(tall, "_matrices", lambda *ts: True)
+    monkeypatch.setattr(tall, "lib", no_kernel)
+    x, w = torch.randn(x), torch.randn(w)
+    b = None if b is None else torch.empty(w.shape[0], device="meta") if b == "meta" else torch.randn(b)
+    assert not tall.product_wanted(x, w, transposed=True, bias=b)
+    if x.dim() == 2 and w.dim() == 2:
+        with pytest.raises(_lib.FgnnError):
+            tall.tall_product(x, w, transposed=True, bias=b)
+    try:
+        want = torch.matmul(x, w.t()) if b is None else torch.matmul(x, w.t()).add_(b)
+    except RuntimeError:
+        with pytest.raises(RuntimeError):
+            dense.tall_linear(x, w, b)
+    else:
+        assert torch.equal(dense.tall_linear(x, w, b), want)
+
+
+def test_products_over_many_rows_check_every_operand(monkeypatch):
+    from ae_mlsys_gnn_amd.operators import tall
+    monkeypatch.setattr(tall, "_plain", lambda *ts: True)
+    monkeypatch.setattr(tall, "_matrices", lambda *ts: True)
+    x, g = torch.randn(4096, 64), torch.randn(4096, 32)
+    col = lambda n, h: (torch.randn(n, h), torch.randn(n, h))
+    assert tall.product_wanted(x, torch.randn(64, 72), h_out=4) and tall.product_wanted(x, torch.randn(72, 64), h_in=4) and tall.reduce_wanted(x, g, 4)
+    assert not tall.product_wanted(x, torch.randn(60, 72), h_out=4) and not tall.product_wanted(x, torch.randn(64, 64), h_in=4)
+    assert not tall.reduce_wanted(x, g[:4000]) and not tall.reduce_wanted(x, g[:, 0])
+    for extra in (None, col(4096, 3), col(4000, 4), (torch.randn(4096, 4), torch.randn(4096, 3)), (torch.randn(4096, 4).double(),) * 2, (torch.randn(4, 4096).t(),) * 2):
+        with pytest.raises(_lib.FgnnError):
+            tall.tall_product(x, torch.randn(72, 64), extra_in=extra)
+        if extra is not None and extra[0].shape != (4096, 3):
+            with pytest.raises(_lib.FgnnError):
+                tall.tall_reduce(x, g, extra)
+    with pytest.raises(_lib.FgnnError):
+        tall.tall_reduce(x, g[:4000])

@@ -1725,6 +1725,26 @@ def test_tall_product(n, k, m, h_in, h_out):
         assert bool(torch.isinf(got[0]).all()) and bool(((got[1:].cpu().double() - ref[1:]).abs() <= tol[1:]).all())
 
 
+@pytest.mark.parametrize("width", [50, 128])
+def test_layers_refuse_inputs_of_another_width(width):
+    """As torch's products do: the kernels in their place read by the sizes of the weights."""
+    from ae_mlsys_gnn_amd.layers import EdgeConv, GATConv, GMMConv, GMMConv_stash
+    from ae_mlsys_gnn_amd.layers.dense import tall_linear
+    g = graphs.add_csc_torch(graphs.rmat_graph(4096, 20000, seed=4)).to(DEV)
+    x, pseudo = torch.randn(g.n, width, device=DEV), torch.randn(g.n_edges, 2, device=DEV)
+    calls = [lambda: GATConv(64, 16, 4).to(DEV)(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, x),
+             lambda: EdgeConv(64, 32).to(DEV)(4, torch.zeros(4 * g.n, dtype=torch.int32, device=DEV), x)]
+    calls += [lambda c=c, fin=fin: c(fin, 16, 2, 2).to(DEV)(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, x, pseudo)
+              for c, fin in ((GMMConv, 64), (GMMConv, 24), (GMMConv_stash, 64))]
+    for grad in (False, True):
+        for call in calls:
+            with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+                call()
+    w = torch.randn(64, width, device=DEV)
+    for bias in (torch.randn(1, device=DEV), torch.randn(1, 64, device=DEV)):
+        assert torch.equal(tall_linear(x, w, bias), torch.matmul(x, w.t()) + bias)
+
+
 # results of one tile to the most tiles a wave takes, rows around a staged block and around a workgroup's share
 @pytest.mark.parametrize("n,a,b,h", [(1, 1, 1, 0), (31, 16, 16, 0), (33, 17, 15, 1), (255, 64, 64, 4), (257, 100, 256, 8), (1025, 256, 48, 1), (4100, 41, 23, 0),
                                      (600, 602, 32, 0), (513, 144, 240, 2), (70000, 20, 4, 0), (300, 48, 200, 0), (90, 4, 512, 2), (2000, 144, 160, 3)])
