@@ -6,15 +6,21 @@ import torch
 from .._lib import FgnnError, as_f32, check, device_guard, lib, ptr, stream_ptr, workspace
 
 
+# Whether torch's own operations are being watched or rewritten (make_fx, fake tensors, functorch): a kernel launched past them would be missing
+# from the record, or be handed no memory.  Where a torch does not have the private names, its public mode stack is asked.
+_modes = getattr(torch._C, "_len_torch_dispatch_stack", None) or (lambda: torch.utils._python_dispatch._get_current_dispatch_mode() is not None)
+_transforms = getattr(torch._C, "_are_functorch_transforms_active", None) or (lambda: False)
+
+
 def _matrices(*ts):
     """fp32 matrices on one GPU with unit column stride."""
-    return all(t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] for t in ts) \
+    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] for t in ts) \
         and all(t.device == ts[0].device for t in ts)
 
 
 def _plain(*ts):
-    """Such matrices outside autocast (which asks for another precision)."""
-    return _matrices(*ts) and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
+    """Such matrices outside autocast (which asks for another precision) and tracing."""
+    return not (_modes() or _transforms() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()) and _matrices(*ts)
 
 
 def _fits(x, k, m, bias=None):

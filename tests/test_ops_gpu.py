@@ -1745,6 +1745,29 @@ def test_layers_refuse_inputs_of_another_width(width):
         assert torch.equal(tall_linear(x, w, bias), torch.matmul(x, w.t()) + bias)
 
 
+def test_products_over_many_rows_leave_traced_calls_to_torch():
+    """make_fx records torch's operations, a fake tensor has no memory: the kernels stay out of both, forward and backward."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from ae_mlsys_gnn_amd.layers.dense import column_sum, reduce_over_rows, tall_linear
+    from ae_mlsys_gnn_amd.operators.tall import product_wanted, reduce_wanted, sum_wanted
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    w, b, n = rnd(64, 64), rnd(64), 131072
+    x, x2, y, g = rnd(n, 64), rnd(n, 64), rnd(n, 64), rnd(n, 64)
+    assert product_wanted(x, w, transposed=True, bias=b) and reduce_wanted(x[:4096], g[:4096]) and sum_wanted(g)
+
+    def step(t, u):
+        with torch.no_grad():
+            return tall_linear(t, w, b), reduce_over_rows(t[:4096], u[:4096]), column_sum(u)
+    want = (y.double() @ w.double().t() + b.double(), y[:4096].double().t() @ g[:4096].double(), g.double().sum(0))
+    for got, ref in zip(make_fx(step)(x, x2)(y, g), want):
+        assert float((got.double() - ref).norm()) <= 1e-5 * float(ref.norm())           # fp32 sums of up to 131072 terms; the trace of x is not y's result
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        fake = mode.from_tensor(y)
+        assert [tuple(t.shape) for t in step(fake, fake)] == [tuple(t.shape) for t in want]
+
+
 # results of one tile to the most tiles a wave takes, rows around a staged block and around a workgroup's share
 @pytest.mark.parametrize("n,a,b,h", [(1, 1, 1, 0), (31, 16, 16, 0), (33, 17, 15, 1), (255, 64, 64, 4), (257, 100, 256, 8), (1025, 256, 48, 1), (4100, 41, 23, 0),
                                      (600, 602, 32, 0), (513, 144, 240, 2), (70000, 20, 4, 0), (300, 48, 200, 0), (90, 4, 512, 2), (2000, 144, 160, 3)])
