@@ -27,6 +27,16 @@ def _flat_list(n, e, row, backward):
     return e >= (1 << 22) and row <= 64 and row % 4 == 0 and 4 * n * row <= ((64 << 20) if backward else (32 << 20))
 
 
+def _sums_in_batches(f, *arrays):
+    """Whether a pass over rows no wider than a wave runs on the kernels that sum a row batch by batch, which take rows of F floats per mixture
+    kernel as 128-bit loads.  The others add all entries of a list item to one chain (up to 2048 of them in a plain list; 8 kernels x 32 floats, error of
+    the summed backward's input gradient, cut / plain: 20 k nodes, 4.4 M edges 2.5e-7 / 3.6e-7, 60 k, 30 M 4.2e-7 / 6.8e-7)."""
+    return f % 4 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in arrays)
+
+
+SUM_KERNELS_MAX = 4     # most mixture kernels that the summed column pass keeps in registers; with more, a pass over K x F floats
+
+
 class gmm_native:
     """gmmconv.gmmconv / gmmconvstash / Gaussian / GaussianBp (src/fused_gmmconv/gmmconv.cc:36-94)."""
 
@@ -63,8 +73,6 @@ class gmm_native:
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), k, e))
         out = torch.empty((n, f), dtype=torch.float32, device=node_feat.device) if sum_kernels else torch.empty_like(node_feat)
         gauss = torch.empty((e, k), dtype=torch.float32, device=node_feat.device) if want_gauss else None
-        # own_order: pseudo (and gauss) are indexed by the schedule's entry order, pseudo_caller[edge_positions(rowptr, colind)]
-        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, e, k * f, False))
         epilogue = bias is not None or residual is not None
         if epilogue:
             if not sum_kernels:
@@ -73,6 +81,9 @@ class gmm_native:
             residual = None if residual is None else as_f32(residual)
             if (bias is not None and tuple(bias.shape) != (f,)) or (residual is not None and tuple(residual.shape) != (n, f)):
                 raise FgnnError("gmmconv: bias must be [%d] and residual [%d, %d]" % (f, n, f))
+        # own_order: pseudo (and gauss) are indexed by the schedule's entry order, pseudo_caller[edge_positions(rowptr, colind)]
+        flat = _flat_list(n, e, k * f, False) and _sums_in_batches(f, node_feat, bias, residual)
+        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=flat)
         with device_guard(node_feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), node_feat.device)
             if proj is not None:
@@ -115,8 +126,9 @@ class gmm_native:
         grad_mu = torch.empty_like(mu)
         grad_sigma = torch.empty_like(sigma)
         # own_order: pseudo, grad_pseudo (and permute) are indexed by the schedule's entry order (gmm_edge_positions(colptr, rowind, True))
+        flat = _flat_list(n, e, f if sum_kernels and k <= SUM_KERNELS_MAX else k * f, True) and _sums_in_batches(f, node_feat, grad_out)
         sched = schedule_for(colptr, idx_tensor=None if (sum_kernels and _plain_list_for_summed_backward(n, e)) else rowind, own_order=own_order, n_cols=n,
-                             flat=_flat_list(n, e, f if sum_kernels else k * f, True))
+                             flat=flat)
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, node_feat, pseudo, (pw, pb), mu, sigma, grad_out, int(sum_kernels), grad_feat, grad_pseudo,
                              grad_mu, grad_sigma, sched, dev)
         return grad_feat, grad_pseudo, grad_mu, grad_sigma
@@ -159,7 +171,7 @@ class gmm_native:
             raise FgnnError("gmmconv_shared: shape mismatch mu %s sigma %s pseudo %s for E=%d" % (
                 tuple(mu.shape), tuple(sigma.shape), tuple(pseudo.shape), e))
         out = torch.empty((n, k, f), dtype=torch.float32, device=feat.device)
-        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, e, f, False))
+        sched = schedule_for(rowptr, idx_tensor=colind, own_order=own_order, n_cols=n, flat=_flat_list(n, e, f, False) and _sums_in_batches(f, feat))
         with device_guard(feat.device):
             ws, wsb = workspace(lib().fgnn_gmm_forward_workspace_bytes(sched.handle, k, f), feat.device)
             if proj is not None:
@@ -197,7 +209,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # same work list as the summed backward, so that one CSC-side copy of own-order edge data serves both kinds of layer
         sched = schedule_for(colptr, idx_tensor=None if _plain_list_for_summed_backward(n, e) else rowind, own_order=own_order, n_cols=n,
-                             flat=_flat_list(n, e, k * f, True))
+                             flat=_flat_list(n, e, k * f, True) and _sums_in_batches(f, feat, grad_out))
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, feat, pseudo, (pw, pb), mu, sigma, grad_out, 2, parts, grad_pseudo, grad_mu, grad_sigma, sched,
                              dev)
         return parts.sum(1), grad_pseudo, grad_mu, grad_sigma

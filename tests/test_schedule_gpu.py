@@ -2,6 +2,8 @@
 split for split the same list, for plain and XCD-aware lists, over segment lengths, bucket cut-offs and graph shapes
 (empty rows, hubs, no edges at all, a single row); malformed pointer arrays are refused by both before any kernel
 walks the index array with them."""
+import math
+
 import pytest
 import torch
 
@@ -209,3 +211,42 @@ def test_flat_list_over_bucketed_order(monkeypatch):
         ref = torch.zeros(g.n, f, dtype=torch.float64, device="cuda:0").index_add_(0, dst, w[:, None] * x.sum(1).double()[g.col_ind.long()])
         mag = torch.zeros(g.n, f, dtype=torch.float64, device="cuda:0").index_add_(0, dst, w[:, None] * x.abs().sum(1).double()[g.col_ind.long()])
         assert bool(((got.double() - ref).abs() <= 64 * 2.0 ** -24 * mag + 1e-30).all())      # chains of at most 64, exp's last bits
+
+
+# kernels past the summed pass' limit, rows past a wave, rows and base addresses off the 128-bit loads (those kernels add an item's entries to one chain),
+# and two forms that do take the plain list
+@pytest.mark.parametrize("k,f,off,summed", [(8, 32, 0, True), (5, 12, 0, True), (2, 16, 1, True), (2, 6, 0, True), (2, 16, 0, True), (2, 16, 2, False), (4, 16, 0, False)])
+def test_plain_list_costs_no_precision(monkeypatch, k, f, off, summed):
+    """On a skewed graph large enough for the rule, the errors against float64 are no larger than with the list cut by source bucket."""
+    from ae_mlsys_gnn_amd.operators import fused_gmmconv
+    from ae_mlsys_gnn_amd.operators.csr2csc import csr2csc
+    dev = "cuda:0"
+    g = graphs.rmat_graph(20000, 4400000, seed=3, device=dev)
+    g.col_ptr, g.row_ind, _ = csr2csc(g.row_ptr, g.col_ind)
+    e = g.n_edges
+    assert e >= 1 << 22
+    gen = torch.Generator(device=dev).manual_seed(k * f)
+    rnd = lambda *s: torch.rand(*s, generator=gen, device=dev)                # positive terms: nothing cancels, and what is lost is lost in the chains
+    shifted = lambda *s: rnd(math.prod(s) + off)[off:].view(*s)
+    x, go, ps = shifted(g.n, k, f), shifted(*((g.n, f) if summed else (g.n, k, f))), rnd(e, 1)
+    mu, sg = torch.zeros(k, 1, device=dev), torch.full((k, 1), 0.5, device=dev)
+    w = torch.exp(-0.5 * (0.5 * ps.double()) ** 2)                              # the weight of every kernel
+
+    def gathered(ptr, idx, rows):
+        out = torch.zeros(g.n, rows.shape[1], dtype=torch.float64, device=dev)
+        dst = torch.repeat_interleave(torch.arange(g.n, device=dev), (ptr[1:] - ptr[:-1]).long())
+        for i in range(0, e, 1 << 19):
+            out.index_add_(0, dst[i:i + (1 << 19)], w[i:i + (1 << 19)] * rows[idx[i:i + (1 << 19)].long()].double())
+        return out
+    fwd = gathered(g.row_ptr, g.col_ind, x.sum(1) if summed else x.reshape(g.n, -1))
+    bwd = gathered(g.col_ptr, g.row_ind, go.reshape(g.n, -1))
+
+    def errors():
+        out = fused_gmmconv.gmm_native.gmmconv(g.row_ptr, g.col_ind, x, ps, mu, sg, sum_kernels=summed)
+        gx = fused_gmmconv.gmm_native.gmmconv_backward(g.col_ptr, g.row_ind, None, x, ps, mu, sg, go, sum_kernels=summed)[0]
+        want = bwd[:, None, :].expand(g.n, k, f) if summed else bwd.view(g.n, k, f)
+        return [float((a.double() - b).norm() / b.norm()) for a, b in ((out, fwd.view(out.shape)), (gx, want))]
+    got = errors()
+    monkeypatch.setattr(fused_gmmconv, "_flat_list", lambda *a: False)
+    for a, b in zip(got, errors()):
+        assert a <= 1.05 * b, (got, b)              # (the same kernel on the same list, or batches whose length does not grow with the item's)
