@@ -193,22 +193,24 @@ class Schedule:
     """Degree-binned work list of one pointer array (row_ptr or col_ptr).  With `idx_tensor` it is
     the XCD-aware form: long rows are cut by source bucket and each XCD gets one bucket."""
 
-    def __init__(self, ptr_tensor, seg_len=0, idx_tensor=None, min_deg=0, with_positions=True, n_cols=None, flat_of=None):
-        """flat_of: an XCD-aware Schedule of the same arrays; the list is then the plain one over its entry order."""
+    def __init__(self, ptr_tensor, seg_len=0, idx_tensor=None, min_deg=0, with_positions=True, n_cols=None, flat_of=None, walked=None):
+        """flat_of: an XCD-aware Schedule of the same arrays; the list is then the plain one over its entry order.
+        walked: the index array that operators walk by a plain list, for the opt-in check alone."""
         require_cuda(ptr_tensor)
         self.ptr_tensor = as_i32(ptr_tensor)      # keeps the device memory alive
         self.flat_of = flat_of                    # ...and the index copy it walks
         self.idx_tensor = None if idx_tensor is None else as_i32(idx_tensor)
+        self.walked = self.idx_tensor if walked is None else as_i32(walked)
         self.n_rows = self.ptr_tensor.numel() - 1
         handle = c_void_p()
         with device_guard(self.ptr_tensor.device):
-            if self.idx_tensor is not None and os.environ.get("FGNN_VALIDATE", "0") not in ("0", ""):
+            if self.walked is not None and os.environ.get("FGNN_VALIDATE", "0") not in ("0", ""):
                 # opt-in: range-check the graph once, when its work list is built, before any gather kernel runs.  The ids
                 # index another array than the pointer array's rows (mhspmm / csrspmm: the gathered matrix), so the bound is
                 # the caller's n_cols; without one only the pointer array and the sign of the ids can be checked
                 bound = int(n_cols) if n_cols is not None else 2147483647
-                check(lib().fgnn_validate_graph(ptr(self.ptr_tensor), ptr(self.idx_tensor), self.n_rows, bound,
-                                                self.idx_tensor.numel(), stream_ptr()), "fgnn_validate_graph")
+                check(lib().fgnn_validate_graph(ptr(self.ptr_tensor), ptr(self.walked), self.n_rows, bound,
+                                                self.walked.numel(), stream_ptr()), "fgnn_validate_graph")
             if flat_of is not None:
                 check(lib().fgnn_schedule_create_flat(flat_of.handle, int(seg_len), stream_ptr(), ctypes.byref(handle)), "fgnn_schedule_create_flat")
             elif self.idx_tensor is None:
@@ -335,10 +337,11 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
     where the per-edge tensors are in that."""
     if seg_len is None:
         seg_len = default_seg_len()
+    walked = None           # the index array of a plain list in caller order: part of its key, so that each is checked
     if flat and idx_tensor is not None and xcd_buckets_enabled(ptr_tensor, idx_tensor.numel()):
         flat_len = seg_len or flat_seg_len(idx_tensor.numel())
         if not own_order:
-            idx_tensor, seg_len = None, flat_len
+            walked, idx_tensor, seg_len = idx_tensor, None, flat_len
     else:
         flat = False
     if idx_tensor is not None and not xcd_buckets_enabled(ptr_tensor, idx_tensor.numel()):
@@ -347,7 +350,8 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
 
     def key(pos):
         return (ptr_tensor.data_ptr(), ptr_tensor.numel(), ptr_tensor.device.index, ptr_tensor._version, int(seg_len),
-                None if idx_tensor is None else (idx_tensor.data_ptr(), idx_tensor._version, min_deg, pos))
+                None if idx_tensor is None else (idx_tensor.data_ptr(), idx_tensor._version, min_deg, pos)) + (
+                    () if walked is None else ("flat", walked.data_ptr(), walked._version))
     if own_order:
         k = key("own")
         s = _sched_cache.get(k)
@@ -371,7 +375,7 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
         k = key(False)
         s = _sched_cache.get(k)
     if s is None:
-        s = Schedule(ptr_tensor, seg_len, idx_tensor, min_deg, with_positions=need_positions, n_cols=n_cols)
+        s = Schedule(ptr_tensor, seg_len, idx_tensor, min_deg, with_positions=need_positions, n_cols=n_cols, walked=walked)
         _sched_cache[k] = s
         while len(_sched_cache) > _SCHED_CACHE_MAX:
             _sched_cache.popitem(last=False)

@@ -275,3 +275,48 @@ def test_products_over_many_rows_check_every_operand(monkeypatch):
                 tall.tall_reduce(x, g, extra)
     with pytest.raises(_lib.FgnnError):
         tall.tall_reduce(x, g[:4000])
+
+
+class _RecordingLib:
+    """The library's work-list calls without a GPU: each call's name and its pointer arguments are kept."""
+
+    def __init__(self):
+        self.calls, self.made = [], 0
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append((name, [a.value for a in args if isinstance(a, ctypes.c_void_p)]))
+            if name.startswith("fgnn_schedule_create"):
+                self.made += 1
+                args[-1]._obj.value = self.made
+            return 8 if name.endswith("num_buckets") else 0
+        return call
+
+
+@pytest.fixture
+def lists_without_gpu(monkeypatch):
+    import contextlib
+    rec = _RecordingLib()
+    monkeypatch.setattr(_lib, "lib", lambda: rec)
+    monkeypatch.setattr(_lib, "_lib", rec)
+    monkeypatch.setattr(_lib, "require_cuda", lambda *ts: None)
+    monkeypatch.setattr(_lib, "device_guard", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream_ptr", lambda: None)
+    monkeypatch.setattr(_lib, "xcd_buckets_enabled", lambda *a: True)               # a skewed graph
+    _lib.clear_schedule_cache()
+    yield rec
+    _lib.clear_schedule_cache()
+
+
+def test_plain_lists_of_skewed_graphs_are_validated(lists_without_gpu, monkeypatch):
+    """FGNN_VALIDATE=1: the ids are checked before the first gather by a plain list too, each index array of a pointer array by itself."""
+    monkeypatch.setenv("FGNN_VALIDATE", "1")
+    row_ptr, one, two = torch.tensor([0, 2, 3], dtype=torch.int32), torch.tensor([0, 1, 1], dtype=torch.int32), torch.tensor([1, 1, 0], dtype=torch.int32)
+    checked = lambda: [args[1] for name, args in lists_without_gpu.calls if name == "fgnn_validate_graph"]
+    for idx in (one, two, one):
+        s = _lib.schedule_for(row_ptr, idx_tensor=idx, n_cols=2, flat=True)
+        assert s.idx_tensor is None
+    assert checked() == [one.data_ptr(), two.data_ptr()]
+    one[0] = 1                                                                          # edited in place: checked again
+    _lib.schedule_for(row_ptr, idx_tensor=one, n_cols=2, flat=True)
+    assert checked() == [one.data_ptr(), two.data_ptr(), one.data_ptr()]

@@ -250,3 +250,20 @@ def test_plain_list_costs_no_precision(monkeypatch, k, f, off, summed):
     monkeypatch.setattr(fused_gmmconv, "_flat_list", lambda *a: False)
     for a, b in zip(got, errors()):
         assert a <= 1.05 * b, (got, b)              # (the same kernel on the same list, or batches whose length does not grow with the item's)
+
+
+def test_plain_list_of_a_skewed_graph_refuses_bad_ids(monkeypatch):
+    """FGNN_VALIDATE=1 stops a bad id before the gather by the plain list as it does before the cut one's."""
+    from ae_mlsys_gnn_amd import _lib
+    from ae_mlsys_gnn_amd.operators import fused_gmmconv
+    monkeypatch.setattr(fused_gmmconv, "_flat_list", lambda *a: True)
+    monkeypatch.setenv("FGNN_VALIDATE", "1")
+    g = graphs.rmat_graph(3000, 400000, seed=3).to("cuda:0")
+    x, ps = torch.randn(g.n, 2, 16, device="cuda:0"), torch.rand(g.n_edges, 2, device="cuda:0")
+    mu, sg = torch.zeros(2, 2, device="cuda:0"), torch.ones(2, 2, device="cuda:0")
+    bad = g.col_ind.clone()
+    bad[7] = g.n
+    call = lambda idx: fused_gmmconv.gmm_native.gmmconv(g.row_ptr, idx, x, ps, mu, sg, sum_kernels=True)
+    with pytest.raises(_lib.FgnnError, match="malformed graph"):
+        call(bad)
+    assert bool(torch.isfinite(call(g.col_ind)).all())
