@@ -260,6 +260,9 @@ class Schedule:
 
 _sched_cache: "collections.OrderedDict" = collections.OrderedDict()
 _SCHED_CACHE_MAX = 32
+# Plain lists of skewed graphs have slots of their own beside those: a graph may hold two lists a direction, and an own-order list cannot be built
+# again once it is dropped.  One over an own-order list is kept under that list's key and goes with it.
+_flat_cache: "collections.OrderedDict" = collections.OrderedDict()
 # The caches below are read and filled by the thread that runs the forward pass and by autograd's backward
 # thread: one re-entrant lock serialises every look-up-then-insert sequence (and the builds inside them).
 _cache_lock = threading.RLock()
@@ -271,6 +274,16 @@ def _locked(fn):
         with _cache_lock:
             return fn(*args, **kwargs)
     return wrapper
+
+
+def _keep(cache, k, s):
+    """Puts s under k as the newest entry and drops the oldest past the limit."""
+    cache[k] = s
+    while len(cache) > _SCHED_CACHE_MAX:
+        old, _ = cache.popitem(last=False)
+        if cache is _sched_cache:
+            _flat_cache.pop(old, None)
+    return s
 
 
 def default_seg_len() -> int:
@@ -360,27 +373,21 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
                             "tensors permuted by its result")
         _sched_cache.move_to_end(k)
         if flat and s.n_buckets > 0:
-            kf = k + ("flat", flat_len)
-            f = _sched_cache.get(kf)
+            f = _flat_cache.get(k)
             if f is None or f.flat_of is not s:
-                f = _sched_cache[kf] = Schedule(ptr_tensor, flat_len, flat_of=s)
-                while len(_sched_cache) > _SCHED_CACHE_MAX:
-                    _sched_cache.popitem(last=False)
-            _sched_cache.move_to_end(kf)
+                return _keep(_flat_cache, k, Schedule(ptr_tensor, flat_len, flat_of=s))
+            _flat_cache.move_to_end(k)
             return f
         return s
     k = key(True)
-    s = _sched_cache.get(k)
+    cache = _sched_cache if walked is None else _flat_cache
+    s = cache.get(k)
     if s is None and not need_positions and idx_tensor is not None:
         k = key(False)
-        s = _sched_cache.get(k)
+        s = cache.get(k)
     if s is None:
-        s = Schedule(ptr_tensor, seg_len, idx_tensor, min_deg, with_positions=need_positions, n_cols=n_cols, walked=walked)
-        _sched_cache[k] = s
-        while len(_sched_cache) > _SCHED_CACHE_MAX:
-            _sched_cache.popitem(last=False)
-    else:
-        _sched_cache.move_to_end(k)
+        return _keep(cache, k, Schedule(ptr_tensor, seg_len, idx_tensor, min_deg, with_positions=need_positions, n_cols=n_cols, walked=walked))
+    cache.move_to_end(k)
     return s
 
 
@@ -403,9 +410,7 @@ def edge_positions(ptr_tensor, idx_tensor, seg_len=None):
     if k in _sched_cache:                   # asked again: the map is a function of the arrays, the cached schedule stays
         _sched_cache.move_to_end(k)
         return pos
-    _sched_cache[k] = s
-    while len(_sched_cache) > _SCHED_CACHE_MAX:
-        _sched_cache.popitem(last=False)
+    _keep(_sched_cache, k, s)
     return pos
 
 
@@ -477,7 +482,7 @@ def schedule_device_bytes() -> int:
     """Device memory held by all cached schedules and column-sum plans: the library allocates it itself, so
     torch's max_memory_allocated does not see it and peak-memory reports add it."""
     with _cache_lock:
-        return sum(s.device_bytes() for s in _sched_cache.values()) + sum(p.device_bytes() for p in _colsum_cache.values())
+        return sum(s.device_bytes() for c in (_sched_cache, _flat_cache) for s in c.values()) + sum(p.device_bytes() for p in _colsum_cache.values())
 
 
 _own_view_cache: "collections.OrderedDict" = collections.OrderedDict()
@@ -531,6 +536,7 @@ def own_order_view(row_ptr, col_ind, col_ptr, row_ind, permute):
 
 def clear_schedule_cache():
     with _cache_lock:
+        _flat_cache.clear()
         _sched_cache.clear()
         _bucket_rule_cache.clear()
         _colsum_cache.clear()

@@ -320,3 +320,31 @@ def test_plain_lists_of_skewed_graphs_are_validated(lists_without_gpu, monkeypat
     one[0] = 1                                                                          # edited in place: checked again
     _lib.schedule_for(row_ptr, idx_tensor=one, n_cols=2, flat=True)
     assert checked() == [one.data_ptr(), two.data_ptr(), one.data_ptr()]
+
+
+def test_own_order_lists_outlive_the_plain_lists_beside_them(lists_without_gpu):
+    """Sixteen graphs with an own-order list a direction fit the cache, whatever plain lists their layers take besides; the plain
+    lists are bounded, and one over an own-order list goes with it."""
+    arrays = [[torch.tensor(v, dtype=torch.int32) for v in ([0, 2, 3], [0, 1, 1])] for _ in range(33)]
+    for ptr, idx in arrays[:32]:
+        _lib.edge_positions(ptr, idx)
+    for _ in range(2):
+        for ptr, idx in arrays[:32]:
+            own = _lib.schedule_for(ptr, idx_tensor=idx, own_order=True)
+            flat = _lib.schedule_for(ptr, idx_tensor=idx, own_order=True, flat=True)
+            assert flat.flat_of is own and _lib.schedule_for(ptr, idx_tensor=idx, own_order=True, flat=True) is flat
+    assert sum(name == "fgnn_schedule_create_flat" for name, _ in lists_without_gpu.calls) == 32         # built once each
+    ptr, idx = arrays[0]
+    assert _lib.schedule_for(ptr, idx_tensor=idx, flat=True) is _lib.schedule_for(ptr, idx_tensor=idx, flat=True)        # the caller's order
+    for p, i in arrays[:32]:
+        _lib.schedule_for(p, idx_tensor=i, own_order=True)
+        _lib.schedule_for(p, idx_tensor=i, flat=True)
+    assert len(_lib._flat_cache) <= 32 and len(_lib._sched_cache) <= 32
+    base = _lib.schedule_for(ptr, idx_tensor=idx, own_order=True)
+    _lib.schedule_for(ptr, idx_tensor=idx, own_order=True, flat=True)
+    for p, i in arrays[1:32]:
+        _lib.schedule_for(p, idx_tensor=i, own_order=True)
+    _lib.edge_positions(*arrays[32])                                                    # one too many: the oldest goes, its plain list with it
+    assert all(f.flat_of is not base for f in _lib._flat_cache.values())
+    with pytest.raises(_lib.FgnnError):
+        _lib.schedule_for(ptr, idx_tensor=idx, own_order=True)
