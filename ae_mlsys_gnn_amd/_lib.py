@@ -68,6 +68,7 @@ _SIGNATURES = {
     "fgnn_gat_unfold_grads": (c_int, [c_int] * 4 + [c_void_p] * 4 + [c_int, c_void_p, c_int] + [c_void_p] * 3 + [c_void_p]),
     "fgnn_tall_product": (c_int, [c_int64, c_int, c_int, c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p,
                                   c_int, c_void_p, c_void_p, c_void_p]),
+    "fgnn_tall_product_workgroups": (c_int64, [c_int64, c_int, c_int, c_int, c_int, c_int]),
     "fgnn_tall_reduce_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
     "fgnn_tall_reduce": (c_int, [c_int64, c_int, c_int, c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "fgnn_knn_graph": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),

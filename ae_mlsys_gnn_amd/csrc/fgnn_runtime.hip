@@ -560,20 +560,26 @@ extern "C" int fgnn_xcd_mapping_for(const char *gcn_arch, int compute_units)
     return gfx950 && compute_units == 32 * FGNN_NUM_XCD ? FGNN_NUM_XCD : 0;
 }
 
-// 1: the current device has the workgroup-to-XCD mapping the bucketed lists assume; 0: it has not (or cannot be asked)
-int fgnn_current_device_has_xcd_mapping()
+// What is asked of the current device, once per device: its compute units (0: it cannot be asked) and whether it has the workgroup-to-XCD
+// mapping the bucketed lists assume.
+struct device_facts { bool asked; int units; bool mapping; };
+static device_facts current_device_facts()
 {
     static std::mutex mu;
-    static int known[64];          // per device: 0 = not asked yet, 1 = no, 2 = yes
+    static device_facts known[64];
     int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return device_facts{};
     std::lock_guard<std::mutex> lock(mu);
-    if (known[dev] == 0) {
+    device_facts &f = known[dev];
+    if (!f.asked) {
         hipDeviceProp_t prop;
-        known[dev] = (hipGetDeviceProperties(&prop, dev) == hipSuccess && fgnn_xcd_mapping_for(prop.gcnArchName, prop.multiProcessorCount) > 0) ? 2 : 1;
+        if (hipGetDeviceProperties(&prop, dev) == hipSuccess) { f.units = prop.multiProcessorCount; f.mapping = fgnn_xcd_mapping_for(prop.gcnArchName, f.units) > 0; }
+        f.asked = true;
     }
-    return known[dev] == 2;
+    return f;
 }
+int fgnn_current_device_has_xcd_mapping() { return current_device_facts().mapping; }
+int fgnn_current_device_compute_units() { return current_device_facts().units; }
 
 extern "C" int fgnn_schedule_create_bucketed(const int32_t *ptr_dev, const int32_t *idx_dev, int n_rows, int seg_len, int min_deg,
                                              int with_positions, void *stream, fgnn_schedule_t **out)

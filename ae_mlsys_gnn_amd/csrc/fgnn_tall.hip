@@ -247,6 +247,41 @@ static inline void tl_dispatch_tiles(int t, Fn &&f)
     }
 }
 
+struct TallPlan { int tiles, splits, waves; int64_t blocks; };   // blocks: workgroups of a column range
+static bool tall_product_plan(int64_t n, int k, int m, int hin, int hout, int cus, TallPlan *pl)
+{
+    const int kk = (k + 15) / 16 + (hin ? 1 : 0), total = (m + 15) / 16 + (hout ? 1 : 0), fit = std::min(18, TL_LDS_MAX / (kk * 1024));
+    if (fit < 1) return false;
+    int splits = (total + fit - 1) / fit, tiles = tl_tiles((total + splits - 1) / splits);
+    while ((size_t)tiles * kk * 1024 > TL_LDS_MAX) {                         // the next number of tiles that a kernel exists for does not fit
+        ++splits;
+        tiles = tl_tiles((total + splits - 1) / splits);
+    }
+    splits = (total + tiles - 1) / tiles;
+    // One workgroup per compute unit, of as many waves (four SIMDs' worth at a time) as give the shortest way through the row tiles:
+    // 4096 tiles are one and a third rounds for 12 waves on 256 units and two for 8, so 24 tile times against 16 (65 k x 64 -> 256: 54 -> 33 us).
+    // A column range gets whole eighths of the units (its workgroups are dealt out by XCD), rounded down: of three ranges 80 on 256 units,
+    // for with 88 eight workgroups of the 264 begin when the others have ended (us, 88 / 80, 180 -> 384 + 12 scores: 70 k rows 216 / 109,
+    // 169 k 401 / 251, 500 k 1216 / 685; library product and score kernel 133, 265, 800).
+    const int64_t rows = (n + 15) / 16, units = std::max(cus / splits / FGNN_NUM_XCD * FGNN_NUM_XCD, FGNN_NUM_XCD);
+    int64_t best = INT64_MAX;
+    for (int w = TL_WAVES(tiles); w >= 4; w -= 4) {
+        const int64_t cost = (rows + units * w - 1) / (units * w) * w;
+        if (cost < best) { best = cost; pl->waves = w; }
+    }
+    const int64_t need = (rows + pl->waves - 1) / pl->waves;
+    pl->blocks = std::min(units, (need + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD * FGNN_NUM_XCD);
+    pl->tiles = tiles; pl->splits = splits;
+    return true;
+}
+
+extern "C" int64_t fgnn_tall_product_workgroups(int64_t n, int k, int m, int hin, int hout, int compute_units)
+{
+    TallPlan pl;
+    if (n < 1 || k < 1 || m < 1 || hin < 0 || hout < 0 || k > (1 << 20) || compute_units < 1 || !tall_product_plan(n, k, m, hin, hout, compute_units, &pl)) return 0;
+    return pl.blocks * pl.splits;
+}
+
 extern "C" int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_t ldx, const float *b, int64_t ldb, int b_transposed, const float *bias,
                                  float *y, int64_t ldy, int hin, const float *xe0, const float *xe1, int hout, float *ye0, float *ye1, void *stream)
 {
@@ -263,30 +298,15 @@ extern "C" int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_
     p.hin = hin; p.xe0 = xe0; p.xe1 = xe1; p.hout = hout; p.ye0 = ye0; p.ye1 = ye1;
     p.kkm = (k + 15) / 16; p.kk = p.kkm + (hin ? 1 : 0);
     p.vecy = ldy % 4 == 0;
-    const int total = (m + 15) / 16 + (hout ? 1 : 0), fit = std::min(18, TL_LDS_MAX / (p.kk * 1024));
-    FGNN_REQUIRE(fit >= 1, FGNN_ERR_LIMIT, "fgnn_tall_product: %d input columns unsupported", k);
-    p.splits = (total + fit - 1) / fit;
-    int tiles = tl_tiles((total + p.splits - 1) / p.splits);
-    while ((size_t)tiles * p.kk * 1024 > TL_LDS_MAX) {                       // the next number of tiles that a kernel exists for does not fit
-        ++p.splits;
-        tiles = tl_tiles((total + p.splits - 1) / p.splits);
-    }
-    p.splits = (total + tiles - 1) / tiles;
-    const size_t lds = (size_t)tiles * p.kk * 1024;
-    // One workgroup per compute unit, of as many waves (four SIMDs' worth at a time) as give the shortest way through the row tiles:
-    // 4096 tiles are one and a third rounds for 12 waves on 256 units and two for 8, so 24 tile times against 16 (65 k x 64 -> 256: 54 -> 33 us).
-    const int64_t rows = (n + 15) / 16, units = std::max(256 / p.splits, 1);
-    int64_t best = INT64_MAX;
-    for (int w = TL_WAVES(tiles); w >= 4; w -= 4) {
-        const int64_t cost = (rows + units * w - 1) / (units * w) * w;
-        if (cost < best) { best = cost; p.waves = w; }
-    }
-    int64_t blocks = std::min<int64_t>((rows + p.waves - 1) / p.waves, units);
-    blocks = (blocks + FGNN_NUM_XCD - 1) / FGNN_NUM_XCD * FGNN_NUM_XCD;
-    const unsigned grid = (unsigned)(blocks * p.splits);
+    const int cus = fgnn_current_device_compute_units();
+    TallPlan pl;
+    FGNN_REQUIRE(tall_product_plan(n, k, m, hin, hout, cus > 0 ? cus : 256, &pl), FGNN_ERR_LIMIT, "fgnn_tall_product: %d input columns unsupported", k);
+    p.splits = pl.splits; p.waves = pl.waves;
+    const size_t lds = (size_t)pl.tiles * p.kk * 1024;
+    const unsigned grid = (unsigned)(pl.blocks * pl.splits);
     hipStream_t st = (hipStream_t)stream;
     FGNN_REQUIRE(hin == 0 || vec == 4, FGNN_ERR_ALIGN, "fgnn_tall_product: extra input columns need x in rows of 16-byte multiples");
-    tl_dispatch_tiles(tiles, [&]<int NT>() {
+    tl_dispatch_tiles(pl.tiles, [&]<int NT>() {
         const dim3 g(grid), w(64 * p.waves);
         if (hin) hipLaunchKernelGGL((tall_product_kernel<NT, 4, true>), g, w, lds, st, p);
         else if (vec == 4) hipLaunchKernelGGL((tall_product_kernel<NT, 4, false>), g, w, lds, st, p);

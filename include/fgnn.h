@@ -297,6 +297,8 @@ int fgnn_gat_unfold_grads(int fin, int H, int F, int pad, const float *W, const 
 int fgnn_tall_product(int64_t n, int k, int m, const float *x, int64_t ldx, const float *b, int64_t ldb, int b_transposed,
                       const float *bias, float *y, int64_t ldy, int hin, const float *xe0, const float *xe1, int hout,
                       float *ye0, float *ye1, void *stream);
+/* Workgroups of that launch on a device of so many compute units (0: unsupported): at most one per unit while a column range has eight. */
+int64_t fgnn_tall_product_workgroups(int64_t n, int k, int m, int hin, int hout, int compute_units);
 size_t fgnn_tall_reduce_workspace_bytes(int64_t n, int ka, int kb, int h);
 int fgnn_tall_reduce(int64_t n, int ka, int kb, const float *x, int64_t ldx, const float *g, int64_t ldg, int h,
                      const float *ge0, const float *ge1, float *c, void *workspace, size_t workspace_bytes, void *stream);

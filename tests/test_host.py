@@ -348,3 +348,16 @@ def test_own_order_lists_outlive_the_plain_lists_beside_them(lists_without_gpu):
     assert all(f.flat_of is not base for f in _lib._flat_cache.values())
     with pytest.raises(_lib.FgnnError):
         _lib.schedule_for(ptr, idx_tensor=idx, own_order=True)
+
+
+@pytest.mark.parametrize("units", [256, 304, 80, 64])
+def test_products_over_many_rows_launch_no_workgroup_past_the_compute_units(units):
+    """A workgroup fills a unit's LDS, and the rows are dealt out over all of them: one too many doubles the time.  One to seven column ranges, with and
+    without extra columns, few rows and many."""
+    count = _lib.lib().fgnn_tall_product_workgroups
+    for n in (1, 17, 4096, 65536, 70001, 169343, 2449029):
+        for k, m, hin, hout in [(64, 64, 0, 0), (180, 384, 0, 6), (275, 256, 0, 4), (520, 128, 0, 1), (602, 64, 2, 0), (100, 256, 0, 8), (256, 100, 8, 0), (1024, 72, 0, 0),
+                                (400, 512, 0, 0), (1024, 112, 0, 0), (16, 16, 0, 0)]:
+            got = count(n, k, m, hin, hout, units)
+            assert 0 < got <= units and got % 8 == 0, (n, k, m, got)
+    assert count(70001, 2561, 16, 0, 0, units) == 0 and count(0, 16, 16, 0, 0, units) == 0
