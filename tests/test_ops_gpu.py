@@ -1869,3 +1869,23 @@ def test_gmm_projected_coordinates(n, e, fin, fout, k, dim, stash, own_order):
         # 2-norm of the error: a few roundings (2^-24 each) of every product and sum; a parameter's gradient is a cancelling sum over the
         # edges, and the composed passes are the measure of it
         assert err <= max(2.0 ** -20, 2 * old + 2.0 ** -22), (i, err, old)
+
+
+@pytest.mark.parametrize("k,dim,f,shared", [(4, 4, 160, False), (4, 4, 256, True), (4, 4, 132, False), (4, 3, 256, False), (3, 4, 256, True)])
+def test_gmm_projected_wide_rows_off_alignment(k, dim, f, shared):
+    """Gradients at a base address off the 128-bit loads: rows of up to 16 slabs beside the sums of the projection in LDS."""
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import GmmProjectedTwoOrders
+    g = graphs.add_csc_torch(graphs.rmat_graph(300, 5000, seed=2)).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(k * f + dim)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    raw = torch.rand(g.n_edges, 2, generator=gen, device=DEV)
+    leaves = [t.requires_grad_() for t in (rnd(g.n, f) if shared else rnd(g.n, k, f), rnd(dim, 2), rnd(dim), rnd(k, dim), rnd(k, dim))]
+    out = GmmProjectedTwoOrders(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, leaves[0], raw, raw[g.permute.long()].contiguous(), *leaves[1:])
+    go = rnd(*out.shape)
+    shifted = torch.empty(go.numel() + 1, device=DEV)[1:].view_as(go).copy_(go)
+    assert shifted.data_ptr() % 16
+    want = torch.autograd.grad(out, leaves, go, retain_graph=True)
+    got = torch.autograd.grad(out, leaves, shifted)
+    for a, b in zip(got, want):
+        # the same products summed in another order: chains of up to 1024 (dot products) and 5000 terms, errors as random walks
+        assert float((a - b).norm()) <= 2e-5 * float(b.norm()) + 1e-12
