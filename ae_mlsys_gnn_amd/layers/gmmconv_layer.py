@@ -6,9 +6,10 @@ import torch as th
 from torch import nn
 from torch.nn import init
 
+from .._lib import xcd_buckets_enabled
 from ..operators.edge_proj import edge_linear_tanh
 from ..operators.fused_gmmconv import (GmmAggregate, GmmAggregateLinear, GmmAggregateTwoOrders, GmmConvFuseSum, GmmConvFuseSumTwoOrders, GmmConvStash,
-                                        GmmConvStashSumTwoOrders, GmmProjectedTwoOrders, gmm_native, project_in_backward)
+                                        GmmConvStashSumTwoOrders, GmmProjectedTwoOrders, gmm_native, project_in_backward, projected_pays)
 from .dense import add_bias, tall_linear
 
 
@@ -59,7 +60,7 @@ class _GMMBase(nn.Module):
         (operators.fused_gmmconv.gmm_edge_positions); without pseudo_csc the layer is forward-only.
         proj: a Linear(2, dim) whose tanh gives the coordinates; pseudo and pseudo_csc are then raw [E, 2] pairs (constant data), and where the
         operators can, they project them on the way."""
-        if proj is not None and not self._projects(feat, pseudo, pseudo_csc, proj, colind):
+        if proj is not None and not self._projects(feat, pseudo, pseudo_csc, proj, colptr, colind):
             apply = lambda t: edge_linear_tanh(t, proj.weight, proj.bias)
             if pseudo_csc is not None:
                 with th.no_grad():
@@ -106,14 +107,18 @@ class _GMMBase(nn.Module):
             rst = rst[..., :self._out_feats]
         return self._finish(rst, feat)
 
-    def _projects(self, feat, raw, raw_csc, proj, colind):
-        """Whether this call leaves the projection to the operators: two orders of constant fp32 pairs, few kernels and coordinates, and not the
-        form of the layer whose backward takes the coordinates' gradient through a projection of the input."""
-        k, fin = self._n_kernels, feat.shape[1]
+    def _projects(self, feat, raw, raw_csc, proj, colptr, colind):
+        """Whether this call leaves the projection to the operators: two orders of constant fp32 pairs, few kernels and coordinates, not the form
+        of the layer whose backward takes the coordinates' gradient through a projection of the input, and edges enough to pay."""
+        k, fin, n, e = self._n_kernels, feat.shape[1], feat.shape[0], colind.numel()
         if (raw_csc is None or not gmm_native.projection_supported(k, self._dim) or raw.requires_grad or raw_csc.requires_grad
                 or any(t.dtype != th.float32 or not t.is_cuda for t in (raw, raw_csc, proj.weight, proj.bias))):
             return False
-        return not (self._aggregate_first(feat) and project_in_backward(k, fin, self._out_feats, feat.requires_grad, feat.shape[0], colind.numel()))
+        first = self._aggregate_first(feat)
+        if first and project_in_backward(k, fin, self._out_feats, feat.requires_grad, n, e):
+            return False
+        row = k * fin if first else (self._out_feats + 3) // 4 * 4
+        return projected_pays(n, e, k, self._dim, row, first, xcd_buckets_enabled(colptr, e))
 
     def _finish(self, rst, feat):
         if self.res_fc is not None:

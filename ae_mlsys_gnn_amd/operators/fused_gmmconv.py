@@ -436,6 +436,28 @@ class GmmProjectedTwoOrdersFunction(torch.autograd.Function):
         return (None, None, None, None, grad_feat, None, None, grad_w, grad_b, grad_mu, grad_sigma, None, None) + _epilogue_grads(ctx, grad_out.contiguous(), 13)
 
 
+def projected_pays(n, e, k, dim, row, aggregate, skewed):
+    """Whether the passes over the edges that project the coordinates themselves are no slower than projecting them beforehand, for n nodes, e edges and
+    a backward that gathers rows of `row` floats (aggregate: of the layer that aggregates its input first).  What they save is per edge; the
+    sums of the parameters' gradients, 2 K dim + 3 dim of them in LDS, cost every wave its start and end, and a wave on rows wider than 64
+    floats has one node's edges.  (us of a layer's forward and backward, formed beforehand / in the passes, 300 k nodes, uniform: 128 floats,
+    5 sums, degree 3 754 / 867, 17 1189 / 1160; 15 sums, degree 8 912 / 1106, 25 1620 / 1551; 44 sums, degree 8 2202 / 2967, 61 ahead; 256
+    floats, 14 sums, degree 8 1.04 of it, 17 0.98; 64 floats, 44 sums, degree 5 1.08, 12 0.95; aggregated rows of 96 floats, 27 sums, degree 3
+    1.4, 21 1.05, 36 0.96.  On skewed graphs half of the columns are nearly empty, and the copies cost more: 256 floats 0.90 to 1.0.)  Few nodes are
+    bound by the host, which the copies' launches cost 45 us."""
+    sums = 2 * k * dim + 3 * dim
+    if row <= 32 or n < 65536 or n * sums < (1 << (22 if skewed else 20)):
+        return True
+    if row <= 64:                           # lane groups: 4 or more nodes a wave
+        return aggregate or e >= n * (sums - 10) / 4
+    least = (10 + sums) * (0.6 if aggregate else 1.0)
+    if row > 128:
+        if skewed and sums <= 30:
+            return True
+        least /= 2
+    return e >= n * least
+
+
 def project_in_backward(k, fin, fout, input_grad, n, e):
     """Which rows the backward of an aggregate-first layer (n nodes, e edges) gathers per edge: K x fin floats, the gradient of the aggregate,
     or the fout floats (rounded up to 4) of the layer's own gradient, for the price of projecting the input again (and of one more

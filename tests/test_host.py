@@ -361,3 +361,30 @@ def test_products_over_many_rows_launch_no_workgroup_past_the_compute_units(unit
             got = count(n, k, m, hin, hout, units)
             assert 0 < got <= units and got % 8 == 0, (n, k, m, got)
     assert count(70001, 2561, 16, 0, 0, units) == 0 and count(0, 16, 16, 0, 0, units) == 0
+
+
+@pytest.mark.parametrize("n,degree,k,dim,row,aggregate,skewed,want", [
+    (300000, 3, 4, 4, 100, False, False, False), (300000, 8, 3, 3, 128, False, False, False), (300000, 60, 4, 4, 128, False, False, True),
+    (300000, 3, 2, 1, 256, False, False, False), (300000, 17, 2, 2, 256, False, False, True), (300000, 3, 2, 2, 256, False, True, True),
+    (500000, 8, 3, 3, 96, True, False, False), (500000, 36, 3, 3, 96, True, True, True), (500000, 3, 4, 4, 64, False, False, False),
+    (500000, 3, 4, 4, 16, False, False, True), (500000, 3, 3, 3, 64, True, False, True), (30000, 3, 4, 4, 128, False, False, True),
+    (90000, 3, 3, 3, 128, False, True, True), (90000, 3, 3, 3, 128, False, False, False), (232965, 490, 2, 1, 16, False, True, True), (169343, 14, 3, 2, 64, False, True, True)])
+def test_projected_coordinates_rule(n, degree, k, dim, row, aggregate, skewed, want):
+    """The measured shapes: few edges a node, many sums and wide rows leave the projection to a pass of its own."""
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import projected_pays
+    assert projected_pays(n, n * degree, k, dim, row, aggregate, skewed) is want
+
+
+def test_layer_asks_the_projection_rule(monkeypatch):
+    """The rule gets the row that the layer's backward gathers: K x in floats where it aggregates first, else the output rounded up to 4."""
+    from types import SimpleNamespace
+    from ae_mlsys_gnn_amd.layers import GMMConv, GMMConv_stash, gmmconv_layer
+    asked = []
+    monkeypatch.setattr(gmmconv_layer, "projected_pays", lambda *a: asked.append(a) or False)
+    monkeypatch.setattr(gmmconv_layer, "xcd_buckets_enabled", lambda *a: True)
+    raw = SimpleNamespace(dtype=torch.float32, is_cuda=True, requires_grad=False)
+    proj = SimpleNamespace(weight=raw, bias=raw)
+    for layer, want in ((GMMConv(32, 40, 3, 3), (96, True)), (GMMConv(256, 41, 3, 3), (44, False)), (GMMConv_stash(32, 40, 3, 3), (40, False))):
+        feat = torch.zeros(500, layer.fc.in_features, requires_grad=True)
+        assert layer._projects(feat, raw, raw, proj, torch.zeros(501, dtype=torch.int32), torch.zeros(1000, dtype=torch.int32)) is False
+        assert asked.pop() == (500, 1000, 3, 3, *want, True) and not asked
