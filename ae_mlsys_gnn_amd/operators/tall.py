@@ -6,21 +6,27 @@ import torch
 from .._lib import FgnnError, as_f32, check, device_guard, lib, ptr, stream_ptr, workspace
 
 
-# Whether torch's own operations are being watched or rewritten (make_fx, fake tensors, functorch): a kernel launched past them would be missing
-# from the record, or be handed no memory.  Where a torch does not have the private names, its public mode stack is asked.
+# Where a torch does not have the private names, its public mode stack is asked.
 _modes = getattr(torch._C, "_len_torch_dispatch_stack", None) or (lambda: torch.utils._python_dispatch._get_current_dispatch_mode() is not None)
 _transforms = getattr(torch._C, "_are_functorch_transforms_active", None) or (lambda: False)
 
 
+def _traced():
+    """Whether torch's own operations are being watched or rewritten (torch.compile, jit.trace, make_fx, fake tensors, functorch): a kernel launched past them
+    would be missing from the record, or be handed no memory.  Asked before any size, so that no size becomes a condition of the record, and the
+    compiler first: it does not follow the questions behind it."""
+    return torch.compiler.is_compiling() or torch.jit.is_tracing() or bool(_modes()) or _transforms()
+
+
 def _matrices(*ts):
     """fp32 matrices on one GPU with unit column stride."""
-    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] for t in ts) \
-        and all(t.device == ts[0].device for t in ts)
+    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1
+               and t.stride(0) >= t.shape[1] for t in ts) and all(t.device == ts[0].device for t in ts)
 
 
 def _plain(*ts):
-    """Such matrices outside autocast (which asks for another precision) and tracing."""
-    return not (_modes() or _transforms() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()) and _matrices(*ts)
+    """Such matrices outside autocast (which asks for another precision)."""
+    return not torch.is_autocast_enabled("cuda") and _matrices(*ts)
 
 
 def _fits(x, k, m, bias=None):
@@ -42,7 +48,7 @@ def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None
     With them, scores included: 16 k x 64 -> 64 + 8 9 / 8, 256 -> 48 + 2 15 / 17, 128 -> 256 + 8 20 / 35; 65 k 18 / 15, 34 / 30, 56 / 57; 169 k 60 / 33,
     85 / 68, 142 / 138; 1 M 231 / 137, 521 / 323, 761 / 601.  Gradients, stacking included: 16 k x 64 + 8 -> 64 11 / 8, 48 + 2 -> 256 16 / 18, 256 + 8 ->
     128 26 / 34; 65 k 26 / 17, 41 / 31, 72 / 65; 1 M 401 / 142, 628 / 348, 1216 / 598."""
-    if b.dim() != 2:
+    if _traced() or b.dim() != 2:
         return False
     k = b.shape[1 if transposed else 0] - 2 * h_in
     if m is None:
@@ -66,7 +72,7 @@ def reduce_wanted(x, g, h=0):
     extra columns: 4 k x 64, 64 + 8 25 / 17, 256, 48 + 2 21 / 30, 128, 256 + 8 24 / 52; 65 k 32 / 21, 34 / 36, 86 / 63; 169 k 69 / 40, 100 / 73, 229 /
     135; 1 M 341 / 184, 444 / 375, 1153 / 684.  On few rows the sum over the workgroups' results is what takes the time, so those are small
     ones there.  Without extra columns 233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116."""
-    if x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
+    if _traced() or x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
         return False
     n, a, b = x.shape[0], x.shape[1], g.shape[1]
     tiles = -(-a // 16) * (-(-b // 16) + (h > 0))
@@ -118,7 +124,7 @@ def tall_reduce(x, g, extra=None):
 def sum_wanted(g):
     """Where tall_sum of g [n, c] is the faster form: two launches for torch's one or two, or five with columns that are no multiple of four (us,
     torch / own, host included: 33 k x 64 11 / 13, 66 k x 16 10 / 11, 169 k x 16 12 / 12, 64 20 / 13, 41 31 / 11, 1 23 / 20, of the GPU 10 / 20)."""
-    return g.dim() == 2 and g.shape[0] >= 131072 and 3 <= g.shape[1] <= 1024 and _plain(g)
+    return not _traced() and g.dim() == 2 and g.shape[0] >= 131072 and 3 <= g.shape[1] <= 1024 and _plain(g)
 
 
 def tall_sum(g):
