@@ -323,9 +323,11 @@ def xcd_buckets_enabled(ptr_tensor, idx_numel=None) -> bool:
     key = (ptr_tensor.data_ptr(), ptr_tensor.numel(), ptr_tensor.device.index, ptr_tensor._version)
     hit = _bucket_rule_cache.get(key)
     if hit is None:
+        require_cuda(ptr_tensor)
+        rows = as_i32(ptr_tensor)
         stats = (ctypes.c_int64 * 2)()
         with device_guard(ptr_tensor.device):
-            check(lib().fgnn_row_length_stats(ptr(ptr_tensor), n_rows, BUCKET_ROW_LEN, ctypes.cast(stats, c_void_p), stream_ptr()),
+            check(lib().fgnn_row_length_stats(ptr(rows), n_rows, BUCKET_ROW_LEN, ctypes.cast(stats, c_void_p), stream_ptr()),
                   "fgnn_row_length_stats")
         n_long, longest = int(stats[0]), int(stats[1])
         n_edges = int(idx_numel) if idx_numel is not None else int(ptr_tensor[-1])

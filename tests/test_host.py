@@ -421,3 +421,22 @@ def test_products_over_many_rows_compile_whole():
     seen = []
     torch.jit.trace(lambda t: (seen.append(tall._traced()), dense.tall_linear(t, w, b))[1], x, check_trace=False)
     assert seen == [True]
+
+
+@pytest.mark.parametrize("ptr", [torch.tensor([0, 2, 3], dtype=torch.int32), torch.tensor([0, 2, 3])])
+def test_row_lengths_are_read_from_the_gpu_only(monkeypatch, ptr):
+    """The kernel that looks a pointer array over gets no host address and no other type; a layer with such an array says so."""
+    from types import SimpleNamespace
+    from ae_mlsys_gnn_amd.layers import GMMConv
+    def no_kernel():
+        raise AssertionError("a kernel was launched")
+    monkeypatch.delenv("FGNN_XCD_BUCKETS", raising=False)
+    monkeypatch.setattr(_lib, "lib", no_kernel)
+    if ptr.dtype != torch.int32:
+        monkeypatch.setattr(_lib, "require_cuda", lambda *ts: None)
+    _lib.clear_schedule_cache()
+    with pytest.raises(_lib.FgnnError):
+        _lib.xcd_buckets_enabled(ptr, 3)
+    raw = SimpleNamespace(dtype=torch.float32, is_cuda=True, requires_grad=False)
+    with pytest.raises(_lib.FgnnError):
+        GMMConv(64, 16, 1, 2)._projects(torch.zeros(2, 64), raw, raw, SimpleNamespace(weight=raw, bias=raw), ptr, torch.zeros(3, dtype=torch.int32))
