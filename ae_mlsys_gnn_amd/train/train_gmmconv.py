@@ -14,6 +14,7 @@ import argparse
 
 import torch
 from torch import nn
+from torch.nn.modules import module as nn_module
 
 from ..layers import GMMConv, GMMConv_stash
 from ..operators import edge_proj
@@ -37,12 +38,17 @@ class PseudoProj(nn.Linear):
         out = pseudo[:, 0:1] * self.weight[:, 0] + pseudo[:, 1:2] * self.weight[:, 1]
         return torch.tanh(out + self.bias)
 
+    def plain(self, layer, *pseudo):
+        """Whether `layer` may apply the projection's parameters itself: a layer of this package that knows how, the fused form's shapes, and nobody
+        hooked to either module, who would see raw coordinates or none."""
+        return (type(self) is PseudoProj and self.out_features <= edge_proj.MAX_OUT and self.bias is not None and type(layer).forward is GMMConv.forward
+                and _untouched(self) and _untouched(layer) and all(t.is_cuda and not t.requires_grad for t in pseudo))
 
-    def plain(self, *pseudo):
-        """Whether a layer may apply the projection's parameters itself: the fused form's shapes, and nobody hooked to the module."""
-        hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
-        return (type(self) is PseudoProj and self.out_features <= edge_proj.MAX_OUT and self.bias is not None and not any(hooks)
-                and all(t.is_cuda and not t.requires_grad for t in pseudo))
+
+def _untouched(module):
+    hooks = (module._forward_hooks, module._forward_pre_hooks, module._backward_hooks, module._backward_pre_hooks)
+    everywhere = (nn_module._global_forward_hooks, nn_module._global_forward_pre_hooks, nn_module._global_backward_hooks, nn_module._global_backward_pre_hooks)
+    return "forward" not in vars(module) and not any(hooks) and not any(everywhere)
 
 
 class MoNet(nn.Module):
@@ -62,7 +68,7 @@ class MoNet(nn.Module):
         for i, (layer, proj) in enumerate(zip(self.layers, self.pseudo_proj)):
             if i:
                 h = self.dropout(h)
-            if pseudo_csc is not None and torch.is_grad_enabled() and proj.plain(pseudo, pseudo_csc):
+            if pseudo_csc is not None and torch.is_grad_enabled() and proj.plain(layer, pseudo, pseudo_csc):
                 h = layer(g.row_ptr, g.col_ind, g.col_ptr, g.row_ind, g.permute, h, pseudo, pseudo_csc=pseudo_csc, own_order=own_order, proj=proj)
             elif pseudo_csc is not None and torch.is_grad_enabled():
                 with torch.no_grad():

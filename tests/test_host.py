@@ -440,3 +440,47 @@ def test_row_lengths_are_read_from_the_gpu_only(monkeypatch, ptr):
     raw = SimpleNamespace(dtype=torch.float32, is_cuda=True, requires_grad=False)
     with pytest.raises(_lib.FgnnError):
         GMMConv(64, 16, 1, 2)._projects(torch.zeros(2, 64), raw, raw, SimpleNamespace(weight=raw, bias=raw), ptr, torch.zeros(3, dtype=torch.int32))
+
+
+def test_monet_projects_for_layers_that_do_not():
+    """A layer of the caller's own, one that overrides the package's, a hooked one, and hooks on every module: the coordinates come projected, through
+    the module."""
+    from types import SimpleNamespace
+    from ae_mlsys_gnn_amd.layers import GMMConv, GMMConv_stash
+    from ae_mlsys_gnn_amd.train.train_gmmconv import MoNet, PseudoProj
+    ps = SimpleNamespace(is_cuda=True, requires_grad=False)
+    proj, seen = PseudoProj(2, 1), []
+
+    class Own(torch.nn.Module):
+        def __init__(self, *sizes):
+            super().__init__()
+
+        def forward(self, rowptr, colind, colptr, rowind, permute, feat, pseudo, pseudo_csc=None, own_order=False):
+            seen.append((pseudo, pseudo_csc))
+            return feat
+
+    class Overridden(GMMConv):
+        def forward(self, *args, **kwargs):
+            return super().forward(*args, **kwargs)
+    for c in (GMMConv, GMMConv_stash):
+        assert proj.plain(c(8, 4, 1, 2), ps, ps)
+    assert not proj.plain(Own(), ps, ps) and not proj.plain(Overridden(8, 4, 1, 2), ps, ps)
+    hooked, patched = GMMConv(8, 4, 1, 2), GMMConv(8, 4, 1, 2)
+    hooked.register_forward_pre_hook(lambda m, args: None)
+    patched.forward = lambda *args, **kwargs: None
+    assert not proj.plain(hooked, ps, ps) and not proj.plain(patched, ps, ps)
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, args, out: None)
+    try:
+        assert not proj.plain(GMMConv(8, 4, 1, 2), ps, ps)
+    finally:
+        handle.remove()
+    model = MoNet(Own, 8, 4, 3, 0, 1, 2, 0.0)
+    real = PseudoProj.forward
+    try:
+        PseudoProj.forward = lambda self, t: torch.ones(t.shape[0], 1)
+        g = SimpleNamespace(row_ptr=None, col_ind=None, col_ptr=None, row_ind=None, permute=None)
+        as_device = SimpleNamespace(is_cuda=True, requires_grad=False, shape=(6, 2))        # coordinates on the GPU, as far as the model can tell
+        model(g, torch.rand(3, 8), as_device, pseudo_csc=as_device)
+    finally:
+        PseudoProj.forward = real
+    assert len(seen) == 2 and all(torch.equal(t, torch.ones(6, 1)) for pair in seen for t in pair)
