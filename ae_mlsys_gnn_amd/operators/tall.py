@@ -19,9 +19,9 @@ def _traced():
 
 
 def _matrices(*ts):
-    """fp32 matrices on one GPU with unit column stride."""
-    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1
-               and t.stride(0) >= t.shape[1] for t in ts) and all(t.device == ts[0].device for t in ts)
+    """fp32 matrices on one GPU with unit column stride (whatever torch calls the stride of a single column)."""
+    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2
+               and (t.stride(1) == 1 or t.shape[1] == 1) and t.stride(0) >= t.shape[1] for t in ts) and all(t.device == ts[0].device for t in ts)
 
 
 def _plain(*ts):

@@ -1725,6 +1725,24 @@ def test_tall_product(n, k, m, h_in, h_out):
         assert bool(torch.isinf(got[0]).all()) and bool(((got[1:].cpu().double() - ref[1:]).abs() <= tol[1:]).all())
 
 
+# waves with several row tiles and a last one that is ragged: loads of 128, 64 and 32 bits, extra columns on either side, one and several column ranges
+@pytest.mark.parametrize("n,k,m,h_in,h_out", [(140003, 100, 64, 0, 8), (140003, 64, 100, 8, 0), (140003, 41, 48, 0, 0), (140003, 50, 32, 0, 2), (140003, 20, 300, 0, 0),
+                                              (140003, 20, 300, 0, 4), (140003, 300, 40, 4, 0), (70001, 180, 384, 0, 6), (270001, 128, 256, 0, 8), (140003, 1, 16, 0, 0)])
+def test_tall_product_of_several_tiles_a_wave(n, k, m, h_in, h_out):
+    from ae_mlsys_gnn_amd.operators.tall import tall_product
+    gen = torch.Generator(device=DEV).manual_seed(n + k)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    x, b, bias, extra = rnd(n, k), rnd(k + 2 * h_in, m + 2 * h_out), rnd(m), [rnd(n, h_in), rnd(n, h_in)] if h_in else None
+    full = torch.cat([x] + (extra or []), 1)
+    ref, tol = full.double() @ b.double(), _bound(full, b, full.shape[1])
+    out = tall_product(x, b, extra_in=extra, extra_out=h_out)
+    got = torch.cat(list(out), 1) if h_out else out
+    assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= tol).all())
+    if not h_out:
+        got = tall_product(x, b.t().contiguous(), transposed=True, extra_in=extra, bias=bias)
+        assert bool(((got.double() - ref - bias.double()).abs() <= tol + 2.0 ** -23 * (ref + bias.double()).abs()).all())
+
+
 @pytest.mark.parametrize("width", [50, 128])
 def test_layers_refuse_inputs_of_another_width(width):
     """As torch's products do: the kernels in their place read by the sizes of the weights."""
@@ -1770,14 +1788,17 @@ def test_products_over_many_rows_leave_traced_calls_to_torch():
 
 # results of one tile to the most tiles a wave takes, rows around a staged block and around a workgroup's share
 @pytest.mark.parametrize("n,a,b,h", [(1, 1, 1, 0), (31, 16, 16, 0), (33, 17, 15, 1), (255, 64, 64, 4), (257, 100, 256, 8), (1025, 256, 48, 1), (4100, 41, 23, 0),
-                                     (600, 602, 32, 0), (513, 144, 240, 2), (70000, 20, 4, 0), (300, 48, 200, 0), (90, 4, 512, 2), (2000, 144, 160, 3)])
+                                     (600, 602, 32, 0), (513, 144, 240, 2), (70000, 20, 4, 0), (300, 48, 200, 0), (90, 4, 512, 2), (2000, 144, 160, 3),
+                                     (70001, 100, 64, 8), (60017, 41, 24, 3), (131075, 50, 30, 0)])
 def test_tall_reduce(n, a, b, h):
     from ae_mlsys_gnn_amd.operators.tall import tall_reduce
     gen = torch.Generator().manual_seed(n * 17 + a)
     rnd = lambda *s: torch.randn(*s, generator=gen)
     x, g, extra = rnd(n, a), rnd(n, b), [rnd(n, h), rnd(n, h)] if h else None
     full = torch.cat([g] + (extra or []), 1)
-    ref, tol = x.double().t() @ full.double(), _bound(x.t(), full, n)
+    # a workgroup's chain: its share of the rows, rounded up to a staged block; the shares are added in 64 bits.  A lost row is past the bound.
+    share = -(-n // min(256, -(-n // 256)))
+    ref, tol = x.double().t() @ full.double(), _bound(x.t(), full, -(-share // 32) * 32)
     dx, dg, de = x.cuda(), g.cuda(), [t.cuda() for t in extra] if h else None
     wide = torch.full((n, b + 3), float("nan"), device="cuda")
     wide[:, :b] = dg
