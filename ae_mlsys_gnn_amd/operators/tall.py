@@ -37,17 +37,22 @@ def _fits(x, k, m, bias=None):
 def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None):
     """Whether tall_product takes x [n, k] and the [k + 2 h_in, m + 2 h_out] matrix b (its transpose when `transposed`) and is the faster
     form; what does not fit goes to the library, which says so.  m: the columns, where b [k, .] is only what the matrix is laid out from.
-    (us, library / own.)  It reads x and
-    writes the result once at 100-110 TFLOP/s, and every workgroup lays b out in LDS first, 5 to 30 us.  The library reaches 60-85 TFLOP/s on
-    thin shapes and more at the sizes it is tuned for, takes 19 of the host at least, and needs a score kernel (10 to 600) or a stacked
-    operand besides for extra columns.
-    No extra columns.  Up to 49 k rows both are within the library's host time: 4 k x 64 -> 64 19 / 8 (5 / 7 of the GPU), 33 k x 64 -> 128 19 / 14
-    (11 / 13), 33 k x 256 -> 128 22 / 31.  Up to 131 k rows: 65 k x 16 -> 64 11 / 8, 64 -> 64 12 / 13, 64 -> 128 18 / 22, 128 -> 128 25 / 31.  Above:
-    169 k x 64 -> 64 48 / 27, 64 -> 128 62 / 44, 128 -> 128 70 / 70, 384 -> 64 171 / 98, 64 -> 256 72 / 77, 128 -> 256 116 / 128; 500 k x 128 -> 128
-    213 / 178; 1 M x 64 -> 256 423 / 360 (at powers of two the library is the better one up to 524 k: 262 k x 128 -> 128 88 / 93).
-    With them, scores included: 16 k x 64 -> 64 + 8 9 / 8, 256 -> 48 + 2 15 / 17, 128 -> 256 + 8 20 / 35; 65 k 18 / 15, 34 / 30, 56 / 57; 169 k 60 / 33,
-    85 / 68, 142 / 138; 1 M 231 / 137, 521 / 323, 761 / 601.  Gradients, stacking included: 16 k x 64 + 8 -> 64 11 / 8, 48 + 2 -> 256 16 / 18, 256 + 8 ->
-    128 26 / 34; 65 k 26 / 17, 41 / 31, 72 / 65; 1 M 401 / 142, 628 / 348, 1216 / 598."""
+    It reads x and writes the result once at 100-110 TFLOP/s, and every workgroup lays b out in LDS first, 5 to 30 us.  The library reaches 60-85
+    TFLOP/s on thin shapes and more at the sizes it is tuned for, takes 19 us of the host at least (this kernel 11), and needs a score kernel (10 to
+    600) or a stacked operand besides for extra columns.  The lines are drawn by the time of a call in a stream of calls, host included; us,
+    library / own, in brackets of the GPU alone, as in a replayed graph, where that is another order.
+    No extra columns.  Up to 49 k rows 4 k x 64 -> 64 21 / 12 (4.4 / 6.6), 16 k x 64 -> 128 20 / 12 (7.3 / 11.5), 33 k x 64 -> 128 21 / 15 (10.8 / 14.4),
+    33 k x 256 -> 128 22 / 31.  Up to 131 k rows: 65 k x 16 -> 64 20 / 11, 64 -> 64 20 / 14 (11.4 / 13.8), 64 -> 128 20 / 23; 131,071 x 64 -> 64 22 / 22,
+    64 -> 128 32 / 35.  Above: 140 k x 64 -> 128 47 / 37, 384 -> 64 85 / 78, 256 -> 128 94 / 100; 169 k x 64 -> 64 48 / 26, 64 -> 128 63 / 43, 128 -> 128
+    87 / 68, 384 -> 64 171 / 97, 64 -> 256 72 / 77, 256 -> 128 108 / 121, 602 -> 48 122 / 138; 300 k x 128 -> 128 129 / 110, 602 -> 48 206 / 221; 700 k x
+    64 -> 128 217 / 141, 602 -> 48 455 / 470; 1 M x 64 -> 256 423 / 360.  A power of two of the library's row tiles is what it is tuned for: 131 k x
+    64 -> 64 22 / 22, 128 -> 64 29 / 32, 256 -> 64 44 / 53; 262 k x 64 -> 64 38 / 34, 64 -> 128 57 / 58, 128 -> 128 87 / 96; 524 k x 64 -> 128 114 / 113,
+    128 -> 128 172 / 179 (a row less 172 / 181); 1 M x 128 -> 64 206 / 192, 256 -> 64 331 / 344.
+    With them, scores included: 4 k x 64 -> 64 + 8 30 / 14, 256 -> 64 + 8 29 / 18 (8.6 / 17.3), 128 -> 256 + 8 29 / 28 (9.7 / 27.6); 16 k x 64 -> 64 + 8
+    29 / 14, 256 -> 48 + 2 29 / 17 (14.5 / 16.9), 128 -> 256 + 8 29 / 33; 65 k 30 / 15, 35 / 29, 54 / 54; 169 k 60 / 33, 85 / 68, 142 / 138; 1 M 231 /
+    137, 521 / 323, 761 / 601.  Gradients, stacking and the weights' included: 4 k x 64 + 8 -> 64 56 / 29; 49 k 48 + 2 -> 256 67 / 58, 256 + 8 -> 128 101 /
+    109; 65,536 x 48 + 2 -> 256 66 / 65, 128 + 16 -> 128 76 / 79, 256 + 8 -> 128 129 / 123; a row more 85 / 79 (8 scores), 110 / 89, 158 / 136; 1 M x 64 + 8
+    -> 64 401 / 142, 48 + 2 -> 256 628 / 348, 256 + 8 -> 128 1216 / 598 (these without the weights' gradient)."""
     if _traced() or b.dim() != 2:
         return False
     k = b.shape[1 if transposed else 0] - 2 * h_in
@@ -61,22 +66,28 @@ def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None
     elif n < 131072:
         most = 8192 if n <= 49152 else 4096
     else:
-        most = 8192 if m > 192 and n < (1 << 19) else 32768
+        tiles = -(-n // 256)
+        most = (4096 if n <= 1 << 18 else 8192) if tiles & (tiles - 1) == 0 else 8192 if m > 192 and n < (1 << 19) else 24576
     return (n > 0 and k > 0 and m > 0 and max(h_in, h_out) <= 8 and (k + 2 * h_in) * (m + 2 * h_out) <= most
             and k <= 1024 and m <= 512 and _plain(x, b) and (not h_in or (k % 4 == 0 and x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0)))
 
 
 def reduce_wanted(x, g, h=0):
     """Where tall_reduce of x [n, a] and g [n, b] (and 2h extra columns) is the faster form: one launch and a small sum for a batched product
-    over chunks, a sum, a remainder, and a stacked operand where there are extra columns (us of the GPU, library / own).  33 k x 64, 128 32 / 23;
-    extra columns: 4 k x 64, 64 + 8 25 / 17, 256, 48 + 2 21 / 30, 128, 256 + 8 24 / 52; 65 k 32 / 21, 34 / 36, 86 / 63; 169 k 69 / 40, 100 / 73, 229 /
-    135; 1 M 341 / 184, 444 / 375, 1153 / 684.  On few rows the sum over the workgroups' results is what takes the time, so those are small
-    ones there.  Without extra columns 233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116."""
+    over chunks, a sum, the rows past the last chunk of 2048, and a stacked operand where there are extra columns (us, library / own, host included;
+    in brackets of the GPU alone where that is another order).  On few rows the sum over the workgroups' results is what takes the time, so those are
+    small ones there: 4 k x 64, 64 28 / 15, 64, 128 28 / 20, 128, 128 28 / 29; 33 k x 64, 128 28 / 21 (14 / 21), 128, 128 27 / 31.  Beyond: 52,001 x 128, 128
+    57 / 33, 131,071 x 192, 128 85 / 72.  Whole chunks leave the library no remainder: 57 k x 128, 128 34 / 32, 65,536 x 64, 64 28 / 18 (15.4 / 17.5), 64, 128
+    28 / 23, 128, 128 28 / 33, 122,880 x 64, 128 35 / 35, 128, 128 44 / 51, 131,072 x 64, 64 27 / 27, 64, 128 28 / 36.  Above 131 k rows either is as fast
+    (233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116).  With extra columns: 4 k x 64, 64 + 8 61 / 18, 65 k x 256, 48 + 2 62 / 35, 128, 256 + 8
+    62 / 62; 169 k x 64, 64 + 8 69 / 40, 256, 48 + 2 100 / 73, 128, 256 + 8 229 / 135; 1 M 341 / 184, 444 / 375, 1153 / 684."""
     if _traced() or x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
         return False
     n, a, b = x.shape[0], x.shape[1], g.shape[1]
     tiles = -(-a // 16) * (-(-b // 16) + (h > 0))
-    return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= (144 if n > 49152 else 36) and (h > 0 or n <= 131072) and _plain(x, g)
+    whole = h == 0 and n >= 65536 and n % (n // 2048) == 0
+    return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= (36 if n <= 49152 or whole else 144)
+            and (h > 0 or n < 131072) and _plain(x, g)
             and all(t.shape[1] % 4 == 0 and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (x, g)))
 
 

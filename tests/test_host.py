@@ -484,3 +484,18 @@ def test_monet_projects_for_layers_that_do_not():
     finally:
         PseudoProj.forward = real
     assert len(seen) == 2 and all(torch.equal(t, torch.ones(6, 1)) for pair in seen for t in pair)
+
+
+@pytest.mark.parametrize("n,k,m,product,reduction", [
+    (16384, 64, 128, True, True), (49152, 256, 48, False, False), (57344, 64, 64, True, True), (65536, 64, 128, False, True), (65536, 128, 128, False, False),
+    (65568, 128, 128, False, False), (65537, 128, 128, False, True), (122880, 256, 64, False, False), (131072, 64, 64, True, False), (131072, 128, 64, False, False),
+    (131073, 128, 64, True, False), (169343, 384, 64, True, False), (169343, 256, 128, False, False), (169343, 64, 256, False, False), (262144, 128, 128, False, False),
+    (524287, 128, 128, False, False), (524288, 64, 128, True, False), (700000, 64, 256, True, False), (700000, 602, 48, False, False)])
+def test_products_over_many_rows_rules(monkeypatch, n, k, m, product, reduction):
+    """The measured shapes, each at the form that a stream of calls runs faster with."""
+    from ae_mlsys_gnn_amd.operators import tall
+    monkeypatch.setattr(tall, "_plain", lambda *ts: True)
+    x, g, w = (torch.empty(s, device="meta") for s in ((n, k), (n, m), (m, k)))
+    assert tall.product_wanted(x, w, transposed=True) is product
+    if m % 4 == k % 4 == 0:
+        assert tall.reduce_wanted(x, g) is reduction
