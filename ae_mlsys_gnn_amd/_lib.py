@@ -292,10 +292,11 @@ def default_seg_len() -> int:
 
 
 def flat_seg_len(n_edges) -> int:
-    """Entries at which the plain list of a skewed graph cuts a hub's row: one eight-thousandth of all (about a resident wave's share), between
-    256 and the usual 2048, so that no hub outlasts the rest (forward pass of 2 x 16 floats, 50 k nodes, 1 M entries: 71 us with 2048, 41
-    so; 169 k nodes, 2.3 M 88 / 62)."""
-    return max(256, min(2048, n_edges // 8192 // 64 * 64))
+    """Entries at which the plain list of a skewed graph (4 M entries and more) cuts a hub's row: one eight-thousandth of all (about a resident
+    wave's share), between 1024 and the usual 2048, so that no hub outlasts the rest (us with 512 / 1024 / 2048, 2 x 16 floats, forward and summed
+    backward: 50 k nodes, 4.4 M entries 61 + 134 / 56 + 124 / 68 + 116; 169 k, 4.7 M 61 + 132 / 53 + 132 / 71 + 132; with 960 / 1024 / 2048, 100 k,
+    8.1 M 78 + 180 / 78 + 183 / 79 + 180; with 256 / 1024 / 1920, 233 k, 16 M 192 + 451 / 145 + 396 / 135 + 383)."""
+    return max(1024, min(2048, n_edges // 8192 // 64 * 64))
 
 
 _bucket_rule_cache: "collections.OrderedDict" = collections.OrderedDict()

@@ -499,3 +499,8 @@ def test_products_over_many_rows_rules(monkeypatch, n, k, m, product, reduction)
     assert tall.product_wanted(x, w, transposed=True) is product
     if m % 4 == k % 4 == 0:
         assert tall.reduce_wanted(x, g) is reduction
+
+
+@pytest.mark.parametrize("entries,want", [(1, 1024), (1 << 22, 1024), (12 << 20, 1536), (115000000, 2048)])
+def test_plain_lists_cut_hubs_by_the_size_of_the_graph(entries, want):
+    assert _lib.flat_seg_len(entries) == want
