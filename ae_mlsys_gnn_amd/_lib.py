@@ -367,8 +367,8 @@ def schedule_for(ptr_tensor, seg_len=None, idx_tensor=None, need_positions=True,
 
     def key(pos):
         return (ptr_tensor.data_ptr(), ptr_tensor.numel(), ptr_tensor.device.index, ptr_tensor._version, int(seg_len),
-                None if idx_tensor is None else (idx_tensor.data_ptr(), idx_tensor._version, min_deg, pos)) + (
-                    () if walked is None else ("flat", walked.data_ptr(), walked._version))
+                (idx_tensor.data_ptr(), idx_tensor._version, min_deg, pos) if idx_tensor is not None else
+                None if walked is None else ("flat", walked.data_ptr(), walked._version))
     if own_order:
         k = key("own")
         s = _sched_cache.get(k)

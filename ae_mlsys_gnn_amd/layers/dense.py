@@ -14,7 +14,7 @@ from ..operators.tall import product_wanted, reduce_wanted, sum_wanted, tall_pro
 def reduce_over_rows(x, g):
     """x^T @ g for tall x [N, a], g [N, b]."""
     if not torch.is_grad_enabled() and reduce_wanted(x, g):        # (a graph of the result is recorded by the operations below)
-        return tall_reduce(x, g)
+        return tall_reduce(x, g, asked=True)
     n = x.shape[0]
     chunks = min(256, n // 2048)
     if chunks < 2:
@@ -66,7 +66,7 @@ class _TallLinear(torch.autograd.Function):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
         if product_wanted(x, weight, transposed=True, bias=bias):
-            return tall_product(x, weight, transposed=True, bias=bias)
+            return tall_product(x, weight, transposed=True, bias=bias, asked=True)
         y = torch.matmul(x, weight.t())
         return y if bias is None else y.add_(bias)
 
@@ -78,7 +78,7 @@ class _TallLinear(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             # where a graph of the gradients is wanted, the operation that records one
             own = not torch.is_grad_enabled() and product_wanted(g, weight)
-            gx = tall_product(g, weight) if own else torch.matmul(g, weight)
+            gx = tall_product(g, weight, asked=True) if own else torch.matmul(g, weight)
         if ctx.needs_input_grad[1]:
             gw = reduce_over_rows(g, x)
         gb = column_sum(g) if (ctx.has_bias and ctx.needs_input_grad[2]) else None

@@ -46,12 +46,12 @@ class _GATBase(nn.Module):
 
 
 class _ProjectScores(torch.autograd.Function):
-    """The dense part of the layer.  The scores are formed as feat @ ((W * attn).sum(-1)): the same
-    sums taken in another order, as one thin product over `feat` instead of two strided reductions over
-    the [N,H,F] projection.  The backward stacks the gradients of the projection and of the scores
-    into one [N, H*F + 2H] operand when the input gradient is wanted, so that it is one GEMM and `feat` is
-    reduced over the nodes once; a first layer reduces the two parts separately instead of copying the wide one.
-    What surrounds the products runs as three kernels: weights folded, scores, gradients unfolded."""
+    """The dense part of the layer.  The scores are formed as feat @ ((W * attn).sum(-1)): the same sums taken in another order, the last
+    columns of the projection's own product where that takes the sizes (operators/tall.py), else one thin product over `feat` instead of two
+    strided reductions over the [N,H,F] projection.  The backward reads the gradients of the projection and of the scores from where they are, in one
+    product for the input's gradient and one reduction over the nodes; where the library has the products, it stacks them into one
+    [N, H*F + 2H] operand when the input gradient is wanted, and a first layer reduces the two parts separately instead of copying the wide one.
+    What surrounds the products runs as kernels of its own: weights folded, gradients unfolded (and the scores beside a library product)."""
 
     @staticmethod
     def forward(ctx, feat, W, attn_l, attn_r, pad):
@@ -59,7 +59,7 @@ class _ProjectScores(torch.autograd.Function):
         own = product_wanted(feat, W, h_out=hh, m=hh * (ff + pad))
         score_wt, w_proj, w_all = gat_dense_native.fold(W, attn_l, attn_r, pad, own or ctx.needs_input_grad[0])
         if own:                                 # the scores are columns of the same product
-            h, row, col = tall_product(feat, w_all, extra_out=hh)
+            h, row, col = tall_product(feat, w_all, extra_out=hh, asked=True)
         else:
             h = torch.matmul(feat, w_proj)
             if gat_dense_native.scores_supported(feat.shape[1], hh):
@@ -90,8 +90,8 @@ class _ProjectScores(torch.autograd.Function):
         if own:                                 # nothing is stacked
             extra = (drow.contiguous(), dcol.contiguous())
             if ctx.needs_input_grad[0]:
-                dfeat = tall_product(dh2, w_all, transposed=True, extra_in=extra)
-            dw_ext = tall_reduce(feat, dh2, extra)                                      # [in, H*Fp + 2H]
+                dfeat = tall_product(dh2, w_all, transposed=True, extra_in=extra, asked=True)
+            dw_ext = tall_reduce(feat, dh2, extra, asked=True)                            # [in, H*Fp + 2H]
             dproj, dscore = dw_ext[:, :hfp], dw_ext[:, hfp:]
         elif ctx.needs_input_grad[0] or dh is None:
             g = torch.cat([zeros(hfp) if dh is None else dh.reshape(n, hfp), zeros(hh) if drow is None else drow,

@@ -532,7 +532,7 @@ class GmmAggregateLinearFunction(torch.autograd.Function):
                               rowptr, colind, agg if ctx.two_orders else None)
         agg = agg.view(-1, k * fin)
         if product_wanted(agg, w, transposed=True, bias=bias):
-            return tall_product(agg, w, transposed=True, bias=bias)
+            return tall_product(agg, w, transposed=True, bias=bias, asked=True)
         y = torch.matmul(agg, w.t())
         return y if bias is None else y + bias
 

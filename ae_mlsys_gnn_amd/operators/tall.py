@@ -9,29 +9,44 @@ from .._lib import FgnnError, as_f32, check, device_guard, lib, ptr, stream_ptr,
 # Where a torch does not have the private names, its public mode stack is asked.
 _modes = getattr(torch._C, "_len_torch_dispatch_stack", None) or (lambda: torch.utils._python_dispatch._get_current_dispatch_mode() is not None)
 _transforms = getattr(torch._C, "_are_functorch_transforms_active", None) or (lambda: False)
+_recording = getattr(torch._C, "_is_tracing", None) or torch.jit.is_tracing
 
 
 def _traced():
     """Whether torch's own operations are being watched or rewritten (torch.compile, jit.trace, make_fx, fake tensors, functorch): a kernel launched past them
     would be missing from the record, or be handed no memory.  Asked before any size, so that no size becomes a condition of the record, and the
     compiler first: it does not follow the questions behind it."""
-    return torch.compiler.is_compiling() or torch.jit.is_tracing() or bool(_modes()) or _transforms()
+    return torch.compiler.is_compiling() or _recording() or bool(_modes()) or _transforms()
 
 
-def _matrices(*ts):
+# These questions stand in front of every product, and small layers are bound by the host: each attribute is asked for once (a product with scores,
+# both rules of a backward and a reduction, host time without the launches: 53 us with generators over the operands, 36 so, nothing asked twice).
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _matrix(t):
+    if not t.is_cuda or t.dtype is not torch.float32 or type(t) not in _TENSORS:
+        return False
+    strides = t.stride()
+    if len(strides) != 2:
+        return False
+    columns = t.shape[1]
+    return (strides[1] == 1 or columns == 1) and strides[0] >= columns
+
+
+def _matrices(x, b=None):
     """fp32 matrices on one GPU with unit column stride (whatever torch calls the stride of a single column)."""
-    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.dim() == 2
-               and (t.stride(1) == 1 or t.shape[1] == 1) and t.stride(0) >= t.shape[1] for t in ts) and all(t.device == ts[0].device for t in ts)
+    return _matrix(x) and (b is None or (_matrix(b) and x.device == b.device))
 
 
-def _plain(*ts):
+def _plain(x, b=None):
     """Such matrices outside autocast (which asks for another precision)."""
-    return not torch.is_autocast_enabled("cuda") and _matrices(*ts)
+    return not torch.is_autocast_enabled("cuda") and _matrices(x, b)
 
 
-def _fits(x, k, m, bias=None):
-    """Whether x has k columns and bias, where there is one, m floats beside x: the kernels read by these sizes alone."""
-    return x.dim() == 2 and x.shape[1] == k and (bias is None or (bias.shape == (m,) and bias.dtype == torch.float32 and bias.device == x.device))
+def _fits(shape, k, m, device, bias):
+    """Whether x of `shape` on `device` has k columns and bias, where there is one, m floats beside it: the kernels read by these sizes alone."""
+    return len(shape) == 2 and shape[1] == k and (bias is None or (bias.shape == (m,) and bias.dtype == torch.float32 and bias.device == device))
 
 
 def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None):
@@ -53,14 +68,17 @@ def product_wanted(x, b, *, transposed=False, bias=None, h_in=0, h_out=0, m=None
     137, 521 / 323, 761 / 601.  Gradients, stacking and the weights' included: 4 k x 64 + 8 -> 64 56 / 29; 49 k 48 + 2 -> 256 67 / 58, 256 + 8 -> 128 101 /
     109; 65,536 x 48 + 2 -> 256 66 / 65, 128 + 16 -> 128 76 / 79, 256 + 8 -> 128 129 / 123; a row more 85 / 79 (8 scores), 110 / 89, 158 / 136; 1 M x 64 + 8
     -> 64 401 / 142, 48 + 2 -> 256 628 / 348, 256 + 8 -> 128 1216 / 598 (these without the weights' gradient)."""
-    if _traced() or b.dim() != 2:
+    if _traced():
         return False
-    k = b.shape[1 if transposed else 0] - 2 * h_in
+    shape, rows = x.shape, b.shape
+    if len(rows) != 2:
+        return False
+    k = rows[1 if transposed else 0] - 2 * h_in
     if m is None:
-        m = b.shape[0 if transposed else 1] - 2 * h_out
-    if not _fits(x, k, m, bias):
+        m = rows[0 if transposed else 1] - 2 * h_out
+    if not _fits(shape, k, m, x.device, bias):
         return False
-    n = x.shape[0]
+    n = shape[0]
     if h_out or h_in:
         most = 73728 if n >= 65536 else 20480 if h_out else 16384
     elif n < 131072:
@@ -81,29 +99,37 @@ def reduce_wanted(x, g, h=0):
     28 / 23, 128, 128 28 / 33, 122,880 x 64, 128 35 / 35, 128, 128 44 / 51, 131,072 x 64, 64 27 / 27, 64, 128 28 / 36.  Above 131 k rows either is as fast
     (233 k x 602, 32 228 / 242, 169 k x 384, 64 112 / 116).  With extra columns: 4 k x 64, 64 + 8 61 / 18, 65 k x 256, 48 + 2 62 / 35, 128, 256 + 8
     62 / 62; 169 k x 64, 64 + 8 69 / 40, 256, 48 + 2 100 / 73, 128, 256 + 8 229 / 135; 1 M 341 / 184, 444 / 375, 1153 / 684."""
-    if _traced() or x.dim() != 2 or g.dim() != 2 or x.shape[0] != g.shape[0]:
+    if _traced():
         return False
-    n, a, b = x.shape[0], x.shape[1], g.shape[1]
+    xs, gs = x.shape, g.shape
+    if len(xs) != 2 or len(gs) != 2 or xs[0] != gs[0]:
+        return False
+    n, a, b = xs[0], xs[1], gs[1]
     tiles = -(-a // 16) * (-(-b // 16) + (h > 0))
     whole = h == 0 and n >= 65536 and n % (n // 2048) == 0
-    return (n > 0 and 0 < a + b <= 1024 and a > 0 and b > 0 and h <= 8 and tiles <= (36 if n <= 49152 or whole else 144)
-            and (h > 0 or n < 131072) and _plain(x, g)
-            and all(t.shape[1] % 4 == 0 and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (x, g)))
+    return (n > 0 and a > 0 and b > 0 and a + b <= 1024 and a % 4 == 0 and b % 4 == 0 and h <= 8 and tiles <= (36 if n <= 49152 or whole else 144)
+            and (h > 0 or n < 131072) and _plain(x, g) and x.stride(0) % 4 == 0 and g.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and g.data_ptr() % 16 == 0)
 
 
 def _columns(x, extra):
     """Whether extra is None or two contiguous [n, h] arrays beside x [n, .]."""
-    return extra is None or all(t.is_contiguous() and t.dtype == torch.float32 and t.device == x.device and t.shape == (x.shape[0], extra[0].shape[1])
-                                for t in extra)
+    if extra is None:
+        return True
+    one, two = extra
+    return (one.is_contiguous() and two.is_contiguous() and one.dtype is two.dtype is torch.float32 and one.device == x.device == two.device
+            and one.shape == two.shape and len(one.shape) == 2 and one.shape[0] == x.shape[0])
 
 
-def tall_product(x, b, *, transposed=False, bias=None, extra_in=None, extra_out=0):
+def tall_product(x, b, *, transposed=False, bias=None, extra_in=None, extra_out=0, asked=False):
     """x [n, k] @ b (b^T when `transposed`) (+ bias).  extra_in: two [n, h] arrays that follow x's columns; extra_out: h, the last 2h
-    columns of the result are returned as two [n, h] arrays of their own."""
-    n, k = x.shape
+    columns of the result are returned as two [n, h] arrays of their own.  asked: product_wanted has just said so of these operands, which are not
+    looked over again (b may be what the weights it saw were laid out in)."""
+    n, k = shape = x.shape
+    rows = b.shape
     hin = 0 if extra_in is None else extra_in[0].shape[1]
-    m = b.shape[0 if transposed else 1] - 2 * extra_out
-    if not _matrices(x, b) or m < 1 or b.shape[1 if transposed else 0] != k + 2 * hin or not _fits(x, k, m, bias) or not _columns(x, extra_in):
+    m = rows[0 if transposed else 1] - 2 * extra_out
+    if not ((asked or (_matrices(x, b) and _fits(shape, k, m, x.device, bias))) and m >= 1 and rows[1 if transposed else 0] == k + 2 * hin
+            and _columns(x, extra_in)):
         raise FgnnError("tall_product: x %s, matrix %s%s, bias %s and %d + %d extra columns do not fit one another" % (
             tuple(x.shape), tuple(b.shape), " (transposed)" if transposed else "", None if bias is None else tuple(bias.shape), hin, extra_out))
     bias = None if bias is None else as_f32(bias)
@@ -117,12 +143,12 @@ def tall_product(x, b, *, transposed=False, bias=None, extra_in=None, extra_out=
     return (y, e0, e1) if extra_out else y
 
 
-def tall_reduce(x, g, extra=None):
-    """x [n, a]^T @ g [n, b] -> [a, b]; extra: two [n, h] arrays that follow g's columns."""
+def tall_reduce(x, g, extra=None, asked=False):
+    """x [n, a]^T @ g [n, b] -> [a, b]; extra: two [n, h] arrays that follow g's columns; asked: of reduce_wanted, as above."""
     n, a = x.shape
     b = g.shape[1]
     h = 0 if extra is None else extra[0].shape[1]
-    if not _matrices(x, g) or g.shape[0] != n or not _columns(x, extra):
+    if not ((asked or (_matrices(x, g) and g.shape[0] == n)) and _columns(x, extra)):
         raise FgnnError("tall_reduce: x %s, g %s and 2 x %d extra columns do not fit one another" % (tuple(x.shape), tuple(g.shape), h))
     c = torch.empty((a, b + 2 * h), dtype=torch.float32, device=x.device)
     e0, e1 = extra if h else (None, None)

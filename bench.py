@@ -3,8 +3,8 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload gat_c2|gat_c5|gat_c5_l2|gat_c5_train|edgeconv_c3|gmm_c4|small_ops_c2|gather_ceiling]
 
-Default workload = benchmark configuration 2: one fused GAT layer forward+backward (dense projection by
-torch.matmul, fused sparse op by libfgnn_hip.so) on a seeded R-MAT power-law graph with 232,965
+Default workload = benchmark configuration 2: one fused GAT layer forward+backward (dense projection, with the
+scores as its last columns, and fused sparse op by libfgnn_hip.so) on a seeded R-MAT power-law graph with 232,965
 nodes and ~114.6 M edges plus self loops, features [N,256], 8 heads x 32, fp32.  A step is one
 layer forward + backward; inputs are resident in HBM before the timed region; graph
 preprocessing (csr2csc, schedules) is reported separately.  One JSON line is printed with the
@@ -403,7 +403,7 @@ def run_gat(args, n, e_target, in_feats, heads, out_feats, workload):
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": workload, "graph": "R-MAT a=0.57 b=0.19 c=0.19 d=0.05 seed 0, unique edges + self loops" + (", node labels permuted" if PERMUTE_LABELS else ""),
                    "nodes": n, "edges": e, "in_feats": in_feats, "heads": heads, "out_feats": out_feats,
-                   "negative_slope": slope, "step": "GATConv forward + backward (torch.matmul projection + fused sparse op)"},
+                   "negative_slope": slope, "step": "GATConv forward + backward (fp32 projection with the scores as its last columns + fused sparse op)"},
         "roofline": roofline_record("gat_fwd_kernel (+gat_fwd_merge_kernel)", b_fwd, ms_fwd, (traffic or {}).get("fwd"), stale),
         "roofline_bwd": roofline_record("gat_bwd_node_kernel + gat_bwd_kernel (+gat_bwd_merge_kernel)", b_bwd, ms_bwd,
                                         (traffic or {}).get("bwd"), stale),
