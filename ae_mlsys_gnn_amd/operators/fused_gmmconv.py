@@ -34,6 +34,13 @@ def _sums_in_batches(f, *arrays):
     return f % 4 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in arrays)
 
 
+def _column_pass_in_batches(k, f):
+    """Whether the column pass over rows of K x F floats has 16 lanes or fewer a row, each kernel's quarter of F rounded up to a power of two of them, and so
+    four rows or more in a batch.  With two, the sums over the batches of an item of 2048 entries are a chain long enough to tell (5 kernels x 12
+    floats, 17 M edges, error of the input gradient, cut / plain list: 6.0e-8 / 7.1e-8; 4 x 16 5.6e-8 / 5.3e-8)."""
+    return f > 0 and k * max(4, 1 << (f - 1).bit_length()) <= 64
+
+
 SUM_KERNELS_MAX = 4     # most mixture kernels that the summed column pass keeps in registers; with more, a pass over K x F floats
 
 
@@ -126,7 +133,8 @@ class gmm_native:
         grad_mu = torch.empty_like(mu)
         grad_sigma = torch.empty_like(sigma)
         # own_order: pseudo, grad_pseudo (and permute) are indexed by the schedule's entry order (gmm_edge_positions(colptr, rowind, True))
-        flat = _flat_list(n, e, f if sum_kernels and k <= SUM_KERNELS_MAX else k * f, True) and _sums_in_batches(f, node_feat, grad_out)
+        summed = sum_kernels and k <= SUM_KERNELS_MAX
+        flat = _flat_list(n, e, f if summed else k * f, True) and (summed or _column_pass_in_batches(k, f)) and _sums_in_batches(f, node_feat, grad_out)
         sched = schedule_for(colptr, idx_tensor=None if (sum_kernels and _plain_list_for_summed_backward(n, e)) else rowind, own_order=own_order, n_cols=n,
                              flat=flat)
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, node_feat, pseudo, (pw, pb), mu, sigma, grad_out, int(sum_kernels), grad_feat, grad_pseudo,
@@ -209,7 +217,7 @@ class gmm_native:
         grad_sigma = torch.empty_like(sigma)
         # same work list as the summed backward, so that one CSC-side copy of own-order edge data serves both kinds of layer
         sched = schedule_for(colptr, idx_tensor=None if _plain_list_for_summed_backward(n, e) else rowind, own_order=own_order, n_cols=n,
-                             flat=_flat_list(n, e, k * f, True) and _sums_in_batches(f, feat, grad_out))
+                             flat=_flat_list(n, e, k * f, True) and _column_pass_in_batches(k, f) and _sums_in_batches(f, feat, grad_out))
         gmm_native._backward(n, e, k, dim, f, colptr, rowind, permute, feat, pseudo, (pw, pb), mu, sigma, grad_out, 2, parts, grad_pseudo, grad_mu, grad_sigma, sched,
                              dev)
         return parts.sum(1), grad_pseudo, grad_mu, grad_sigma

@@ -504,3 +504,10 @@ def test_products_over_many_rows_rules(monkeypatch, n, k, m, product, reduction)
 @pytest.mark.parametrize("entries,want", [(1, 1024), (1 << 22, 1024), (12 << 20, 1536), (115000000, 2048)])
 def test_plain_lists_cut_hubs_by_the_size_of_the_graph(entries, want):
     assert _lib.flat_seg_len(entries) == want
+
+
+@pytest.mark.parametrize("k,f,want", [(1, 4, True), (4, 16, True), (2, 28, True), (1, 64, True), (5, 12, False), (3, 20, False), (4, 12, True), (2, 36, False), (16, 4, True), (17, 4, False)])
+def test_column_pass_batches(k, f, want):
+    """Four rows or more in a batch: K times F, rounded up to a power of two, within the 64 floats of 16 lanes."""
+    from ae_mlsys_gnn_amd.operators.fused_gmmconv import _column_pass_in_batches
+    assert _column_pass_in_batches(k, f) is want

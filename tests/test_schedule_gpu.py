@@ -215,7 +215,7 @@ def test_flat_list_over_bucketed_order(monkeypatch):
 
 # kernels past the summed pass' limit, rows past a wave, rows and base addresses off the 128-bit loads (those kernels add an item's entries to one chain),
 # and two forms that do take the plain list
-@pytest.mark.parametrize("k,f,off,summed", [(8, 32, 0, True), (5, 12, 0, True), (2, 16, 1, True), (2, 6, 0, True), (2, 16, 0, True), (2, 16, 2, False), (4, 16, 0, False)])
+@pytest.mark.parametrize("k,f,off,summed", [(8, 32, 0, True), (5, 12, 0, True), (2, 16, 1, True), (2, 6, 0, True), (2, 16, 0, True), (2, 16, 2, False), (4, 16, 0, False), (3, 20, 0, False)])
 def test_plain_list_costs_no_precision(monkeypatch, k, f, off, summed):
     """On a skewed graph large enough for the rule, the errors against float64 are no larger than with the list cut by source bucket."""
     from ae_mlsys_gnn_amd.operators import fused_gmmconv
