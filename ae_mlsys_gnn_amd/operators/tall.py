@@ -19,8 +19,8 @@ def _traced():
     return torch.compiler.is_compiling() or _recording() or bool(_modes()) or _transforms()
 
 
-# These questions stand in front of every product, and small layers are bound by the host: each attribute is asked for once (a product with scores,
-# both rules of a backward and a reduction, host time without the launches: 53 us with generators over the operands, 36 so, nothing asked twice).
+# These questions stand in front of every product, and small layers are bound by the host: each attribute is asked for once, and nothing twice (host time
+# of the three rules and three wrappers of a layer with scores, launches left out: 65 us with generators over the operands and both asking, 39 so).
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -123,13 +123,14 @@ def _columns(x, extra):
 def tall_product(x, b, *, transposed=False, bias=None, extra_in=None, extra_out=0, asked=False):
     """x [n, k] @ b (b^T when `transposed`) (+ bias).  extra_in: two [n, h] arrays that follow x's columns; extra_out: h, the last 2h
     columns of the result are returned as two [n, h] arrays of their own.  asked: product_wanted has just said so of these operands, which are not
-    looked over again (b may be what the weights it saw were laid out in)."""
+    looked over again (b may be what the weights it saw were laid out in); extra_in are the gradients of two fp32 [n, h] outputs, made contiguous,
+    whose shape and device autograd has seen to."""
     n, k = shape = x.shape
     rows = b.shape
     hin = 0 if extra_in is None else extra_in[0].shape[1]
     m = rows[0 if transposed else 1] - 2 * extra_out
-    if not ((asked or (_matrices(x, b) and _fits(shape, k, m, x.device, bias))) and m >= 1 and rows[1 if transposed else 0] == k + 2 * hin
-            and _columns(x, extra_in)):
+    if not ((asked or (_matrices(x, b) and _fits(shape, k, m, x.device, bias) and _columns(x, extra_in))) and m >= 1
+            and rows[1 if transposed else 0] == k + 2 * hin):
         raise FgnnError("tall_product: x %s, matrix %s%s, bias %s and %d + %d extra columns do not fit one another" % (
             tuple(x.shape), tuple(b.shape), " (transposed)" if transposed else "", None if bias is None else tuple(bias.shape), hin, extra_out))
     bias = None if bias is None else as_f32(bias)
@@ -148,7 +149,7 @@ def tall_reduce(x, g, extra=None, asked=False):
     n, a = x.shape
     b = g.shape[1]
     h = 0 if extra is None else extra[0].shape[1]
-    if not ((asked or (_matrices(x, g) and g.shape[0] == n)) and _columns(x, extra)):
+    if not (asked or (_matrices(x, g) and g.shape[0] == n and _columns(x, extra))):
         raise FgnnError("tall_reduce: x %s, g %s and 2 x %d extra columns do not fit one another" % (tuple(x.shape), tuple(g.shape), h))
     c = torch.empty((a, b + 2 * h), dtype=torch.float32, device=x.device)
     e0, e1 = extra if h else (None, None)
